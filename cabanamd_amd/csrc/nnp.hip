@@ -8,11 +8,11 @@
 //                positions), radial functions with lanes over neighbours and
 //                angular functions with lanes over neighbour pairs; per-lane
 //                partial sums are combined with a reduce-scatter butterfly.
-//   k_nnp_mlp    per element, 16 atoms per wave: the two hidden layers and
-//                the backward pass as BF16 MFMA GEMMs (16x16x16, FP32
-//                accumulate) over the scaled symmetry functions; output
-//                layer, tanh and scaling on the VALU.  k_nnp_mlp_f32 is the
-//                same network in FP32 (one atom per lane).
+//   k_nnp_mlp    all elements in one launch, 16 atoms of one element per
+//                wave: the two hidden layers and the backward pass on the
+//                matrix cores over the scaled symmetry functions (split BF16
+//                products, or FP32 ones); output layer, tanh and scaling on
+//                the VALU.
 //   k_nnp_force  one wave per atom: dE/dG chained into dG/dr on the same
 //                pairs; reactions on neighbours gather in LDS and reach
 //                f by FP64 atomics (ghost rows included, folded by
@@ -73,12 +73,17 @@ struct NnpElemPlan
     float a_eta[AG_MAX], a_rs[AG_MAX];
     float a_lam[AP_MAX], a_zeta[AP_MAX], a_lpref[AP_MAX]; // lpref = 1 - zeta
     int a_out[AG_MAX][AP_MAX];     // model index of angular (g, p)
-    float g_mul[NSF_LD], g_add[NSF_LD]; // Gs = g_mul * G + g_add
+    alignas( 16 ) float g_mul[NSF_LD]; // Gs = g_mul * G + g_add
+    alignas( 16 ) float g_add[NSF_LD];
     int h1, h2;
     int act1, act2, act3; // 1 = tanh, 0 = linear
-    float W1[HPAD][KPAD]; // [out][in], zero padded
+    // layer weights, zero padded: [out][in] as the forward products' B
+    // operands read them, [in][out] for the backward ones
+    alignas( 16 ) float W1[HPAD][KPAD];
+    alignas( 16 ) float W1T[KPAD][HPAD];
     float b1[HPAD];
-    float W2[HPAD][HPAD];
+    alignas( 16 ) float W2[HPAD][HPAD];
+    alignas( 16 ) float W2T[HPAD][HPAD];
     float b2[HPAD];
     float w3[HPAD];
     float b3;
@@ -133,7 +138,7 @@ struct cmd_nnp
     bool plan_ok = false;
     int prec = CMD_PREC_MIXED; // MIXED: BF16 MFMA layers; FP64: FP32 layers
     cmd::DevBuf<float> G, dEdG, Ei;
-    cmd::DevBuf<int> elist, ecount, flag;
+    cmd::DevBuf<int> flag;
     cmd::DevBuf<double> part;
     cmd::DevBuf<int4> terms; // per atom: neighbours, triplets, element (last compute)
     int cap = 0;
@@ -341,6 +346,7 @@ static cmd_status build_plan( const cmd_nnp_model &m, NnpPlan &P )
             for ( int k = 0; k < KPAD; ++k )
             {
                 unsigned short part[3];
+                Q.W1T[k][o] = Q.W1[o][k];
                 bf16_split3( Q.W1[o][k], part );
                 for ( int q = 0; q < 3; ++q )
                 {
@@ -351,6 +357,7 @@ static cmd_status build_plan( const cmd_nnp_model &m, NnpPlan &P )
             for ( int k = 0; k < HPAD; ++k )
             {
                 unsigned short part[3];
+                Q.W2T[k][o] = Q.W2[o][k];
                 bf16_split3( Q.W2[o][k], part );
                 for ( int q = 0; q < 3; ++q )
                 {
@@ -875,50 +882,124 @@ __device__ __forceinline__ f32x4 mfma_split( const float *a8, const unsigned sho
     return c;
 }
 
+// The same K block in FP32 on the 16x16x4 FP32 MFMA.  Any order of k serves
+// the sum, so MFMA (j, u) takes k = 16 j + 4 (l / 16) + u in lane l and both
+// operands are read 16 bytes at a time.
+__device__ __forceinline__ f32x4 mfma_f32( const float *a, const float *w, f32x4 c )
+{
+#pragma unroll
+    for ( int j = 0; j < 2; ++j )
+    {
+        const f32x4 av = *reinterpret_cast<const f32x4 *>( a + 16 * j );
+        const f32x4 wv = *reinterpret_cast<const f32x4 *>( w + 16 * j );
+#pragma unroll
+        for ( int u = 0; u < 4; ++u )
+            c = __builtin_amdgcn_mfma_f32_16x16x4f32( av[u], wv[u], c, 0, 0, 0 );
+    }
+    return c;
+}
+
+// The network of every element in one launch: energies and dE/dG, forward
+// and backward, 16 atoms of one element per wave.  A block takes 64
+// consecutive atoms and groups them by element in LDS (sum_e ceil(c_e / 16)
+// <= 3 + nelem tiles, one per wave), so no grouping pass over the system and
+// no per-element launch is needed.  F32 runs the products on the FP32 MFMA
+// (FP32 operands and sums, as the per-atom dot products it replaces), else
+// on split BF16 parts.  A tile is a serial chain of five products and two
+// activations: latency bounds it, so the tiles of a block sit in separate
+// waves and K ends at the element's function count.  Against one launch per
+// element after a grouping pass, and one atom per lane in FP32, a whole step
+// took: 19,652 atoms, 27-24-24-1, FP32 layers 437 -> 237 us; 3,000 atoms,
+// two 70-25-25-1 networks, BF16 parts 288 -> 243 us (192,000 atoms: 5.63 ->
+// 5.53 ms).
+//
 // MFMA 16x16x32 operand layout (per lane l): A[row = l % 16][k = 8 (l / 16)
 // + 0..7], B[k = 8 (l / 16) + 0..7][col = l % 16], D[row = 4 (l / 16) + 0..3]
-// [col = l % 16].
-__global__ __launch_bounds__( 256 ) void k_nnp_mlp( int elem, const int *__restrict__ list,
-                                                   const int *__restrict__ count,
-                                                   const float *__restrict__ G,
-                                                   const NnpPlan *__restrict__ P,
-                                                   float *__restrict__ dEdG,
-                                                   float *__restrict__ Ei )
+// [col = l % 16]; 16x16x4: A[row = l % 16][k = l / 16], B[k = l / 16]
+// [col = l % 16], D as above.
+constexpr int MLP_ATOMS = 64; // atoms per block
+constexpr int MLP_WAVES = MLP_ATOMS / 16 + NNP_MAXEL - 1;
+
+template <bool F32>
+__global__ __launch_bounds__( 64 * MLP_WAVES ) void k_nnp_mlp(
+    int n_local, int nelem, const double4 *__restrict__ x, const float *__restrict__ G,
+    const NnpPlan *__restrict__ P, float *__restrict__ dEdG, float *__restrict__ Ei )
 {
-    __shared__ float sA[4][16][KPAD + 4]; // per wave: row-major 16 x K
+    extern __shared__ __align__( 16 ) float s_mlp[]; // per wave: row-major 16 x (KPAD + 4)
+    __shared__ int s_atom[MLP_ATOMS];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int t0 = ( blockIdx.x * 4 + wv ) * 16;
-    const int cnt = count[elem];
-    if ( t0 >= cnt )
+    // every wave groups the block's atoms the same way: rank of each atom in
+    // element order, and the element and atoms of this wave's tile
+    const int at = blockIdx.x * MLP_ATOMS + lane;
+    const int el = at < n_local ? (int)x[at].w : -1;
+    int elem = -1, first = 0, cnt = 0; // this wave's tile: s_atom[first ..)
+    {
+        int base = 0, tile = 0;
+        for ( int e = 0; e < nelem; ++e )
+        {
+            const unsigned long long m = __ballot( el == e );
+            const int c = (int)__popcll( m );
+            if ( wv == 0 && el == e )
+                s_atom[base + (int)__builtin_amdgcn_mbcnt_hi(
+                                  (unsigned)( m >> 32 ),
+                                  __builtin_amdgcn_mbcnt_lo( (unsigned)m, 0u ) )] = at;
+            const int nt = ( c + 15 ) >> 4;
+            if ( wv >= tile && wv < tile + nt )
+            {
+                elem = e;
+                first = base + 16 * ( wv - tile );
+                cnt = min( 16, c - 16 * ( wv - tile ) );
+            }
+            tile += nt;
+            base += c;
+        }
+    }
+    __syncthreads();
+    elem = __builtin_amdgcn_readfirstlane( elem );
+    if ( elem < 0 )
         return;
     const NnpElemPlan &Q = P->el[elem];
-    float( *A )[KPAD + 4] = sA[wv];
+    constexpr int LDA = KPAD + 4;
+    float *A = s_mlp + wv * 16 * LDA;
     const int row = lane & 15, kq = ( lane >> 4 ) * 4, k8 = ( lane >> 4 ) * 8;
-    // scaled inputs, row-major in LDS
-    for ( int k = lane; k < 16 * KPAD; k += 64 )
+    const int ka = F32 ? kq : k8; // first k of the lane in a 32-deep block
+    const int nsf = Q.nsf, nkb = ( nsf + 31 ) >> 5;
+    // scaled inputs, row-major in LDS, zero past nsf and past the tile's
+    // atoms: lane group l / 16 takes every fourth quad of row l % 16
     {
-        const int r = k / KPAD, c = k % KPAD;
-        float v = 0.0f;
-        if ( t0 + r < cnt && c < Q.nsf )
+        const bool have = row < cnt;
+        const float *Gi = G + (size_t)s_atom[first + ( have ? row : 0 )] * NSF_LD;
+        for ( int c = kq; c < 32 * nkb; c += 16 )
         {
-            const int at = list[t0 + r];
-            v = Q.g_mul[c] * G[(size_t)at * NSF_LD + c] + Q.g_add[c];
+            const f32x4 g = *reinterpret_cast<const f32x4 *>( Gi + c );
+            const f32x4 mu = *reinterpret_cast<const f32x4 *>( Q.g_mul + c );
+            const f32x4 ad = *reinterpret_cast<const f32x4 *>( Q.g_add + c );
+            f32x4 v;
+#pragma unroll
+            for ( int u = 0; u < 4; ++u )
+                v[u] = have && c + u < nsf ? mu[u] * g[u] + ad[u] : 0.f;
+            *reinterpret_cast<f32x4 *>( A + row * LDA + c ) = v;
         }
-        A[r][c] = v;
     }
     __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
-    // layer 1: h1[16 x 32] = Gs[16 x 96] W1^T, B[k][col] = W1[col][k]
-    f32x4 h1[2];
-#pragma unroll
-    for ( int nt = 0; nt < 2; ++nt )
+    // one 32-deep K block: A row at k0, W in [col][k] order (split parts Ws)
+    auto block = [&]( int k0, const float *W, const unsigned short *Ws, size_t stride, int ld,
+                      int col, f32x4 c ) -> f32x4
     {
-        f32x4 c = { 0.f, 0.f, 0.f, 0.f };
+        if constexpr ( F32 )
+            return mfma_f32( A + row * LDA + k0 + ka, W + (size_t)col * ld + k0 + ka, c );
+        else
+            return mfma_split( A + row * LDA + k0 + ka, Ws + (size_t)col * ld + k0 + ka, stride,
+                               c );
+    };
+    const f32x4 zero = { 0.f, 0.f, 0.f, 0.f };
+    // layer 1: h1[16 x 32] = Gs[16 x K] W1^T, B[k][col] = W1[col][k]
+    f32x4 h1[2] = { zero, zero };
+    for ( int kb = 0; kb < nkb; ++kb )
 #pragma unroll
-        for ( int kb = 0; kb < KPAD / 32; ++kb )
-            c = mfma_split( &A[row][kb * 32 + k8], &Q.W1s[0][nt * 16 + row][kb * 32 + k8],
-                            (size_t)HPAD * KPAD, c );
-        h1[nt] = c;
-    }
+        for ( int nt = 0; nt < 2; ++nt )
+            h1[nt] = block( kb * 32, &Q.W1[0][0], &Q.W1s[0][0][0], (size_t)HPAD * KPAD, KPAD,
+                            nt * 16 + row, h1[nt] );
     __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
     // bias + activation; h1 to LDS (row-major 16 x 32)
 #pragma unroll
@@ -930,15 +1011,15 @@ __global__ __launch_bounds__( 256 ) void k_nnp_mlp( int elem, const int *__restr
             const float z = h1[nt][u] + ( col < Q.h1 ? Q.b1[col] : 0.f );
             const float h = col < Q.h1 ? act_f( z, Q.act1 ) : 0.f;
             h1[nt][u] = h;
-            A[r][col] = h;
+            A[r * LDA + col] = h;
         }
     __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
     // layer 2: h2[16 x 32] = h1 W2^T, B[k][col] = W2[col][k]
     f32x4 h2[2];
 #pragma unroll
     for ( int nt = 0; nt < 2; ++nt )
-        h2[nt] = mfma_split( &A[row][k8], &Q.W2s[0][nt * 16 + row][k8], (size_t)HPAD * HPAD,
-                             f32x4{ 0.f, 0.f, 0.f, 0.f } );
+        h2[nt] = block( 0, &Q.W2[0][0], &Q.W2s[0][0][0], (size_t)HPAD * HPAD, HPAD,
+                        nt * 16 + row, zero );
     __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
     // output layer and the first backward step (VALU, FP32):
     // E = w3 . h2 + b3; delta2 = w3 * act'(z2)
@@ -953,7 +1034,7 @@ __global__ __launch_bounds__( 256 ) void k_nnp_mlp( int elem, const int *__restr
             const float h = col < Q.h2 ? act_f( z, Q.act2 ) : 0.f;
             const float w = col < Q.h2 ? Q.w3[col] : 0.f;
             epart[u] += h * w;
-            A[r][col] = Q.act2 ? w * ( 1.f - h * h ) : w; // delta2, row-major
+            A[r * LDA + col] = Q.act2 ? w * ( 1.f - h * h ) : w; // delta2, row-major
         }
     // sum the 16 columns held by the 16 lanes of each row group
 #pragma unroll
@@ -968,15 +1049,15 @@ __global__ __launch_bounds__( 256 ) void k_nnp_mlp( int elem, const int *__restr
     if ( row == 0 )
 #pragma unroll
         for ( int u = 0; u < 4; ++u )
-            if ( t0 + kq + u < cnt )
-                Ei[list[t0 + kq + u]] = epart[u] + Q.b3;
+            if ( kq + u < cnt )
+                Ei[s_atom[first + kq + u]] = epart[u] + Q.b3;
     __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
     // delta1[16 x 32] = (delta2 W2) * act'(z1): B[k][col] = W2[k][col]
     f32x4 d1[2];
 #pragma unroll
     for ( int nt = 0; nt < 2; ++nt )
-        d1[nt] = mfma_split( &A[row][k8], &Q.W2Ts[0][nt * 16 + row][k8], (size_t)HPAD * HPAD,
-                             f32x4{ 0.f, 0.f, 0.f, 0.f } );
+        d1[nt] = block( 0, &Q.W2T[0][0], &Q.W2Ts[0][0][0], (size_t)HPAD * HPAD, HPAD,
+                        nt * 16 + row, zero );
     __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
 #pragma unroll
     for ( int nt = 0; nt < 2; ++nt )
@@ -985,74 +1066,20 @@ __global__ __launch_bounds__( 256 ) void k_nnp_mlp( int elem, const int *__restr
         {
             const int r = kq + u, col = nt * 16 + row;
             const float h = h1[nt][u];
-            A[r][col] = col < Q.h1 ? ( Q.act1 ? d1[nt][u] * ( 1.f - h * h ) : d1[nt][u] ) : 0.f;
+            A[r * LDA + col] =
+                col < Q.h1 ? ( Q.act1 ? d1[nt][u] * ( 1.f - h * h ) : d1[nt][u] ) : 0.f;
         }
     __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
-    // dE/dGs[16 x 96] = delta1 W1: B[k][col] = W1[k][col]
-#pragma unroll
-    for ( int nt = 0; nt < KPAD / 16; ++nt )
+    // dE/dGs[16 x nsf] = delta1 W1: B[k][col] = W1[k][col]
+    for ( int nt = 0; 16 * nt < nsf; ++nt )
     {
-        const f32x4 c = mfma_split( &A[row][k8], &Q.W1Ts[0][nt * 16 + row][k8],
-                                    (size_t)KPAD * HPAD, f32x4{ 0.f, 0.f, 0.f, 0.f } );
+        const f32x4 c = block( 0, &Q.W1T[0][0], &Q.W1Ts[0][0][0], (size_t)KPAD * HPAD, HPAD,
+                               nt * 16 + row, zero );
         const int col = nt * 16 + row;
 #pragma unroll
         for ( int u = 0; u < 4; ++u )
-            if ( t0 + kq + u < cnt && col < Q.nsf )
-                dEdG[(size_t)list[t0 + kq + u] * NSF_LD + col] = c[u] * Q.g_mul[col];
-    }
-}
-
-// The same network in FP32 on the VALU, one atom per lane.
-__global__ __launch_bounds__( 256 ) void k_nnp_mlp_f32( int n_local,
-                                                       const double4 *__restrict__ x,
-                                                       const float *__restrict__ G,
-                                                       const NnpPlan *__restrict__ P,
-                                                       float *__restrict__ dEdG,
-                                                       float *__restrict__ Ei )
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if ( i >= n_local )
-        return;
-    const NnpElemPlan &Q = P->el[(int)x[i].w];
-    const float *Gi = G + (size_t)i * NSF_LD;
-    float gs[KPAD];
-    for ( int k = 0; k < Q.nsf; ++k )
-        gs[k] = Q.g_mul[k] * Gi[k] + Q.g_add[k];
-    float h1[HPAD], h2[HPAD];
-    for ( int o = 0; o < Q.h1; ++o )
-    {
-        float z = Q.b1[o];
-        for ( int k = 0; k < Q.nsf; ++k )
-            z = fmaf( Q.W1[o][k], gs[k], z );
-        h1[o] = act_f( z, Q.act1 );
-    }
-    float e = Q.b3;
-    for ( int o = 0; o < Q.h2; ++o )
-    {
-        float z = Q.b2[o];
-        for ( int k = 0; k < Q.h1; ++k )
-            z = fmaf( Q.W2[o][k], h1[k], z );
-        h2[o] = act_f( z, Q.act2 );
-        e = fmaf( Q.w3[o], h2[o], e );
-    }
-    Ei[i] = e;
-    float d2[HPAD], d1[HPAD];
-    for ( int o = 0; o < Q.h2; ++o )
-        d2[o] = Q.act2 ? Q.w3[o] * ( 1.f - h2[o] * h2[o] ) : Q.w3[o];
-    for ( int k = 0; k < Q.h1; ++k )
-    {
-        float s = 0.f;
-        for ( int o = 0; o < Q.h2; ++o )
-            s = fmaf( Q.W2[o][k], d2[o], s );
-        d1[k] = Q.act1 ? s * ( 1.f - h1[k] * h1[k] ) : s;
-    }
-    float *Di = dEdG + (size_t)i * NSF_LD;
-    for ( int k = 0; k < Q.nsf; ++k )
-    {
-        float s = 0.f;
-        for ( int o = 0; o < Q.h1; ++o )
-            s = fmaf( Q.W1[o][k], d1[o], s );
-        Di[k] = s * Q.g_mul[k];
+            if ( kq + u < cnt && col < nsf )
+                dEdG[(size_t)s_atom[first + kq + u] * NSF_LD + col] = c[u] * Q.g_mul[col];
     }
 }
 
@@ -1340,33 +1367,6 @@ __global__ __launch_bounds__( NNP_TPB ) void k_nnp_force(
     }
 }
 
-// Atoms grouped by element for the per-element network GEMMs; one atomic
-// per element and wave (the order inside a group does not matter).
-__global__ void k_nnp_group( int n_local, const double4 *__restrict__ x,
-                             int cap, int *__restrict__ list, int *__restrict__ count )
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int lane = threadIdx.x & 63;
-    const int e = i < n_local ? (int)x[i].w : -1;
-    for ( int el = 0; el < NNP_MAXEL; ++el )
-    {
-        const unsigned long long m = __ballot( e == el );
-        if ( !m )
-            continue;
-        const int leader = __ffsll( (long long)m ) - 1;
-        int base = 0;
-        if ( lane == leader )
-            base = atomicAdd( &count[el], (int)__popcll( m ) );
-        base = __shfl( base, leader, 64 );
-        if ( e == el )
-        {
-            const int r = (int)__builtin_amdgcn_mbcnt_hi(
-                (unsigned)( m >> 32 ), __builtin_amdgcn_mbcnt_lo( (unsigned)m, 0u ) );
-            list[(size_t)el * cap + base + r] = i;
-        }
-    }
-}
-
 __global__ void k_nnp_esum( int n, const float *__restrict__ Ei,
                             double *__restrict__ part )
 {
@@ -1402,9 +1402,7 @@ static cmd_status nnp_prepare( cmd_nnp *M, int n_local, hipStream_t st )
         CMD_TRY( M->G.reserve( (size_t)n * NSF_LD ) );
         CMD_TRY( M->dEdG.reserve( (size_t)n * NSF_LD ) );
         CMD_TRY( M->Ei.reserve( n ) );
-        CMD_TRY( M->elist.reserve( (size_t)n * NNP_MAXEL ) );
     }
-    CMD_TRY( M->ecount.reserve( NNP_MAXEL ) );
     CMD_TRY( M->flag.reserve( 1 ) );
     return CMD_OK;
 }
@@ -1460,25 +1458,16 @@ cmd_status nnp_compute( cmd_nnp *M, cmd_system *S, cmd_neigh *N )
         CMD_SF( 0, 0, false );
 #undef CMD_SF
     CMD_LAUNCH_CHECK();
-    if ( M->prec == CMD_PREC_MIXED )
     {
-        CMD_TRY( fill_i32( M->ecount.p, 0, NNP_MAXEL, st ) );
-        k_nnp_group<<<( n + 255 ) / 256, 256, 0, st>>>( n, S->x.p, M->cap,
-                                                       M->elist.p, M->ecount.p );
-        CMD_LAUNCH_CHECK();
-        for ( int e = 0; e < M->plan.nelem; ++e )
-        {
-            k_nnp_mlp<<<( n + 63 ) / 64, 256, 0, st>>>(
-                e, M->elist.p + (size_t)e * M->cap, M->ecount.p, M->G.p,
-                M->dplan.p, M->dEdG.p, M->Ei.p );
-            CMD_LAUNCH_CHECK();
-        }
-    }
-    else
-    {
-        k_nnp_mlp_f32<<<( n + 255 ) / 256, 256, 0, st>>>( n, S->x.p, M->G.p,
-                                                         M->dplan.p, M->dEdG.p,
-                                                         M->Ei.p );
+        const int nb = ( n + MLP_ATOMS - 1 ) / MLP_ATOMS;
+        const int waves = MLP_ATOMS / 16 + M->plan.nelem - 1;
+        const size_t lds = (size_t)waves * 16 * ( KPAD + 4 ) * sizeof( float );
+        if ( M->prec == CMD_PREC_MIXED )
+            k_nnp_mlp<false><<<nb, 64 * waves, lds, st>>>( n, M->plan.nelem, S->x.p, M->G.p,
+                                                           M->dplan.p, M->dEdG.p, M->Ei.p );
+        else
+            k_nnp_mlp<true><<<nb, 64 * waves, lds, st>>>( n, M->plan.nelem, S->x.p, M->G.p,
+                                                          M->dplan.p, M->dEdG.p, M->Ei.p );
         CMD_LAUNCH_CHECK();
     }
 #define CMD_FORCE( A, P, R )                                                               \

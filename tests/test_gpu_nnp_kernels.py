@@ -1,0 +1,99 @@
+"""NNP kernels at the sizes where their block and grid mappings can go wrong,
+against the FP64 NNP oracle on open clusters (no periodic images in reach).
+
+Bars: FP32 symmetry functions and sums carry 6e-8 relative per operation over
+chains of at most a few hundred terms, so 2e-5 of each function's scale and
+1e-4 of the energy and force scales leave a factor of ten.
+"""
+import numpy as np
+import pytest
+
+import pyoracle as O
+from test_gpu_nnp import _engine_model, _system
+from nnp_models import to_oracle
+
+pytestmark = pytest.mark.gpu
+
+BOX = 60.0
+
+
+def _cluster(n, nelem, seed):
+    """n atoms at least 0.9 apart in the middle of the box."""
+    rng = np.random.default_rng(seed)
+    side = max(2.0, (1.6 * n) ** (1.0 / 3.0))
+    x = np.empty((0, 3))
+    while len(x) < n:
+        p = rng.uniform(0, side, 3)
+        if len(x) == 0 or np.min(np.linalg.norm(x - p, axis=1)) >= 0.9:
+            x = np.vstack([x, p])
+    return x + 0.5 * (BOX - side), rng.integers(0, nelem, n).astype(np.int32)
+
+
+def _model(nelem, etas, pl, ang_rs=0.0, rc=3.0, hidden=(7, 5), seed=3):
+    """Radial functions on any neighbour and the (eta) x (zeta, lambda)
+    angular grid for every element, in a shuffled order."""
+    rng = np.random.default_rng(seed)
+    m = dict(nelem=nelem, hidden=list(hidden), act="ttl", smin=0.0, smax=1.0,
+             scale=True, sf=[], gmin=[], gmax=[], W=[], b=[],
+             atom_energy=[0.0] * nelem)
+    for e in range(nelem):
+        sf = [(2, -1, -1, eta, 0.3 * k, 0.0, 0.0, rc)
+              for k, eta in enumerate((0.05, 0.4))]
+        sf += [(3, -1, -1, eta, ang_rs, lam, z, rc) for eta in etas
+               for z, lam in pl]
+        sf = [sf[k] for k in rng.permutation(len(sf))]
+        n = len(sf)
+        sizes = [n] + list(hidden) + [1]
+        m["sf"].append(sf)
+        m["gmin"].append(rng.uniform(0.0, 0.2, n))
+        m["gmax"].append(m["gmin"][-1] + rng.uniform(1.0, 3.0, n))
+        m["W"].append([rng.normal(0, 1, (sizes[l + 1], sizes[l])) /
+                       np.sqrt(sizes[l]) for l in range(3)])
+        m["b"].append([rng.normal(0, 0.1, sizes[l + 1]) for l in range(3)])
+    return m
+
+
+def _check(M, m, x, t, prec):
+    nelem = m["nelem"]
+    s, comm, nl = _system(M, x, t, [BOX] * 3, 3.3, ntypes=nelem)
+    F = M.ForceNNP(_engine_model(M, m),
+                   M.PREC_FP64 if prec == "fp32" else M.PREC_MIXED)
+    F.compute(s, nl)
+    f = s.download()[2][:len(x)]
+    G, _, E = F.atomic(s, 96)
+    off, idx = nl.get()
+    _, Eo, Go, _, fo = to_oracle(O, m).compute(s.download()[0], t, len(x), off,
+                                               idx, ld=96)
+    for e in range(nelem):
+        k = t == e
+        if k.any():
+            ns = len(m["sf"][e])
+            scale = np.maximum(np.abs(Go[k][:, :ns]).max(axis=0), 1e-3)
+            assert (np.abs(G[k][:, :ns] - Go[k][:, :ns]) / scale).max() < 2e-5
+    assert np.abs(E - Eo).max() < 1e-4 * max(np.abs(Eo).max(), 1e-3)
+    fs = max(np.sqrt((fo[:len(x)] ** 2).sum(1).mean()), 1e-6)
+    assert np.sqrt(((f - fo[:len(x)]) ** 2).sum(1)).max() < 1e-4 * fs
+
+
+PL = [(z, lam) for z in (1.0, 3.0) for lam in (-1.0, 1.0)]
+
+
+@pytest.mark.parametrize("prec", ["fp32", "bf16"])
+@pytest.mark.parametrize("nelem,n", [(1, 1), (1, 16), (1, 65), (2, 63),
+                                     (2, 130), (3, 64), (4, 66), (4, 200)])
+def test_network_tiles(gpu, nelem, n, prec):
+    """The network kernel's blocks of 64 atoms and tiles of 16 atoms of one
+    element: part-full tiles and blocks, one to four elements."""
+    x, t = _cluster(n, nelem, 10 * n + nelem)
+    _check(gpu, _model(nelem, (0.01, 0.2), PL), x, t, prec)
+
+
+@pytest.mark.parametrize("prec", ["fp32", "bf16"])
+@pytest.mark.parametrize("neta", [1, 7, 8])
+def test_network_input_widths(gpu, neta, prec):
+    """Function counts around the 32-deep blocks of the first product: 10,
+    58 and 66 inputs, and hidden layers of 32 and 1 nodes."""
+    pl = [(z, lam) for z in (1.0, 2.0, 3.0, 5.0) for lam in (-1.0, 1.0)]
+    etas = [0.02 * (k + 1) for k in range(neta)]
+    x, t = _cluster(50, 2, neta)
+    _check(gpu, _model(2, etas, pl, hidden=(32, 1)), x, t, prec)
