@@ -60,8 +60,13 @@ static constexpr int NSF_LD = 96;              // row stride of G / dE/dG
 static constexpr int KPAD = 96;                // MFMA K of layer 1 (6 x 16)
 static constexpr int HPAD = 32;                // hidden width (2 x 16)
 static constexpr int NN_MAX = 128;             // neighbours inside rc
-static constexpr int TCAP = 512;               // compacted neighbour pairs per wave
+static constexpr int TCAP = 1024;              // compacted neighbour pairs per wave
 static constexpr int NNP_TPB = 256;
+// The (lambda, zeta) grid of zeta = 1, 2, 4, 16 and both signs of lambda:
+// its powers are a few squarings, so it has kernels of its own.  Entry p:
+// lambda = -1 for p < 4, else +1; zeta = POW_ZETA[p % 4].
+static constexpr double POW_ZETA[4] = { 1.0, 2.0, 4.0, 16.0 };
+static constexpr int POW_NAP = 8;
 
 struct NnpElemPlan
 {
@@ -73,6 +78,7 @@ struct NnpElemPlan
     float a_eta[AG_MAX], a_rs[AG_MAX];
     float a_lam[AP_MAX], a_zeta[AP_MAX], a_lpref[AP_MAX]; // lpref = 1 - zeta
     int a_out[AG_MAX][AP_MAX];     // model index of angular (g, p)
+    int pow2;                      // (lambda, zeta) are the POW_* grid, in its order
     alignas( 16 ) float g_mul[NSF_LD]; // Gs = g_mul * G + g_add
     alignas( 16 ) float g_add[NSF_LD];
     int h1, h2;
@@ -240,6 +246,17 @@ static cmd_status build_plan( const cmd_nnp_model &m, NnpPlan &P )
                 return CMD_ERR_ARG;
             }
         }
+        // the power-of-two grid in its own order, whatever the model's
+        Q.pow2 = (int)ap.size() == POW_NAP;
+        std::vector<std::pair<double, double>> pg;
+        for ( int p = 0; p < POW_NAP; ++p )
+        {
+            pg.push_back( { p < 4 ? -1.0 : 1.0, POW_ZETA[p % 4] } );
+            if ( std::find( ap.begin(), ap.end(), pg.back() ) == ap.end() )
+                Q.pow2 = 0;
+        }
+        if ( Q.pow2 )
+            ap = pg;
         CMD_REQUIRE( (int)rg.size() <= RG_MAX && (int)re.size() <= RE_MAX &&
                          (int)ag.size() <= AG_MAX && (int)ap.size() <= AP_MAX,
                      CMD_ERR_ARG, "symmetry-function grid too large" );
@@ -486,20 +503,60 @@ __device__ __forceinline__ void ang_powers( const AngK &K, float cs, float *Pw, 
 // Reduce-scatter across the 64 lanes: in: v[S] per lane; out: v[0] of
 // lane l = the sum over lanes of value l (S = 64) or l & 31 (S = 32).
 // Each halving step keeps the half selected by one lane bit and sends the
-// other half to the partner lane, so S values cost S - 1 shuffles in all.
+// other half to the partner lane, so S values cost S - 1 exchanges in all.
+// The 32- and 16-lane exchanges are one swap of the two halves' registers
+// (after it, one register holds the kept value of every lane and the other
+// the received one); the shorter ones go through the row rotations and quad
+// permutes of the adder's operand, so no step waits on LDS.
+template <int CTRL>
+__device__ __forceinline__ float dpp_f( float v )
+{
+    return __builtin_bit_cast( float, __builtin_amdgcn_update_dpp(
+                                          0, __builtin_bit_cast( int, v ), CTRL, 0xf, 0xf, true ) );
+}
+
+template <int O>
+__device__ __forceinline__ float lane_xor( float v )
+{
+    if constexpr ( O == 8 )
+        return dpp_f<0x128>( v ); // row_ror:8
+    else if constexpr ( O == 2 )
+        return dpp_f<0x4e>( v ); // quad_perm [2,3,0,1]
+    else if constexpr ( O == 1 )
+        return dpp_f<0xb1>( v ); // quad_perm [1,0,3,2]
+    else
+        return __shfl_xor( v, O, 64 );
+}
+
 template <int M>
 __device__ __forceinline__ void rs_step( float *v, int lane )
 {
     if constexpr ( M > 1 )
     {
         constexpr int O = M / 2;
-        const bool hi = lane & O;
-#pragma unroll
-        for ( int k = 0; k < O; ++k )
+        if constexpr ( O >= 16 )
         {
-            const float keep = hi ? v[O + k] : v[k];
-            const float send = hi ? v[k] : v[O + k];
-            v[k] = keep + __shfl_xor( send, O, 64 );
+#pragma unroll
+            for ( int k = 0; k < O; ++k )
+            {
+                const unsigned a = __builtin_bit_cast( unsigned, v[k] ),
+                               b = __builtin_bit_cast( unsigned, v[O + k] );
+                const auto r = O == 32 ? __builtin_amdgcn_permlane32_swap( a, b, false, false )
+                                       : __builtin_amdgcn_permlane16_swap( a, b, false, false );
+                v[k] = __builtin_bit_cast( float, (unsigned)r[0] ) +
+                       __builtin_bit_cast( float, (unsigned)r[1] );
+            }
+        }
+        else
+        {
+            const bool hi = lane & O;
+#pragma unroll
+            for ( int k = 0; k < O; ++k )
+            {
+                const float keep = hi ? v[O + k] : v[k];
+                const float send = hi ? v[k] : v[O + k];
+                v[k] = keep + lane_xor<O>( send );
+            }
         }
         rs_step<O>( v, lane );
     }
@@ -594,7 +651,7 @@ __device__ __forceinline__ void pair_of( int p, int n, int &a, int &q )
 
 // The neighbour pairs (a < q) of the gathered list whose third side is
 // inside the cutoff, |x_q - x_a| < rc: tested 64 at a time and compacted
-// into buf (TCAP entries per wave, a | q << 16), then handed to body(a, q)
+// into buf (TCAP entries per wave, a | q << 8; NN_MAX <= 256), then handed to body(a, q)
 // with every lane busy (lane l takes entries l*per .. l*per + per - 1).
 // Used where the body keeps many accumulators in registers.
 // With PAIRS the body takes two pairs at once, (a0, q0) and (a1, q1), the
@@ -602,7 +659,8 @@ __device__ __forceinline__ void pair_of( int p, int n, int &a, int &q )
 // chains are independent, so their latencies overlap.
 template <bool PAIRS = false, class Body>
 __device__ __forceinline__ void for_triplets( const NbLds &L, int n, float rc2,
-                                             unsigned *buf, Body body, int *count = nullptr )
+                                             unsigned short *buf, Body body,
+                                             int *count = nullptr )
 {
     const int lane = threadIdx.x & 63;
     // candidate pairs, 64 per test: with n <= 64 rows a and n - 2 - a side
@@ -617,7 +675,7 @@ __device__ __forceinline__ void for_triplets( const NbLds &L, int n, float rc2,
         while ( cnt <= TCAP - 64 && it < nit )
         {
             bool ok = false;
-            unsigned code = 0u;
+            unsigned short code = 0;
             int a = 0, q = 0;
             bool have;
             if ( rows )
@@ -650,7 +708,7 @@ __device__ __forceinline__ void for_triplets( const NbLds &L, int n, float rc2,
                 const float4 A = L.d[a], B = L.d[q];
                 const float cx = B.x - A.x, cy = B.y - A.y, cz = B.z - A.z;
                 ok = cx * cx + cy * cy + cz * cz < rc2;
-                code = (unsigned)a | ( (unsigned)q << 16 );
+                code = (unsigned short)( a | ( q << 8 ) );
             }
             const unsigned long long m = __ballot( ok );
             if ( ok )
@@ -674,8 +732,8 @@ __device__ __forceinline__ void for_triplets( const NbLds &L, int n, float rc2,
                     const unsigned c0 = buf[e];
                     const bool ok1 = j + 1 < per && e + 1 < cnt;
                     const unsigned c1 = ok1 ? buf[e + 1] : c0;
-                    body( (int)( c0 & 0xffffu ), (int)( c0 >> 16 ), (int)( c1 & 0xffffu ),
-                          (int)( c1 >> 16 ), ok1 );
+                    body( (int)( c0 & 0xffu ), (int)( c0 >> 8 ), (int)( c1 & 0xffu ),
+                          (int)( c1 >> 8 ), ok1 );
                 }
             }
         }
@@ -687,11 +745,48 @@ __device__ __forceinline__ void for_triplets( const NbLds &L, int n, float rc2,
                 if ( e < cnt )
                 {
                     const unsigned c = buf[e];
-                    body( (int)( c & 0xffffu ), (int)( c >> 16 ) );
+                    body( (int)( c & 0xffu ), (int)( c >> 8 ) );
                 }
             }
         }
         __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
+    }
+}
+
+// Radial symmetry functions of one atom, lanes over its neighbours.
+__device__ __forceinline__ void radial_sf( const NnpElemPlan &Q, const NbLds &L, int n,
+                                           float *__restrict__ Gi )
+{
+    const int lane = threadIdx.x & 63;
+    float acc[NR_MAX];
+#pragma unroll
+    for ( int s = 0; s < NR_MAX; ++s )
+        acc[s] = 0.0f;
+    for ( int a = lane; a < n; a += 64 )
+    {
+        const float4 Ea = L.e[a];
+        const float r = L.d[a].w, fc = Ea.y;
+        const int ej = __builtin_bit_cast( int, Ea.w );
+#pragma unroll
+        for ( int g = 0; g < RG_MAX; ++g )
+        {
+            if ( g < Q.nrg )
+            {
+                const float t = r - Q.r_rs[g];
+                const float v = __expf( -Q.r_eta[g] * t * t ) * fc;
+#pragma unroll
+                for ( int k = 0; k < RE_MAX; ++k )
+                    if ( k < Q.nre && ( Q.r_el[k] < 0 || Q.r_el[k] == ej ) )
+                        acc[g * RE_MAX + k] += v;
+            }
+        }
+    }
+    wave_reduce_scatter<NR_MAX>( acc );
+    if ( lane < NR_MAX )
+    {
+        const int g = lane / RE_MAX, k = lane % RE_MAX;
+        if ( g < Q.nrg && k < Q.nre )
+            Gi[Q.r_out[g][k]] = acc[0];
     }
 }
 
@@ -708,7 +803,7 @@ __global__ __launch_bounds__( NNP_TPB ) void k_nnp_sf(
     float *__restrict__ G, int *__restrict__ flag, int4 *__restrict__ terms )
 {
     __shared__ NbLds lds[NNP_TPB / 64];
-    __shared__ unsigned tbuf[NNP_TPB / 64][TCAP];
+    __shared__ unsigned short tbuf[NNP_TPB / 64][TCAP];
     __shared__ float kst[NNP_TPB / 64][64];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int i = blockIdx.x * ( NNP_TPB / 64 ) + wv;
@@ -725,39 +820,7 @@ __global__ __launch_bounds__( NNP_TPB ) void k_nnp_sf(
     if constexpr ( NAP > 0 )
         K.nap = NAP;
     float *Gi = G + (size_t)i * NSF_LD;
-    // radial: lanes over neighbours
-    {
-        float acc[NR_MAX];
-#pragma unroll
-        for ( int s = 0; s < NR_MAX; ++s )
-            acc[s] = 0.0f;
-        for ( int a = lane; a < n; a += 64 )
-        {
-            const float4 Ea = L.e[a];
-            const float r = L.d[a].w, fc = Ea.y;
-            const int ej = __builtin_bit_cast( int, Ea.w );
-#pragma unroll
-            for ( int g = 0; g < RG_MAX; ++g )
-            {
-                if ( g < Q.nrg )
-                {
-                    const float t = r - Q.r_rs[g];
-                    const float v = __expf( -Q.r_eta[g] * t * t ) * fc;
-#pragma unroll
-                    for ( int k = 0; k < RE_MAX; ++k )
-                        if ( k < Q.nre && ( Q.r_el[k] < 0 || Q.r_el[k] == ej ) )
-                            acc[g * RE_MAX + k] += v;
-                }
-            }
-        }
-        wave_reduce_scatter<NR_MAX>( acc );
-        if ( lane < NR_MAX )
-        {
-            const int g = lane / RE_MAX, k = lane % RE_MAX;
-            if ( g < Q.nrg && k < Q.nre )
-                Gi[Q.r_out[g][k]] = acc[0];
-        }
-    }
+    radial_sf( Q, L, n, Gi );
     // angular: lanes over the compacted neighbour pairs
     {
         float acc[NA_MAX];
@@ -822,6 +885,98 @@ __global__ __launch_bounds__( NNP_TPB ) void k_nnp_sf(
         if ( g < Q.nag && pp < Q.nap )
             Gi[Q.a_out[g][pp]] = acc[0];
     }
+}
+
+// ---- the power-of-two (lambda, zeta) grid, angular rs = 0
+//
+// Both kernels below run on the models whose every element has the POW_*
+// grid, NAG (the number of angular etas, the same for all elements) and
+// angular rs of 0 -- the usual n2p2 form -- in place of the general ones.
+// They are bound by FP32 VALU issue, so they are written for few operations
+// per triplet: (1 + lambda cos)^zeta by squarings (no log2 and exp2, and
+// exact to a few roundings for zeta = 16), 2^(1 - zeta) applied to the
+// finished sum or the coefficients, one reciprocal square root for r_jk and
+// 1 / r_jk, and constants in scalar registers.
+
+// A constant of the lane-held table t as a wave-uniform value.
+__device__ __forceinline__ float lane_value( float t, int k )
+{
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_readlane( __builtin_bit_cast( int, t ), k ) );
+}
+
+// b^1, b^2, b^4, b^16
+__device__ __forceinline__ void pow_grid( float b, float *p )
+{
+    p[0] = b;
+    p[1] = b * b;
+    p[2] = p[1] * p[1];
+    const float b8 = p[2] * p[2];
+    p[3] = b8 * b8;
+}
+
+template <int NAG>
+__global__ __launch_bounds__( NNP_TPB ) void k_nnp_sf_pow(
+    int n_local, const double4 *__restrict__ x, const int64_t *__restrict__ off,
+    const int *__restrict__ idx, const NnpPlan *__restrict__ P,
+    float *__restrict__ G, int *__restrict__ flag, int4 *__restrict__ terms )
+{
+    __shared__ NbLds lds[NNP_TPB / 64];
+    __shared__ unsigned short tbuf[NNP_TPB / 64][TCAP];
+    const int wv = __builtin_amdgcn_readfirstlane( threadIdx.x >> 6 ), lane = threadIdx.x & 63;
+    const int i = blockIdx.x * ( NNP_TPB / 64 ) + wv;
+    if ( i >= n_local )
+        return;
+    NbLds &L = lds[wv];
+    const float rc = P->rc, rc2 = P->rc2, kpi = P->pi_rc;
+    const int n = gather_neighbours( i, x, off, idx, rc, rc2, kpi, L, flag );
+    const int e = __builtin_amdgcn_readfirstlane( (int)x[i].w );
+    const NnpElemPlan &Q = P->el[e];
+    float *Gi = G + (size_t)i * NSF_LD;
+    radial_sf( Q, L, n, Gi );
+    // exp(-eta s) = exp2(k s)
+    const float kl = -1.44269504f * Q.a_eta[lane & ( AG_MAX - 1 )];
+    float ke[NAG];
+#pragma unroll
+    for ( int g = 0; g < NAG; ++g )
+        ke[g] = lane_value( kl, g );
+    const float kcos = 0.5f / rc; // cos(pi r / rc) in revolutions
+    float acc[NA_MAX];
+#pragma unroll
+    for ( int s = 0; s < NA_MAX; ++s )
+        acc[s] = 0.0f;
+    int ntrip = 0;
+    for_triplets(
+        L, n, rc2, tbuf[wv],
+        [&]( int a, int q ) {
+            const float4 A = L.d[a], B = L.d[q], Ea = L.e[a], Eb = L.e[q];
+            const float cx = B.x - A.x, cy = B.y - A.y, cz = B.z - A.z;
+            const float c2 = cx * cx + cy * cy + cz * cz;
+            const float f3 =
+                0.5f + 0.5f * __builtin_amdgcn_cosf( __builtin_amdgcn_sqrtf( c2 ) * kcos );
+            const float F = Ea.y * Eb.y * f3;
+            const float cs = ( A.x * B.x + A.y * B.y + A.z * B.z ) * ( Ea.x * Eb.x );
+            const float s2 = A.w * A.w + ( B.w * B.w + c2 );
+            float Pw[POW_NAP];
+            pow_grid( fmaxf( 1.0f - cs, 0.0f ), Pw );
+            pow_grid( fmaxf( 1.0f + cs, 0.0f ), Pw + 4 );
+#pragma unroll
+            for ( int g = 0; g < NAG; ++g )
+            {
+                const float EgF = __builtin_amdgcn_exp2f( ke[g] * s2 ) * F;
+#pragma unroll
+                for ( int pp = 0; pp < POW_NAP; ++pp )
+                    acc[g * AP_MAX + pp] += EgF * Pw[pp];
+            }
+        },
+        &ntrip );
+    // the work model's term counts, as in k_nnp_sf
+    if ( terms && lane == 0 )
+        terms[i] = make_int4( n, ntrip, e, 0 );
+    wave_reduce_scatter<NA_MAX>( acc );
+    const int g = lane / AP_MAX, pp = lane % AP_MAX;
+    if ( g < NAG )
+        Gi[Q.a_out[g][pp]] = acc[0] * __builtin_amdgcn_exp2f( Q.a_lpref[pp] );
 }
 
 // ---- network: split-BF16 MFMA, 16 atoms of one element per wave
@@ -1084,6 +1239,33 @@ __global__ __launch_bounds__( 64 * MLP_WAVES ) void k_nnp_mlp(
 }
 
 // ---- forces
+// sum_s c_s dG_s/dr / r of the radial functions for neighbour a.
+__device__ __forceinline__ float radial_force( const NnpElemPlan &Q, const NbLds &L, int a,
+                                               const float *c )
+{
+    const float4 Ea = L.e[a];
+    const float r = L.d[a].w, fc = Ea.y, dfc = Ea.z;
+    const int ej = __builtin_bit_cast( int, Ea.w );
+    float gsum = 0.f;
+#pragma unroll
+    for ( int g = 0; g < RG_MAX; ++g )
+    {
+        if ( g < Q.nrg )
+        {
+            const float t = r - Q.r_rs[g];
+            const float ex = __expf( -Q.r_eta[g] * t * t );
+            const float d = ex * ( -2.f * Q.r_eta[g] * t * fc + dfc );
+            float cw = 0.f;
+#pragma unroll
+            for ( int k = 0; k < RE_MAX; ++k )
+                if ( k < Q.nre && ( Q.r_el[k] < 0 || Q.r_el[k] == ej ) )
+                    cw += c[Q.r_out[g][k]];
+            gsum = fmaf( cw, d, gsum );
+        }
+    }
+    return gsum * Ea.x;
+}
+
 template <int NAG, int NAP, bool RS0>
 __global__ __launch_bounds__( NNP_TPB ) void k_nnp_force(
     int n_local, int fcap, const double4 *__restrict__ x,
@@ -1095,7 +1277,7 @@ __global__ __launch_bounds__( NNP_TPB ) void k_nnp_force(
     __shared__ float sF[NNP_TPB / 64][NN_MAX][3];
     __shared__ float sC[NNP_TPB / 64][NSF_LD];
     __shared__ float4 sCg[NNP_TPB / 64][NA_MAX / 4]; // c of angular (g, p) in grid order
-    __shared__ unsigned tbuf[NNP_TPB / 64][TCAP];
+    __shared__ unsigned short tbuf[NNP_TPB / 64][TCAP];
     __shared__ float kst[NNP_TPB / 64][64];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int i = blockIdx.x * ( NNP_TPB / 64 ) + wv;
@@ -1125,27 +1307,8 @@ __global__ __launch_bounds__( NNP_TPB ) void k_nnp_force(
     // radial
     for ( int a = lane; a < n; a += 64 )
     {
-        const float4 A = L.d[a], Ea = L.e[a];
-        const float r = A.w, fc = Ea.y, dfc = Ea.z;
-        const int ej = __builtin_bit_cast( int, Ea.w );
-        float gsum = 0.f; // sum_s c_s dG_s/dr
-#pragma unroll
-        for ( int g = 0; g < RG_MAX; ++g )
-        {
-            if ( g < Q.nrg )
-            {
-                const float t = r - Q.r_rs[g];
-                const float ex = __expf( -Q.r_eta[g] * t * t );
-                const float d = ex * ( -2.f * Q.r_eta[g] * t * fc + dfc );
-                float cw = 0.f;
-#pragma unroll
-                for ( int k = 0; k < RE_MAX; ++k )
-                    if ( k < Q.nre && ( Q.r_el[k] < 0 || Q.r_el[k] == ej ) )
-                        cw += c[Q.r_out[g][k]];
-                gsum = fmaf( cw, d, gsum );
-            }
-        }
-        const float s = gsum * Ea.x;
+        const float4 A = L.d[a];
+        const float s = radial_force( Q, L, a, c );
         const float vx = s * A.x, vy = s * A.y, vz = s * A.z;
         // dG/dx_j = g' u; F_j -= c g' u, F_i += c g' u
         sF[wv][a][0] -= vx;
@@ -1367,6 +1530,176 @@ __global__ __launch_bounds__( NNP_TPB ) void k_nnp_force(
     }
 }
 
+// Forces of the power-of-two grid (see k_nnp_sf_pow).  With T = sum_s c_s
+// T_s of a triplet (i, a, q), A = x_a - x_i and B = x_q - x_i, the gradients
+// are combinations of A and B alone,
+//   dT/dA = pa A + pm B,  dT/dB = pb B + pm A,
+//   pm = F T' / (r1 r2) - s3,
+//   pa = F M + s3 - F T' cos / r1^2 + S f2 f3 fc'(r1) / r1  (pb likewise),
+//   s3 = F M + S f1 f2 fc'(r3) / r3,
+// where S, T' and M are the coefficient sums of P E, (dP/dcos) E and
+// -2 eta P E: two scalars per neighbour and triplet in place of gradients by
+// component.  The atom's own force is minus the sum of its neighbours'
+// reactions.
+template <int NAG>
+__global__ __launch_bounds__( NNP_TPB ) void k_nnp_force_pow(
+    int n_local, int fcap, const double4 *__restrict__ x,
+    const int64_t *__restrict__ off, const int *__restrict__ idx,
+    const NnpPlan *__restrict__ P, const float *__restrict__ dEdG,
+    double *__restrict__ f, int *__restrict__ flag )
+{
+    __shared__ NbLds lds[NNP_TPB / 64];
+    __shared__ float sF[NNP_TPB / 64][NN_MAX][3];
+    __shared__ float sC[NNP_TPB / 64][NSF_LD];
+    __shared__ unsigned short tbuf[NNP_TPB / 64][TCAP];
+    const int wv = __builtin_amdgcn_readfirstlane( threadIdx.x >> 6 ), lane = threadIdx.x & 63;
+    const int i = blockIdx.x * ( NNP_TPB / 64 ) + wv;
+    if ( i >= n_local )
+        return;
+    NbLds &L = lds[wv];
+    const float rc = P->rc, rc2 = P->rc2, kpi = P->pi_rc;
+    const int n = gather_neighbours( i, x, off, idx, rc, rc2, kpi, L, flag );
+    const int e = __builtin_amdgcn_readfirstlane( (int)x[i].w );
+    const NnpElemPlan &Q = P->el[e];
+    const float *c = sC[wv];
+    for ( int k = lane; k < NSF_LD; k += 64 )
+        sC[wv][k] = k < Q.nsf ? dEdG[(size_t)i * NSF_LD + k] : 0.f;
+    __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
+    // the radial reactions start each neighbour's sum; e.z becomes fc' / r
+    for ( int a = lane; a < n; a += 64 )
+    {
+        const float4 A = L.d[a];
+        const float s = radial_force( Q, L, a, c );
+        sF[wv][a][0] = -s * A.x;
+        sF[wv][a][1] = -s * A.y;
+        sF[wv][a][2] = -s * A.z;
+        L.e[a].z *= L.e[a].x;
+    }
+    // lane g * 8 + p holds c_gp 2^(1 - zeta_p); exp(-eta s) = exp2(k s)
+    const int lg = lane / AP_MAX, lp = lane % AP_MAX;
+    const float cl = lg < NAG ? c[Q.a_out[lg][lp]] * __builtin_amdgcn_exp2f( Q.a_lpref[lp] ) : 0.f;
+    const float kl = -1.44269504f * Q.a_eta[lane & ( AG_MAX - 1 )];
+    const float ml = -2.0f * Q.a_eta[lane & ( AG_MAX - 1 )];
+    float cg[NAG][POW_NAP], ke[NAG], me[NAG];
+#pragma unroll
+    for ( int g = 0; g < NAG; ++g )
+    {
+        ke[g] = lane_value( kl, g );
+        me[g] = lane_value( ml, g );
+#pragma unroll
+        for ( int pp = 0; pp < POW_NAP; ++pp )
+            cg[g][pp] = lane_value( cl, g * AP_MAX + pp );
+    }
+    __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
+    const float krev = 0.5f / rc; // pi r / rc in revolutions
+    const float kd = -0.5f * kpi;
+    // each lane takes a contiguous block of the compacted (a-major) pair
+    // list: the sums of pa and pm B of the row atom stay in registers until
+    // a changes, the reaction on q goes to LDS
+    int cur = -1;
+    float spa = 0.f, bx = 0.f, by = 0.f, bz = 0.f;
+    auto flush = [&]()
+    {
+        const float4 A = L.d[cur];
+        atomicAdd( &sF[wv][cur][0], -( spa * A.x + bx ) );
+        atomicAdd( &sF[wv][cur][1], -( spa * A.y + by ) );
+        atomicAdd( &sF[wv][cur][2], -( spa * A.z + bz ) );
+    };
+    for_triplets( L, n, rc2, tbuf[wv], [&]( int a, int q ) {
+        const float4 A = L.d[a], Ea = L.e[a];
+        const float4 B = L.d[q], Eb = L.e[q];
+        const float cx = B.x - A.x, cy = B.y - A.y, cz = B.z - A.z;
+        const float c2 = cx * cx + cy * cy + cz * cz;
+        const float ic = __builtin_amdgcn_rsqf( c2 );
+        const float rev = c2 * ic * krev;
+        const float f3 = 0.5f + 0.5f * __builtin_amdgcn_cosf( rev );
+        const float d3 = kd * __builtin_amdgcn_sinf( rev ) * ic; // fc'(r3) / r3
+        const float f12 = Ea.y * Eb.y, F = f12 * f3;
+        const float inv12 = Ea.x * Eb.x;
+        const float cs = ( A.x * B.x + A.y * B.y + A.z * B.z ) * inv12;
+        const float s2 = A.w * A.w + ( B.w * B.w + c2 );
+        // S_g = sum_p c_gp P_p and T_p = sum_g c_gp E_g
+        float Pw[POW_NAP], T[POW_NAP];
+        const float bm = fmaxf( 1.0f - cs, 0.0f ), bp = fmaxf( 1.0f + cs, 0.0f );
+        pow_grid( bm, Pw );
+        pow_grid( bp, Pw + 4 );
+#pragma unroll
+        for ( int pp = 0; pp < POW_NAP; ++pp )
+            T[pp] = 0.f;
+        float S = 0.f, Mg = 0.f;
+#pragma unroll
+        for ( int g = 0; g < NAG; ++g )
+        {
+            const float Eg = __builtin_amdgcn_exp2f( ke[g] * s2 );
+            float sg = 0.f;
+#pragma unroll
+            for ( int pp = 0; pp < POW_NAP; ++pp )
+            {
+                sg = fmaf( cg[g][pp], Pw[pp], sg );
+                T[pp] = fmaf( cg[g][pp], Eg, T[pp] );
+            }
+            const float w = sg * Eg;
+            S += w;
+            Mg = fmaf( me[g], w, Mg );
+        }
+        // T' = sum_p T_p zeta lambda b^(zeta - 1), b^3 and b^15 from the grid
+        const float m3 = Pw[1] * bm, p3 = Pw[5] * bp;
+        const float m15 = Pw[2] * Pw[2] * Pw[2] * m3, p15 = Pw[6] * Pw[6] * Pw[6] * p3;
+        float Td = T[4] - T[0];
+        Td = fmaf( 2.f, T[5] * bp - T[1] * bm, Td );
+        Td = fmaf( 4.f, T[6] * p3 - T[2] * m3, Td );
+        Td = fmaf( 16.f, T[7] * p15 - T[3] * m15, Td );
+        const float X = F * Td, FM = F * Mg;
+        const float s3 = fmaf( S * f12, d3, FM );
+        const float pm = fmaf( X, inv12, -s3 );
+        const float Xc = X * cs, Sf3 = S * f3, base = FM + s3;
+        const float pa = fmaf( Sf3 * Eb.y, Ea.z, fmaf( -Xc * Ea.x, Ea.x, base ) );
+        const float pb = fmaf( Sf3 * Ea.y, Eb.z, fmaf( -Xc * Eb.x, Eb.x, base ) );
+        if ( a != cur )
+        {
+            if ( cur >= 0 )
+                flush();
+            cur = a;
+            spa = bx = by = bz = 0.f;
+        }
+        spa += pa;
+        bx = fmaf( pm, B.x, bx );
+        by = fmaf( pm, B.y, by );
+        bz = fmaf( pm, B.z, bz );
+        atomicAdd( &sF[wv][q][0], -fmaf( pb, B.x, pm * A.x ) );
+        atomicAdd( &sF[wv][q][1], -fmaf( pb, B.y, pm * A.y ) );
+        atomicAdd( &sF[wv][q][2], -fmaf( pb, B.z, pm * A.z ) );
+    } );
+    if ( cur >= 0 )
+        flush();
+    __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
+    float fix = 0.f, fiy = 0.f, fiz = 0.f;
+    for ( int a = lane; a < n; a += 64 )
+    {
+        const int j = L.j[a];
+        const float rx = sF[wv][a][0], ry = sF[wv][a][1], rz = sF[wv][a][2];
+        fix -= rx;
+        fiy -= ry;
+        fiz -= rz;
+        unsafeAtomicAdd( &f[j], (double)rx );
+        unsafeAtomicAdd( &f[fcap + j], (double)ry );
+        unsafeAtomicAdd( &f[2 * fcap + j], (double)rz );
+    }
+#pragma unroll
+    for ( int o = 32; o > 0; o >>= 1 )
+    {
+        fix += __shfl_xor( fix, o, 64 );
+        fiy += __shfl_xor( fiy, o, 64 );
+        fiz += __shfl_xor( fiz, o, 64 );
+    }
+    if ( lane == 0 )
+    {
+        unsafeAtomicAdd( &f[i], (double)fix );
+        unsafeAtomicAdd( &f[fcap + i], (double)fiy );
+        unsafeAtomicAdd( &f[2 * fcap + i], (double)fiz );
+    }
+}
+
 __global__ void k_nnp_esum( int n, const float *__restrict__ Ei,
                             double *__restrict__ part )
 {
@@ -1432,20 +1765,49 @@ cmd_status nnp_compute( cmd_nnp *M, cmd_system *S, cmd_neigh *N )
     CMD_TRY( M->terms.reserve( std::max( n, 1 ) ) );
     M->n_last = n;
     const int nbw = ( n + NNP_TPB / 64 - 1 ) / ( NNP_TPB / 64 );
-    // the angular grid of every element, for the kernels compiled for it:
-    // its size (5 x 8) and whether all its rs are 0
-    bool g58 = M->plan.nelem > 0, rs0 = true;
+    // the angular grid of every element: its number of etas where they
+    // agree (0: they do not), whether all its rs are 0 and whether its
+    // (lambda, zeta) are the power-of-two grid
+    int nag = M->plan.nelem > 0 ? M->plan.el[0].nag : 0;
+    bool nap8 = true, rs0 = true, pow2 = true;
     for ( int e = 0; e < M->plan.nelem; ++e )
     {
         const NnpElemPlan &Q = M->plan.el[e];
-        g58 = g58 && Q.nag == 5 && Q.nap == 8;
+        if ( Q.nag != nag )
+            nag = 0;
+        nap8 = nap8 && Q.nap == 8;
+        pow2 = pow2 && Q.pow2;
         for ( int g = 0; g < Q.nag; ++g )
             rs0 = rs0 && Q.a_rs[g] == 0.f;
     }
+    // squarings in place of log2 and exp2 and fixed grid sizes: the fewest
+    // operations wherever the grid allows them
+    const bool pow = nag >= 1 && rs0 && pow2;
+    const bool g58 = nag == 5 && nap8;
+#define CMD_POW( LAUNCH )                                                                 \
+    switch ( nag )                                                                        \
+    {                                                                                     \
+    case 1: LAUNCH( 1 ); break;                                                           \
+    case 2: LAUNCH( 2 ); break;                                                           \
+    case 3: LAUNCH( 3 ); break;                                                           \
+    case 4: LAUNCH( 4 ); break;                                                           \
+    case 5: LAUNCH( 5 ); break;                                                           \
+    case 6: LAUNCH( 6 ); break;                                                           \
+    case 7: LAUNCH( 7 ); break;                                                           \
+    default: LAUNCH( 8 ); break;                                                          \
+    }
+#define CMD_SF_POW( A )                                                                   \
+    k_nnp_sf_pow<A><<<nbw, NNP_TPB, 0, st>>>( n, S->x.p, N->offsets.p, N->idx.p, M->dplan.p, \
+                                              M->G.p, M->flag.p, M->terms.p )
+#define CMD_FORCE_POW( A )                                                                \
+    k_nnp_force_pow<A><<<nbw, NNP_TPB, 0, st>>>( n, S->cap, S->x.p, N->offsets.p, N->idx.p, \
+                                                 M->dplan.p, M->dEdG.p, S->f.p, M->flag.p )
 #define CMD_SF( A, P, R )                                                                 \
     k_nnp_sf<A, P, R><<<nbw, NNP_TPB, 0, st>>>( n, S->x.p, N->offsets.p, N->idx.p, M->dplan.p, \
                                                 M->G.p, M->flag.p, M->terms.p )
-    if ( g58 )
+    if ( pow )
+        CMD_POW( CMD_SF_POW )
+    else if ( g58 )
     {
         if ( rs0 )
             CMD_SF( 5, 8, true );
@@ -1473,7 +1835,9 @@ cmd_status nnp_compute( cmd_nnp *M, cmd_system *S, cmd_neigh *N )
 #define CMD_FORCE( A, P, R )                                                               \
     k_nnp_force<A, P, R><<<nbw, NNP_TPB, 0, st>>>( n, S->cap, S->x.p, N->offsets.p, N->idx.p, \
                                                    M->dplan.p, M->dEdG.p, S->f.p, M->flag.p )
-    if ( g58 )
+    if ( pow )
+        CMD_POW( CMD_FORCE_POW )
+    else if ( g58 )
     {
         if ( rs0 )
             CMD_FORCE( 5, 8, true );
@@ -1485,6 +1849,9 @@ cmd_status nnp_compute( cmd_nnp *M, cmd_system *S, cmd_neigh *N )
     else
         CMD_FORCE( 0, 0, false );
 #undef CMD_FORCE
+#undef CMD_POW
+#undef CMD_SF_POW
+#undef CMD_FORCE_POW
     CMD_LAUNCH_CHECK();
     int fl = 0;
     CMD_HIP( hipMemcpyAsync( &fl, M->flag.p, sizeof( int ),

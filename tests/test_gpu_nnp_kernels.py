@@ -55,13 +55,23 @@ def _model(nelem, etas, pl, ang_rs=0.0, rc=3.0, hidden=(7, 5), seed=3):
 
 def _check(M, m, x, t, prec):
     nelem = m["nelem"]
-    s, comm, nl = _system(M, x, t, [BOX] * 3, 3.3, ntypes=nelem)
+    cut = m["sf"][0][0][7] + 0.3
+    s, comm, nl = _system(M, x, t, [BOX] * 3, cut, ntypes=nelem)
+    # scale every function to the cluster's own range, as a fitted model does
+    # (far outside it the layers saturate and 1 - tanh^2 cancels)
+    off, idx = nl.get()
+    _, _, G0, _, _ = to_oracle(O, m).compute(s.download()[0], t, len(x), off,
+                                             idx, ld=96)
+    for e in range(nelem):
+        if (t == e).any():
+            g = G0[t == e][:, :len(m["sf"][e])]
+            m["gmin"][e] = g.min(axis=0)
+            m["gmax"][e] = np.maximum(g.max(axis=0), g.min(axis=0) + 0.5)
     F = M.ForceNNP(_engine_model(M, m),
                    M.PREC_FP64 if prec == "fp32" else M.PREC_MIXED)
     F.compute(s, nl)
     f = s.download()[2][:len(x)]
     G, _, E = F.atomic(s, 96)
-    off, idx = nl.get()
     _, Eo, Go, _, fo = to_oracle(O, m).compute(s.download()[0], t, len(x), off,
                                                idx, ld=96)
     for e in range(nelem):
@@ -97,3 +107,27 @@ def test_network_input_widths(gpu, neta, prec):
     etas = [0.02 * (k + 1) for k in range(neta)]
     x, t = _cluster(50, 2, neta)
     _check(gpu, _model(2, etas, pl, hidden=(32, 1)), x, t, prec)
+
+
+POW2 = [(z, lam) for lam in (1.0, -1.0) for z in (16.0, 1.0, 4.0, 2.0)]
+
+
+@pytest.mark.parametrize("neta", range(1, 9))
+def test_power_of_two_grid(gpu, neta):
+    """zeta 1, 2, 4, 16 with both lambdas (the squaring kernels), one to
+    eight etas, functions in any order; 15 to 20 neighbours per atom."""
+    etas = [0.02 * (k + 1) for k in range(neta)]
+    x, t = _cluster(60, 2, 100 + neta)
+    _check(gpu, _model(2, etas, POW2), x, t, "bf16")
+
+
+@pytest.mark.parametrize("n", [2, 3, 64, 65, 66, 100, 129])
+@pytest.mark.parametrize("pl", ["pow2", "general"])
+def test_neighbour_counts(gpu, n, pl):
+    """Every atom of the cluster a neighbour of every other: 1, 2, 63, 64, 65
+    and 128 neighbours, where the pair walk changes form and the buffer of
+    pairs is emptied one or more times."""
+    x, t = _cluster(n, 1, n)
+    x = BOX / 2 + (x - BOX / 2) * min(1.0, 4.0 / np.ptp(x, axis=0).max())
+    m = _model(1, (0.01, 0.05), POW2 if pl == "pow2" else PL, rc=8.0)
+    _check(gpu, m, x, t, "fp32")
