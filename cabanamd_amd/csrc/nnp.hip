@@ -60,7 +60,7 @@ static constexpr int NSF_LD = 96;              // row stride of G / dE/dG
 static constexpr int KPAD = 96;                // MFMA K of layer 1 (6 x 16)
 static constexpr int HPAD = 32;                // hidden width (2 x 16)
 static constexpr int NN_MAX = 128;             // neighbours inside rc
-static constexpr int TCAP = 1024;              // compacted neighbour pairs per wave
+static constexpr int TCAP = 512;               // compacted neighbour pairs per wave
 static constexpr int NNP_TPB = 256;
 // The (lambda, zeta) grid of zeta = 1, 2, 4, 16 and both signs of lambda:
 // its powers are a few squarings, so it has kernels of its own.  Entry p:
@@ -651,13 +651,13 @@ __device__ __forceinline__ void pair_of( int p, int n, int &a, int &q )
 
 // The neighbour pairs (a < q) of the gathered list whose third side is
 // inside the cutoff, |x_q - x_a| < rc: tested 64 at a time and compacted
-// into buf (TCAP entries per wave, a | q << 8; NN_MAX <= 256), then handed to body(a, q)
+// into buf (CAP entries per wave, a | q << 8; NN_MAX <= 256), then handed to body(a, q)
 // with every lane busy (lane l takes entries l*per .. l*per + per - 1).
 // Used where the body keeps many accumulators in registers.
 // With PAIRS the body takes two pairs at once, (a0, q0) and (a1, q1), the
 // second valid when ok1 (else a repeat of the first): the two gradient
 // chains are independent, so their latencies overlap.
-template <bool PAIRS = false, class Body>
+template <bool PAIRS = false, int CAP = TCAP, class Body>
 __device__ __forceinline__ void for_triplets( const NbLds &L, int n, float rc2,
                                              unsigned short *buf, Body body,
                                              int *count = nullptr )
@@ -672,7 +672,7 @@ __device__ __forceinline__ void for_triplets( const NbLds &L, int n, float rc2,
     for ( int it = 0; it < nit; )
     {
         int cnt = 0;
-        while ( cnt <= TCAP - 64 && it < nit )
+        while ( cnt <= CAP - 64 && it < nit )
         {
             bool ok = false;
             unsigned short code = 0;
@@ -751,6 +751,110 @@ __device__ __forceinline__ void for_triplets( const NbLds &L, int n, float rc2,
         }
         __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
     }
+}
+
+// Walk of the neighbour pairs of an atom with n <= 64 neighbours whose third
+// side is inside the cutoff, with every lane busy and no atomics.  Row d
+// (1 <= d <= n / 2) pairs neighbour l with neighbour (l + d) mod n in lane l,
+// so a row's test reads the partners from consecutive LDS records and its
+// valid pairs are one 64-bit mask.  The valid pairs of consecutive rows are
+// compacted into a ring of PAIR_RING codes; step(slot, l, p) runs on 64 of
+// them at a time.  Once all pairs of a row are done, row(d, mask, start) may
+// collect what step left at ring slots start, start + 1, ... (one per mask
+// bit in lane order) -- each neighbour meets each of its pairs there in its
+// own lane, which replaces reactions added with LDS atomics: at 192,000 atoms
+// those took half of the force kernel's 3794 us, which the ring, the matrix
+// products of the coefficients (k_nnp_force_pow) and six blocks per CU brought
+// to 1795 us, 87 % of them VALU issue; the symmetry functions, which use the
+// steps alone, went from 996 to 893 us.
+constexpr int PAIR_RING = 256;
+
+// set bits of m below the lane's
+__device__ __forceinline__ int lanes_below( unsigned long long m )
+{
+    return (int)__builtin_amdgcn_mbcnt_hi( (unsigned)( m >> 32 ),
+                                           __builtin_amdgcn_mbcnt_lo( (unsigned)m, 0u ) );
+}
+
+// the partner (l + d) mod n, for l < n and d < n
+__device__ __forceinline__ int pair_partner( int l, int d, int n )
+{
+    const int p = l + d;
+    return p >= n ? p - n : p;
+}
+
+// Without ROWS only the steps run (row is not called).
+template <bool ROWS, class Step, class Row>
+__device__ __forceinline__ int pair_ring( const NbLds &L, int n, float rc2,
+                                          unsigned short *code, Step step, Row row )
+{
+    const int lane = threadIdx.x & 63;
+    const int nrow = n / 2;
+    const float4 own = L.d[lane]; // lanes past n are masked out
+    // prod pairs compacted, comp of them stepped; rows below made are
+    // compacted, rows below done are collected and first is where row done
+    // starts: a ring slot is reused only after its row is collected
+    int prod = 0, comp = 0, made = 1, done = 1, first = 0;
+    int mlo = 0, mhi = 0, mst = 0; // row d's mask and start in lane d - 1
+    while ( ROWS ? done <= nrow : ( made <= nrow || comp < prod ) )
+    {
+        if ( !ROWS )
+            first = comp;
+        while ( made <= nrow && prod - first <= PAIR_RING - 64 )
+        {
+            const int p = pair_partner( lane, made, n );
+            // the middle row of an even n holds each pair once in its first
+            // half
+            const int lim = 2 * made == n ? made : n;
+            bool ok = false;
+            if ( lane < lim )
+            {
+                const float4 B = L.d[p];
+                const float cx = B.x - own.x, cy = B.y - own.y, cz = B.z - own.z;
+                ok = cx * cx + cy * cy + cz * cz < rc2;
+            }
+            const unsigned long long m = __ballot( ok );
+            if ( ok )
+                code[( prod + lanes_below( m ) ) & ( PAIR_RING - 1 )] =
+                    (unsigned short)( lane | ( p << 8 ) );
+            if ( ROWS )
+            {
+                const bool mine = lane == made - 1;
+                mlo = mine ? (int)m : mlo;
+                mhi = mine ? (int)( m >> 32 ) : mhi;
+                mst = mine ? prod : mst;
+            }
+            prod += (int)__popcll( m );
+            ++made;
+        }
+        __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
+        while ( prod - comp >= 64 || ( made > nrow && comp < prod ) )
+        {
+            const int e = comp + lane;
+            if ( e < prod )
+            {
+                const int slot = e & ( PAIR_RING - 1 );
+                const unsigned c = code[slot];
+                step( slot, (int)( c & 0xffu ), (int)( c >> 8 ) );
+            }
+            comp = min( comp + 64, prod );
+        }
+        __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
+        while ( ROWS && done < made )
+        {
+            const unsigned lo = __builtin_amdgcn_readlane( mlo, done - 1 ),
+                           hi = __builtin_amdgcn_readlane( mhi, done - 1 );
+            const unsigned long long mu = lo | ( (unsigned long long)hi << 32 );
+            first = __builtin_amdgcn_readlane( mst, done - 1 );
+            const int end = first + (int)__popcll( mu );
+            if ( end > comp )
+                break;
+            row( done, mu, first );
+            first = end;
+            ++done;
+        }
+    }
+    return prod;
 }
 
 // Radial symmetry functions of one atom, lanes over its neighbours.
@@ -945,31 +1049,35 @@ __global__ __launch_bounds__( NNP_TPB ) void k_nnp_sf_pow(
 #pragma unroll
     for ( int s = 0; s < NA_MAX; ++s )
         acc[s] = 0.0f;
+    auto triplet = [&]( int a, int q )
+    {
+        const float4 A = L.d[a], B = L.d[q], Ea = L.e[a], Eb = L.e[q];
+        const float cx = B.x - A.x, cy = B.y - A.y, cz = B.z - A.z;
+        const float c2 = cx * cx + cy * cy + cz * cz;
+        const float f3 =
+            0.5f + 0.5f * __builtin_amdgcn_cosf( __builtin_amdgcn_sqrtf( c2 ) * kcos );
+        const float F = Ea.y * Eb.y * f3;
+        const float cs = ( A.x * B.x + A.y * B.y + A.z * B.z ) * ( Ea.x * Eb.x );
+        const float s2 = A.w * A.w + ( B.w * B.w + c2 );
+        float Pw[POW_NAP];
+        pow_grid( fmaxf( 1.0f - cs, 0.0f ), Pw );
+        pow_grid( fmaxf( 1.0f + cs, 0.0f ), Pw + 4 );
+#pragma unroll
+        for ( int g = 0; g < NAG; ++g )
+        {
+            const float EgF = __builtin_amdgcn_exp2f( ke[g] * s2 ) * F;
+#pragma unroll
+            for ( int pp = 0; pp < POW_NAP; ++pp )
+                acc[g * AP_MAX + pp] += EgF * Pw[pp];
+        }
+    };
     int ntrip = 0;
-    for_triplets(
-        L, n, rc2, tbuf[wv],
-        [&]( int a, int q ) {
-            const float4 A = L.d[a], B = L.d[q], Ea = L.e[a], Eb = L.e[q];
-            const float cx = B.x - A.x, cy = B.y - A.y, cz = B.z - A.z;
-            const float c2 = cx * cx + cy * cy + cz * cz;
-            const float f3 =
-                0.5f + 0.5f * __builtin_amdgcn_cosf( __builtin_amdgcn_sqrtf( c2 ) * kcos );
-            const float F = Ea.y * Eb.y * f3;
-            const float cs = ( A.x * B.x + A.y * B.y + A.z * B.z ) * ( Ea.x * Eb.x );
-            const float s2 = A.w * A.w + ( B.w * B.w + c2 );
-            float Pw[POW_NAP];
-            pow_grid( fmaxf( 1.0f - cs, 0.0f ), Pw );
-            pow_grid( fmaxf( 1.0f + cs, 0.0f ), Pw + 4 );
-#pragma unroll
-            for ( int g = 0; g < NAG; ++g )
-            {
-                const float EgF = __builtin_amdgcn_exp2f( ke[g] * s2 ) * F;
-#pragma unroll
-                for ( int pp = 0; pp < POW_NAP; ++pp )
-                    acc[g * AP_MAX + pp] += EgF * Pw[pp];
-            }
-        },
-        &ntrip );
+    if ( n <= 64 )
+        ntrip = pair_ring<false>(
+            L, n, rc2, tbuf[wv], [&]( int, int a, int q ) { triplet( a, q ); },
+            []( int, unsigned long long, int ) {} );
+    else
+        for_triplets( L, n, rc2, tbuf[wv], triplet, &ntrip );
     // the work model's term counts, as in k_nnp_sf
     if ( terms && lane == 0 )
         terms[i] = make_int4( n, ntrip, e, 0 );
@@ -1530,6 +1638,26 @@ __global__ __launch_bounds__( NNP_TPB ) void k_nnp_force(
     }
 }
 
+// LDS of a wave's pair walk beyond its neighbours'.  Up to 64 neighbours
+// leave the upper halves of L.d and L.e free: the ring's records (pa, pm,
+// pb) lie there and here, which keeps five blocks on a CU.
+union ForceBuf
+{
+    float coef[NSF_LD];
+    struct
+    {
+        float pb[PAIR_RING];
+        unsigned short code[PAIR_RING];
+    } ring;
+    struct
+    {
+        float f[NN_MAX][3];
+        unsigned short code[PAIR_RING];
+    } flat;
+};
+static_assert( PAIR_RING * sizeof( float ) == ( NN_MAX - 64 ) * sizeof( float4 ),
+               "a ring of floats fits the upper half of L.d" );
+
 // Forces of the power-of-two grid (see k_nnp_sf_pow).  With T = sum_s c_s
 // T_s of a triplet (i, a, q), A = x_a - x_i and B = x_q - x_i, the gradients
 // are combinations of A and B alone,
@@ -1542,16 +1670,14 @@ __global__ __launch_bounds__( NNP_TPB ) void k_nnp_force(
 // component.  The atom's own force is minus the sum of its neighbours'
 // reactions.
 template <int NAG>
-__global__ __launch_bounds__( NNP_TPB ) void k_nnp_force_pow(
+__global__ __launch_bounds__( NNP_TPB, 5 ) void k_nnp_force_pow(
     int n_local, int fcap, const double4 *__restrict__ x,
     const int64_t *__restrict__ off, const int *__restrict__ idx,
     const NnpPlan *__restrict__ P, const float *__restrict__ dEdG,
     double *__restrict__ f, int *__restrict__ flag )
 {
     __shared__ NbLds lds[NNP_TPB / 64];
-    __shared__ float sF[NNP_TPB / 64][NN_MAX][3];
-    __shared__ float sC[NNP_TPB / 64][NSF_LD];
-    __shared__ unsigned short tbuf[NNP_TPB / 64][TCAP];
+    __shared__ ForceBuf buf[NNP_TPB / 64];
     const int wv = __builtin_amdgcn_readfirstlane( threadIdx.x >> 6 ), lane = threadIdx.x & 63;
     const int i = blockIdx.x * ( NNP_TPB / 64 ) + wv;
     if ( i >= n_local )
@@ -1561,53 +1687,50 @@ __global__ __launch_bounds__( NNP_TPB ) void k_nnp_force_pow(
     const int n = gather_neighbours( i, x, off, idx, rc, rc2, kpi, L, flag );
     const int e = __builtin_amdgcn_readfirstlane( (int)x[i].w );
     const NnpElemPlan &Q = P->el[e];
-    const float *c = sC[wv];
+    // dE/dG of the atom, in LDS until the coefficients below are read
+    float *c = buf[wv].coef;
     for ( int k = lane; k < NSF_LD; k += 64 )
-        sC[wv][k] = k < Q.nsf ? dEdG[(size_t)i * NSF_LD + k] : 0.f;
+        c[k] = k < Q.nsf ? dEdG[(size_t)i * NSF_LD + k] : 0.f;
     __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
-    // the radial reactions start each neighbour's sum; e.z becomes fc' / r
-    for ( int a = lane; a < n; a += 64 )
+    // the radial factors, kept for the end; e.z becomes fc' / r, d.w r^2
+    float srad[NN_MAX / 64];
+#pragma unroll
+    for ( int u = 0; u < NN_MAX / 64; ++u )
     {
-        const float4 A = L.d[a];
-        const float s = radial_force( Q, L, a, c );
-        sF[wv][a][0] = -s * A.x;
-        sF[wv][a][1] = -s * A.y;
-        sF[wv][a][2] = -s * A.z;
-        L.e[a].z *= L.e[a].x;
+        const int a = lane + 64 * u;
+        srad[u] = 0.f;
+        if ( a < n )
+        {
+            srad[u] = radial_force( Q, L, a, c );
+            L.e[a].z *= L.e[a].x;
+            L.d[a].w *= L.d[a].w;
+        }
     }
-    // lane g * 8 + p holds c_gp 2^(1 - zeta_p); exp(-eta s) = exp2(k s)
-    const int lg = lane / AP_MAX, lp = lane % AP_MAX;
-    const float cl = lg < NAG ? c[Q.a_out[lg][lp]] * __builtin_amdgcn_exp2f( Q.a_lpref[lp] ) : 0.f;
+    // the coefficients as rows of 4x4x1 MFMAs: lane l holds row l % 4, that
+    // is c_gp 2^(1 - zeta_p) for p = l % 4 (half 0) and 4 + l % 4 (half 1);
+    // exp(-eta s) = exp2(k s)
     const float kl = -1.44269504f * Q.a_eta[lane & ( AG_MAX - 1 )];
     const float ml = -2.0f * Q.a_eta[lane & ( AG_MAX - 1 )];
-    float cg[NAG][POW_NAP], ke[NAG], me[NAG];
+    float ct[NAG][2], ke[NAG], me[NAG];
 #pragma unroll
     for ( int g = 0; g < NAG; ++g )
     {
         ke[g] = lane_value( kl, g );
         me[g] = lane_value( ml, g );
 #pragma unroll
-        for ( int pp = 0; pp < POW_NAP; ++pp )
-            cg[g][pp] = lane_value( cl, g * AP_MAX + pp );
+        for ( int h = 0; h < 2; ++h )
+        {
+            const int pp = 4 * h + ( lane & 3 );
+            ct[g][h] = c[Q.a_out[g][pp]] * __builtin_amdgcn_exp2f( Q.a_lpref[pp] );
+        }
     }
     __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
     const float krev = 0.5f / rc; // pi r / rc in revolutions
     const float kd = -0.5f * kpi;
-    // each lane takes a contiguous block of the compacted (a-major) pair
-    // list: the sums of pa and pm B of the row atom stay in registers until
-    // a changes, the reaction on q goes to LDS
-    int cur = -1;
-    float spa = 0.f, bx = 0.f, by = 0.f, bz = 0.f;
-    auto flush = [&]()
+    // pa, pb and pm of the triplet (i, a, q)
+    auto grad = [&]( const float4 &A, const float4 &B, const float4 &Ea, const float4 &Eb,
+                     float &pa, float &pb, float &pm )
     {
-        const float4 A = L.d[cur];
-        atomicAdd( &sF[wv][cur][0], -( spa * A.x + bx ) );
-        atomicAdd( &sF[wv][cur][1], -( spa * A.y + by ) );
-        atomicAdd( &sF[wv][cur][2], -( spa * A.z + bz ) );
-    };
-    for_triplets( L, n, rc2, tbuf[wv], [&]( int a, int q ) {
-        const float4 A = L.d[a], Ea = L.e[a];
-        const float4 B = L.d[q], Eb = L.e[q];
         const float cx = B.x - A.x, cy = B.y - A.y, cz = B.z - A.z;
         const float c2 = cx * cx + cy * cy + cz * cz;
         const float ic = __builtin_amdgcn_rsqf( c2 );
@@ -1617,73 +1740,165 @@ __global__ __launch_bounds__( NNP_TPB ) void k_nnp_force_pow(
         const float f12 = Ea.y * Eb.y, F = f12 * f3;
         const float inv12 = Ea.x * Eb.x;
         const float cs = ( A.x * B.x + A.y * B.y + A.z * B.z ) * inv12;
-        const float s2 = A.w * A.w + ( B.w * B.w + c2 );
-        // S_g = sum_p c_gp P_p and T_p = sum_g c_gp E_g
-        float Pw[POW_NAP], T[POW_NAP];
+        const float s2 = A.w + B.w + c2;
+        float Pw[POW_NAP];
         const float bm = fmaxf( 1.0f - cs, 0.0f ), bp = fmaxf( 1.0f + cs, 0.0f );
         pow_grid( bm, Pw );
         pow_grid( bp, Pw + 4 );
-#pragma unroll
-        for ( int pp = 0; pp < POW_NAP; ++pp )
-            T[pp] = 0.f;
-        float S = 0.f, Mg = 0.f;
+        // T_p = sum_g c_gp E_g and U_p = sum_g -2 eta_g c_gp E_g on the FP32
+        // matrix cores: in 16 blocks of 4 x 4 with the coefficients as rows
+        // and the Gaussians as columns, lane l is column l % 4 of block
+        // l / 4 and receives its own triplet's four sums, so no operand
+        // changes lanes (a lane outside the exec mask fills only its own)
+        f32x4 T[2] = { { 0.f, 0.f, 0.f, 0.f }, { 0.f, 0.f, 0.f, 0.f } }, U[2] = { T[0], T[0] };
 #pragma unroll
         for ( int g = 0; g < NAG; ++g )
         {
-            const float Eg = __builtin_amdgcn_exp2f( ke[g] * s2 );
-            float sg = 0.f;
+            const float Eg = __builtin_amdgcn_exp2f( ke[g] * s2 ), Mg = me[g] * Eg;
 #pragma unroll
-            for ( int pp = 0; pp < POW_NAP; ++pp )
+            for ( int h = 0; h < 2; ++h )
             {
-                sg = fmaf( cg[g][pp], Pw[pp], sg );
-                T[pp] = fmaf( cg[g][pp], Eg, T[pp] );
+                T[h] = __builtin_amdgcn_mfma_f32_4x4x1f32( ct[g][h], Eg, T[h], 0, 0, 0 );
+                U[h] = __builtin_amdgcn_mfma_f32_4x4x1f32( ct[g][h], Mg, U[h], 0, 0, 0 );
             }
-            const float w = sg * Eg;
-            S += w;
-            Mg = fmaf( me[g], w, Mg );
         }
-        // T' = sum_p T_p zeta lambda b^(zeta - 1), b^3 and b^15 from the grid
+        // S = sum_p T_p P_p, M = sum_p U_p P_p and T' = sum_p T_p zeta lambda
+        // b^(zeta - 1), b^3 and b^15 from the grid
+        float S = 0.f, Mg = 0.f;
+#pragma unroll
+        for ( int u = 0; u < 4; ++u )
+        {
+            S = fmaf( T[1][u], Pw[4 + u], fmaf( T[0][u], Pw[u], S ) );
+            Mg = fmaf( U[1][u], Pw[4 + u], fmaf( U[0][u], Pw[u], Mg ) );
+        }
         const float m3 = Pw[1] * bm, p3 = Pw[5] * bp;
         const float m15 = Pw[2] * Pw[2] * Pw[2] * m3, p15 = Pw[6] * Pw[6] * Pw[6] * p3;
-        float Td = T[4] - T[0];
-        Td = fmaf( 2.f, T[5] * bp - T[1] * bm, Td );
-        Td = fmaf( 4.f, T[6] * p3 - T[2] * m3, Td );
-        Td = fmaf( 16.f, T[7] * p15 - T[3] * m15, Td );
+        float Td = T[1][0] - T[0][0];
+        Td = fmaf( 2.f, T[1][1] * bp - T[0][1] * bm, Td );
+        Td = fmaf( 4.f, T[1][2] * p3 - T[0][2] * m3, Td );
+        Td = fmaf( 16.f, T[1][3] * p15 - T[0][3] * m15, Td );
         const float X = F * Td, FM = F * Mg;
         const float s3 = fmaf( S * f12, d3, FM );
-        const float pm = fmaf( X, inv12, -s3 );
         const float Xc = X * cs, Sf3 = S * f3, base = FM + s3;
-        const float pa = fmaf( Sf3 * Eb.y, Ea.z, fmaf( -Xc * Ea.x, Ea.x, base ) );
-        const float pb = fmaf( Sf3 * Ea.y, Eb.z, fmaf( -Xc * Eb.x, Eb.x, base ) );
-        if ( a != cur )
-        {
-            if ( cur >= 0 )
-                flush();
-            cur = a;
-            spa = bx = by = bz = 0.f;
-        }
-        spa += pa;
-        bx = fmaf( pm, B.x, bx );
-        by = fmaf( pm, B.y, by );
-        bz = fmaf( pm, B.z, bz );
-        atomicAdd( &sF[wv][q][0], -fmaf( pb, B.x, pm * A.x ) );
-        atomicAdd( &sF[wv][q][1], -fmaf( pb, B.y, pm * A.y ) );
-        atomicAdd( &sF[wv][q][2], -fmaf( pb, B.z, pm * A.z ) );
-    } );
-    if ( cur >= 0 )
-        flush();
-    __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
+        pm = fmaf( X, inv12, -s3 );
+        pa = fmaf( Sf3 * Eb.y, Ea.z, fmaf( -Xc * Ea.x, Ea.x, base ) );
+        pb = fmaf( Sf3 * Ea.y, Eb.z, fmaf( -Xc * Eb.x, Eb.x, base ) );
+    };
     float fix = 0.f, fiy = 0.f, fiz = 0.f;
-    for ( int a = lane; a < n; a += 64 )
+    auto finish = [&]( int a, float rx, float ry, float rz )
     {
         const int j = L.j[a];
-        const float rx = sF[wv][a][0], ry = sF[wv][a][1], rz = sF[wv][a][2];
         fix -= rx;
         fiy -= ry;
         fiz -= rz;
         unsafeAtomicAdd( &f[j], (double)rx );
         unsafeAtomicAdd( &f[fcap + j], (double)ry );
         unsafeAtomicAdd( &f[2 * fcap + j], (double)rz );
+    };
+    if ( n <= 64 )
+    {
+        float *rpa = reinterpret_cast<float *>( L.d + 64 ),
+              *rpm = reinterpret_cast<float *>( L.e + 64 ), *rpb = buf[wv].ring.pb;
+        // of the lane's neighbour: sum of its pa (or pb), sum of pm X_partner
+        float sp = srad[0], sx = 0.f, sy = 0.f, sz = 0.f;
+        pair_ring<true>(
+            L, n, rc2, buf[wv].ring.code,
+            [&]( int slot, int a, int q ) {
+                float pa, pb, pm;
+                grad( L.d[a], L.d[q], L.e[a], L.e[q], pa, pb, pm );
+                rpa[slot] = pa;
+                rpm[slot] = pm;
+                rpb[slot] = pb;
+            },
+            [&]( int d, unsigned long long m, int s0 ) {
+                // as the pair's first neighbour, the partner d further on
+                if ( __builtin_amdgcn_inverse_ballot_w64( m ) )
+                {
+                    const int k = ( s0 + lanes_below( m ) ) & ( PAIR_RING - 1 );
+                    const float4 X = L.d[pair_partner( lane, d, n )];
+                    const float w = rpm[k];
+                    sp += rpa[k];
+                    sx = fmaf( w, X.x, sx );
+                    sy = fmaf( w, X.y, sy );
+                    sz = fmaf( w, X.z, sz );
+                }
+                // as its second, the first neighbour p d before: lanes from
+                // d on have p = lane - d, those below p = lane - d + n, so
+                // the row's mask turns by d within n bits
+                const unsigned long long up = m << d, wrap = m >> ( n - d );
+                const unsigned long long turned =
+                    ( up & ( ~0ull >> ( 64 - n ) ) ) | wrap;
+                if ( __builtin_amdgcn_inverse_ballot_w64( turned ) )
+                {
+                    const int nw = (int)__popcll( wrap );
+                    const int before = s0 + ( lane >= d ? -nw : (int)__popcll( m ) - nw );
+                    const int k = ( before + lanes_below( turned ) ) & ( PAIR_RING - 1 );
+                    const float4 X = L.d[pair_partner( lane, n - d, n )];
+                    const float w = rpm[k];
+                    sp += rpb[k];
+                    sx = fmaf( w, X.x, sx );
+                    sy = fmaf( w, X.y, sy );
+                    sz = fmaf( w, X.z, sz );
+                }
+            } );
+        if ( lane < n )
+        {
+            const float4 A = L.d[lane];
+            finish( lane, -fmaf( sp, A.x, sx ), -fmaf( sp, A.y, sy ), -fmaf( sp, A.z, sz ) );
+        }
+    }
+    else
+    {
+        // more neighbours than lanes: each lane takes a contiguous block of
+        // the compacted (a-major) pair list, the sums of pa and pm B of the
+        // row atom stay in registers until a changes and the reaction on q
+        // goes to LDS
+        float( *sF )[3] = buf[wv].flat.f;
+        for ( int a = lane; a < n; a += 64 )
+            sF[a][0] = sF[a][1] = sF[a][2] = 0.f;
+        __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
+        int cur = -1;
+        float spa = 0.f, bx = 0.f, by = 0.f, bz = 0.f;
+        auto flush = [&]()
+        {
+            const float4 A = L.d[cur];
+            atomicAdd( &sF[cur][0], -( spa * A.x + bx ) );
+            atomicAdd( &sF[cur][1], -( spa * A.y + by ) );
+            atomicAdd( &sF[cur][2], -( spa * A.z + bz ) );
+        };
+        for_triplets<false, PAIR_RING>( L, n, rc2, buf[wv].flat.code, [&]( int a, int q ) {
+            const float4 A = L.d[a], B = L.d[q];
+            float pa, pb, pm;
+            grad( A, B, L.e[a], L.e[q], pa, pb, pm );
+            if ( a != cur )
+            {
+                if ( cur >= 0 )
+                    flush();
+                cur = a;
+                spa = bx = by = bz = 0.f;
+            }
+            spa += pa;
+            bx = fmaf( pm, B.x, bx );
+            by = fmaf( pm, B.y, by );
+            bz = fmaf( pm, B.z, bz );
+            atomicAdd( &sF[q][0], -fmaf( pb, B.x, pm * A.x ) );
+            atomicAdd( &sF[q][1], -fmaf( pb, B.y, pm * A.y ) );
+            atomicAdd( &sF[q][2], -fmaf( pb, B.z, pm * A.z ) );
+        } );
+        if ( cur >= 0 )
+            flush();
+        __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
+#pragma unroll
+        for ( int u = 0; u < NN_MAX / 64; ++u )
+        {
+            const int a = lane + 64 * u;
+            if ( a < n )
+            {
+                const float4 A = L.d[a];
+                finish( a, fmaf( -srad[u], A.x, sF[a][0] ), fmaf( -srad[u], A.y, sF[a][1] ),
+                        fmaf( -srad[u], A.z, sF[a][2] ) );
+            }
+        }
     }
 #pragma unroll
     for ( int o = 32; o > 0; o >>= 1 )
