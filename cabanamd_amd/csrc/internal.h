@@ -457,7 +457,12 @@ cmd_status lj_energy_virial( const cmd_force *F, cmd_system *S,
                              const cmd_neigh *N, double *pe, double *w );
 
 // NNP force (nnp.hip)
-cmd_status nnp_compute( cmd_nnp *M, cmd_system *S, cmd_neigh *N );
+// check: wait for the result and report an atom with too many neighbours; a
+// time loop passes false and brackets its calls with nnp_check_begin and
+// nnp_check_end, so that its steps queue without a host wait.
+cmd_status nnp_compute( cmd_nnp *M, cmd_system *S, cmd_neigh *N, bool check = true );
+cmd_status nnp_check_begin( cmd_nnp *M, hipStream_t st );
+cmd_status nnp_check_end( cmd_nnp *M, hipStream_t st );
 cmd_status nnp_reference_energy( cmd_nnp *M, cmd_system *S, double *pe );
 cmd_status nnp_energy_sum( cmd_nnp *M, cmd_system *S, double *sum );
 // Atomic energies E_i of the last compute as FP64 into out[0..n) (device).

@@ -654,13 +654,14 @@ __device__ __forceinline__ void pair_of( int p, int n, int &a, int &q )
 // into buf (CAP entries per wave, a | q << 8; NN_MAX <= 256), then handed to body(a, q)
 // with every lane busy (lane l takes entries l*per .. l*per + per - 1).
 // Used where the body keeps many accumulators in registers.
+// A wave that shares the atom with others takes every its-th test from it0.
 // With PAIRS the body takes two pairs at once, (a0, q0) and (a1, q1), the
 // second valid when ok1 (else a repeat of the first): the two gradient
 // chains are independent, so their latencies overlap.
 template <bool PAIRS = false, int CAP = TCAP, class Body>
 __device__ __forceinline__ void for_triplets( const NbLds &L, int n, float rc2,
                                              unsigned short *buf, Body body,
-                                             int *count = nullptr )
+                                             int *count = nullptr, int it0 = 0, int its = 1 )
 {
     const int lane = threadIdx.x & 63;
     // candidate pairs, 64 per test: with n <= 64 rows a and n - 2 - a side
@@ -669,7 +670,7 @@ __device__ __forceinline__ void for_triplets( const NbLds &L, int n, float rc2,
     const bool rows = n <= 64;
     const int np = n * ( n - 1 ) / 2;
     const int nit = rows ? n / 2 : ( np + 63 ) / 64; // rows: pairs of rows
-    for ( int it = 0; it < nit; )
+    for ( int it = it0; it < nit; )
     {
         int cnt = 0;
         while ( cnt <= CAP - 64 && it < nit )
@@ -716,7 +717,7 @@ __device__ __forceinline__ void for_triplets( const NbLds &L, int n, float rc2,
                               (unsigned)( m >> 32 ),
                               __builtin_amdgcn_mbcnt_lo( (unsigned)m, 0u ) )] = code;
             cnt += (int)__popcll( m );
-            ++it;
+            it += its;
         }
         __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
         if ( count )
@@ -783,29 +784,32 @@ __device__ __forceinline__ int pair_partner( int l, int d, int n )
     return p >= n ? p - n : p;
 }
 
-// Without ROWS only the steps run (row is not called).
-template <bool ROWS, class Step, class Row>
-__device__ __forceinline__ int pair_ring( const NbLds &L, int n, float rc2,
+// Without ROWS only the steps run (row is not called).  With WPA waves on an
+// atom, wave `part` takes the rows part + 1, part + 1 + WPA, ...
+template <bool ROWS, int WPA, class Step, class Row>
+__device__ __forceinline__ int pair_ring( const NbLds &L, int n, float rc2, int part,
                                           unsigned short *code, Step step, Row row )
 {
     const int lane = threadIdx.x & 63;
-    const int nrow = n / 2;
+    const int nrow = ( n / 2 + WPA - 1 - part ) / WPA; // this wave's rows
     const float4 own = L.d[lane]; // lanes past n are masked out
     // prod pairs compacted, comp of them stepped; rows below made are
     // compacted, rows below done are collected and first is where row done
     // starts: a ring slot is reused only after its row is collected
     int prod = 0, comp = 0, made = 1, done = 1, first = 0;
-    int mlo = 0, mhi = 0, mst = 0; // row d's mask and start in lane d - 1
+    int mlo = 0, mhi = 0, mst = 0; // the k-th row's mask and start in lane k - 1
+    auto row_d = [&]( int k ) { return part + 1 + WPA * ( k - 1 ); };
     while ( ROWS ? done <= nrow : ( made <= nrow || comp < prod ) )
     {
         if ( !ROWS )
             first = comp;
         while ( made <= nrow && prod - first <= PAIR_RING - 64 )
         {
-            const int p = pair_partner( lane, made, n );
+            const int d = row_d( made );
+            const int p = pair_partner( lane, d, n );
             // the middle row of an even n holds each pair once in its first
             // half
-            const int lim = 2 * made == n ? made : n;
+            const int lim = 2 * d == n ? d : n;
             bool ok = false;
             if ( lane < lim )
             {
@@ -849,7 +853,7 @@ __device__ __forceinline__ int pair_ring( const NbLds &L, int n, float rc2,
             const int end = first + (int)__popcll( mu );
             if ( end > comp )
                 break;
-            row( done, mu, first );
+            row( row_d( done ), mu, first );
             first = end;
             ++done;
         }
@@ -894,6 +898,24 @@ __device__ __forceinline__ void radial_sf( const NnpElemPlan &Q, const NbLds &L,
     }
 }
 
+// f = 0 over the nt local and ghost rows and the G columns past the atom's
+// functions, by the first kernel of a force call (no launches of their own).
+__device__ __forceinline__ void zero_forces( double *__restrict__ f, int fcap, int nt )
+{
+    for ( int k = blockIdx.x * blockDim.x + threadIdx.x; k < nt; k += gridDim.x * blockDim.x )
+    {
+        f[k] = 0.0;
+        f[fcap + k] = 0.0;
+        f[2 * fcap + k] = 0.0;
+    }
+}
+
+__device__ __forceinline__ void zero_tail( const NnpElemPlan &Q, float *__restrict__ Gi )
+{
+    for ( int k = Q.nsf + ( threadIdx.x & 63 ); k < NSF_LD; k += 64 )
+        Gi[k] = 0.f;
+}
+
 // NAG, NAP > 0: the angular (eta, rs) and (lambda, zeta) grid sizes of
 // every element, fixed at compile time (loops unrolled straight); 0: read
 // from the plan.  RS0: every element's angular rs are 0, so the Gaussian
@@ -904,12 +926,14 @@ template <int NAG, int NAP, bool RS0>
 __global__ __launch_bounds__( NNP_TPB ) void k_nnp_sf(
     int n_local, const double4 *__restrict__ x, const int64_t *__restrict__ off,
     const int *__restrict__ idx, const NnpPlan *__restrict__ P,
-    float *__restrict__ G, int *__restrict__ flag, int4 *__restrict__ terms )
+    float *__restrict__ G, int *__restrict__ flag, int4 *__restrict__ terms,
+    double *__restrict__ f, int fcap, int nt )
 {
     __shared__ NbLds lds[NNP_TPB / 64];
     __shared__ unsigned short tbuf[NNP_TPB / 64][TCAP];
     __shared__ float kst[NNP_TPB / 64][64];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    zero_forces( f, fcap, nt );
     const int i = blockIdx.x * ( NNP_TPB / 64 ) + wv;
     if ( i >= n_local )
         return;
@@ -924,6 +948,7 @@ __global__ __launch_bounds__( NNP_TPB ) void k_nnp_sf(
     if constexpr ( NAP > 0 )
         K.nap = NAP;
     float *Gi = G + (size_t)i * NSF_LD;
+    zero_tail( Q, Gi );
     radial_sf( Q, L, n, Gi );
     // angular: lanes over the compacted neighbour pairs
     {
@@ -1019,16 +1044,20 @@ __device__ __forceinline__ void pow_grid( float b, float *p )
     p[3] = b8 * b8;
 }
 
-template <int NAG>
+template <int NAG, int WPA>
 __global__ __launch_bounds__( NNP_TPB ) void k_nnp_sf_pow(
     int n_local, const double4 *__restrict__ x, const int64_t *__restrict__ off,
     const int *__restrict__ idx, const NnpPlan *__restrict__ P,
-    float *__restrict__ G, int *__restrict__ flag, int4 *__restrict__ terms )
+    float *__restrict__ G, int *__restrict__ flag, int4 *__restrict__ terms,
+    double *__restrict__ f, int fcap, int nt )
 {
     __shared__ NbLds lds[NNP_TPB / 64];
     __shared__ unsigned short tbuf[NNP_TPB / 64][TCAP];
     const int wv = __builtin_amdgcn_readfirstlane( threadIdx.x >> 6 ), lane = threadIdx.x & 63;
-    const int i = blockIdx.x * ( NNP_TPB / 64 ) + wv;
+    zero_forces( f, fcap, nt );
+    // with WPA = 4 the block's waves share an atom (one exit for all)
+    const int part = WPA > 1 ? wv : 0;
+    const int i = WPA > 1 ? (int)blockIdx.x : blockIdx.x * ( NNP_TPB / 64 ) + wv;
     if ( i >= n_local )
         return;
     NbLds &L = lds[wv];
@@ -1037,7 +1066,11 @@ __global__ __launch_bounds__( NNP_TPB ) void k_nnp_sf_pow(
     const int e = __builtin_amdgcn_readfirstlane( (int)x[i].w );
     const NnpElemPlan &Q = P->el[e];
     float *Gi = G + (size_t)i * NSF_LD;
-    radial_sf( Q, L, n, Gi );
+    if ( part == 0 )
+    {
+        zero_tail( Q, Gi );
+        radial_sf( Q, L, n, Gi );
+    }
     // exp(-eta s) = exp2(k s)
     const float kl = -1.44269504f * Q.a_eta[lane & ( AG_MAX - 1 )];
     float ke[NAG];
@@ -1073,15 +1106,30 @@ __global__ __launch_bounds__( NNP_TPB ) void k_nnp_sf_pow(
     };
     int ntrip = 0;
     if ( n <= 64 )
-        ntrip = pair_ring<false>(
-            L, n, rc2, tbuf[wv], [&]( int, int a, int q ) { triplet( a, q ); },
+        ntrip = pair_ring<false, WPA>(
+            L, n, rc2, part, tbuf[wv], [&]( int, int a, int q ) { triplet( a, q ); },
             []( int, unsigned long long, int ) {} );
     else
-        for_triplets( L, n, rc2, tbuf[wv], triplet, &ntrip );
+        for_triplets( L, n, rc2, tbuf[wv], triplet, &ntrip, part, WPA );
+    wave_reduce_scatter<NA_MAX>( acc );
+    if constexpr ( WPA > 1 )
+    {
+        // the waves' sums and counts, through the neighbour tables
+        lds[wv].e[lane].x = acc[0];
+        if ( lane == 0 )
+            lds[wv].j[0] = ntrip;
+        __syncthreads();
+        if ( part != 0 )
+            return;
+        for ( int w = 1; w < WPA; ++w )
+        {
+            acc[0] += lds[w].e[lane].x;
+            ntrip += lds[w].j[0];
+        }
+    }
     // the work model's term counts, as in k_nnp_sf
     if ( terms && lane == 0 )
         terms[i] = make_int4( n, ntrip, e, 0 );
-    wave_reduce_scatter<NA_MAX>( acc );
     const int g = lane / AP_MAX, pp = lane % AP_MAX;
     if ( g < NAG )
         Gi[Q.a_out[g][pp]] = acc[0] * __builtin_amdgcn_exp2f( Q.a_lpref[pp] );
@@ -1669,7 +1717,7 @@ static_assert( PAIR_RING * sizeof( float ) == ( NN_MAX - 64 ) * sizeof( float4 )
 // -2 eta P E: two scalars per neighbour and triplet in place of gradients by
 // component.  The atom's own force is minus the sum of its neighbours'
 // reactions.
-template <int NAG>
+template <int NAG, int WPA>
 __global__ __launch_bounds__( NNP_TPB, 5 ) void k_nnp_force_pow(
     int n_local, int fcap, const double4 *__restrict__ x,
     const int64_t *__restrict__ off, const int *__restrict__ idx,
@@ -1679,7 +1727,9 @@ __global__ __launch_bounds__( NNP_TPB, 5 ) void k_nnp_force_pow(
     __shared__ NbLds lds[NNP_TPB / 64];
     __shared__ ForceBuf buf[NNP_TPB / 64];
     const int wv = __builtin_amdgcn_readfirstlane( threadIdx.x >> 6 ), lane = threadIdx.x & 63;
-    const int i = blockIdx.x * ( NNP_TPB / 64 ) + wv;
+    // with WPA = 4 the block's waves share an atom (one exit for all)
+    const int part = WPA > 1 ? wv : 0;
+    const int i = WPA > 1 ? (int)blockIdx.x : blockIdx.x * ( NNP_TPB / 64 ) + wv;
     if ( i >= n_local )
         return;
     NbLds &L = lds[wv];
@@ -1701,7 +1751,8 @@ __global__ __launch_bounds__( NNP_TPB, 5 ) void k_nnp_force_pow(
         srad[u] = 0.f;
         if ( a < n )
         {
-            srad[u] = radial_force( Q, L, a, c );
+            if ( part == 0 )
+                srad[u] = radial_force( Q, L, a, c );
             L.e[a].z *= L.e[a].x;
             L.d[a].w *= L.d[a].w;
         }
@@ -1801,8 +1852,8 @@ __global__ __launch_bounds__( NNP_TPB, 5 ) void k_nnp_force_pow(
               *rpm = reinterpret_cast<float *>( L.e + 64 ), *rpb = buf[wv].ring.pb;
         // of the lane's neighbour: sum of its pa (or pb), sum of pm X_partner
         float sp = srad[0], sx = 0.f, sy = 0.f, sz = 0.f;
-        pair_ring<true>(
-            L, n, rc2, buf[wv].ring.code,
+        pair_ring<true, WPA>(
+            L, n, rc2, part, buf[wv].ring.code,
             [&]( int slot, int a, int q ) {
                 float pa, pb, pm;
                 grad( L.d[a], L.d[q], L.e[a], L.e[q], pa, pb, pm );
@@ -1841,6 +1892,22 @@ __global__ __launch_bounds__( NNP_TPB, 5 ) void k_nnp_force_pow(
                     sz = fmaf( w, X.z, sz );
                 }
             } );
+        if constexpr ( WPA > 1 )
+        {
+            // the waves' sums meet in the first wave
+            L.e[lane] = make_float4( sp, sx, sy, sz );
+            __syncthreads();
+            if ( part != 0 )
+                return;
+            for ( int w = 1; w < WPA; ++w )
+            {
+                const float4 o = lds[w].e[lane];
+                sp += o.x;
+                sx += o.y;
+                sy += o.z;
+                sz += o.w;
+            }
+        }
         if ( lane < n )
         {
             const float4 A = L.d[lane];
@@ -1884,10 +1951,20 @@ __global__ __launch_bounds__( NNP_TPB, 5 ) void k_nnp_force_pow(
             atomicAdd( &sF[q][0], -fmaf( pb, B.x, pm * A.x ) );
             atomicAdd( &sF[q][1], -fmaf( pb, B.y, pm * A.y ) );
             atomicAdd( &sF[q][2], -fmaf( pb, B.z, pm * A.z ) );
-        } );
+        }, nullptr, part, WPA );
         if ( cur >= 0 )
             flush();
         __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
+        if constexpr ( WPA > 1 )
+        {
+            __syncthreads();
+            if ( part != 0 )
+                return;
+            for ( int a = lane; a < n; a += 64 )
+                for ( int w = 1; w < WPA; ++w )
+                    for ( int k = 0; k < 3; ++k )
+                        sF[a][k] += buf[w].flat.f[a][k];
+        }
 #pragma unroll
         for ( int u = 0; u < NN_MAX / 64; ++u )
         {
@@ -1955,7 +2032,36 @@ static cmd_status nnp_prepare( cmd_nnp *M, int n_local, hipStream_t st )
     return CMD_OK;
 }
 
-cmd_status nnp_compute( cmd_nnp *M, cmd_system *S, cmd_neigh *N )
+// The neighbour-count check of one or several force calls: begin clears the
+// flag that the kernels raise, end waits for the stream and reads it.
+cmd_status nnp_check_begin( cmd_nnp *M, hipStream_t st )
+{
+    CMD_TRY( M->flag.reserve( 1 ) );
+    return fill_i32( M->flag.p, 0, 1, st );
+}
+
+cmd_status nnp_check_end( cmd_nnp *M, hipStream_t st )
+{
+    int fl = 0;
+    CMD_HIP( hipMemcpyAsync( &fl, M->flag.p, sizeof( int ),
+                             hipMemcpyDeviceToHost, st ) );
+    CMD_HIP( hipStreamSynchronize( st ) );
+    CMD_REQUIRE( fl == 0, CMD_ERR_CAPACITY,
+                 "an atom has more than %d neighbours inside the NNP cutoff",
+                 NN_MAX );
+    return CMD_OK;
+}
+
+// Up to this many atoms, and from this many listed neighbours on average, the
+// power-of-two kernels put four waves on an atom: one wave each leaves SIMDs
+// with too few waves to cover their latencies, but the gather and set-up are
+// repeated, which costs more where there are few pairs or many atoms.
+// Forces / symmetry functions, one wave and four: 512 atoms of 62 neighbours
+// 49 / 30 and 27 / 15 us, 3,000 atoms 61 / 39 and 59 / 34 us, 5,832 atoms
+// 86 / 56 and 91 / 53 us; 2,048 atoms of 23 neighbours 12 / 8 and 19 / 13 us.
+static constexpr int NNP_SPLIT_MAX = 3072, NNP_SPLIT_NEIGH = 48;
+
+cmd_status nnp_compute( cmd_nnp *M, cmd_system *S, cmd_neigh *N, bool check )
 {
     const hipStream_t st = S->stream;
     const int n = S->n_local;
@@ -1971,12 +2077,10 @@ cmd_status nnp_compute( cmd_nnp *M, cmd_system *S, cmd_neigh *N )
     // 3.9 + skin against rc 7.37 in input/nnp/input.nn).
     CMD_TRY( neigh_csr( N ) );
     const int nt = S->n_local + S->n_ghost;
-    for ( int c = 0; c < 3; ++c )
-        CMD_TRY( fill_f64( S->f.p + (size_t)c * S->cap, 0.0, nt, st ) );
-    CMD_TRY( fill_i32( M->flag.p, 0, 1, st ) );
+    if ( check )
+        CMD_TRY( nnp_check_begin( M, st ) );
     if ( n == 0 )
-        return CMD_OK;
-    CMD_TRY( fill_i32( reinterpret_cast<int *>( M->G.p ), 0, (size_t)n * NSF_LD, st ) );
+        return CMD_OK; // no atoms, no ghosts: no force rows
     CMD_TRY( M->terms.reserve( std::max( n, 1 ) ) );
     M->n_last = n;
     const int nbw = ( n + NNP_TPB / 64 - 1 ) / ( NNP_TPB / 64 );
@@ -1999,6 +2103,7 @@ cmd_status nnp_compute( cmd_nnp *M, cmd_system *S, cmd_neigh *N )
     // operations wherever the grid allows them
     const bool pow = nag >= 1 && rs0 && pow2;
     const bool g58 = nag == 5 && nap8;
+    const bool split = n <= NNP_SPLIT_MAX && N->nnz >= (int64_t)NNP_SPLIT_NEIGH * n;
 #define CMD_POW( LAUNCH )                                                                 \
     switch ( nag )                                                                        \
     {                                                                                     \
@@ -2012,14 +2117,27 @@ cmd_status nnp_compute( cmd_nnp *M, cmd_system *S, cmd_neigh *N )
     default: LAUNCH( 8 ); break;                                                          \
     }
 #define CMD_SF_POW( A )                                                                   \
-    k_nnp_sf_pow<A><<<nbw, NNP_TPB, 0, st>>>( n, S->x.p, N->offsets.p, N->idx.p, M->dplan.p, \
-                                              M->G.p, M->flag.p, M->terms.p )
+    if ( split )                                                                          \
+        k_nnp_sf_pow<A, 4><<<n, NNP_TPB, 0, st>>>( n, S->x.p, N->offsets.p, N->idx.p,      \
+                                                   M->dplan.p, M->G.p, M->flag.p,         \
+                                                   M->terms.p, S->f.p, S->cap, nt );      \
+    else                                                                                  \
+        k_nnp_sf_pow<A, 1><<<nbw, NNP_TPB, 0, st>>>( n, S->x.p, N->offsets.p, N->idx.p,    \
+                                                     M->dplan.p, M->G.p, M->flag.p,       \
+                                                     M->terms.p, S->f.p, S->cap, nt )
 #define CMD_FORCE_POW( A )                                                                \
-    k_nnp_force_pow<A><<<nbw, NNP_TPB, 0, st>>>( n, S->cap, S->x.p, N->offsets.p, N->idx.p, \
-                                                 M->dplan.p, M->dEdG.p, S->f.p, M->flag.p )
+    if ( split )                                                                          \
+        k_nnp_force_pow<A, 4><<<n, NNP_TPB, 0, st>>>( n, S->cap, S->x.p, N->offsets.p,     \
+                                                      N->idx.p, M->dplan.p, M->dEdG.p,    \
+                                                      S->f.p, M->flag.p );                \
+    else                                                                                  \
+        k_nnp_force_pow<A, 1><<<nbw, NNP_TPB, 0, st>>>( n, S->cap, S->x.p, N->offsets.p,   \
+                                                        N->idx.p, M->dplan.p, M->dEdG.p,  \
+                                                        S->f.p, M->flag.p )
 #define CMD_SF( A, P, R )                                                                 \
     k_nnp_sf<A, P, R><<<nbw, NNP_TPB, 0, st>>>( n, S->x.p, N->offsets.p, N->idx.p, M->dplan.p, \
-                                                M->G.p, M->flag.p, M->terms.p )
+                                                M->G.p, M->flag.p, M->terms.p, S->f.p,    \
+                                                S->cap, nt )
     if ( pow )
         CMD_POW( CMD_SF_POW )
     else if ( g58 )
@@ -2068,14 +2186,7 @@ cmd_status nnp_compute( cmd_nnp *M, cmd_system *S, cmd_neigh *N )
 #undef CMD_SF_POW
 #undef CMD_FORCE_POW
     CMD_LAUNCH_CHECK();
-    int fl = 0;
-    CMD_HIP( hipMemcpyAsync( &fl, M->flag.p, sizeof( int ),
-                             hipMemcpyDeviceToHost, st ) );
-    CMD_HIP( hipStreamSynchronize( st ) );
-    CMD_REQUIRE( fl == 0, CMD_ERR_CAPACITY,
-                 "an atom has more than %d neighbours inside the NNP cutoff",
-                 NN_MAX );
-    return CMD_OK;
+    return check ? nnp_check_end( M, st ) : CMD_OK;
 }
 
 // Sum of the atomic network outputs (FP64 reduction).
