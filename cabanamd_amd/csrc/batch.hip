@@ -759,13 +759,14 @@ cmd_status thermo( cmd_batch *B, const std::vector<char> *which )
 
 // Forces of the current positions with the current list (CbnMD::init's
 // first compute; for NNP also the ghost-force fold, cabanamd_impl.h:218-223).
-cmd_status forces( cmd_batch *B )
+// check as in nnp_compute.
+cmd_status forces( cmd_batch *B, bool check = true )
 {
     if ( B->S->n_local == 0 )
         return CMD_OK;
     if ( B->nnp )
     {
-        CMD_TRY( cmd_force_compute( B->F, B->S, B->N ) );
+        CMD_TRY( nnp_compute( B->F->nnp, B->S, B->N, check ) );
         return cmd_comm_update_force( B->S );
     }
     StepCtl ctl{};
@@ -1175,11 +1176,21 @@ cmd_status cmd_batch_run( cmd_batch *b, int nsteps )
     const int s0 = b->step + 1, s1 = b->step + nsteps;
     if ( b->nnp )
     {
-        // CbnMD::run's order (cabanamd_impl.h:285-399) step by step
+        // CbnMD::run's order (cabanamd_impl.h:285-399); a step's final half
+        // kick and the next one's half kick and drift are one kernel except
+        // at a thermo row, and the force's check is read at the end
+        StepCtl ctl{};
+        ctl.dtf = 0.5 * S->dt / S->mvv2e;
+        ctl.dtv = S->dt;
+        ctl.do_final = 1;
+        ctl.do_next_initial = 1;
+        CMD_TRY( nnp_check_begin( b->F->nnp, st ) );
+        bool started = false;
         for ( int s = s0; s <= s1; ++s )
         {
             b->step = s;
-            CMD_TRY( cmd_nve_initial( S ) );
+            if ( !started )
+                CMD_TRY( cmd_nve_initial( S ) );
             if ( s % p.every == 0 )
             {
                 CMD_TRY( wrap( b, S->x.p ) );
@@ -1187,12 +1198,22 @@ cmd_status cmd_batch_run( cmd_batch *b, int nsteps )
             }
             else
                 CMD_TRY( refresh( b ) );
-            CMD_TRY( forces( b ) );
-            CMD_TRY( cmd_nve_final( S ) );
-            if ( s == s1 || ( p.thermo_rate > 0 && s % p.thermo_rate == 0 ) )
+            CMD_TRY( forces( b, false ) );
+            const bool th = s == s1 || ( p.thermo_rate > 0 && s % p.thermo_rate == 0 );
+            started = !th;
+            if ( started )
+            {
+                CMD_TRY( S->x_alt.reserve( S->cap ) );
+                CMD_TRY( nve_final_initial( S, ctl, S->x_alt.p, nullptr, nullptr ) );
+                S->x.swap( S->x_alt );
+            }
+            else
+            {
+                CMD_TRY( cmd_nve_final( S ) );
                 CMD_TRY( thermo( b, nullptr ) );
+            }
         }
-        CMD_HIP( hipStreamSynchronize( st ) );
+        CMD_TRY( nnp_check_end( b->F->nnp, st ) );
         b->timers[1] += now_s() - t0;
         return CMD_OK;
     }

@@ -210,26 +210,44 @@ static cmd_status thermo_now( cmd_md *md, int step )
     return CMD_OK;
 }
 
-// The reference's step order without fusion (cabanamd_impl.h:285-399), used
-// for the NNP force, whose cost dwarfs the integrator's.
+// The reference's step order (cabanamd_impl.h:285-399) for the NNP force.
+// The final half kick of a step and the half kick and drift of the next (with
+// the wrap before a rebuild) run as one kernel, except around a thermo row;
+// no step waits on the device: the force's neighbour-count check is read at
+// the end of the call.
 static cmd_status run_steps_plain( cmd_md *md, int nsteps )
 {
     cmd_system *S = md->S;
     const cmd_params &p = md->p;
     const int s0 = md->step + 1, s1 = md->step + nsteps;
     auto t0 = std::chrono::steady_clock::now();
+    StepCtl ctl{};
+    ctl.dtf = 0.5 * S->dt / S->mvv2e;
+    ctl.dtv = S->dt;
+    for ( int k = 0; k < 3; ++k )
+        ctl.L[k] = S->dom.L[k];
+    ctl.do_final = 1;
+    ctl.do_next_initial = 1;
+    CMD_TRY( nnp_check_begin( md->F->nnp, S->stream ) );
+    bool started = false; // the last step's kernel began this one
     for ( int s = s0; s <= s1; ++s )
     {
-        int k = md->begin( PH_INT );
-        CMD_TRY( cmd_nve_initial( S ) );
-        md->end( k );
-        if ( s % p.every == 0 )
+        const bool rb = s % p.every == 0;
+        int k;
+        if ( !started )
         {
-            k = md->begin( PH_COMM );
-            CMD_TRY( cmd_comm_exchange( S ) );
+            k = md->begin( PH_INT );
+            CMD_TRY( cmd_nve_initial( S ) );
             md->end( k );
-            CMD_TRY( rebuild( md ) );
+            if ( rb )
+            {
+                k = md->begin( PH_COMM );
+                CMD_TRY( cmd_comm_exchange( S ) );
+                md->end( k );
+            }
         }
+        if ( rb )
+            CMD_TRY( rebuild( md ) );
         else
         {
             k = md->begin( PH_COMM );
@@ -237,18 +255,34 @@ static cmd_status run_steps_plain( cmd_md *md, int nsteps )
             md->end( k );
         }
         k = md->begin( PH_FORCE );
-        CMD_TRY( cmd_force_compute( md->F, S, md->N ) );
+        CMD_TRY( nnp_compute( md->F->nnp, S, md->N, false ) );
         md->end( k );
         k = md->begin( PH_COMM );
         CMD_TRY( cmd_comm_update_force( S ) );
         md->end( k );
+        const bool th = p.thermo_rate > 0 && s % p.thermo_rate == 0;
+        started = s < s1 && !th && S->n_local > 0;
         k = md->begin( PH_INT );
-        CMD_TRY( cmd_nve_final( S ) );
+        if ( started )
+        {
+            ctl.wrap_next = ( s + 1 ) % p.every == 0 ? 1 : 0;
+            CMD_TRY( S->x_alt.reserve( S->cap ) );
+            CMD_TRY( nve_final_initial( S, ctl, S->x_alt.p, nullptr, nullptr ) );
+            S->x.swap( S->x_alt );
+            S->bin_grid_valid = false; // atoms leave the cells they were sorted into
+            if ( ctl.wrap_next )
+            {
+                S->n_ghost = 0; // Comm::exchange resizes to N_local
+                S->xg_valid = false;
+            }
+        }
+        else
+            CMD_TRY( cmd_nve_final( S ) );
         md->end( k );
-        if ( p.thermo_rate > 0 && s % p.thermo_rate == 0 )
+        if ( th )
             CMD_TRY( thermo_now( md, s ) );
     }
-    CMD_HIP( hipStreamSynchronize( S->stream ) );
+    CMD_TRY( nnp_check_end( md->F->nnp, S->stream ) );
     md->timers[5] +=
         std::chrono::duration<double>( std::chrono::steady_clock::now() - t0 )
             .count();

@@ -131,3 +131,52 @@ def test_neighbour_counts(gpu, n, pl):
     x = BOX / 2 + (x - BOX / 2) * min(1.0, 4.0 / np.ptp(x, axis=0).max())
     m = _model(1, (0.01, 0.05), POW2 if pl == "pow2" else PL, rc=8.0)
     _check(gpu, m, x, t, "fp32")
+
+
+def test_one_wave_per_atom_at_62_neighbours(gpu):
+    """3,375 atoms, past the sizes that put four waves on an atom: the ring
+    walk with most lanes in use, forces within 1e-5 of the oracle."""
+    from test_gpu_nnp import _fitted_benchmark_model, _run
+    M = gpu
+    x, t, _ = M.nnp_lattice((15, 15, 15), spacing=2.5, jitter=0.1, seed=5)
+    L = [37.5] * 3
+    model = _fitted_benchmark_model(M, x, t, L)
+    m = model.describe(2)
+    m.update(act="ttl", smin=0.0, smax=1.0, scale=True)
+    s, comm, nl = _system(M, x, t, L, 6.3)
+    r = _run(M, s, comm, nl, M.ForceNNP(model, M.PREC_MIXED), m)
+    assert (np.linalg.norm(r["f"] - r["fo"]) <
+            1e-5 * np.linalg.norm(r["fo"]))
+
+
+@pytest.mark.parametrize("batch", [False, True])
+def test_joined_kicks_match_separate_ones(gpu, batch):
+    """A run whose steps join the final and the next first half kick against
+    one with a thermo row (separate kicks) every step, over two rebuilds:
+    equal up to the order of the force atomics (1e-16 a step, 45 steps)."""
+    M = gpu
+    m = _model(2, (0.01, 0.05), POW2, rc=4.0)
+    x, t, ids = M.nnp_lattice((6, 6, 7), spacing=2.0, jitter=0.1, seed=3)
+    L = [12.0, 12.0, 14.0]
+    x = np.mod(x, L)
+    v = np.random.default_rng(1).normal(0, 0.5, x.shape)
+    out = []
+    for thermo in (1, 100):
+        p = M.nnp_params(cutoff=4.0, thermo=thermo, dt=0.002)
+        if batch:
+            B = M.Batch(p, M.PREC_MIXED, nnp_model=_engine_model(M, m))
+            h = B.add(x, t, [0, 0, 0], L, v=v, id=ids)
+            B.run(45)
+            out.append(B.download(h)[:3])
+        else:
+            md = M.CbnMD(p, M.PREC_MIXED)
+            md.set_nnp_model(_engine_model(M, m))
+            md.set_initial_state(x, t, [0, 0, 0], L, v=v, id=ids)
+            md.init()
+            md.run(45)
+            n = md.n_local
+            a = md.arrays()
+            o = np.argsort(a[4][:n])
+            out.append([k[:n][o] for k in a[:3]])
+    for a, b in zip(*out):
+        assert np.abs(a - b).max() < 1e-11 * np.abs(b).max()
