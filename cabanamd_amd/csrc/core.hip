@@ -191,6 +191,76 @@ __global__ void k_scan_tile_apply( const InT *__restrict__ in, int n,
     }
 }
 
+// The whole scan in one block, for inputs of one round (8 elements a thread,
+// read 16 bytes at a time; in is 16-byte aligned, as device allocations are):
+// three launches cost more.  2,744 counts (the cells of 32,000 atoms): 10 us
+// in three kernels; a second round would lose that again.  Sums in the type
+// of the result.
+static constexpr int SCAN_ONE_TPB = 1024;
+static constexpr int SCAN_ONE_MAX = SCAN_ONE_TPB * SCAN_ITEMS;
+
+template <class OutT>
+__global__ __launch_bounds__( SCAN_ONE_TPB ) void k_scan_one( const int *__restrict__ in, int n,
+                                                            OutT *__restrict__ out,
+                                                            int64_t *__restrict__ total_slot )
+{
+    constexpr int NW = SCAN_ONE_TPB / 64;
+    __shared__ OutT wsum[NW];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int i0 = (int)threadIdx.x * SCAN_ITEMS;
+    int vals[SCAN_ITEMS];
+    if ( i0 + SCAN_ITEMS <= n )
+    {
+        const int4 a = *reinterpret_cast<const int4 *>( in + i0 );
+        const int4 b = *reinterpret_cast<const int4 *>( in + i0 + 4 );
+        vals[0] = a.x, vals[1] = a.y, vals[2] = a.z, vals[3] = a.w;
+        vals[4] = b.x, vals[5] = b.y, vals[6] = b.z, vals[7] = b.w;
+    }
+    else
+    {
+#pragma unroll
+        for ( int k = 0; k < SCAN_ITEMS; ++k )
+            vals[k] = i0 + k < n ? in[i0 + k] : 0;
+    }
+    OutT own = 0;
+#pragma unroll
+    for ( int k = 0; k < SCAN_ITEMS; ++k )
+        own += vals[k];
+    OutT s = own;
+#pragma unroll
+    for ( int o = 1; o < 64; o <<= 1 )
+    {
+        const OutT t = __shfl_up( s, o, 64 );
+        if ( lane >= o )
+            s += t;
+    }
+    if ( lane == 63 )
+        wsum[wid] = s;
+    __syncthreads();
+    OutT e = s - own, total = 0;
+#pragma unroll
+    for ( int w = 0; w < NW; ++w )
+    {
+        const OutT ws = wsum[w];
+        if ( w < wid )
+            e += ws;
+        total += ws;
+    }
+#pragma unroll
+    for ( int k = 0; k < SCAN_ITEMS; ++k )
+    {
+        if ( i0 + k < n )
+            out[i0 + k] = e;
+        e += vals[k];
+    }
+    if ( threadIdx.x == 0 )
+    {
+        out[n] = total;
+        if ( total_slot )
+            *total_slot = (int64_t)total;
+    }
+}
+
 template <class OutT>
 static cmd_status scan_impl( const int *in, OutT *out, int n, Scratch &sc,
                              hipStream_t st, int64_t *total_host )
@@ -198,24 +268,25 @@ static cmd_status scan_impl( const int *in, OutT *out, int n, Scratch &sc,
     const int nblk = std::max( 1, ( n + SCAN_TILE - 1 ) / SCAN_TILE );
     CMD_TRY( sc.blk.reserve( nblk + 2 ) );
     int64_t *slot = sc.blk.p + nblk + 1;
-    if ( n > 0 )
+    if ( n <= SCAN_ONE_MAX && ( (uintptr_t)in & 15 ) == 0 )
     {
-        k_scan_tile_sums<int><<<nblk, TPB, 0, st>>>( in, n, sc.blk.p );
+        k_scan_one<OutT><<<1, SCAN_ONE_TPB, 0, st>>>( in, n, out, slot );
         CMD_LAUNCH_CHECK();
+        if ( total_host )
+        {
+            CMD_HIP( hipMemcpyAsync( total_host, slot, sizeof( int64_t ),
+                                     hipMemcpyDeviceToHost, st ) );
+            CMD_HIP( hipStreamSynchronize( st ) );
+        }
+        return CMD_OK;
     }
-    else
-    {
-        CMD_TRY( fill_i32( (int *)sc.blk.p, 0, 2, st ) );
-    }
-    k_scan_tile_offsets<OutT><<<1, TPB, 0, st>>>( sc.blk.p, n > 0 ? nblk : 0,
-                                                  out, n, slot );
+    // (n may be 0: one empty tile)
+    k_scan_tile_sums<int><<<nblk, TPB, 0, st>>>( in, n, sc.blk.p );
     CMD_LAUNCH_CHECK();
-    if ( n > 0 )
-    {
-        k_scan_tile_apply<int, OutT><<<nblk, TPB, 0, st>>>( in, n, sc.blk.p,
-                                                            out );
-        CMD_LAUNCH_CHECK();
-    }
+    k_scan_tile_offsets<OutT><<<1, TPB, 0, st>>>( sc.blk.p, nblk, out, n, slot );
+    CMD_LAUNCH_CHECK();
+    k_scan_tile_apply<int, OutT><<<nblk, TPB, 0, st>>>( in, n, sc.blk.p, out );
+    CMD_LAUNCH_CHECK();
     if ( total_host )
     {
         CMD_HIP( hipMemcpyAsync( total_host, slot, sizeof( int64_t ),
@@ -525,7 +596,7 @@ __global__ void k_final_initial( int n, int cap, const double4 *__restrict__ x,
             // comm_mpi_impl.h:369-408): the drifted position, shifted per
             // image, at the image's sorted ghost slot
             if ( ctl.xg_next )
-                for ( int m = ctl.img_start[i]; m < ctl.img_start[i + 1]; ++m )
+                for ( int m = ctl.img_rng[i].x; m < ctl.img_rng[i].y; ++m )
                 {
                     const unsigned e = (unsigned)ctl.img_pk[m];
                     const unsigned code = e >> IMG_CODE_SHIFT;
@@ -767,6 +838,12 @@ __global__ __launch_bounds__( TPB ) void k_halo_count( int n, const double4 *__r
 // past the ghost rows the host sized, and block 0 sets *flag when a set's
 // images differ from its total.  The images' velocity and force rows are
 // zeroed (cap: the planes' stride).
+//
+// Each local atom gets a range of image entries, img_rng[i] = (first, past
+// the last), one per image and in atom order (the images of earlier blocks
+// are, set by set, what the scan counts before this block), and each ghost
+// its entry img_pos[k] in its root's range.  The entries' contents follow
+// once the ghosts are sorted.
 __global__ __launch_bounds__( TPB ) void k_halo_fill( int n, int cap, double4 *__restrict__ x,
                                                       double *__restrict__ v,
                                                       double *__restrict__ f,
@@ -777,7 +854,9 @@ __global__ __launch_bounds__( TPB ) void k_halo_fill( int n, int cap, double4 *_
                                                       int *__restrict__ root,
                                                       int *__restrict__ code,
                                                       const int *__restrict__ pre, int ng,
-                                                      int *__restrict__ flag )
+                                                      int *__restrict__ flag,
+                                                      int2 *__restrict__ img_rng,
+                                                      int *__restrict__ img_pos )
 {
     __shared__ int s_w[HALO_SETS][TPB / 64];
     if ( pre )
@@ -809,7 +888,11 @@ __global__ __launch_bounds__( TPB ) void k_halo_fill( int n, int cap, double4 *_
     }
     __syncthreads();
     if ( !any )
+    {
+        if ( i < n )
+            img_rng[i] = make_int2( 0, 0 );
         return;
+    }
     double4 p0 = make_double4( 0.0, 0.0, 0.0, 0.0 );
     int idv = 0;
     if ( m )
@@ -817,6 +900,34 @@ __global__ __launch_bounds__( TPB ) void k_halo_fill( int n, int cap, double4 *_
         p0 = x[i];
         idv = id[i];
     }
+    // images of the atom (one per set its mask holds) and their entries
+    int nimg = 0;
+#pragma unroll
+    for ( int j = 0; j < HALO_SETS; ++j )
+        nimg += ( m & halo_set( j ) ) == halo_set( j ) ? 1 : 0;
+    int inc = nimg;
+#pragma unroll
+    for ( int o = 1; o < 64; o <<= 1 )
+    {
+        const int t = __shfl_up( inc, o, 64 );
+        if ( lane >= o )
+            inc += t;
+    }
+    // lane j: set j's images in earlier blocks and in this block's earlier
+    // waves
+    int before = 0;
+    if ( lane < HALO_SETS )
+    {
+        before = off[lane * nblk + blockIdx.x] - off[lane * nblk];
+        for ( int w = 0; w < wv; ++w )
+            before += s_w[lane][w];
+    }
+#pragma unroll
+    for ( int o = 32; o > 0; o >>= 1 )
+        before += __shfl_xor( before, o, 64 );
+    int img = before + inc - nimg;
+    if ( i < n )
+        img_rng[i] = nimg ? make_int2( img, img + nimg ) : make_int2( 0, 0 );
     int pos[HALO_SETS];
 #pragma unroll
     for ( int j = 0; j < HALO_SETS; ++j )
@@ -855,6 +966,7 @@ __global__ __launch_bounds__( TPB ) void k_halo_fill( int n, int cap, double4 *_
             }
             root[k] = i;
             code[k] = c;
+            img_pos[k] = img++;
             send_idx[k] = halo_source( j ) < 0 ? i : n + pos[halo_source( j ) < 0 ? 0 : halo_source( j )];
         }
     }
@@ -1346,6 +1458,7 @@ cmd_status cmd_system_upload( cmd_system *s, int n_local, int n_ghost,
     s->n_local = n_local;
     s->n_ghost = n_ghost;
     s->N = n_local;
+    s->halo_locals = s->halo_ghosts = -1;
     s->bin_grid_valid = false;
     s->xg_valid = false;
     for ( int k = 0; k < 6; ++k )
@@ -1515,12 +1628,15 @@ cmd_status cmd_comm_exchange_halo( cmd_system *s, double comm_depth )
     // the halo gathers positions and types only (comm_mpi_impl.h:346-347);
     // the ghosts' velocity and force rows are set to zero so that downloads
     // are defined and full-list kernels, which never write them, leave them 0
+    CMD_TRY( s->img_rng.reserve( n ) );
+    CMD_TRY( s->img_pos.reserve( std::max( ng, 1 ) ) );
+    s->img_valid = false; // the entries are written with the ghost sort
     if ( ng > 0 || pre )
     {
         k_halo_fill<<<nblk, TPB, 0, s->stream>>>(
             n, s->cap, s->x.p, s->v.p, s->f.p, s->id.p, mask, nblk, off, H, s->send_idx.p,
             s->ghost_root.p, s->ghost_code.p, pre ? s->halo_pre_tot.p : nullptr, ng,
-            pre ? s->hw.d + HW_HALO_FLAG : nullptr );
+            pre ? s->hw.d + HW_HALO_FLAG : nullptr, s->img_rng.p, s->img_pos.p );
         CMD_LAUNCH_CHECK();
     }
     if ( pre )
@@ -1529,6 +1645,8 @@ cmd_status cmd_comm_exchange_halo( cmd_system *s, double comm_depth )
         s->halo_pre_check = true;
     }
     s->n_ghost = ng;
+    s->halo_locals = n;
+    s->halo_ghosts = ng;
     return CMD_OK;
 }
 

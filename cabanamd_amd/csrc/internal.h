@@ -200,6 +200,7 @@ cmd_status fill_f64( double *p, double v, size_t n, hipStream_t st );
 struct MassTable
 {
     double m[CMD_MAX_TYPES];
+    double dtfm[CMD_MAX_TYPES]; // the half kick's 0.5 dt / mvv2e / m
 };
 
 // Linked-cell grid: cell = floor((x - min) * rd) per dimension, with the
@@ -295,6 +296,8 @@ struct cmd_system
     cmd::DevBuf<int> halo_pre_tot;
     bool halo_pre = false;       // the totals await the next halo pass
     bool halo_pre_check = false; // that pass's mismatch flag is still unread
+    // atoms and ghosts of the last halo pass (-1: none since an upload)
+    int halo_locals = -1, halo_ghosts = -1;
     int halo_pre_n = 0;
     double halo_pre_depth = 0.0;
     cmd::HostWords hw;
@@ -309,12 +312,15 @@ struct cmd_system
     cmd::DevBuf<double4> xg;
     bool xg_valid = false;
     // the fused step writes the next step's sorted ghosts into xg_alt: local
-    // atom i has images img_pk[gimg.start[i] .. gimg.start[i + 1]), each the
+    // atom i has images img_pk[img_rng[i].x .. img_rng[i].y), each the
     // sorted slot | shift code << IMG_CODE_SHIFT; the system's own ghost rows
-    // are then stale until the next refresh
+    // are then stale until the next refresh.  The halo pass lays out the
+    // ranges and each ghost's entry img_pos; the ghost sort writes them.
     cmd::DevBuf<double4> xg_alt;
-    cmd::CellSort gimg;
-    cmd::DevBuf<int> img_pk;
+    cmd::DevBuf<int2> img_rng;
+    cmd::DevBuf<int> img_pos, img_pk;
+    // 1 when a sorted ghost lies outside the binning grid
+    cmd::DevBuf<int> ghost_out;
     bool img_valid = false; // img_pk matches the current ghosts
     bool ghosts_x_stale = false;
     cmd::Scratch sc;
@@ -322,8 +328,12 @@ struct cmd_system
     cmd::MassTable mass_table() const
     {
         cmd::MassTable t;
+        const double dtf = 0.5 * dt / mvv2e;
         for ( int k = 0; k < CMD_MAX_TYPES; ++k )
+        {
             t.m[k] = mass[k];
+            t.dtfm[k] = dtf / mass[k];
+        }
         return t;
     }
     cmd_status reserve( int n ); // keeps the first n_local+n_ghost atoms
@@ -377,7 +387,7 @@ struct cmd_neigh
     struct Spec
     {
         bool valid = false;
-        int G = 0, half = 0, W = 0, E = 0, bw_req = 0, cap = 0;
+        int G = 0, half = 0, W = 0, E = 0, E_req = 0, bw_req = 0, cap = 0;
         int slot_cap = 0;   // build planes: staged slots + sentinel
         int rows = 0;       // build rows: atoms of one atom column
         int slab_waves = 0; // slab waves of all tiles
@@ -443,7 +453,7 @@ struct StepCtl
     // every local atom is also written, shifted per its images' codes, to
     // xg_next at its sorted ghost slots: the next step's ghost refresh
     double4 *xg_next = nullptr;
-    const int *img_start = nullptr; // per local atom, into img_pk
+    const int2 *img_rng = nullptr;  // per local atom: first and past-the-last entry of img_pk
     const int *img_pk = nullptr;    // sorted slot | code << IMG_CODE_SHIFT
 };
 
@@ -519,7 +529,7 @@ enum
     TILE_RES_INFO = 0,     // 5 words, k_tile_info
     TILE_RES_MAXROW = 5,   // longest row of the build
     TILE_RES_OVER = 6,     // 1: a block's needs exceeded the launch sizes
-    TILE_RES_INSIDE = 7,   // 1: every position lies in the binning grid
+    TILE_RES_OUTSIDE = 7,  // 1: a ghost lies outside the binning grid
     TILE_RES_WAVES = 8,    // slab waves of all tiles (written by the build)
     TILE_RES_WORDS = 9
 };

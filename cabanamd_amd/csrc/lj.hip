@@ -263,9 +263,10 @@ __device__ __forceinline__ void walk_row( const int *__restrict__ row, int nr,
 // -- integrator_nve.h:91-110 and comm_mpi.h:141-168 -- adding m v^2 to mv2.
 // With G >= 4 lanes per atom lane s handles component s; otherwise lane 0
 // does all three.  Both orders run the same operations on the same values.
-// vin, when given, holds the velocity components the lane would load
+// The half kick's factor dtf / m comes divided per type from the host (the
+// same IEEE quotient).  vin, when given, holds the velocity components the lane would load
 // (component s, or all three), read early so their latency is hidden.
-template <int G, bool FUSED>
+template <int G, bool FUSED, bool ONE_TYPE = false>
 __device__ __forceinline__ void finish_atom( bool active, int s, int i,
                                              const double4 &xi, double fx,
                                              double fy, double fz, int scap,
@@ -292,8 +293,8 @@ __device__ __forceinline__ void finish_atom( bool active, int s, int i,
                 double *xn = reinterpret_cast<double *>( x_next + i );
                 if ( c < 3 )
                 {
-                    const double m = mt.m[(int)xi.w];
-                    const double dtfm = ctl.dtf / m;
+                    const int ty = ONE_TYPE ? 0 : (int)xi.w;
+                    const double m = mt.m[ty], dtfm = mt.dtfm[ty];
                     double vc = ( vin ? vin[0] : v[c * scap + i] ) + dtfm * fc;
                     mv2 += vc * vc * m;
                     if ( ctl.do_next_initial )
@@ -345,8 +346,8 @@ __device__ __forceinline__ void finish_atom( bool active, int s, int i,
         }
         if ( FUSED && ctl.do_final )
         {
-            const double m = mt.m[(int)xi.w];
-            const double dtfm = ctl.dtf / m;
+            const int ty = ONE_TYPE ? 0 : (int)xi.w;
+            const double m = mt.m[ty], dtfm = mt.dtfm[ty];
             double vx = ( vin ? vin[0] : v[i] ) + dtfm * fx;
             double vy = ( vin ? vin[1] : v[scap + i] ) + dtfm * fy;
             double vz = ( vin ? vin[2] : v[2 * scap + i] ) + dtfm * fz;
@@ -478,26 +479,26 @@ __global__ __launch_bounds__( 512 ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 )
     double *__restrict__ partial )
 {
     extern __shared__ double s_rec[];
-    __shared__ TileHead H;
     constexpr int APW = 64 / G;
     const int t = xcd_tile( blockIdx.x, gridDim.x );
-    // staging waves issue first: a block's tile head and records are on
-    // the critical path of all its waves (1 % faster than equal priority)
+    // staging waves issue first: a block's records are on the critical path
+    // of all its waves (1 % faster than equal priority)
     __builtin_amdgcn_s_setprio( 2 );
-    load_head( info, t, T.W, H );
+    // the tile's info words, read at wave-uniform places (no copy in LDS)
+    const int *__restrict__ I = info + (size_t)t * TI_WORDS;
     const char *s_byte = reinterpret_cast<const char *>( s_rec );
-    const int *s_t = reinterpret_cast<const int *>( s_rec + 3 * slot_cap );
+    int *s_t = reinterpret_cast<int *>( s_rec + 3 * slot_cap );
     const int R4 = ( ( lcap + G - 1 ) / G + 3 ) / 4;
     const int wbase = woff[t];
     const unsigned short *st = slab + (size_t)wbase * R4 * 256;
     const int nw = woff[t + 1] - wbase;
-    const int nat = H.info[TI_NAT];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int nat = I[TI_NAT], total = I[TI_TOTAL];
+    const int lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane( threadIdx.x >> 6 );
     const int nwb = blockDim.x >> 6;
     // four sentinel entries: the word a lane past the tile's atoms walks
     constexpr int REC = F32REC ? TILE_REC32 : TILE_REC;
-    const unsigned long long sent4 =
-        0x0001000100010001ull * (unsigned)( H.segoff[H.nseg] * REC );
+    const unsigned long long sent4 = 0x0001000100010001ull * (unsigned)( total * REC );
     // FP32 records: coordinates about the centre of the staged region
     double ox = 0.0, oy = 0.0, oz = 0.0;
     if constexpr ( F32REC )
@@ -522,8 +523,16 @@ __global__ __launch_bounds__( 512 ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 )
         sub = lane / apw;
         const int ta = w * APW + a;
         active = a < APW && ta < nat;
-        // lanes past the atoms take the tile's first atom (nat >= 1 here)
-        i = tile_atom( H, T.W, active ? ta : 0 );
+        // the atom's column is the last one starting at or before ta; lanes
+        // past the atoms take the tile's first atom (nat >= 1 here)
+        const int tq = active ? ta : 0;
+        int base = I[TI_AL];
+        for ( int c = 1; c < T.W * T.W; ++c )
+        {
+            const int ao = I[TI_AOFF + c];
+            base = tq >= ao ? I[TI_AL + c] - ao : base;
+        }
+        i = base + tq;
     };
     auto row_of = [&]( int w ) -> const unsigned long long *
     {
@@ -552,10 +561,37 @@ __global__ __launch_bounds__( 512 ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 )
     WaveIn P;
     if ( wid < nw )
         prep( wid, P );
+    const int nseg = 2 * tile_q( T.W );
     if constexpr ( F32REC )
-        stage_records32( H, x, xg, reinterpret_cast<float4 *>( s_rec ), ox, oy, oz );
+    {
+        float4 *rec = reinterpret_cast<float4 *>( s_rec );
+        stage_chunks( I, nseg, wid, nwb, x, xg, [&]( int k, const double4 &p ) {
+            rec[k] = make_float4( (float)( p.x - ox ), (float)( p.y - oy ), (float)( p.z - oz ),
+                                  __int_as_float( (int)p.w ) );
+        } );
+        if ( threadIdx.x == 0 )
+            rec[total] = make_float4( (float)TILE_FAR, (float)TILE_FAR, (float)TILE_FAR,
+                                      __int_as_float( 0 ) );
+    }
     else
-        stage_records<!ONE_TYPE>( H, x, xg, s_rec, slot_cap );
+    {
+        stage_chunks( I, nseg, wid, nwb, x, xg, [&]( int k, const double4 &p ) {
+            s_rec[3 * k] = p.x;
+            s_rec[3 * k + 1] = p.y;
+            s_rec[3 * k + 2] = p.z;
+            if ( !ONE_TYPE )
+                s_t[k] = (int)p.w;
+        } );
+        if ( threadIdx.x == 0 )
+        {
+            s_rec[3 * total] = TILE_FAR;
+            s_rec[3 * total + 1] = TILE_FAR;
+            s_rec[3 * total + 2] = TILE_FAR;
+            if ( !ONE_TYPE )
+                s_t[total] = 0;
+        }
+    }
+    __syncthreads();
     __builtin_amdgcn_s_setprio( 0 );
     for ( int w = wid; w < nw; w += nwb )
     {
@@ -570,10 +606,7 @@ __global__ __launch_bounds__( 512 ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 )
         const int n = active ? P.n : 0;
         double fx = 0.0, fy = 0.0, fz = 0.0;
         int nr = n > sub ? ( n - sub + gw - 1 ) / gw : 0;
-#pragma unroll
-        for ( int o = 32; o > 0; o >>= 1 )
-            nr = max( nr, __shfl_xor( nr, o, 64 ) );
-        nr = __builtin_amdgcn_readfirstlane( nr );
+        nr = wave_max_i32( nr );
         const unsigned long long *row8 = row_of( w );
         // the velocities and ghost image range the epilogue needs, loaded
         // before the pair loop
@@ -594,8 +627,9 @@ __global__ __launch_bounds__( 512 ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 )
             }
             if ( ctl.xg_next && ( G >= 4 ? sub < 4 : sub == 0 ) )
             {
-                img_b = ctl.img_start[i];
-                img_e = ctl.img_start[i + 1];
+                const int2 r = ctl.img_rng[i];
+                img_b = r.x;
+                img_e = r.y;
             }
         }
         // the atom about the tile's centre for FP32 records (inactive lanes
@@ -709,13 +743,8 @@ __global__ __launch_bounds__( 512 ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 )
                 quad( q2 );
             q2 = word( k + 5 );
         }
-        for ( int o = apw; o < 64; o <<= 1 )
-        {
-            fx += __shfl_xor( fx, o, 64 );
-            fy += __shfl_xor( fy, o, 64 );
-            fz += __shfl_xor( fz, o, 64 );
-        }
-        finish_atom<G, FUSED>( active, sub, i, xi, fx, fy, fz, scap, x_next, v,
+        sum_atom_lanes( apw, fx, fy, fz );
+        finish_atom<G, FUSED, ONE_TYPE>( active, sub, i, xi, fx, fy, fz, scap, x_next, v,
                                f, mt, ctl, mv2, vpre, img_b, img_e );
     }
     if ( FUSED && ENERGY )
@@ -766,11 +795,11 @@ __global__ __launch_bounds__( 512 ) void k_tile_half(
     // reaction records, then (energy only) a ghost flag per slot
     char *s_acc = s_byte + half_acc_offset( slot_cap, ONE_TYPE );
     int *s_gh = reinterpret_cast<int *>( s_acc + (size_t)slot_cap * TILE_REC );
-    const int total = H.segoff[H.nseg];
+    const int total = H.segoff()[H.nseg];
     if ( ENERGY )
     {
         for ( int k = threadIdx.x; k < slot_cap; k += blockDim.x )
-            s_gh[k] = k < total && ( find_seg( H.segoff, H.nseg, k ) & 1 );
+            s_gh[k] = k < total && ( find_seg( H.segoff(), H.nseg, k ) & 1 );
     }
     const int R4 = ( ( lcap + G - 1 ) / G + 3 ) / 4;
     const unsigned short *st = slab + (size_t)woff[t] * R4 * 256;
@@ -779,7 +808,7 @@ __global__ __launch_bounds__( 512 ) void k_tile_half(
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const int nwb = blockDim.x >> 6;
     const unsigned long long sent4 =
-        0x0001000100010001ull * (unsigned)( H.segoff[H.nseg] * TILE_REC );
+        0x0001000100010001ull * (unsigned)( H.segoff()[H.nseg] * TILE_REC );
     // the lane's atom in slab wave w: gw lanes per atom (G, or more in a
     // part-full wave), the atom, and the LDS slot it is staged at (its
     // staged column's local run); lanes past the atoms take the tile's
@@ -794,11 +823,11 @@ __global__ __launch_bounds__( 512 ) void k_tile_half(
         active = a < APW && ta < nat;
         const int tq = active ? ta : 0;
         int ac = 0;
-        while ( ac + 1 < T.W * T.W && tq >= H.aoff[ac + 1] )
+        while ( ac + 1 < T.W * T.W && tq >= H.aoff()[ac + 1] )
             ++ac;
-        i = H.info[TI_AL + ac] + ( tq - H.aoff[ac] );
+        i = H.info[TI_AL + ac] + ( tq - H.aoff()[ac] );
         const int qc = atom_col_q( T.W, ac );
-        islot = H.segoff[2 * qc] + ( i - H.info[TI_LB + qc] );
+        islot = H.segoff()[2 * qc] + ( i - H.info[TI_LB + qc] );
     };
     auto row_of = [&]( int w ) -> const unsigned long long *
     {
@@ -937,8 +966,8 @@ __global__ __launch_bounds__( 512 ) void k_tile_half(
             const double ax = r[0], ay = r[1], az = r[2];
             if ( ax == 0.0 && ay == 0.0 && az == 0.0 )
                 continue;
-            const int seg = find_seg( H.segoff, H.nseg, k );
-            const int q = seg >> 1, o = k - H.segoff[seg];
+            const int seg = find_seg( H.segoff(), H.nseg, k );
+            const int q = seg >> 1, o = k - H.segoff()[seg];
             const int idx = ( seg & 1 ) ? ghost_root[gperm[H.info[TI_GB + q] + o]]
                                         : H.info[TI_LB + q] + o;
             unsafeAtomicAdd( &f[idx], ax );

@@ -370,7 +370,7 @@ static cmd_status run_steps( cmd_md *md, int nsteps )
         {
             CMD_TRY( S->xg_alt.reserve( S->n_ghost ) );
             ctl.xg_next = S->xg_alt.p;
-            ctl.img_start = S->gimg.start.p;
+            ctl.img_rng = S->img_rng.p;
             ctl.img_pk = S->img_pk.p;
         }
         ghosts_next = ctl.xg_next != nullptr;

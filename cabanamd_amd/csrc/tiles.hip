@@ -62,14 +62,28 @@ static int max_force_slots( int rec )
 // in an interior cell of the grid), slots[2] the most slab waves of one
 // tile, slots[3] the largest staged count of one atom column's 3 x 3
 // columns (the list build's neighbourhood), slots[4] the most atoms of one
-// atom column (the list build's rows).
-__global__ void k_tile_info( TileGrid T, const int *__restrict__ ls,
-                             const int *__restrict__ gs, int apw,
-                             int *__restrict__ info, int *__restrict__ waves,
-                             int *__restrict__ slots )
+// atom column (the list build's rows); slots[TILE_RES_OUTSIDE] is copied
+// from the ghost sort's flag.
+//
+// One wave per tile, lane q = staged column q (25 at most): a thread per
+// tile ran through about a hundred dependent loads (12 us at 144 tiles, 20
+// us at 6,912; one wave per tile 4 and 7 us).  The maxima are joined in LDS
+// first, so the five result words see one atomic per 16 tiles.
+static constexpr int INFO_TPB = 1024;
+
+__global__ __launch_bounds__( INFO_TPB ) void k_tile_info(
+    TileGrid T, const int *__restrict__ ls, const int *__restrict__ gs, int apw,
+    const int *__restrict__ ghost_out, int *__restrict__ info, int *__restrict__ waves,
+    int *__restrict__ slots )
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    int total = 0, nat = 0, nwv = 0, bmax = 0, cmax = 0;
+    __shared__ int s_max[5];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    if ( threadIdx.x < 5 )
+        s_max[threadIdx.x] = 0;
+    if ( blockIdx.x == 0 && threadIdx.x == 0 )
+        slots[TILE_RES_OUTSIDE] = *ghost_out;
+    __syncthreads();
+    const int t = blockIdx.x * ( INFO_TPB / 64 ) + wid;
     if ( t < T.ntiles )
     {
         int a0, b0, e0, e1;
@@ -77,11 +91,11 @@ __global__ void k_tile_info( TileGrid T, const int *__restrict__ ls,
         const int ea = max( e0 - 1, 0 ), eb = min( e1 + 1, T.g.n[2] );
         const int S = T.W + 2;
         int *I = info + (size_t)t * TI_WORDS;
-        int len[TILE_QMAX];
-        for ( int q = 0; q < TILE_QMAX; ++q )
+        int len = 0, ll = 0;
+        if ( lane < TILE_QMAX )
         {
-            const int a = a0 - 1 + q / S, b = b0 - 1 + q % S;
-            int lb = 0, ll = 0, gb = 0, gl = 0;
+            const int q = lane, a = a0 - 1 + q / S, b = b0 - 1 + q % S;
+            int lb = 0, gb = 0, gl = 0;
             if ( q < S * S && a < T.g.n[0] && b < T.g.n[1] )
             {
                 const int c = col_base( T, a, b );
@@ -94,58 +108,77 @@ __global__ void k_tile_info( TileGrid T, const int *__restrict__ ls,
             I[TI_LLEN + q] = ll;
             I[TI_GB + q] = gb;
             I[TI_GLEN + q] = gl;
-            len[q] = ll + gl;
-            total += ll + gl;
+            len = ll + gl;
         }
-        for ( int c = 0; c < TILE_CMAX; ++c )
+        // lane c: atom column c, its atoms and its 3 x 3 columns' length
+        const int c = lane, ca = c / T.W, cb = c % T.W;
+        int an = 0, s9 = 0;
+        for ( int da = 0; da < 3; ++da )
+            for ( int db = 0; db < 3; ++db )
+                s9 += __shfl( len, ( ( ca + da ) * S + cb + db ) & 63, 64 );
+        const bool col =
+            c < T.W * T.W && a0 + ca <= T.g.n[0] - 2 && b0 + cb <= T.g.n[1] - 2;
+        if ( c < TILE_CMAX )
         {
-            const int ca = c / T.W, cb = c % T.W;
-            int al = 0, an = 0;
-            if ( c < T.W * T.W && a0 + ca <= T.g.n[0] - 2 && b0 + cb <= T.g.n[1] - 2 )
+            int al = 0;
+            if ( col )
             {
                 const int cc = col_base( T, a0 + ca, b0 + cb );
                 al = ls[cc + e0];
                 an = ls[cc + e1] - al;
-                int s9 = 0;
-                for ( int da = 0; da < 3; ++da )
-                    for ( int db = 0; db < 3; ++db )
-                        s9 += len[( ca + da ) * S + cb + db];
-                bmax = max( bmax, s9 );
             }
             I[TI_AL + c] = al;
             I[TI_AN + c] = an;
-            nat += an;
-            cmax = max( cmax, an );
         }
-        I[TI_NAT] = nat;
-        I[TI_TOTAL] = total;
-        I[TI_EA] = ea;
-        I[TI_NST] = eb - ea;
-        nwv = ( nat + apw - 1 ) / apw;
-        waves[t] = nwv;
-    }
-    int m = total;
+        // segment and atom-column offsets
+        int seg = len, ao = an;
 #pragma unroll
-    for ( int o = 32; o > 0; o >>= 1 )
-    {
-        m = max( m, __shfl_xor( m, o, 64 ) );
-        nat += __shfl_xor( nat, o, 64 );
-        nwv = max( nwv, __shfl_xor( nwv, o, 64 ) );
-        bmax = max( bmax, __shfl_xor( bmax, o, 64 ) );
-        cmax = max( cmax, __shfl_xor( cmax, o, 64 ) );
+        for ( int o = 1; o < 32; o <<= 1 )
+        {
+            const int u = __shfl_up( seg, o, 64 ), v = __shfl_up( ao, o, 64 );
+            seg += lane >= o ? u : 0;
+            ao += lane >= o ? v : 0;
+        }
+        if ( lane < TILE_QMAX )
+        {
+            I[TI_SEG + 2 * lane] = seg - len;
+            I[TI_SEG + 2 * lane + 1] = seg - len + ll;
+        }
+        else if ( lane == TILE_QMAX )
+            I[TI_SEG + TILE_SEGS] = seg; // the lanes past the columns add nothing
+        if ( lane <= TILE_CMAX )
+            I[TI_AOFF + lane] = ao - an;
+        int total = len, nat = an, bmax = col ? s9 : 0, cmax = an;
+#pragma unroll
+        for ( int o = 32; o > 0; o >>= 1 )
+        {
+            total += __shfl_xor( total, o, 64 );
+            nat += __shfl_xor( nat, o, 64 );
+            bmax = max( bmax, __shfl_xor( bmax, o, 64 ) );
+            cmax = max( cmax, __shfl_xor( cmax, o, 64 ) );
+        }
+        if ( lane == 0 )
+        {
+            const int nwv = ( nat + apw - 1 ) / apw;
+            I[TI_NAT] = nat;
+            I[TI_TOTAL] = total;
+            I[TI_EA] = ea;
+            I[TI_NST] = eb - ea;
+            waves[t] = nwv;
+            atomicMax( &s_max[0], total );
+            atomicAdd( &s_max[1], nat );
+            atomicMax( &s_max[2], nwv );
+            atomicMax( &s_max[3], bmax );
+            atomicMax( &s_max[4], cmax );
+        }
     }
-    if ( ( threadIdx.x & 63 ) == 0 )
+    __syncthreads();
+    if ( threadIdx.x < 5 && s_max[threadIdx.x] > 0 )
     {
-        if ( m > 0 )
-            atomicMax( &slots[0], m );
-        if ( nat > 0 )
-            atomicAdd( &slots[1], nat );
-        if ( nwv > 0 )
-            atomicMax( &slots[2], nwv );
-        if ( bmax > 0 )
-            atomicMax( &slots[3], bmax );
-        if ( cmax > 0 )
-            atomicMax( &slots[4], cmax );
+        if ( threadIdx.x == 1 )
+            atomicAdd( &slots[1], s_max[1] );
+        else
+            atomicMax( &slots[threadIdx.x], s_max[threadIdx.x] );
     }
 }
 
@@ -475,10 +508,10 @@ __global__ __launch_bounds__( BTPB ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 
         {
             const int qf = ( ca + qb / 3 ) * S + cb + qb % 3;
             s_bseg[2 * qb] = off;
-            s_dl[qb] = H.segoff[2 * qf] - off;
+            s_dl[qb] = H.segoff()[2 * qf] - off;
             off += H.info[TI_LLEN + qf];
             s_bseg[2 * qb + 1] = off;
-            s_dg[qb] = H.segoff[2 * qf + 1] - off;
+            s_dg[qb] = H.segoff()[2 * qf + 1] - off;
             off += H.info[TI_GLEN + qf];
         }
         s_bseg[18] = off;
@@ -560,7 +593,7 @@ __global__ __launch_bounds__( BTPB ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 
     const int al = H.info[TI_AL + c];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int nwv = blockDim.x >> 6;
-    const int fsent = H.segoff[H.nseg]; // the force tile's sentinel slot
+    const int fsent = H.segoff()[H.nseg]; // the force tile's sentinel slot
     // rows start as the force tile's sentinel record
     {
         const unsigned sent = (unsigned)( fsent * rec );
@@ -797,7 +830,7 @@ __global__ __launch_bounds__( BTPB ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 
         // wave's atom L % (64 / gw).  Only the words of this atom column's
         // atoms (tile atoms ta0 .. ta0 + nat_c - 1) are written; entries at
         // or past cap are the sentinel.
-        const int nat = H.info[TI_NAT], ta0 = H.aoff[c];
+        const int nat = H.info[TI_NAT], ta0 = H.aoff()[c];
         const int w0 = ta0 / APW, w1 = ( ta0 + nat_c - 1 ) / APW;
         const unsigned short sent = (unsigned short)( fsent * rec );
         for ( int sw = w0; sw <= w1; ++sw )
@@ -860,8 +893,8 @@ __global__ __launch_bounds__( TPB ) void k_tile_to_csr(
             const int r = k / gw, lane = ( k % gw ) * apw + aw;
             const int sj =
                 st[( ( w * R4 + ( r >> 2 ) ) * 64 + lane ) * 4 + ( r & 3 )] / rec;
-            const int seg = find_seg( H.segoff, H.nseg, sj );
-            const int q = seg >> 1, off = sj - H.segoff[seg];
+            const int seg = find_seg( H.segoff(), H.nseg, sj );
+            const int q = seg >> 1, off = sj - H.segoff()[seg];
             idx[o + k] = ( seg & 1 ) ? n_local + gperm[H.info[TI_GB + q] + off]
                                      : H.info[TI_LB + q] + off;
         }
@@ -901,37 +934,34 @@ __global__ void k_ghost_refresh_sorted( int n_local, int n_ghost,
     xg[k] = p;
 }
 
+// Positions of the sorted ghosts, the image entry of each (its sorted slot
+// and shift code, at its place in its root's range; pk null: no ranges) and
+// whether one lies outside the binning grid.  A place past the entries
+// (a halo pass that found other totals than its rows were sized for leaves
+// old ones; the rebuild then fails) is skipped.
 __global__ void k_gather_ghosts( int n_local, int n_ghost,
                                  const int *__restrict__ gperm,
                                  const double4 *__restrict__ x,
-                                 double4 *__restrict__ xg )
+                                 double4 *__restrict__ xg, const int *__restrict__ img_pos,
+                                 const int *__restrict__ code, int *__restrict__ pk,
+                                 double3 glo, double3 ghi, int *__restrict__ outside )
 {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if ( k < n_ghost )
-        xg[k] = x[n_local + gperm[k]];
-}
-
-// Root of the ghost at each sorted slot: the key that groups the slots by
-// local atom (the images the fused step writes).
-__global__ void k_image_roots( int n_ghost, const int *__restrict__ gperm,
-                               const int *__restrict__ root, int *__restrict__ key )
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if ( k < n_ghost )
-        key[k] = root[gperm[k]];
-}
-
-// Image entries in root order: sorted slot and shift code in one word.
-__global__ void k_image_pack( int n_ghost, const int *__restrict__ slot,
-                              const int *__restrict__ gperm,
-                              const int *__restrict__ code, int *__restrict__ pk )
-{
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if ( m < n_ghost )
+    if ( k >= n_ghost )
+        return;
+    const int g = gperm[k];
+    const double4 p = x[n_local + g];
+    xg[k] = p;
+    if ( pk )
     {
-        const int k = slot[m];
-        pk[m] = (int)( (unsigned)k | ( (unsigned)code[gperm[k]] << IMG_CODE_SHIFT ) );
+        const int m = img_pos[g];
+        if ( (unsigned)m < (unsigned)n_ghost )
+            pk[m] = (int)( (unsigned)k | ( (unsigned)code[g] << IMG_CODE_SHIFT ) );
     }
+    // (written so that a NaN counts as outside)
+    if ( !( p.x >= glo.x && p.y >= glo.y && p.z >= glo.z && p.x < ghi.x && p.y < ghi.y &&
+            p.z < ghi.z ) )
+        *outside = 1;
 }
 
 cmd_status tiles_prepare_ghosts( cmd_system *S )
@@ -944,31 +974,23 @@ cmd_status tiles_prepare_ghosts( cmd_system *S )
                         S->stream ) );
     CMD_TRY( S->xg.reserve( std::max( ng, 1 ) ) );
     CMD_TRY( S->xg_alt.reserve( std::max( ng, 1 ) ) );
+    CMD_TRY( S->img_pk.reserve( std::max( ng, 1 ) ) );
+    CMD_TRY( S->ghost_out.reserve( 1 ) );
+    CMD_TRY( fill_i32( S->ghost_out.p, 0, 1, S->stream ) );
+    // the image ranges are those of the halo pass that made these ghosts
+    S->img_valid = ng <= IMG_SLOT_MASK + 1 && S->halo_ghosts == ng &&
+                   S->halo_locals == S->n_local;
     if ( ng > 0 )
     {
+        const CellGrid &g = S->bin_grid;
         k_gather_ghosts<<<( ng + TPB - 1 ) / TPB, TPB, 0, S->stream>>>(
-            S->n_local, ng, S->gsort.perm.p, S->x.p, S->xg.p );
+            S->n_local, ng, S->gsort.perm.p, S->x.p, S->xg.p, S->img_pos.p, S->ghost_code.p,
+            S->img_valid ? S->img_pk.p : nullptr,
+            make_double3( g.min[0], g.min[1], g.min[2] ),
+            make_double3( g.min[0] + g.n[0] / g.rd[0], g.min[1] + g.n[1] / g.rd[1],
+                          g.min[2] + g.n[2] / g.rd[2] ),
+            S->ghost_out.p );
         CMD_LAUNCH_CHECK();
-    }
-    // sorted ghost slots grouped by their local atom
-    CMD_TRY( S->gimg.cell_of.reserve( std::max( ng, 1 ) ) );
-    if ( ng > 0 )
-    {
-        k_image_roots<<<( ng + TPB - 1 ) / TPB, TPB, 0, S->stream>>>(
-            ng, S->gsort.perm.p, S->ghost_root.p, S->gimg.cell_of.p );
-        CMD_LAUNCH_CHECK();
-    }
-    CMD_TRY( cell_sort_ids( ng, std::max( S->n_local, 1 ), S->gimg, S->sc, S->stream ) );
-    S->img_valid = ng <= IMG_SLOT_MASK + 1;
-    if ( S->img_valid )
-    {
-        CMD_TRY( S->img_pk.reserve( std::max( ng, 1 ) ) );
-        if ( ng > 0 )
-        {
-            k_image_pack<<<( ng + TPB - 1 ) / TPB, TPB, 0, S->stream>>>(
-                ng, S->gimg.perm.p, S->gsort.perm.p, S->ghost_code.p, S->img_pk.p );
-            CMD_LAUNCH_CHECK();
-        }
     }
     S->xg_valid = true;
     S->ghosts_x_stale = false;
@@ -1012,13 +1034,13 @@ static cmd_status tile_info_launch( cmd_neigh *N, cmd_system *S, int W, int E )
     DevBuf<int> &waves = N->grid_sort.cursor; // scratch: waves per tile
     CMD_TRY( waves.reserve( T.ntiles + 1 ) );
     CMD_TRY( N->grid_sort.start.reserve( T.ntiles + 1 ) ); // scan of waves
-    CMD_TRY( fill_i32( S->sc.ires.p + TILE_RES_INFO, 0, 5, S->stream ) );
+    // the maxima and the build's own words (longest row, capacity flag)
+    CMD_TRY( fill_i32( S->sc.ires.p, 0, TILE_RES_WORDS, S->stream ) );
     const int apw = 64 / N->lanes;
-    // one wave per block: a thread does a whole tile (about a hundred
-    // dependent loads), so the tiles are spread over as many CUs as possible
-    k_tile_info<<<( T.ntiles + 63 ) / 64, 64, 0, S->stream>>>(
-        T, S->bins.start.p, S->gsort.start.p, apw, N->tile_info.p, waves.p,
-        S->sc.ires.p + TILE_RES_INFO );
+    constexpr int per = INFO_TPB / 64;
+    k_tile_info<<<( T.ntiles + per - 1 ) / per, INFO_TPB, 0, S->stream>>>(
+        T, S->bins.start.p, S->gsort.start.p, apw, S->ghost_out.p, N->tile_info.p, waves.p,
+        S->sc.ires.p );
     CMD_LAUNCH_CHECK();
     CMD_TRY( scan_exclusive( waves.p, N->grid_sort.start.p, T.ntiles, S->sc,
                              S->stream, nullptr ) );
@@ -1150,9 +1172,6 @@ static void launch_build( cmd_neigh *N, cmd_system *S, int slot_cap, int rows_ca
 static cmd_status launch_build_g( cmd_neigh *N, cmd_system *S, int slot_cap, int rows_cap,
                                   int waves_cap, size_t lds )
 {
-    // the build's result words start at zero (the device test of the
-    // bounding box, when used, is left as it was written)
-    CMD_TRY( fill_i32( S->sc.ires.p + TILE_RES_MAXROW, 0, 2, S->stream ) );
     switch ( N->lanes )
     {
     case 2:
@@ -1214,18 +1233,23 @@ static void record_spec( cmd_neigh *N, int W, int E, const int h[6], int mr, siz
 {
     cmd_neigh::Spec &P = N->spec;
     P.valid = false;
-    if ( E != requested_height( N, W ) )
-        return; // a lowered height is chosen afresh at each build
     P.G = N->lanes;
     P.half = N->half;
     P.W = W;
     P.E = E;
+    P.E_req = requested_height( N, W ); // E may be a lowered one
     P.bw_req = N->tile_bw;
     P.cap = N->cap;
     if ( mr + std::max( 4, mr / 16 ) > P.cap )
         P.cap = mr + std::max( 8, mr / 8 );
-    P.slot_cap = std::min( h[3] + 1 + std::max( 16, h[3] / 32 ), MAX_SLOTS + 1 );
-    P.rows = h[4] + std::max( 2, h[4] / 20 );
+    // few tiles: their maxima are no extremes of many, and move by about the
+    // square root of the count from build to build (a box of 256 atoms went
+    // through the exact path at four rebuilds in five)
+    const bool few = N->tg.ntiles < 64;
+    auto dev = [&]( int v ) { return few ? (int)std::lround( 3.0 * std::sqrt( (double)v ) ) : 0; };
+    P.slot_cap =
+        std::min( h[3] + 1 + std::max( { 16, h[3] / 32, dev( h[3] ) } ), MAX_SLOTS + 1 );
+    P.rows = h[4] + std::max( { 2, h[4] / 20, dev( h[4] ) } );
     P.slab_waves = h[5] + std::max( 64, h[5] / 50 );
     P.lds = build_lds_cap( N->lanes, P.cap, P.slot_cap, P.rows );
     P.valid = P.lds <= hard;
@@ -1322,8 +1346,8 @@ cmd_status tiles_build( cmd_neigh *N, cmd_system *S, bool *built )
 
 // The tiled build launched with the sizes of the last one (record_spec) and
 // read back once, after the build: tile maxima, longest row, the capacity
-// flag of the build blocks and the device's bounding-box test (written by
-// the caller into TILE_RES_INSIDE).  Built only when every test passes and
+// flag of the build blocks and whether a ghost lies outside the grid (a
+// local atom outside it is one the tiles do not cover).  Built only when every test passes and
 // the layout is the one tiles_build would choose from these maxima;
 // otherwise *built stays false and the caller builds afresh.
 cmd_status tiles_build_spec( cmd_neigh *N, cmd_system *S, bool *built )
@@ -1335,7 +1359,7 @@ cmd_status tiles_build_spec( cmd_neigh *N, cmd_system *S, bool *built )
          P.half != N->half || P.cap < N->cap || P.bw_req != N->tile_bw )
         return CMD_OK;
     const int W = N->tile_w > 0 ? N->tile_w : 2;
-    if ( P.W != W || P.E != requested_height( N, W ) )
+    if ( P.W != W || P.E_req != requested_height( N, W ) )
         return CMD_OK;
     N->cap = P.cap; // grown ahead of the rows (record_spec)
     CMD_TRY( tile_info_launch( N, S, P.W, P.E ) );
@@ -1345,7 +1369,7 @@ cmd_status tiles_build_spec( cmd_neigh *N, cmd_system *S, bool *built )
     CMD_TRY( tile_results( N, S, res, &h[5], true ) );
     for ( int k = 0; k < 5; ++k )
         h[k] = res[TILE_RES_INFO + k];
-    if ( res[TILE_RES_INSIDE] != 1 || res[TILE_RES_OVER] != 0 || h[1] != S->n_local )
+    if ( res[TILE_RES_OUTSIDE] != 0 || res[TILE_RES_OVER] != 0 || h[1] != S->n_local )
         return CMD_OK;
     size_t hard = 0, lds_cu = 0;
     lds_limits( &hard, &lds_cu );

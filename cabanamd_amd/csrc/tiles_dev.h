@@ -18,7 +18,7 @@ namespace cmd
 constexpr int TILE_WMAX = 3;
 constexpr int TILE_QMAX = ( TILE_WMAX + 2 ) * ( TILE_WMAX + 2 ); // staged columns
 constexpr int TILE_CMAX = TILE_WMAX * TILE_WMAX;                 // atom columns
-static constexpr int TI_WORDS = 4 * TILE_QMAX + 2 * TILE_CMAX + 4;
+static constexpr int TILE_SEGS = 2 * TILE_QMAX; // segments: locals and ghosts of each column
 enum
 {
     TI_LB = 0,                         // [Q] first local index of each staged column run
@@ -30,7 +30,12 @@ enum
     TI_NAT = 4 * TILE_QMAX + 2 * TILE_CMAX, // atoms in the tile
     TI_TOTAL,                               // staged positions
     TI_EA,                                  // first staged cell (e0 - 1, clamped)
-    TI_NST                                  // staged cells per column
+    TI_NST,                                 // staged cells per column
+    TI_SEG,                                 // [SEGS + 1] segment offsets in slots (segment
+                                            // 2q = locals of staged column q, 2q + 1 = its
+                                            // ghosts; TOTAL past the tile's segments)
+    TI_AOFF = TI_SEG + TILE_SEGS + 1,       // [C + 1] tile-atom offsets of the atom columns
+    TI_WORDS = TI_AOFF + TILE_CMAX + 1
 };
 
 constexpr int TILE_STRIP = 4;
@@ -66,15 +71,14 @@ __device__ __forceinline__ int xcd_tile( int b, int nb )
     return ( xcd < r ) ? xcd * ( q + 1 ) + k : r * ( q + 1 ) + ( xcd - r ) * q + k;
 }
 
-// Shared tile header: info words, the segment offsets in LDS slots
-// (segment 2q = locals of staged column q, 2q + 1 = its ghosts) and the
-// tile-atom offsets of the atom columns.
+// Shared tile header: the info words (the segment offsets and atom-column
+// offsets are among them, laid out by k_tile_info).
 struct TileHead
 {
     int info[TI_WORDS];
-    int segoff[2 * TILE_QMAX + 1];
-    int aoff[TILE_CMAX + 1];
     int nseg; // 2 (W + 2)^2
+    __device__ const int *segoff() const { return info + TI_SEG; }
+    __device__ const int *aoff() const { return info + TI_AOFF; }
 };
 
 __device__ inline void load_head( const int *__restrict__ info, int t, int W, TileHead &H )
@@ -82,28 +86,8 @@ __device__ inline void load_head( const int *__restrict__ info, int t, int W, Ti
     const int *I = info + (size_t)t * TI_WORDS;
     for ( int k = threadIdx.x; k < TI_WORDS; k += blockDim.x )
         H.info[k] = I[k];
-    __syncthreads();
     if ( threadIdx.x == 0 )
-    {
-        const int nq = tile_q( W );
-        int off = 0;
-        for ( int q = 0; q < nq; ++q )
-        {
-            H.segoff[2 * q] = off;
-            off += H.info[TI_LLEN + q];
-            H.segoff[2 * q + 1] = off;
-            off += H.info[TI_GLEN + q];
-        }
-        H.segoff[2 * nq] = off;
-        H.nseg = 2 * nq;
-        int a = 0;
-        for ( int c = 0; c < W * W; ++c )
-        {
-            H.aoff[c] = a;
-            a += H.info[TI_AN + c];
-        }
-        H.aoff[W * W] = a;
-    }
+        H.nseg = 2 * tile_q( W );
     __syncthreads();
 }
 
@@ -111,9 +95,9 @@ __device__ inline void load_head( const int *__restrict__ info, int t, int W, Ti
 __device__ __forceinline__ int tile_atom( const TileHead &H, int W, int ta )
 {
     int c = 0;
-    while ( c + 1 < W * W && ta >= H.aoff[c + 1] )
+    while ( c + 1 < W * W && ta >= H.aoff()[c + 1] )
         ++c;
-    return H.info[TI_AL + c] + ( ta - H.aoff[c] );
+    return H.info[TI_AL + c] + ( ta - H.aoff()[c] );
 }
 
 // Staged column of atom column c.
@@ -175,7 +159,7 @@ __device__ inline void stage_records( const TileHead &H, const double4 *__restri
                                       double *__restrict__ zero = nullptr, int nzero = 0 )
 {
     int *s_t = reinterpret_cast<int *>( s_rec + 3 * cap );
-    const int total = H.segoff[H.nseg];
+    const int total = H.segoff()[H.nseg];
     constexpr int B = 8; // slots per thread whose loads are in flight together
     auto clear = [&]()
     {
@@ -190,8 +174,8 @@ __device__ inline void stage_records( const TileHead &H, const double4 *__restri
         {
             // past the end: reload the last slot (in bounds)
             const int k = min( k0 + u * (int)blockDim.x, total - 1 );
-            const int seg = find_seg( H.segoff, H.nseg, k );
-            const int q = seg >> 1, off = k - H.segoff[seg];
+            const int seg = find_seg( H.segoff(), H.nseg, k );
+            const int q = seg >> 1, off = k - H.segoff()[seg];
             const double4 *__restrict__ base = ( seg & 1 ) ? xg : x;
             const int idx = ( ( seg & 1 ) ? H.info[TI_GB + q] : H.info[TI_LB + q] ) + off;
             p[u] = base[idx];
@@ -225,46 +209,137 @@ __device__ inline void stage_records( const TileHead &H, const double4 *__restri
     __syncthreads();
 }
 
-// The same neighbourhood staged as 16-byte FP32 records for the
-// mixed-precision full-list kernel: x, y, z about the tile's centre (ox, oy,
-// oz; the staged region spans a few cells, so the coordinates keep about
-// 1e-7 of a cell in absolute precision) and the type's bits in w, followed
-// by the sentinel record.  Ends with a barrier.
-__device__ inline void stage_records32( const TileHead &H, const double4 *__restrict__ x,
-                                        const double4 *__restrict__ xg,
-                                        float4 *__restrict__ s_rec, double ox, double oy,
-                                        double oz )
+// Largest value of the wave's lanes (values >= 0), in row shifts and row
+// broadcasts of the adder's operand rather than LDS permutes.
+__device__ __forceinline__ int wave_max_i32( int v )
 {
-    const int total = H.segoff[H.nseg];
-    constexpr int B = 8; // slots per thread whose loads are in flight together
-    for ( int k0 = threadIdx.x; k0 < total; k0 += B * blockDim.x )
+#define CMD_MAX_DPP( CTRL )                                                                \
+    v = max( v, __builtin_amdgcn_update_dpp( 0, v, CTRL, 0xf, 0xf, true ) )
+    CMD_MAX_DPP( 0x111 ); // row_shr 1, 2, 4, 8: lane 15 of each row holds its maximum
+    CMD_MAX_DPP( 0x112 );
+    CMD_MAX_DPP( 0x114 );
+    CMD_MAX_DPP( 0x118 );
+    CMD_MAX_DPP( 0x142 ); // row_bcast 15, then 31: lane 63 holds the wave's
+    CMD_MAX_DPP( 0x143 );
+#undef CMD_MAX_DPP
+    return __builtin_amdgcn_readlane( v, 63 );
+}
+
+// v plus the value of the lane O away (lane ^ O), O = 8, 16 or 32.
+template <int O>
+__device__ __forceinline__ double add_lane_xor( double v )
+{
+    const unsigned long long b = (unsigned long long)__double_as_longlong( v );
+    const unsigned lo = (unsigned)b, hi = (unsigned)( b >> 32 );
+    auto join = []( unsigned l, unsigned h )
+    { return __longlong_as_double( (long long)( ( (unsigned long long)h << 32 ) | l ) ); };
+    if constexpr ( O == 8 )
+    {
+        // row_ror:8 turns each row of 16 lanes by half
+        const unsigned l = (unsigned)__builtin_amdgcn_update_dpp( 0, (int)lo, 0x128, 0xf, 0xf, true );
+        const unsigned h = (unsigned)__builtin_amdgcn_update_dpp( 0, (int)hi, 0x128, 0xf, 0xf, true );
+        return v + join( l, h );
+    }
+    else
+    {
+        // the swap leaves one half's (or row pair's) values in all lanes of
+        // one result and the other's in the other
+        const auto l = O == 32 ? __builtin_amdgcn_permlane32_swap( lo, lo, false, false )
+                               : __builtin_amdgcn_permlane16_swap( lo, lo, false, false );
+        const auto h = O == 32 ? __builtin_amdgcn_permlane32_swap( hi, hi, false, false )
+                               : __builtin_amdgcn_permlane16_swap( hi, hi, false, false );
+        return join( l[0], h[0] ) + join( l[1], h[1] );
+    }
+}
+
+// Sum over the lanes of one atom: lane pairs apw, 2 apw, ... apart (apw = 8,
+// 16 or 32 atoms per wave; wave-uniform).
+__device__ __forceinline__ void sum_atom_lanes( int apw, double &a, double &b, double &c )
+{
+    if ( apw <= 8 )
+    {
+        a = add_lane_xor<8>( a );
+        b = add_lane_xor<8>( b );
+        c = add_lane_xor<8>( c );
+    }
+    if ( apw <= 16 )
+    {
+        a = add_lane_xor<16>( a );
+        b = add_lane_xor<16>( b );
+        c = add_lane_xor<16>( c );
+    }
+    a = add_lane_xor<32>( a );
+    b = add_lane_xor<32>( b );
+    c = add_lane_xor<32>( c );
+}
+
+// Walk of a tile's staged positions for the full-list force kernel, straight
+// from the tile's info words: the segments (lane s of a wave holds segment
+// s: 50 at most) are cut into chunks of 64 and wave w of nw takes chunks w,
+// w + nw, ...; put(slot, p) gets each lane's position with its slot.  A
+// chunk's segment is the number of segments that end at or before it (one
+// compare and a scalar count), so no lane searches for its segment, the
+// loads of a wave are consecutive, and up to B chunks are in flight.  A block
+// that first copied the info words to LDS, chained the segment offsets in one
+// thread and searched them per slot spent about a tenth of its time there:
+// with this walk and the cross-lane sums above the force kernel went from 222
+// to 194 us (2,048,000 atoms, mixed), 152 to 133 us (864,000, FP64) and 17.2
+// to 13.1 us (48,000, two types, mixed).
+template <class Put>
+__device__ __forceinline__ void stage_chunks( const int *__restrict__ I, int nseg, int wid,
+                                              int nw, const double4 *__restrict__ x,
+                                              const double4 *__restrict__ xg, Put put )
+{
+    const int lane = threadIdx.x & 63;
+    int src = 0, len = 0, dst = 0;
+    if ( lane < nseg )
+    {
+        const int q = lane >> 1, g = lane & 1;
+        src = I[( g ? TI_GB : TI_LB ) + q];
+        len = I[( g ? TI_GLEN : TI_LLEN ) + q];
+        dst = I[TI_SEG + lane];
+    }
+    // chunks of the segments up to and including the lane's
+    int inc = ( len + 63 ) >> 6;
+#define CMD_SCAN_DPP( CTRL, ROWS )                                                         \
+    inc += __builtin_amdgcn_update_dpp( 0, inc, CTRL, ROWS, 0xf, true )
+    CMD_SCAN_DPP( 0x111, 0xf );
+    CMD_SCAN_DPP( 0x112, 0xf );
+    CMD_SCAN_DPP( 0x114, 0xf );
+    CMD_SCAN_DPP( 0x118, 0xf );
+    CMD_SCAN_DPP( 0x142, 0xa ); // rows 1 and 3 take the row before's total
+    CMD_SCAN_DPP( 0x143, 0xc ); // rows 2 and 3 take the first half's
+#undef CMD_SCAN_DPP
+    const int nch = __builtin_amdgcn_readlane( inc, 63 );
+    constexpr int B = 8; // chunks of a wave in flight together
+    for ( int c0 = wid; c0 < nch; c0 += B * nw )
     {
         double4 p[B];
+        int slot[B];
 #pragma unroll
         for ( int u = 0; u < B; ++u )
         {
-            // past the end: reload the last slot (in bounds)
-            const int k = min( k0 + u * (int)blockDim.x, total - 1 );
-            const int seg = find_seg( H.segoff, H.nseg, k );
-            const int q = seg >> 1, off = k - H.segoff[seg];
-            const double4 *__restrict__ base = ( seg & 1 ) ? xg : x;
-            const int idx = ( ( seg & 1 ) ? H.info[TI_GB + q] : H.info[TI_LB + q] ) + off;
-            p[u] = base[idx];
+            const int c = c0 + u * nw;
+            slot[u] = -1;
+            if ( c < nch ) // wave-uniform
+            {
+                const int s =
+                    (int)__popcll( __builtin_amdgcn_ballot_w64( inc <= c ) );
+                const int sl = __builtin_amdgcn_readlane( len, s );
+                const int first = __builtin_amdgcn_readlane( inc, s ) - ( ( sl + 63 ) >> 6 );
+                const int o = ( ( c - first ) << 6 ) + lane;
+                const double4 *__restrict__ base = ( s & 1 ) ? xg : x;
+                // lanes past the segment's end reload its last position
+                p[u] = base[__builtin_amdgcn_readlane( src, s ) + min( o, sl - 1 )];
+                if ( o < sl )
+                    slot[u] = __builtin_amdgcn_readlane( dst, s ) + o;
+            }
         }
-        // stores past the end go to the sentinel record, rewritten below
 #pragma unroll
         for ( int u = 0; u < B; ++u )
-        {
-            const int k = min( k0 + u * (int)blockDim.x, total );
-            s_rec[k] = make_float4( (float)( p[u].x - ox ), (float)( p[u].y - oy ),
-                                    (float)( p[u].z - oz ), __int_as_float( (int)p[u].w ) );
-        }
+            if ( slot[u] >= 0 )
+                put( slot[u], p[u] );
     }
-    __syncthreads();
-    if ( threadIdx.x == 0 )
-        s_rec[total] = make_float4( (float)TILE_FAR, (float)TILE_FAR, (float)TILE_FAR,
-                                    __int_as_float( 0 ) );
-    __syncthreads();
 }
 
 // Centre of tile t's staged region, the origin of its FP32 records.
