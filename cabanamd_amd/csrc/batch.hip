@@ -343,8 +343,8 @@ __global__ __launch_bounds__( 256 ) void k_b_neigh_cell(
 #pragma unroll
     for ( int o = 32; o > 0; o >>= 1 )
         mrow = max( mrow, __shfl_xor( mrow, o, 64 ) );
-    if ( lane == 0 && mrow > 0 )
-        atomicMax( max_row, mrow );
+    if ( lane == 0 )
+        raise_max( max_row, mrow );
 }
 
 // Per-atom thermo terms in FP64: pe_i = 1/2 sum_j shifted LJ over the full

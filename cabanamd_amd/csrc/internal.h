@@ -213,6 +213,15 @@ struct CellGrid
     int floor_mode; // 1: floor() (Cabana LinkedCellList); 0: truncation
 };
 
+// Raise the maximum at p (device memory, every block's) to v.  The atomics of
+// one address are served one after another, and after a kernel's first few
+// blocks hardly any raises a maximum, so the value is looked at first.
+__device__ __forceinline__ void raise_max( int *p, int v )
+{
+    if ( v > __hip_atomic_load( p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT ) )
+        atomicMax( p, v );
+}
+
 __device__ __forceinline__ int cell_coord( double c, double mn, double rd,
                                            int n, int floor_mode )
 {
@@ -351,6 +360,12 @@ struct cmd_neigh
     int max_row = 0;
     cmd::DevBuf<int> slab;   // lane-interleaved rows, see neighbor.hip
     cmd::DevBuf<int> counts; // per-row lengths
+    // Tiled half lists hold every neighbour of an atom (forces walk the full
+    // rows, with no reactions to add), an entry's low bit marking the pairs of
+    // the half list: fcounts are the full rows' lengths, counts the half
+    // list's.
+    cmd::DevBuf<int> fcounts;
+    const int *row_counts() const { return tiled && half ? fcounts.p : counts.p; }
     bool csr_valid = false;
     cmd::DevBuf<int64_t> offsets; // CSR view (on demand)
     cmd::DevBuf<int> idx;
@@ -447,8 +462,6 @@ struct StepCtl
     int wrap_next;        // wrap the drifted positions (next step rebuilds)
     int thermo;           // accumulate KE, PE and virial partials
     int write_f;          // store f
-    int zero_f;           // (integrator) clear f after reading it: the next
-                          // step's forces accumulate into it
     // when set (with do_next_initial and no wrap), the drifted position of
     // every local atom is also written, shifted per its images' codes, to
     // xg_next at its sorted ghost slots: the next step's ghost refresh
@@ -531,7 +544,8 @@ enum
     TILE_RES_OVER = 6,     // 1: a block's needs exceeded the launch sizes
     TILE_RES_OUTSIDE = 7,  // 1: a ghost lies outside the binning grid
     TILE_RES_WAVES = 8,    // slab waves of all tiles (written by the build)
-    TILE_RES_WORDS = 9
+    TILE_RES_MAXHALF = 9,  // longest row of a half list
+    TILE_RES_WORDS = 10
 };
 static_assert( HW_TILE + TILE_RES_WORDS <= HW_WORDS, "tile results fit the pinned words" );
 cmd_status tiles_csr( cmd_neigh *N, int64_t *nnz );

@@ -496,9 +496,6 @@ __global__ __launch_bounds__( 512 ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 )
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane( threadIdx.x >> 6 );
     const int nwb = blockDim.x >> 6;
-    // four sentinel entries: the word a lane past the tile's atoms walks
-    constexpr int REC = F32REC ? TILE_REC32 : TILE_REC;
-    const unsigned long long sent4 = 0x0001000100010001ull * (unsigned)( total * REC );
     // FP32 records: coordinates about the centre of the staged region
     double ox = 0.0, oy = 0.0, oz = 0.0;
     if constexpr ( F32REC )
@@ -665,7 +662,11 @@ __global__ __launch_bounds__( 512 ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 )
             fy = __builtin_fma( (double)dy, fpd, fy );
             fz = __builtin_fma( (double)dz, fpd, fz );
         };
-        auto body = [&]( const double4 &xj )
+        // FP64 records.  A half list's rows hold its pairs from both sides,
+        // entries of ghosts marked (bit 1): its energy counts a pair with a
+        // ghost 1/2, another 1 (compute_energy_half), so before the factor
+        // 1/2 of a pair seen twice a marked one weighs 1/2.
+        auto body = [&]( const double4 &xj, bool ghost )
         {
             const double dx = xi.x - xj.x;
             const double dy = xi.y - xj.y;
@@ -674,7 +675,10 @@ __global__ __launch_bounds__( 512 ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 )
                                    ? dx * dx + dy * dy + dz * dz
                                    : __builtin_fma( dx, dx, __builtin_fma( dy, dy, dz * dz ) );
             const PairCoef c = coef<ONE_TYPE>( Pd, one, ti, (int)xj.w );
-            const double fpair = lj_pair<PREC, ENERGY>( rsq, c, pe, vir );
+            double e = 0.0;
+            const double fpair = lj_pair<PREC, ENERGY>( rsq, c, e, vir );
+            if ( ENERGY )
+                pe += ghost ? 0.5 * e : e;
             accumulate<PREC>( fx, fy, fz, dx, dy, dz, fpair );
         };
         // four records per 8-byte word of byte offsets; all four LDS reads
@@ -692,10 +696,11 @@ __global__ __launch_bounds__( 512 ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 )
         // (a rotation through registers would wait for the newest load).
         // Every lane loads from its own column of the wave's slab, which
         // holds at least max(nq, 1) words for all 64 lanes; lanes past the
-        // tile's atoms use the sentinel word in place of what their column
-        // holds.  Loads are issued unconditionally (indexes past the last
+        // tile's atoms walk record 0 from their far point instead (keep, which
+        // also takes off a half list's marks).  Loads are issued unconditionally (indexes past the last
         // word re-read it), so the count of loads in flight is the same on
         // every path and the wait before a use covers only that word.
+        const unsigned long long keep = active ? 0xfff8fff8fff8fff8ull : 0ull;
         const int nq = ( nr + 3 ) / 4;
         const int klast = max( nq - 1, 0 );
         auto word = [&]( int k ) -> unsigned long long
@@ -707,7 +712,7 @@ __global__ __launch_bounds__( 512 ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 )
         };
         auto quad = [&]( unsigned long long wd )
         {
-            const unsigned long long cur = active ? wd : sent4;
+            const unsigned long long cur = wd & keep;
             if constexpr ( F32REC )
             {
                 const float4 p0 = fetch32( cur, 0 );
@@ -725,10 +730,10 @@ __global__ __launch_bounds__( 512 ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 )
                 const double4 p1 = fetch( cur, 1 );
                 const double4 p2 = fetch( cur, 2 );
                 const double4 p3 = fetch( cur, 3 );
-                body( p0 );
-                body( p1 );
-                body( p2 );
-                body( p3 );
+                body( p0, ENERGY && ( wd & 2 ) );
+                body( p1, ENERGY && ( wd >> 16 & 2 ) );
+                body( p2, ENERGY && ( wd >> 32 & 2 ) );
+                body( p3, ENERGY && ( wd >> 48 & 2 ) );
             }
         };
         unsigned long long q0 = P.q0, q1 = P.q1, q2 = P.q2;
@@ -755,228 +760,6 @@ __global__ __launch_bounds__( 512 ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 )
         block_sum4_in( mv2, 0.5 * pe, 0.5 * vir, 0.0, partial + 4 * blockIdx.x,
                        reinterpret_cast<double( * )[8]>( s_rec ) );
     }
-}
-
-// LDS bytes before the reaction records of the tiled half-list kernel: the
-// position records and, with several types, an int type per slot.
-__host__ __device__ constexpr size_t half_acc_offset( int slot_cap, bool one_type )
-{
-    return ( (size_t)slot_cap * TILE_REC + ( one_type ? 0 : (size_t)slot_cap * sizeof( int ) ) +
-             7 ) & ~(size_t)7;
-}
-
-// Tiled half list (compute_force_half, force_lj_cabana_neigh_impl.h:205-259):
-// each listed pair once, both sides accumulated.  The block stages its
-// tile's neighbourhood as records, with an FP64 reaction record per staged
-// slot in LDS at the same byte offset in a second area.  A pair adds d fpair
-// to atom i (registers) and subtracts it from slot j's reaction record (LDS
-// atomics); the atom's own total joins its slot's record.  When every row
-// of the tile is done, each slot with a nonzero record adds it to f of its
-// atom with global atomics (an atom is staged by several tiles); ghost
-// slots go to the local atoms they image, so update_force's fold has
-// nothing left to add.  Energy weights follow compute_energy_half: 1 for a
-// local j, 1/2 for a ghost j.
-template <int G, int PREC, bool ONE_TYPE, bool ENERGY>
-__global__ __launch_bounds__( 512 ) void k_tile_half(
-    TileGrid T, const int *__restrict__ info, const int *__restrict__ woff,
-    int lcap, int scap, int slot_cap, const double4 *__restrict__ x,
-    const double4 *__restrict__ xg, const int *__restrict__ gperm,
-    const int *__restrict__ ghost_root, double *__restrict__ f,
-    const int *__restrict__ counts, const unsigned short *__restrict__ slab,
-    const LJParams *__restrict__ Pd, PairCoef one, double *__restrict__ partial )
-{
-    extern __shared__ double s_rec[];
-    __shared__ TileHead H;
-    constexpr int APW = 64 / G;
-    const int t = xcd_tile( blockIdx.x, gridDim.x );
-    load_head( info, t, T.W, H );
-    char *s_byte = reinterpret_cast<char *>( s_rec );
-    const int *s_t = reinterpret_cast<const int *>( s_rec + 3 * slot_cap );
-    // reaction records, then (energy only) a ghost flag per slot
-    char *s_acc = s_byte + half_acc_offset( slot_cap, ONE_TYPE );
-    int *s_gh = reinterpret_cast<int *>( s_acc + (size_t)slot_cap * TILE_REC );
-    const int total = H.segoff()[H.nseg];
-    if ( ENERGY )
-    {
-        for ( int k = threadIdx.x; k < slot_cap; k += blockDim.x )
-            s_gh[k] = k < total && ( find_seg( H.segoff(), H.nseg, k ) & 1 );
-    }
-    const int R4 = ( ( lcap + G - 1 ) / G + 3 ) / 4;
-    const unsigned short *st = slab + (size_t)woff[t] * R4 * 256;
-    const int nw = woff[t + 1] - woff[t];
-    const int nat = H.info[TI_NAT];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const int nwb = blockDim.x >> 6;
-    const unsigned long long sent4 =
-        0x0001000100010001ull * (unsigned)( H.segoff()[H.nseg] * TILE_REC );
-    // the lane's atom in slab wave w: gw lanes per atom (G, or more in a
-    // part-full wave), the atom, and the LDS slot it is staged at (its
-    // staged column's local run); lanes past the atoms take the tile's
-    // first atom
-    auto lane_map = [&]( int w, int &gw, int &apw, int &sub, int &i, int &islot, bool &active )
-    {
-        gw = wave_lanes( G, nat, w );
-        apw = 64 / gw;
-        const int a = lane % apw;
-        sub = lane / apw;
-        const int ta = w * APW + a;
-        active = a < APW && ta < nat;
-        const int tq = active ? ta : 0;
-        int ac = 0;
-        while ( ac + 1 < T.W * T.W && tq >= H.aoff()[ac + 1] )
-            ++ac;
-        i = H.info[TI_AL + ac] + ( tq - H.aoff()[ac] );
-        const int qc = atom_col_q( T.W, ac );
-        islot = H.segoff()[2 * qc] + ( i - H.info[TI_LB + qc] );
-    };
-    auto row_of = [&]( int w ) -> const unsigned long long *
-    {
-        return reinterpret_cast<const unsigned long long *>(
-            st + ( (size_t)w * R4 * 64 + lane ) * 4 );
-    };
-    // the atom's position, row length and first three list words, loaded
-    // before the staging so that their memory latency overlaps it (words
-    // past a row's end are loaded but not used)
-    struct WaveIn
-    {
-        double4 xi;
-        int n;
-        unsigned long long q0, q1, q2;
-    };
-    auto prep = [&]( int w, WaveIn &P )
-    {
-        int gw, apw, sub, i, islot;
-        bool active;
-        lane_map( w, gw, apw, sub, i, islot, active );
-        P.xi = x[i];
-        P.n = counts[i];
-        const unsigned long long *row8 = row_of( w );
-        P.q0 = __builtin_nontemporal_load( row8 );
-        __builtin_amdgcn_sched_barrier( 0 );
-        P.q1 = __builtin_nontemporal_load( row8 + (size_t)min( 1, R4 - 1 ) * 64 );
-        __builtin_amdgcn_sched_barrier( 0 );
-        P.q2 = __builtin_nontemporal_load( row8 + (size_t)min( 2, R4 - 1 ) * 64 );
-        __builtin_amdgcn_sched_barrier( 0 );
-    };
-    WaveIn P;
-    if ( wid < nw )
-        prep( wid, P );
-    // the reaction records are cleared while the staging loads are in flight
-    stage_records<!ONE_TYPE>( H, x, xg, s_rec, slot_cap, reinterpret_cast<double *>( s_acc ),
-                              3 * slot_cap ); // ends with a barrier
-    double pe = 0.0, vir = 0.0;
-    for ( int w = wid; w < nw; w += nwb )
-    {
-        if ( w != wid )
-            prep( w, P );
-        int gw, apw, sub, i, islot;
-        bool active;
-        lane_map( w, gw, apw, sub, i, islot, active );
-        double fx = 0.0, fy = 0.0, fz = 0.0;
-        const double4 xi =
-            active ? P.xi : make_double4( -TILE_FAR, -TILE_FAR, -TILE_FAR, 0.0 );
-        const int ti = (int)xi.w;
-        const int n = active ? P.n : 0;
-        int nr = n > sub ? ( n - sub + gw - 1 ) / gw : 0;
-#pragma unroll
-        for ( int o = 32; o > 0; o >>= 1 )
-            nr = max( nr, __shfl_xor( nr, o, 64 ) );
-        nr = __builtin_amdgcn_readfirstlane( nr );
-        const unsigned long long *row8 = row_of( w );
-        auto body = [&]( unsigned off )
-        {
-            const double *p = reinterpret_cast<const double *>( s_byte + off );
-            const double dx = xi.x - p[0];
-            const double dy = xi.y - p[1];
-            const double dz = xi.z - p[2];
-            const double rsq = dx * dx + dy * dy + dz * dz;
-            const PairCoef c =
-                coef<ONE_TYPE>( Pd, one, ti, ONE_TYPE ? 0 : s_t[off / TILE_REC] );
-            double ep = 0.0, wp = 0.0;
-            const double fpair = lj_pair<PREC, ENERGY>( rsq, c, ep, wp );
-            if ( ENERGY )
-            {
-                pe += ( s_gh[off / TILE_REC] ? 0.5 : 1.0 ) * ep;
-                vir += wp;
-            }
-            if ( rsq < c.cs )
-            {
-                const double ax = dx * fpair, ay = dy * fpair, az = dz * fpair;
-                fx += ax;
-                fy += ay;
-                fz += az;
-                double *r = reinterpret_cast<double *>( s_acc + off );
-                unsafeAtomicAdd( r, -ax );
-                unsafeAtomicAdd( r + 1, -ay );
-                unsafeAtomicAdd( r + 2, -az );
-            }
-        };
-        // list words three loads ahead, as in the full-list kernel: every
-        // lane loads from its own column of the wave's slab (indexes past
-        // the row's last word re-read it) and lanes past the tile's atoms
-        // walk the sentinel in place of what their column holds
-        const int nq = ( nr + 3 ) / 4;
-        const int klast = max( nq - 1, 0 );
-        auto word = [&]( int k ) -> unsigned long long
-        { return __builtin_nontemporal_load( row8 + (size_t)min( k, klast ) * 64 ); };
-        auto quad = [&]( unsigned long long w8 )
-        {
-            const unsigned long long wd = active ? w8 : sent4;
-            body( (unsigned)( wd & 0xffffull ) );
-            body( (unsigned)( ( wd >> 16 ) & 0xffffull ) );
-            body( (unsigned)( ( wd >> 32 ) & 0xffffull ) );
-            body( (unsigned)( wd >> 48 ) );
-        };
-        unsigned long long q0 = P.q0, q1 = P.q1, q2 = P.q2;
-        for ( int k = 0; k < nq; k += 3 )
-        {
-            quad( q0 );
-            q0 = word( k + 3 );
-            if ( k + 1 < nq )
-                quad( q1 );
-            q1 = word( k + 4 );
-            if ( k + 2 < nq )
-                quad( q2 );
-            q2 = word( k + 5 );
-        }
-        for ( int o = apw; o < 64; o <<= 1 )
-        {
-            fx += __shfl_xor( fx, o, 64 );
-            fy += __shfl_xor( fy, o, 64 );
-            fz += __shfl_xor( fz, o, 64 );
-        }
-        if ( active && sub == 0 )
-        {
-            double *r = reinterpret_cast<double *>( s_acc + islot * TILE_REC );
-            unsafeAtomicAdd( r, fx );
-            unsafeAtomicAdd( r + 1, fy );
-            unsafeAtomicAdd( r + 2, fz );
-        }
-    }
-    __syncthreads();
-    // every staged slot with a reaction: locals by run start, ghosts through
-    // the ghost sort permutation to the local atoms they image (a ghost's
-    // force is its source atom's, which is what update_force's fold of the
-    // ghost rows gives: the ghost rows are left untouched, and a fold adds
-    // nothing)
-    {
-        for ( int k = threadIdx.x; k < total; k += blockDim.x )
-        {
-            const double *r = reinterpret_cast<const double *>( s_acc + k * TILE_REC );
-            const double ax = r[0], ay = r[1], az = r[2];
-            if ( ax == 0.0 && ay == 0.0 && az == 0.0 )
-                continue;
-            const int seg = find_seg( H.segoff(), H.nseg, k );
-            const int q = seg >> 1, o = k - H.segoff()[seg];
-            const int idx = ( seg & 1 ) ? ghost_root[gperm[H.info[TI_GB + q] + o]]
-                                        : H.info[TI_LB + q] + o;
-            unsafeAtomicAdd( &f[idx], ax );
-            unsafeAtomicAdd( &f[scap + idx], ay );
-            unsafeAtomicAdd( &f[2 * scap + idx], az );
-        }
-    }
-    if ( ENERGY )
-        block_sum4( 0.0, pe, vir, 0.0, partial + 4 * blockIdx.x );
 }
 
 // Half list: each listed pair once; the reaction goes to j by atomics
@@ -1224,7 +1007,7 @@ static void launch_tile_k( cmd_neigh *N, cmd_system *S, double4 *xn,
             k_tile_force<G, PREC, ONE, FUSED, ENERGY, true>
                 <<<N->tg.ntiles, 64 * N->tg.bw, lds, S->stream>>>(
                     N->tg, N->tile_info.p, N->grid_sort.start.p, N->cap, S->cap, slot_cap,
-                    S->x.p, S->xg.p, xn, S->v.p, S->f.p, N->counts.p, N->tslab.p, Pd, c, mt,
+                    S->x.p, S->xg.p, xn, S->v.p, S->f.p, N->row_counts(), N->tslab.p, Pd, c, mt,
                     ctl, partial );
             return;
         }
@@ -1234,7 +1017,7 @@ static void launch_tile_k( cmd_neigh *N, cmd_system *S, double4 *xn,
         (size_t)slot_cap * ( TILE_REC + ( ONE ? 0 : sizeof( int ) ) ), 32 * sizeof( double ) );
     k_tile_force<G, PREC, ONE, FUSED, ENERGY, false><<<N->tg.ntiles, 64 * N->tg.bw, lds, S->stream>>>(
         N->tg, N->tile_info.p, N->grid_sort.start.p, N->cap, S->cap, slot_cap,
-        S->x.p, S->xg.p, xn, S->v.p, S->f.p, N->counts.p, N->tslab.p, Pd, c, mt,
+        S->x.p, S->xg.p, xn, S->v.p, S->f.p, N->row_counts(), N->tslab.p, Pd, c, mt,
         ctl, partial );
 }
 
@@ -1396,69 +1179,12 @@ static void launch_half_t( const cmd_force *F, cmd_system *S, const cmd_neigh *N
     }
 }
 
-template <int G, int PREC, bool ONE, bool ENERGY>
-static void launch_tile_half_k( const cmd_neigh *N, cmd_system *S, const LJParams *Pd,
-                                const PairCoef &c, double *partial )
-{
-    const int slot_cap = std::max( N->max_tile_slots, 1 ) + 1;
-    const size_t lds = half_acc_offset( slot_cap, ONE ) + (size_t)slot_cap * TILE_REC +
-                       ( ENERGY ? (size_t)slot_cap * sizeof( int ) : 0 );
-    k_tile_half<G, PREC, ONE, ENERGY><<<N->tg.ntiles, 64 * N->tg.bw, lds, S->stream>>>(
-        N->tg, N->tile_info.p, N->grid_sort.start.p, N->cap, S->cap, slot_cap, S->x.p,
-        S->xg.p, S->gsort.perm.p, S->ghost_root.p, S->f.p, N->counts.p, N->tslab.p, Pd, c,
-        partial );
-}
-
-template <int G, int PREC>
-static void launch_tile_half_t( const cmd_neigh *N, cmd_system *S, bool one, bool thermo,
-                                const LJParams *Pd, const PairCoef &c, double *partial )
-{
-    if ( one )
-    {
-        if ( thermo )
-            launch_tile_half_k<G, PREC, true, true>( N, S, Pd, c, partial );
-        else
-            launch_tile_half_k<G, PREC, true, false>( N, S, Pd, c, partial );
-    }
-    else
-    {
-        if ( thermo )
-            launch_tile_half_k<G, PREC, false, true>( N, S, Pd, c, partial );
-        else
-            launch_tile_half_k<G, PREC, false, false>( N, S, Pd, c, partial );
-    }
-}
-
-template <int PREC>
-static cmd_status launch_tile_half( const cmd_neigh *N, cmd_system *S, bool one,
-                                    bool thermo, const LJParams *Pd, const PairCoef &c,
-                                    double *partial )
-{
-    switch ( N->lanes )
-    {
-    case 2:
-        launch_tile_half_t<2, PREC>( N, S, one, thermo, Pd, c, partial );
-        break;
-    case 4:
-        launch_tile_half_t<4, PREC>( N, S, one, thermo, Pd, c, partial );
-        break;
-    case 8:
-        launch_tile_half_t<8, PREC>( N, S, one, thermo, Pd, c, partial );
-        break;
-    default:
-        set_error( "tiled lists need 2, 4 or 8 lanes per atom" );
-        return CMD_ERR_ARG;
-    }
-    CMD_LAUNCH_CHECK();
-    return CMD_OK;
-}
-
 cmd_status lj_half( const cmd_force *F, cmd_system *S, const cmd_neigh *N,
                     int thermo, double *partial, int *nblocks_out )
 {
     const int n = S->n_local;
     const int G = N->lanes;
-    const int nb = N->tiled ? N->tg.ntiles : blocks_for( n, G );
+    const int nb = blocks_for( n, G );
     if ( nblocks_out )
         *nblocks_out = nb;
     if ( n == 0 )
@@ -1469,15 +1195,6 @@ cmd_status lj_half( const cmd_force *F, cmd_system *S, const cmd_neigh *N,
     LJParams *Pd = nullptr;
     if ( F->ntypes != 1 )
         CMD_TRY( upload_params( F, S->stream, &Pd ) );
-    if ( N->tiled )
-    {
-        CMD_REQUIRE( S->xg_valid, CMD_ERR_STATE,
-                     "tiled list needs the sorted ghosts of its build" );
-        const bool one = F->ntypes == 1;
-        if ( F->prec == CMD_PREC_FP64 )
-            return launch_tile_half<CMD_PREC_FP64>( N, S, one, thermo != 0, Pd, c, partial );
-        return launch_tile_half<CMD_PREC_MIXED>( N, S, one, thermo != 0, Pd, c, partial );
-    }
     switch ( G )
     {
     case 1:
@@ -1706,7 +1423,7 @@ cmd_status force_compute_plain( cmd_force *F, cmd_system *S, cmd_neigh *N )
     // f = 0 over local and ghost atoms (cabanamd_impl.h:336-338)
     for ( int k = 0; k < 3; ++k )
         CMD_TRY( fill_f64( S->f.p + (size_t)k * S->cap, 0.0, nt, S->stream ) );
-    if ( N->half )
+    if ( N->half && !N->tiled )
         return lj_half( F, S, N, 0, nullptr, nullptr );
     StepCtl ctl{};
     return lj_full( F, S, N, ctl, nullptr, nullptr, nullptr );

@@ -300,7 +300,6 @@ static cmd_status run_steps( cmd_md *md, int nsteps )
     cmd_force *F = md->F;
     const cmd_params &p = md->p;
     const hipStream_t st = S->stream;
-    const bool half = N->half != 0;
     const int s0 = md->step + 1, s1 = md->step + nsteps;
     const int nthermo = p.thermo_rate > 0 ? nsteps / p.thermo_rate + 2 : 0;
     CMD_TRY( md->trows.reserve( 8 * (size_t)std::max( nthermo, 1 ) ) );
@@ -348,6 +347,8 @@ static cmd_status run_steps( cmd_md *md, int nsteps )
         }
         const bool th = p.thermo_rate > 0 && ( s % p.thermo_rate == 0 );
         const bool last = ( s == s1 );
+        // tiled half lists hold full rows and run the fused step too
+        const bool half = N->half && !N->tiled;
         ctl.do_final = 1;
         ctl.do_next_initial = last ? 0 : 1;
         ctl.wrap_next = ( !last && ( ( s + 1 ) % p.every == 0 ) ) ? 1 : 0;
@@ -383,33 +384,18 @@ static cmd_status run_steps( cmd_md *md, int nsteps )
         }
         else
         {
-            // tiled half lists: the force kernel adds each ghost's reaction
-            // to the atom it images (nothing left to fold), and the
-            // integrator clears the forces it has read for the next step's
-            // sums, so f is cleared here only at the call's first step (it
-            // held the last call's forces for the first half-kick) and after
-            // a list rebuild (new ghost rows)
-            const bool tiled = N->tiled;
             int k = md->begin( PH_FORCE );
-            if ( !tiled || rb || s == s0 )
-            {
-                const int nt = S->n_local + S->n_ghost;
-                for ( int c = 0; c < 3; ++c )
-                    CMD_TRY( fill_f64( S->f.p + (size_t)c * S->cap, 0.0, nt, st ) );
-            }
+            const int nt = S->n_local + S->n_ghost;
+            for ( int c = 0; c < 3; ++c )
+                CMD_TRY( fill_f64( S->f.p + (size_t)c * S->cap, 0.0, nt, st ) );
             CMD_TRY( lj_half( F, S, N, ctl.thermo, md->partA.p, &nb_force ) );
             md->end( k );
-            if ( !tiled )
-            {
-                k = md->begin( PH_COMM );
-                CMD_TRY( cmd_comm_update_force( S ) );
-                md->end( k );
-            }
+            k = md->begin( PH_COMM );
+            CMD_TRY( cmd_comm_update_force( S ) );
+            md->end( k );
             k = md->begin( PH_INT );
-            ctl.zero_f = tiled && !last ? 1 : 0;
             CMD_TRY( nve_final_initial( S, ctl, S->x_alt.p, md->partB.p,
                                         &nb_int ) );
-            ctl.zero_f = 0;
             md->end( k );
         }
         if ( th )

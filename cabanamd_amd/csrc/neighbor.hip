@@ -185,8 +185,8 @@ __global__ __launch_bounds__( TPB ) void k_neigh_slab(
 #pragma unroll
     for ( int o = 32; o > 0; o >>= 1 )
         m = max( m, __shfl_xor( m, o, 64 ) );
-    if ( ( threadIdx.x & 63 ) == 0 && m > 0 )
-        atomicMax( max_row, m );
+    if ( ( threadIdx.x & 63 ) == 0 )
+        raise_max( max_row, m );
 }
 
 // CSR view: row i of the slab copied to idx[offsets[i] ...].

@@ -240,12 +240,12 @@ struct ExactCtx
 };
 
 // Of the lanes in q (candidates at build slot sj, the atom at local index
-// ia), those within rc in FP64 (and, HALF, above the atom).
-template <bool HALF>
+// ia), those within rc in FP64 (returned) and those above the atom (up).
 __device__ __forceinline__ unsigned long long exact_lanes( const ExactCtx &X,
-                                                           unsigned long long q, int sj, int ia )
+                                                           unsigned long long q, int sj, int ia,
+                                                           unsigned long long &up )
 {
-    bool ok = false;
+    bool ok = false, above = false;
     if ( __builtin_amdgcn_inverse_ballot_w64( q ) )
     {
         const int seg = find_seg( X.bseg, 18, sj );
@@ -258,10 +258,10 @@ __device__ __forceinline__ unsigned long long exact_lanes( const ExactCtx &X,
         const double dy = a.y - c.y;
         const double dz = a.z - c.z;
         ok = dx * dx + dy * dy + dz * dz <= X.rc2;
-        if ( HALF )
-            ok = ok && ( ( c.x > a.x ) |
-                         ( ( c.x == a.x ) & ( ( c.y > a.y ) | ( ( c.y == a.y ) & ( c.z > a.z ) ) ) ) );
+        above = ( c.x > a.x ) |
+                ( ( c.x == a.x ) & ( ( c.y > a.y ) | ( ( c.y == a.y ) & ( c.z > a.z ) ) ) );
     }
+    up = __builtin_amdgcn_ballot_w64( above ) & q;
     return __builtin_amdgcn_ballot_w64( ok ) & q;
 }
 
@@ -269,6 +269,8 @@ __device__ __forceinline__ unsigned long long exact_lanes( const ExactCtx &X,
 // indices ia and ia + 1) against NC register chunks, their operations
 // interleaved so that each dependent operation has the other atom's
 // independent one beside it; lanes in the band are settled by exact_lanes.
+// HALF: near is nonzero when an accepted candidate's x difference is within
+// eps, so that its sign in FP32 may not be its sign in FP64.
 template <int NC, bool HALF>
 __device__ __forceinline__ void test_pair32( const float ( &px )[BCH], const float ( &py )[BCH],
                                              const float ( &pz )[BCH], const float4 pa,
@@ -276,7 +278,8 @@ __device__ __forceinline__ void test_pair32( const float ( &px )[BCH], const flo
                                              float eps, const ExactCtx &X,
                                              const int ( &dj )[BCH], int v0, int ia,
                                              unsigned long long ( &ma )[NC],
-                                             unsigned long long ( &mb )[NC] )
+                                             unsigned long long ( &mb )[NC],
+                                             unsigned long long &near )
 {
     const int csa = vs >> 6, csb = ( vs + 1 ) >> 6;
     const unsigned long long nsa = ~( 1ull << ( vs & 63 ) );
@@ -290,43 +293,34 @@ __device__ __forceinline__ void test_pair32( const float ( &px )[BCH], const flo
         const float dza = pa.z - pz[c], dzb = pb.z - pz[c];
         const float ra = fmaf( dza, dza, fmaf( dya, dya, dxa * dxa ) );
         const float rb = fmaf( dzb, dzb, fmaf( dyb, dyb, dxb * dxb ) );
-        unsigned long long sa, sb, qa, qb;
-        if ( HALF )
-        {
-            // settled: inside lo with a certain x direction
-            const bool ka = ( ra <= lo ) & ( fabsf( dxa ) > eps );
-            const bool kb = ( rb <= lo ) & ( fabsf( dxb ) > eps );
-            sa = __builtin_amdgcn_ballot_w64( ka & ( dxa < 0.f ) );
-            sb = __builtin_amdgcn_ballot_w64( kb & ( dxb < 0.f ) );
-            qa = __builtin_amdgcn_ballot_w64( ra <= hi ) & ~__builtin_amdgcn_ballot_w64( ka );
-            qb = __builtin_amdgcn_ballot_w64( rb <= hi ) & ~__builtin_amdgcn_ballot_w64( kb );
-        }
-        else
-        {
-            sa = __builtin_amdgcn_ballot_w64( ra <= lo );
-            sb = __builtin_amdgcn_ballot_w64( rb <= lo );
-            qa = __builtin_amdgcn_ballot_w64( ra <= hi ) & ~sa;
-            qb = __builtin_amdgcn_ballot_w64( rb <= hi ) & ~sb;
-        }
+        unsigned long long sa = __builtin_amdgcn_ballot_w64( ra <= lo );
+        unsigned long long sb = __builtin_amdgcn_ballot_w64( rb <= lo );
+        const unsigned long long qa = __builtin_amdgcn_ballot_w64( ra <= hi ) & ~sa;
+        const unsigned long long qb = __builtin_amdgcn_ballot_w64( rb <= hi ) & ~sb;
         if ( qa | qb )
         {
             const int sj = v0 + c * 64 + lane + dj[c];
+            unsigned long long up;
             if ( qa )
-                sa |= exact_lanes<HALF>( X, qa, sj, ia );
+                sa |= exact_lanes( X, qa, sj, ia, up );
             if ( qb )
-                sb |= exact_lanes<HALF>( X, qb, sj, ia + 1 );
+                sb |= exact_lanes( X, qb, sj, ia + 1, up );
         }
         ma[c] = sa & ( c == csa ? nsa : ~0ull );
         mb[c] = sb & ( c == csb ? nsb : ~0ull );
+        if ( HALF )
+            near |= ( __builtin_amdgcn_ballot_w64( fabsf( dxa ) <= eps ) & ma[c] ) |
+                    ( __builtin_amdgcn_ballot_w64( fabsf( dxb ) <= eps ) & mb[c] );
     }
 }
 
 template <int NC, bool HALF>
 __device__ __forceinline__ void test_chunks32( const float ( &px )[BCH], const float ( &py )[BCH],
                                                const float ( &pz )[BCH], const float4 pa, int vs,
-                                               float lo, float hi, float eps, const ExactCtx &X,
-                                               const int ( &dj )[BCH], int v0, int ia,
-                                               unsigned long long ( &m )[NC] )
+                                               float lo, float hi, float eps,
+                                               const ExactCtx &X, const int ( &dj )[BCH],
+                                               int v0, int ia, unsigned long long ( &m )[NC],
+                                               unsigned long long &near )
 {
     const int cself = vs >> 6;
     const unsigned long long notself = ~( 1ull << ( vs & 63 ) );
@@ -338,30 +332,35 @@ __device__ __forceinline__ void test_chunks32( const float ( &px )[BCH], const f
         const float dy = pa.y - py[c];
         const float dz = pa.z - pz[c];
         const float r = fmaf( dz, dz, fmaf( dy, dy, dx * dx ) );
-        unsigned long long sa, q;
-        if ( HALF )
-        {
-            const bool k = ( r <= lo ) & ( fabsf( dx ) > eps );
-            sa = __builtin_amdgcn_ballot_w64( k & ( dx < 0.f ) );
-            q = __builtin_amdgcn_ballot_w64( r <= hi ) & ~__builtin_amdgcn_ballot_w64( k );
-        }
-        else
-        {
-            sa = __builtin_amdgcn_ballot_w64( r <= lo );
-            q = __builtin_amdgcn_ballot_w64( r <= hi ) & ~sa;
-        }
+        unsigned long long sa = __builtin_amdgcn_ballot_w64( r <= lo );
+        const unsigned long long q = __builtin_amdgcn_ballot_w64( r <= hi ) & ~sa;
+        unsigned long long up;
         if ( q )
-            sa |= exact_lanes<HALF>( X, q, v0 + c * 64 + lane + dj[c], ia );
+            sa |= exact_lanes( X, q, v0 + c * 64 + lane + dj[c], ia, up );
         m[c] = sa & ( c == cself ? notself : ~0ull );
+        if ( HALF )
+            near |= __builtin_amdgcn_ballot_w64( fabsf( dx ) <= eps ) & m[c];
     }
 }
 
-// The accepted candidates of one atom's masks appended to its row in chunk
-// order.  A row holds cap entries and a spare slot at index cap: lanes that
-// do not accept, and accepted entries that would fall past the row's
-// capacity (the row length is still counted, and the list is rebuilt with
-// larger rows), store into the spare slot, so the stores need no branch.
-// Returns the new row length.
+// The accepted candidates m of one chunk appended to a row of length k0.  A
+// row holds cap entries and a spare slot at index cap: lanes that do not
+// accept, and accepted entries that would fall past the row's capacity (the
+// row length is still counted, and the list is rebuilt with larger rows),
+// store into the spare slot, so the store needs no branch.
+__device__ __forceinline__ void place_chunk( int po, unsigned long long m, unsigned short *row,
+                                             unsigned &k0, unsigned cap )
+{
+    unsigned e = cap;
+    if ( __builtin_amdgcn_inverse_ballot_w64( m ) )
+        e = min( __builtin_amdgcn_mbcnt_hi( (unsigned)( m >> 32 ),
+                                            __builtin_amdgcn_mbcnt_lo( (unsigned)m, k0 ) ),
+                 cap );
+    row[e] = (unsigned short)po;
+    k0 += (unsigned)__popcll( m );
+}
+
+// One atom's masks appended to its row in chunk order; the new row length.
 template <int NC>
 __device__ __forceinline__ unsigned place_row( const int ( &po )[BCH],
                                                const unsigned long long ( &m )[NC],
@@ -369,31 +368,44 @@ __device__ __forceinline__ unsigned place_row( const int ( &po )[BCH],
 {
 #pragma unroll
     for ( int c = 0; c < NC; ++c )
-    {
-        unsigned e = cap;
-        if ( __builtin_amdgcn_inverse_ballot_w64( m[c] ) )
-            e = min( __builtin_amdgcn_mbcnt_hi( (unsigned)( m[c] >> 32 ),
-                                                __builtin_amdgcn_mbcnt_lo( (unsigned)m[c], k0 ) ),
-                     cap );
-        row[e] = (unsigned short)po[c];
-        k0 += (unsigned)__popcll( m[c] );
-    }
+        place_chunk( po[c], m[c], row, k0, cap );
     return k0;
 }
 
-// Lane l's value of v, as a wave-uniform (scalar) value.
-__device__ __forceinline__ double readlane_f64( double v, int l )
+// The same for a half list (the atom at pa, local index ia): the rows hold
+// every neighbour, and an entry's low bit (record offsets are multiples of 8;
+// po brings bit 1, set for ghosts) says that the half list holds the pair,
+// that is, that the candidate is above the atom: by the sign of the x
+// difference, and with NEAR in FP64 where that is within eps.  kh counts the
+// marked entries.
+template <int NC, bool NEAR>
+__device__ __forceinline__ unsigned place_half( const float ( &px )[BCH], const int ( &po )[BCH],
+                                                const float4 &pa, float eps, const ExactCtx &X,
+                                                const int ( &dj )[BCH], int v0, int ia,
+                                                const unsigned long long ( &m )[NC],
+                                                unsigned short *row, unsigned k0, unsigned cap,
+                                                unsigned &kh )
 {
-    const unsigned long long b = (unsigned long long)__double_as_longlong( v );
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane( (int)(unsigned)b, l );
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane( (int)(unsigned)( b >> 32 ), l );
-    return __longlong_as_double( (long long)( ( (unsigned long long)hi << 32 ) | lo ) );
-}
-
-__device__ __forceinline__ double4 lane_pos( const double4 &a, int l )
-{
-    return make_double4( readlane_f64( a.x, l ), readlane_f64( a.y, l ),
-                         readlane_f64( a.z, l ), 0.0 );
+#pragma unroll
+    for ( int c = 0; c < NC; ++c )
+    {
+        unsigned long long u = __builtin_amdgcn_ballot_w64( pa.x < px[c] );
+        if ( NEAR )
+        {
+            const unsigned long long d =
+                __builtin_amdgcn_ballot_w64( fabsf( pa.x - px[c] ) <= eps ) & m[c];
+            if ( d )
+            {
+                unsigned long long up;
+                exact_lanes( X, d, v0 + c * 64 + ( threadIdx.x & 63 ) + dj[c], ia, up );
+                u = ( u & ~d ) | ( up & d );
+            }
+        }
+        place_chunk( po[c] + ( __builtin_amdgcn_inverse_ballot_w64( u ) ? 1 : 0 ), m[c], row,
+                     k0, cap );
+        kh += (unsigned)__popcll( m[c] & u );
+    }
+    return k0;
 }
 
 __device__ __forceinline__ float readlane_f32( float v, int l )
@@ -412,48 +424,81 @@ __device__ __forceinline__ float4 lane_pos( const float4 &a, int l )
 // against NC register chunks of candidates, two atoms at a time.  An atom's
 // position and row length are read out of their lanes as wave-uniform
 // values, so the loop waits on no memory.  Lane l of cnt holds atom l's row
-// length.  Coordinates are FP32 about the block's origin, with the band of
-// B (and, HALF, the x-direction bound eps; pass start v0, local index i0 of
-// the group's first atom) settled in FP64 (ExactCtx, dj: the chunks'
-// candidate-to-slot offsets).
+// length (cnth: of a half list, its marked entries).  Coordinates are FP32
+// about the block's origin, with the band of B (and, HALF, the x-direction
+// bound eps; pass start v0, local index i0 of the group's first atom) settled
+// in FP64 (ExactCtx, dj: the chunks' candidate-to-slot offsets).
 struct BandArgs
 {
     float lo, hi, eps;
     int v0, i0;
 };
-
-template <int NC, int G, bool HALF, class PT, class P4>
-__device__ __forceinline__ void build_atoms( const PT ( &px )[BCH], const PT ( &py )[BCH],
-                                             const PT ( &pz )[BCH], const int ( &po )[BCH],
-                                             const P4 &at, int na, int vs0,
-                                             unsigned short *row0, int RS, double rc2,
-                                             unsigned cap, int &cnt, const ExactCtx &X,
-                                             const int ( &dj )[BCH], const BandArgs &B )
+template <int NC, bool HALF>
+__device__ __forceinline__ void build_atoms( const float ( &px )[BCH], const float ( &py )[BCH],
+                                             const float ( &pz )[BCH], const int ( &po )[BCH],
+                                             const float4 &at, int na, int vs0,
+                                             unsigned short *row0, int RS,
+                                             unsigned cap, int &cnt, int &cnth,
+                                             const ExactCtx &X, const int ( &dj )[BCH],
+                                             const BandArgs &B )
 {
+    const int lane = threadIdx.x & 63;
     int l = 0;
     for ( ; l + 1 < na; l += 2 )
     {
-        const P4 pa = lane_pos( at, l ), pb = lane_pos( at, l + 1 );
+        const float4 pa = lane_pos( at, l ), pb = lane_pos( at, l + 1 );
         const unsigned ka0 = (unsigned)__builtin_amdgcn_readlane( cnt, l );
         const unsigned kb0 = (unsigned)__builtin_amdgcn_readlane( cnt, l + 1 );
-        unsigned long long ma[NC], mb[NC];
+        unsigned short *ra = row0 + l * RS, *rb = ra + RS;
+        unsigned long long ma[NC], mb[NC], near = 0;
+        unsigned ka, kb;
         test_pair32<NC, HALF>( px, py, pz, pa, pb, vs0 + l, B.lo, B.hi, B.eps, X, dj, B.v0,
-                               B.i0 + l, ma, mb );
-        const unsigned ka = place_row<NC>( po, ma, row0 + l * RS, ka0, cap );
-        const unsigned kb = place_row<NC>( po, mb, row0 + ( l + 1 ) * RS, kb0, cap );
-        const int lane = threadIdx.x & 63;
+                               B.i0 + l, ma, mb, near );
+        if constexpr ( HALF )
+        {
+            unsigned ha = 0, hb = 0;
+            if ( near )
+            {
+                ka = place_half<NC, true>( px, po, pa, B.eps, X, dj, B.v0, B.i0 + l, ma, ra, ka0,
+                                           cap, ha );
+                kb = place_half<NC, true>( px, po, pb, B.eps, X, dj, B.v0, B.i0 + l + 1, mb, rb,
+                                           kb0, cap, hb );
+            }
+            else
+            {
+                ka = place_half<NC, false>( px, po, pa, B.eps, X, dj, B.v0, B.i0 + l, ma, ra, ka0,
+                                            cap, ha );
+                kb = place_half<NC, false>( px, po, pb, B.eps, X, dj, B.v0, B.i0 + l + 1, mb, rb,
+                                            kb0, cap, hb );
+            }
+            cnth += lane == l ? (int)ha : ( lane == l + 1 ? (int)hb : 0 );
+        }
+        else
+        {
+            ka = place_row<NC>( po, ma, ra, ka0, cap );
+            kb = place_row<NC>( po, mb, rb, kb0, cap );
+        }
         cnt = lane == l ? (int)ka : ( lane == l + 1 ? (int)kb : cnt );
     }
     if ( l < na )
     {
-        const P4 pa = lane_pos( at, l );
-        unsigned long long ma[NC];
+        const float4 pa = lane_pos( at, l );
+        const unsigned ka0 = (unsigned)__builtin_amdgcn_readlane( cnt, l );
+        unsigned short *ra = row0 + l * RS;
+        unsigned long long ma[NC], near = 0;
+        unsigned ka;
         test_chunks32<NC, HALF>( px, py, pz, pa, vs0 + l, B.lo, B.hi, B.eps, X, dj, B.v0,
-                                 B.i0 + l, ma );
-        const unsigned ka = place_row<NC>( po, ma, row0 + l * RS,
-                                           (unsigned)__builtin_amdgcn_readlane( cnt, l ), cap );
-        if ( ( threadIdx.x & 63 ) == l )
-            cnt = (int)ka;
+                                 B.i0 + l, ma, near );
+        if constexpr ( HALF )
+        {
+            unsigned ha = 0;
+            ka = place_half<NC, true>( px, po, pa, B.eps, X, dj, B.v0, B.i0 + l, ma, ra, ka0, cap,
+                                       ha );
+            cnth += lane == l ? (int)ha : 0;
+        }
+        else
+            ka = place_row<NC>( po, ma, ra, ka0, cap );
+        cnt = lane == l ? (int)ka : cnt;
     }
 }
 
@@ -466,8 +511,9 @@ __global__ __launch_bounds__( BTPB ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 
     const int *__restrict__ info, const int *__restrict__ woff,
     const double4 *__restrict__ x, const double4 *__restrict__ xg, double rc2, int rec,
     int cap, int slot_cap, int rows_cap, int waves_cap, unsigned short *__restrict__ slab,
-    int *__restrict__ counts, int *__restrict__ max_row, int *__restrict__ over,
-    int *__restrict__ waves_total, float band_lo, float band_hi, float band_eps )
+    int *__restrict__ counts, int *__restrict__ hcounts, int *__restrict__ max_row,
+    int *__restrict__ max_half, int *__restrict__ over, int *__restrict__ waves_total,
+    float band_lo, float band_hi, float band_eps )
 {
     // coordinate planes in FP32 about the block's origin (tests above)
     using PT = float;
@@ -604,7 +650,7 @@ __global__ __launch_bounds__( BTPB ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 
             reinterpret_cast<uint4 *>( chunk )[k] = fill;
     }
     __syncthreads();
-    int mrow = 0;
+    int mrow = 0, mhalf = 0;
     int *rs = s_rs[wv], *rf = s_rf[wv], *rp = s_rp[wv];
     const int bsent = btotal;
     const ExactCtx X{ x, xg, s_bseg, H.info, ca, cb, S, rc2 };
@@ -676,7 +722,7 @@ __global__ __launch_bounds__( BTPB ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 
                 if ( !gh )
                 {
                     rs[off] = s_lcs[lane][elo];
-                    rf[off] = s_lcs[lane][elo] + s_dl[lane];
+                    rf[off] = ( s_lcs[lane][elo] + s_dl[lane] ) * ( HALF ? 2 : 1 );
                     rp[off + 1] = s_lcs[lane][ehi + 1] - s_lcs[lane][elo];
                 }
                 else
@@ -688,6 +734,11 @@ __global__ __launch_bounds__( BTPB ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 
                         rp[off + 1] = s_lcs[lane][c2 + 1] - s_lcs[lane][c2];
                         rs[off + 1] = s_gcs[lane][c2];
                         rf[off + 1] = s_gcs[lane][c2] + s_dg[lane];
+                        if ( HALF ) // bit 0: ghosts
+                        {
+                            rf[off] *= 2;
+                            rf[off + 1] = 2 * rf[off + 1] + 1;
+                        }
                         rp[off + 2] = s_gcs[lane][c2 + 1] - s_gcs[lane][c2];
                         off += 2;
                     }
@@ -709,7 +760,8 @@ __global__ __launch_bounds__( BTPB ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 
             {
                 t_p = inc - len;
                 t_dj = rs[lane] - t_p;
-                t_df = ( rf[lane] - t_p ) * rec;
+                t_df = HALF ? ( ( rf[lane] >> 1 ) - t_p ) * rec + 2 * ( rf[lane] & 1 )
+                            : ( rf[lane] - t_p ) * rec;
             }
             // candidate index of the cell's first atom, in the centre
             // column's (lane 4's) ranges: the locals of cell ce, its range
@@ -741,7 +793,7 @@ __global__ __launch_bounds__( BTPB ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 
             at.y = s_y[sa];
             at.z = s_z[sa];
             at.w = 0;
-            int cnt = 0; // row length of atom i0 + lane
+            int cnt = 0, cnth = 0; // row length (and half-list entries) of atom i0 + lane
             int cur = 0; // range holding the pass's first candidate
             for ( int v0 = 0; v0 < total; v0 += BCH * 64 )
             {
@@ -798,25 +850,30 @@ __global__ __launch_bounds__( BTPB ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 
                 const unsigned ucap = (unsigned)cap;
                 const BandArgs B{ band_lo, band_hi, band_eps, v0, i0 };
                 if ( nch <= 4 )
-                    build_atoms<4, G, HALF>( px, py, pz, po, at, na, vs0, row0, RS, rc2,
-                                             ucap, cnt, X, dj, B );
+                    build_atoms<4, HALF>( px, py, pz, po, at, na, vs0, row0, RS,
+                                             ucap, cnt, cnth, X, dj, B );
                 else if ( nch <= 6 )
-                    build_atoms<6, G, HALF>( px, py, pz, po, at, na, vs0, row0, RS, rc2,
-                                             ucap, cnt, X, dj, B );
+                    build_atoms<6, HALF>( px, py, pz, po, at, na, vs0, row0, RS,
+                                             ucap, cnt, cnth, X, dj, B );
                 else if ( nch <= 8 )
-                    build_atoms<8, G, HALF>( px, py, pz, po, at, na, vs0, row0, RS, rc2,
-                                             ucap, cnt, X, dj, B );
+                    build_atoms<8, HALF>( px, py, pz, po, at, na, vs0, row0, RS,
+                                             ucap, cnt, cnth, X, dj, B );
                 else if ( nch == 9 )
-                    build_atoms<9, G, HALF>( px, py, pz, po, at, na, vs0, row0, RS, rc2,
-                                             ucap, cnt, X, dj, B );
+                    build_atoms<9, HALF>( px, py, pz, po, at, na, vs0, row0, RS,
+                                             ucap, cnt, cnth, X, dj, B );
                 else
-                    build_atoms<BCH, G, HALF>( px, py, pz, po, at, na, vs0, row0, RS,
-                                               rc2, ucap, cnt, X, dj, B );
+                    build_atoms<BCH, HALF>( px, py, pz, po, at, na, vs0, row0, RS,
+                                             ucap, cnt, cnth, X, dj, B );
             }
             if ( lane < na )
             {
                 counts[i0 + lane] = cnt;
                 mrow = max( mrow, cnt );
+                if ( HALF )
+                {
+                    hcounts[i0 + lane] = cnth;
+                    mhalf = max( mhalf, cnth );
+                }
             }
         }
         // the range tables are rewritten for the next cell
@@ -858,11 +915,15 @@ __global__ __launch_bounds__( BTPB ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 
             }
         }
     }
-#pragma unroll
-    for ( int o = 32; o > 0; o >>= 1 )
-        mrow = max( mrow, __shfl_xor( mrow, o, 64 ) );
-    if ( lane == 0 && mrow > 0 )
-        atomicMax( max_row, mrow );
+    mrow = wave_max_i32( mrow );
+    if ( lane == 0 )
+        raise_max( max_row, mrow );
+    if ( HALF )
+    {
+        mhalf = wave_max_i32( mhalf );
+        if ( lane == 0 )
+            raise_max( max_half, mhalf );
+    }
 }
 
 // CSR view: slots mapped back to system indices (locals by run start,
@@ -870,7 +931,7 @@ __global__ __launch_bounds__( BTPB ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 
 template <int G>
 __global__ __launch_bounds__( TPB ) void k_tile_to_csr(
     TileGrid T, const int *__restrict__ info, const int *__restrict__ woff,
-    int cap, int n_local, int rec, const unsigned short *__restrict__ slab,
+    int cap, int n_local, int rec, int half, const unsigned short *__restrict__ slab,
     const int *__restrict__ counts, const int *__restrict__ gperm,
     const int64_t *__restrict__ offsets, int *__restrict__ idx )
 {
@@ -887,16 +948,18 @@ __global__ __launch_bounds__( TPB ) void k_tile_to_csr(
         const int w = ta / APW, aw = ta % APW;
         const int gw = wave_lanes( G, nat, w ), apw = 64 / gw;
         const int n = counts[i];
-        const int64_t o = offsets[i];
+        int64_t o = offsets[i];
         for ( int k = 0; k < n; ++k )
         {
             const int r = k / gw, lane = ( k % gw ) * apw + aw;
-            const int sj =
-                st[( ( w * R4 + ( r >> 2 ) ) * 64 + lane ) * 4 + ( r & 3 )] / rec;
+            const int en = st[( ( w * R4 + ( r >> 2 ) ) * 64 + lane ) * 4 + ( r & 3 )];
+            if ( half && !( en & 1 ) )
+                continue; // the pair is its other atom's
+            const int sj = en / rec;
             const int seg = find_seg( H.segoff(), H.nseg, sj );
             const int q = seg >> 1, off = sj - H.segoff()[seg];
-            idx[o + k] = ( seg & 1 ) ? n_local + gperm[H.info[TI_GB + q] + off]
-                                     : H.info[TI_LB + q] + off;
+            idx[o++] = ( seg & 1 ) ? n_local + gperm[H.info[TI_GB + q] + off]
+                                   : H.info[TI_LB + q] + off;
         }
     }
 }
@@ -1120,12 +1183,11 @@ static void lds_limits( size_t *block, size_t *cu )
 
 // LDS of the force kernels on tiles with `slots` staged atoms: a position
 // record and, with several types, a type per slot (lj.hip; FP32 records
-// hold the type); the half list adds a reaction record and an energy weight
-// per slot.
-static size_t force_lds( int slots, bool half, int rec )
+// hold the type).
+static size_t force_lds( int slots, int rec )
 {
     const size_t per = rec == TILE_REC32 ? (size_t)TILE_REC32 : TILE_REC + sizeof( int );
-    return (size_t)( slots + 1 ) * per * ( half ? 2 : 1 ) + 16;
+    return (size_t)( slots + 1 ) * per + 16;
 }
 
 template <int G>
@@ -1159,19 +1221,23 @@ static void launch_build( cmd_neigh *N, cmd_system *S, int slot_cap, int rows_ca
         k_tile_build<G, true><<<nb, threads, lds, S->stream>>>(
             N->tg, S->bins.start.p, S->gsort.start.p, N->tile_info.p,
             N->grid_sort.start.p, S->x.p, S->xg.p, rc2, N->rec, N->cap, slot_cap, rows_cap,
-            waves_cap, N->tslab.p, N->counts.p, res + TILE_RES_MAXROW, res + TILE_RES_OVER,
-            res + TILE_RES_WAVES, lo, hi, eps );
+            waves_cap, N->tslab.p, N->fcounts.p, N->counts.p, res + TILE_RES_MAXROW,
+            res + TILE_RES_MAXHALF, res + TILE_RES_OVER, res + TILE_RES_WAVES, lo, hi, eps );
     else
         k_tile_build<G, false><<<nb, threads, lds, S->stream>>>(
             N->tg, S->bins.start.p, S->gsort.start.p, N->tile_info.p,
             N->grid_sort.start.p, S->x.p, S->xg.p, rc2, N->rec, N->cap, slot_cap, rows_cap,
-            waves_cap, N->tslab.p, N->counts.p, res + TILE_RES_MAXROW, res + TILE_RES_OVER,
-            res + TILE_RES_WAVES, lo, hi, eps );
+            waves_cap, N->tslab.p, N->counts.p, nullptr, res + TILE_RES_MAXROW,
+            res + TILE_RES_MAXHALF, res + TILE_RES_OVER, res + TILE_RES_WAVES, lo, hi, eps );
 }
 
 static cmd_status launch_build_g( cmd_neigh *N, cmd_system *S, int slot_cap, int rows_cap,
                                   int waves_cap, size_t lds )
 {
+    // a half list's rows hold the full neighbourhood: their lengths go to
+    // fcounts, the half list's own to counts
+    if ( N->half )
+        CMD_TRY( N->fcounts.reserve( std::max( S->n_local, 1 ) ) );
     switch ( N->lanes )
     {
     case 2:
@@ -1216,7 +1282,7 @@ static int requested_height( const cmd_neigh *N, int W )
 static bool layout_ok( const cmd_neigh *N, const int h[6], size_t lds, size_t hard,
                        size_t lds_cu, int E, bool *fits, int *blocks )
 {
-    const size_t flds = force_lds( h[0], N->half != 0, N->rec );
+    const size_t flds = force_lds( h[0], N->rec );
     *fits = h[0] <= max_force_slots( N->rec ) && lds <= hard && flds <= hard;
     // blocks per CU of the force kernel (its static tables included)
     *blocks = (int)std::min( lds_cu / ( flds + 1024 ), (size_t)( 32 / N->tg.bw ) );
@@ -1270,12 +1336,21 @@ static void report_layout( const cmd_neigh *N, const char *how, int W, int E, co
                   build_lds );
 }
 
+// The longest row of the list (a half list's own rows, not the full ones
+// behind them) and the reference's guess: 1.1 times it when it is longer.
+static void list_rows( cmd_neigh *N, const int *res )
+{
+    N->max_row = res[N->half ? TILE_RES_MAXHALF : TILE_RES_MAXROW];
+    if ( N->max_row > N->max_neigh_guess )
+        N->max_neigh_guess = (int)( N->max_row * 1.1 );
+}
+
 cmd_status tiles_build( cmd_neigh *N, cmd_system *S, bool *built )
 {
     *built = false;
     N->spec.valid = false;
     if ( N->half )
-        N->rec = TILE_REC; // the half-list kernel stages FP64 records
+        N->rec = TILE_REC; // half lists address FP64 records
     if ( !S->bin_grid_valid || !S->xg_valid || N->lanes < 2 )
         return CMD_OK;
     if ( N->cap < 1 )
@@ -1324,9 +1399,7 @@ cmd_status tiles_build( cmd_neigh *N, cmd_system *S, bool *built )
         CMD_TRY( launch_build_g( N, S, h[3] + 1, h[4], h[5], lds ) );
         CMD_TRY( tile_results( N, S, res, &h[5], true ) );
         const int mr = res[TILE_RES_MAXROW];
-        N->max_row = mr;
-        if ( mr > N->max_neigh_guess )
-            N->max_neigh_guess = (int)( mr * 1.1 );
+        list_rows( N, res );
         if ( mr <= N->cap )
         {
             *built = true;
@@ -1338,7 +1411,7 @@ cmd_status tiles_build( cmd_neigh *N, cmd_system *S, bool *built )
             return CMD_OK;
         }
         // rows overflowed: larger rows, and the LDS fit rechecked
-        N->cap = std::max( N->max_neigh_guess, mr );
+        N->cap = std::max( N->max_neigh_guess, (int)( mr * 1.1 ) );
     }
     set_error( "neighbour rows kept growing during the tiled build" );
     return CMD_ERR_CAPACITY;
@@ -1379,13 +1452,11 @@ cmd_status tiles_build_spec( cmd_neigh *N, cmd_system *S, bool *built )
     if ( !layout_ok( N, h, build_lds( N, h[3] + 1, h[4] ), hard, lds_cu, P.E, &fits, &blocks ) )
         return CMD_OK;
     const int mr = res[TILE_RES_MAXROW];
-    N->max_row = mr;
-    if ( mr > N->max_neigh_guess )
-        N->max_neigh_guess = (int)( mr * 1.1 );
+    list_rows( N, res );
     if ( mr > N->cap )
     {
         // rows overflowed: the caller's build starts at the grown rows
-        N->cap = std::max( N->max_neigh_guess, mr );
+        N->cap = std::max( N->max_neigh_guess, (int)( mr * 1.1 ) );
         return CMD_OK;
     }
     N->tile_blocks = blocks;
@@ -1408,17 +1479,17 @@ cmd_status tiles_csr( cmd_neigh *N, int64_t *nnz_out )
     case 2:
         k_tile_to_csr<2><<<nt, TPB, 0, N->stream>>>(
             N->tg, N->tile_info.p, N->grid_sort.start.p, N->cap, N->n_rows, N->built_rec,
-            N->tslab.p, N->counts.p, N->gperm_view, N->offsets.p, N->idx.p );
+            N->half, N->tslab.p, N->row_counts(), N->gperm_view, N->offsets.p, N->idx.p );
         break;
     case 4:
         k_tile_to_csr<4><<<nt, TPB, 0, N->stream>>>(
             N->tg, N->tile_info.p, N->grid_sort.start.p, N->cap, N->n_rows, N->built_rec,
-            N->tslab.p, N->counts.p, N->gperm_view, N->offsets.p, N->idx.p );
+            N->half, N->tslab.p, N->row_counts(), N->gperm_view, N->offsets.p, N->idx.p );
         break;
     default:
         k_tile_to_csr<8><<<nt, TPB, 0, N->stream>>>(
             N->tg, N->tile_info.p, N->grid_sort.start.p, N->cap, N->n_rows, N->built_rec,
-            N->tslab.p, N->counts.p, N->gperm_view, N->offsets.p, N->idx.p );
+            N->half, N->tslab.p, N->row_counts(), N->gperm_view, N->offsets.p, N->idx.p );
         break;
     }
     CMD_LAUNCH_CHECK();

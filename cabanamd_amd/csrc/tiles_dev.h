@@ -145,70 +145,6 @@ __device__ __forceinline__ int find_seg( const int *off, int nseg, int k )
     return lo;
 }
 
-// Copy the staged runs of positions (locals from x, ghosts from xg) into LDS
-// as 24-byte records, followed by the sentinel record; with WITH_TYPE the
-// types follow as ints, `cap` records on.  Each thread has up to B loads in
-// flight, so a tile's neighbourhood (about a thousand records) arrives in
-// one round of memory latency for blocks of 256 threads and more.  The
-// `nzero` doubles at `zero` (an LDS area of the caller's) are cleared while
-// the first round's loads are in flight.  Ends with a barrier.
-template <bool WITH_TYPE>
-__device__ inline void stage_records( const TileHead &H, const double4 *__restrict__ x,
-                                      const double4 *__restrict__ xg,
-                                      double *__restrict__ s_rec, int cap,
-                                      double *__restrict__ zero = nullptr, int nzero = 0 )
-{
-    int *s_t = reinterpret_cast<int *>( s_rec + 3 * cap );
-    const int total = H.segoff()[H.nseg];
-    constexpr int B = 8; // slots per thread whose loads are in flight together
-    auto clear = [&]()
-    {
-        for ( int k = threadIdx.x; k < nzero; k += blockDim.x )
-            zero[k] = 0.0;
-    };
-    for ( int k0 = threadIdx.x; k0 < total; k0 += B * blockDim.x )
-    {
-        double4 p[B];
-#pragma unroll
-        for ( int u = 0; u < B; ++u )
-        {
-            // past the end: reload the last slot (in bounds)
-            const int k = min( k0 + u * (int)blockDim.x, total - 1 );
-            const int seg = find_seg( H.segoff(), H.nseg, k );
-            const int q = seg >> 1, off = k - H.segoff()[seg];
-            const double4 *__restrict__ base = ( seg & 1 ) ? xg : x;
-            const int idx = ( ( seg & 1 ) ? H.info[TI_GB + q] : H.info[TI_LB + q] ) + off;
-            p[u] = base[idx];
-        }
-        if ( k0 == (int)threadIdx.x )
-            clear();
-        // stores past the end go to the sentinel record, rewritten below
-#pragma unroll
-        for ( int u = 0; u < B; ++u )
-        {
-            const int k = min( k0 + u * (int)blockDim.x, total );
-            s_rec[3 * k] = p[u].x;
-            s_rec[3 * k + 1] = p[u].y;
-            s_rec[3 * k + 2] = p[u].z;
-            if ( WITH_TYPE )
-                s_t[k] = (int)p[u].w;
-        }
-    }
-    // threads past the records clear their share too
-    if ( (int)threadIdx.x >= total )
-        clear();
-    __syncthreads();
-    if ( threadIdx.x == 0 )
-    {
-        s_rec[3 * total] = TILE_FAR;
-        s_rec[3 * total + 1] = TILE_FAR;
-        s_rec[3 * total + 2] = TILE_FAR;
-        if ( WITH_TYPE )
-            s_t[total] = 0;
-    }
-    __syncthreads();
-}
-
 // Largest value of the wave's lanes (values >= 0), in row shifts and row
 // broadcasts of the adder's operand rather than LDS permutes.
 __device__ __forceinline__ int wave_max_i32( int v )
