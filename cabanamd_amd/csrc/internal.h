@@ -213,6 +213,24 @@ struct CellGrid
     int floor_mode; // 1: floor() (Cabana LinkedCellList); 0: truncation
 };
 
+// Round-robin dispatch puts block b on XCD b % 8; give XCD k the k-th
+// contiguous slice of logical blocks instead.
+__device__ __forceinline__ int xcd_remap( int b, int nb )
+{
+    const int q = nb >> 3, r = nb & 7;
+    const int xcd = b & 7, k = b >> 3;
+    return ( xcd < r ) ? xcd * ( q + 1 ) + k : r * ( q + 1 ) + ( xcd - r ) * q + k;
+}
+
+// Lane l's value of v (l wave-uniform), as a wave-uniform value.
+__device__ __forceinline__ double readlane_f64( double v, int l )
+{
+    const unsigned long long b = (unsigned long long)__double_as_longlong( v );
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane( (int)(unsigned)b, l );
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane( (int)(unsigned)( b >> 32 ), l );
+    return __longlong_as_double( (long long)( ( (unsigned long long)hi << 32 ) | lo ) );
+}
+
 // Raise the maximum at p (device memory, every block's) to v.  The atomics of
 // one address are served one after another, and after a kernel's first few
 // blocks hardly any raises a maximum, so the value is looked at first.

@@ -26,15 +26,6 @@ namespace cmd
 {
 static constexpr int TPB = 256;
 
-// Round-robin dispatch puts block b on XCD b % 8; give XCD k the k-th
-// contiguous slice of logical blocks instead.
-__device__ __forceinline__ int xcd_remap( int b, int nb )
-{
-    const int q = nb >> 3, r = nb & 7;
-    const int xcd = b & 7, k = b >> 3;
-    return ( xcd < r ) ? xcd * ( q + 1 ) + k : r * ( q + 1 ) + ( xcd - r ) * q + k;
-}
-
 LJParams lj_params( const cmd_force *F )
 {
     LJParams P;
@@ -828,7 +819,8 @@ __global__ __launch_bounds__( TPB ) void k_lj_energy(
     constexpr int APW = 64 / G;
     const SlabLane L = slab_lane<G>( blockIdx.x );
     const int i = L.i;
-    double pe = 0.0, vir = 0.0;
+    // pe6: six times the unshifted energies (one division at the end)
+    double pe6 = 0.0, esh = 0.0, vir = 0.0;
     if ( i < n_local )
     {
         const double4 xi = x[i];
@@ -837,10 +829,8 @@ __global__ __launch_bounds__( TPB ) void k_lj_energy(
         const int nr = n > L.s ? ( n - L.s + G - 1 ) / G : 0;
         const int R = ( lcap + G - 1 ) / G;
         const int *row = slab + (size_t)L.wave * R * 64 + L.s * APW + L.a;
-        for ( int r = 0; r < nr; ++r )
+        auto body = [&]( int j, const double4 &xj )
         {
-            const int j = row[r * 64];
-            const double4 xj = x[j];
             const double dx = xi.x - xj.x;
             const double dy = xi.y - xj.y;
             const double dz = xi.z - xj.z;
@@ -851,14 +841,15 @@ __global__ __launch_bounds__( TPB ) void k_lj_energy(
                 const double fac = half ? ( ( j < n_local ) ? 1.0 : 0.5 ) : 0.5;
                 const double r2inv = 1.0 / rsq;
                 const double r6inv = r2inv * r2inv * r2inv;
-                pe += fac * r6inv * ( 0.5 * c.lj1 * r6inv - c.lj2 ) / 6.0;
-                pe -= fac * c.esh;
+                pe6 += fac * r6inv * ( 0.5 * c.lj1 * r6inv - c.lj2 );
+                esh += fac * c.esh;
                 const double fpair = ( r6inv * ( c.lj1 * r6inv - c.lj2 ) ) * r2inv;
                 vir += ( half ? 1.0 : 0.5 ) * rsq * fpair;
             }
-        }
+        };
+        walk_row<G, ONE_TYPE>( row, nr, x, body );
     }
-    block_sum4( 0.0, pe, vir, 0.0, partial + 4 * blockIdx.x );
+    block_sum4( 0.0, pe6 / 6.0 - esh, vir, 0.0, partial + 4 * blockIdx.x );
 }
 
 // compute_energy over a CSR view (used for tiled lists).

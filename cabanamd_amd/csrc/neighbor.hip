@@ -116,76 +116,152 @@ __global__ void k_gather_sorted( int n, const int *__restrict__ perm,
     xs[k] = p;
 }
 
-__device__ __forceinline__ bool accept_pair( const double4 &pi, const double4 &pj,
-                                             int i, int j, double rc2, int half )
-{
-    if ( i == j )
-        return false;
-    if ( half &&
-         !( ( pj.x > pi.x ) ||
-            ( ( pj.x == pi.x ) &&
-              ( ( pj.y > pi.y ) || ( ( pj.y == pi.y ) && ( pj.z > pi.z ) ) ) ) ) )
-        return false;
-    const double dx = pi.x - pj.x;
-    const double dy = pi.y - pj.y;
-    const double dz = pi.z - pj.z;
-    const double rsq = dx * dx + dy * dy + dz * dz;
-    return rsq <= rc2;
-}
-
-
-// One lane per local atom i; lanes of a wave are consecutive atoms, which
-// after binning sit in neighbouring cells and walk overlapping stencils.
-template <int G>
-__global__ __launch_bounds__( TPB ) void k_neigh_slab(
-    int n_local, const double4 *__restrict__ x, const double4 *__restrict__ xs,
-    const int *__restrict__ start, CellGrid g, double rc2, int half, int cap,
+// Rows of the local atoms among the grid-sorted atoms xs[s0, s0 + per) of one
+// wave.  Per cell that the wave's atoms lie in, the candidates (nine runs of
+// xs: columns a - 1 .. a + 1, b - 1 .. b + 1, cells e - 1 .. e + 1) are loaded
+// into registers, one per lane, NB_CH chunks at a time; each atom, its
+// position read out of its lane, is tested against a chunk in one go, and
+// the accepted candidates take the next places of its row, so rows keep the
+// order of the walk.  Bound by the FP64 tests (about 18 instructions for 64
+// of them) and, in small systems, by the latency of a wave's walk: a wave
+// takes fewer atoms there (slots_per_wave).  Neighbouring blocks run on one
+// XCD, whose L2 joins the 4-byte stores of a slab wave's rows (171 us at
+// 256,000 atoms without, 154 us with).  A lane per atom, walking its
+// candidates one load after another, took 350 us at 256,000 atoms and 239 us
+// at the 3,000 atoms of an NNP box (this: 18 us).
+constexpr int NB_CH = 10;
+template <int G, bool HALF>
+__global__ __launch_bounds__( TPB ) void k_neigh_rows(
+    int nt, int n_local, int per, const double4 *__restrict__ xs,
+    const int *__restrict__ start, CellGrid g, double rc2, int cap,
     int *__restrict__ counts, int *__restrict__ slab, int *__restrict__ max_row )
 {
     constexpr int APW = 64 / G;
-    const int i = blockIdx.x * TPB + (int)threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int s0 = __builtin_amdgcn_readfirstlane(
+        ( xcd_remap( blockIdx.x, gridDim.x ) * ( TPB / 64 ) + (int)( threadIdx.x >> 6 ) ) *
+        per );
+    if ( s0 >= nt )
+        return;
+    // lane l: sorted atom s0 + l and its cell
+    const int s = s0 + lane;
+    const double4 me = xs[min( s, nt - 1 )];
+    const int id = (int)me.w;
+    const int a = cell_coord( me.x, g.min[0], g.rd[0], g.n[0], g.floor_mode );
+    const int b = cell_coord( me.y, g.min[1], g.rd[1], g.n[1], g.floor_mode );
+    const int e = cell_coord( me.z, g.min[2], g.rd[2], g.n[2], g.floor_mode );
+    const int cell = ( a * g.n[1] + b ) * g.n[2] + e;
+    const bool mine = lane < per && s < nt && id < n_local;
+    const int R = ( cap + G - 1 ) / G;
     int cnt = 0;
-    if ( i < n_local )
+    unsigned long long todo = __builtin_amdgcn_ballot_w64( mine );
+    while ( todo )
     {
-        const double4 pi = x[i];
-        const int a = cell_coord( pi.x, g.min[0], g.rd[0], g.n[0], g.floor_mode );
-        const int b = cell_coord( pi.y, g.min[1], g.rd[1], g.n[1], g.floor_mode );
-        const int e = cell_coord( pi.z, g.min[2], g.rd[2], g.n[2], g.floor_mode );
-        const int e0 = e > 0 ? e - 1 : 0;
-        const int e1 = e < g.n[2] - 1 ? e + 1 : g.n[2] - 1;
-        const int R = ( cap + G - 1 ) / G;
-        const int w = i / APW, ai = i % APW;
-        int *out = slab + (size_t)w * R * 64 + ai;
-        for ( int aa = a - 1; aa <= a + 1; ++aa )
+        const int l0 = __builtin_ctzll( todo );
+        const unsigned long long grp =
+            __builtin_amdgcn_ballot_w64( cell == __builtin_amdgcn_readlane( cell, l0 ) ) & todo;
+        todo &= ~grp;
+        const int ca = __builtin_amdgcn_readlane( a, l0 );
+        const int cb = __builtin_amdgcn_readlane( b, l0 );
+        const int ce = __builtin_amdgcn_readlane( e, l0 );
+        // column q = lane (< 9): its run [rs, rs + len) of candidates
+        int rs = 0, len = 0;
+        if ( lane < 9 )
         {
-            if ( aa < 0 || aa >= g.n[0] )
-                continue;
-            for ( int bb = b - 1; bb <= b + 1; ++bb )
+            const int aa = ca + lane / 3 - 1, bb = cb + lane % 3 - 1;
+            if ( aa >= 0 && aa < g.n[0] && bb >= 0 && bb < g.n[1] )
             {
-                if ( bb < 0 || bb >= g.n[1] )
-                    continue;
                 const int base = ( aa * g.n[1] + bb ) * g.n[2];
-                const int s1 = start[base + e1 + 1];
-                for ( int s = start[base + e0]; s < s1; ++s )
-                {
-                    const double4 pj = xs[s];
-                    const int j = (int)pj.w;
-                    if ( accept_pair( pi, pj, i, j, rc2, half ) )
-                    {
-                        if ( cnt < cap )
-                            out[( cnt / G ) * 64 + ( cnt % G ) * APW] = j;
-                        ++cnt;
-                    }
-                }
+                rs = start[base + max( ce - 1, 0 )];
+                len = start[base + min( ce + 1, g.n[2] - 1 ) + 1] - rs;
             }
         }
-        counts[i] = cnt;
+        int inc = len;
+#pragma unroll
+        for ( int o = 1; o < 16; o <<= 1 )
+        {
+            const int u = __shfl_up( inc, o, 64 );
+            if ( lane >= o )
+                inc += u;
+        }
+        // run q starts at candidate P[q]; candidate v of run q is xs[v + D[q]]
+        int P[9], D[9];
+#pragma unroll
+        for ( int q = 0; q < 9; ++q )
+        {
+            P[q] = __builtin_amdgcn_readlane( inc - len, q );
+            D[q] = __builtin_amdgcn_readlane( rs, q ) - P[q];
+        }
+        const int total = __builtin_amdgcn_readlane( inc, 8 );
+        for ( int v0 = 0; v0 < total; v0 += NB_CH * 64 )
+        {
+            double px[NB_CH], py[NB_CH], pz[NB_CH];
+            int pj[NB_CH];
+#pragma unroll
+            for ( int k = 0; k < NB_CH; ++k )
+            {
+                const int v = v0 + k * 64 + lane;
+                // lanes past the last candidate: outside every cutoff
+                px[k] = py[k] = pz[k] = 1.0e30;
+                pj[k] = -1;
+                if ( v < total )
+                {
+                    int d = D[0];
+#pragma unroll
+                    for ( int q = 1; q < 9; ++q )
+                        d = v >= P[q] ? D[q] : d;
+                    const double4 p = xs[v + d];
+                    px[k] = p.x;
+                    py[k] = p.y;
+                    pz[k] = p.z;
+                    pj[k] = (int)p.w;
+                }
+            }
+            const int nch = min( NB_CH, ( total - v0 + 63 ) >> 6 );
+            for ( unsigned long long left = grp; left; left &= left - 1 )
+            {
+                const int l = __builtin_ctzll( left );
+                const double ax = readlane_f64( me.x, l );
+                const double ay = readlane_f64( me.y, l );
+                const double az = readlane_f64( me.z, l );
+                const int i = __builtin_amdgcn_readlane( id, l );
+                int *out = slab + (size_t)( i / APW ) * R * 64 + i % APW;
+                unsigned k0 = (unsigned)__builtin_amdgcn_readlane( cnt, l );
+#pragma unroll
+                for ( int k = 0; k < NB_CH; ++k )
+                {
+                    if ( k < nch )
+                    {
+                        const double dx = ax - px[k];
+                        const double dy = ay - py[k];
+                        const double dz = az - pz[k];
+                        const double rsq = dx * dx + dy * dy + dz * dz;
+                        unsigned long long m = __builtin_amdgcn_ballot_w64( rsq <= rc2 ) &
+                                               __builtin_amdgcn_ballot_w64( pj[k] != i );
+                        if ( HALF )
+                            m &= __builtin_amdgcn_ballot_w64(
+                                ( px[k] > ax ) |
+                                ( ( px[k] == ax ) &
+                                  ( ( py[k] > ay ) | ( ( py[k] == ay ) & ( pz[k] > az ) ) ) ) );
+                        const unsigned kk = __builtin_amdgcn_mbcnt_hi(
+                            (unsigned)( m >> 32 ),
+                            __builtin_amdgcn_mbcnt_lo( (unsigned)m, k0 ) );
+                        if ( __builtin_amdgcn_inverse_ballot_w64( m ) && kk < (unsigned)cap )
+                            out[( kk / G ) * 64 + ( kk % G ) * APW] = pj[k];
+                        k0 += (unsigned)__popcll( m );
+                    }
+                }
+                cnt = lane == l ? (int)k0 : cnt;
+            }
+        }
     }
-    int m = cnt;
+    if ( mine )
+        counts[id] = cnt;
+    int m = cnt; // 0 where no local atom is
 #pragma unroll
     for ( int o = 32; o > 0; o >>= 1 )
         m = max( m, __shfl_xor( m, o, 64 ) );
-    if ( ( threadIdx.x & 63 ) == 0 )
+    if ( lane == 0 )
         raise_max( max_row, m );
 }
 
@@ -236,15 +312,27 @@ static void neigh_grid( const double lo[3], const double hi[3], double rc,
         rcell[k] = ng[k] / std::max( ext[k], 1e-300 );
 }
 
+// Sorted atoms per wave of the list build.  More of a cell's atoms share the
+// load of its candidates, fewer give more waves and a shorter last one:
+// 256,000 LJ atoms take 163 us at 8 atoms, 171 us at 16 and 237 us at 32
+// (before the blocks' XCD order); small systems take 4, so that every CU has
+// waves.
+static int slots_per_wave( int nt )
+{
+    int per = 4;
+    while ( per < 16 && nt / ( 2 * per ) >= 8192 )
+        per *= 2;
+    return per;
+}
+
 static cmd_status launch_slab( cmd_neigh *N, cmd_system *S, const CellGrid &g,
-                               int n_local, int cap, int *max_row_dev )
+                               int n_local, int nt, int cap, int *max_row_dev )
 {
     const double rc2 = N->neigh_cut * N->neigh_cut;
-    const int nb = std::max( 1, ( n_local + TPB - 1 ) / TPB );
-#define CMD_SLAB( GG )                                                        \
-    k_neigh_slab<GG><<<nb, TPB, 0, S->stream>>>(                              \
-        n_local, S->x.p, N->xs.p, N->grid_sort.start.p, g, rc2, N->half, cap, \
-        N->counts.p, N->slab.p, max_row_dev )
+    const int per = slots_per_wave( nt );
+    const int nb = ( ( nt + per - 1 ) / per + TPB / 64 - 1 ) / ( TPB / 64 );
+#define CMD_SLAB_H( GG, HALF )                                                    k_neigh_rows<GG, HALF><<<nb, TPB, 0, S->stream>>>(                                nt, n_local, per, N->xs.p, N->grid_sort.start.p, g, rc2, cap,                 N->counts.p, N->slab.p, max_row_dev )
+#define CMD_SLAB( GG )                                                            if ( N->half )                                                                    CMD_SLAB_H( GG, true );                                                   else                                                                              CMD_SLAB_H( GG, false )
     switch ( N->lanes )
     {
     case 1:
@@ -264,6 +352,7 @@ static cmd_status launch_slab( cmd_neigh *N, cmd_system *S, const CellGrid &g,
         return CMD_ERR_ARG;
     }
 #undef CMD_SLAB
+#undef CMD_SLAB_H
     CMD_LAUNCH_CHECK();
     return CMD_OK;
 }
@@ -393,7 +482,7 @@ cmd_status neigh_build( cmd_neigh *N, cmd_system *S )
     {
         CMD_TRY( N->slab.reserve( slab_entries( n_local, N->cap, N->lanes ) ) );
         CMD_TRY( fill_i32( S->sc.ires.p, 0, 1, st ) );
-        CMD_TRY( launch_slab( N, S, g, n_local, N->cap, S->sc.ires.p ) );
+        CMD_TRY( launch_slab( N, S, g, n_local, nt, N->cap, S->sc.ires.p ) );
         int mr = 0;
         CMD_HIP( hipMemcpyAsync( &mr, S->sc.ires.p, sizeof( int ),
                                  hipMemcpyDeviceToHost, st ) );
