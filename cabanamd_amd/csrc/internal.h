@@ -272,6 +272,20 @@ struct TileGrid
     int E, tpc;   // tile height in cells, tiles per column
     int ntiles;
     int bw;       // waves per block of the tiled force kernels
+    int cell0, tile0; // first cell and tile (grids of a batch share both spaces)
+};
+
+// What a tiled build reads besides the atoms: the cell starts of the local
+// atoms and of the sorted ghosts, the ghosts' positions, and for a batch the
+// grid of each system and of each tile.
+struct TileSrc
+{
+    const TileGrid *grids; // nullptr: one grid, the list's own
+    const int *grid_of;    // grid of each tile
+    const int *ls, *gs;
+    const double4 *xg;
+    const int *ghost_out; // nullptr: every ghost lies in its grid
+    double amax;          // bound of a staged coordinate about a build block's origin
 };
 
 // Counting sort of n positions into grid cells, stable by index.  Produces
@@ -338,6 +352,9 @@ struct cmd_system
     cmd::CellSort gsort;
     cmd::DevBuf<double4> xg;
     bool xg_valid = false;
+    // a batch keeps its ghosts in cell order behind the local atoms instead
+    bool ghosts_in_x = false;
+    const double4 *tile_ghosts() const { return ghosts_in_x ? x.p + n_local : xg.p; }
     // the fused step writes the next step's sorted ghosts into xg_alt: local
     // atom i has images img_pk[img_rng[i].x .. img_rng[i].y), each the
     // sorted slot | shift code << IMG_CODE_SHIFT; the system's own ghost rows
@@ -550,6 +567,10 @@ cmd_status tiles_prepare_ghosts( cmd_system *S );
 cmd_status binning_create( cmd_system *s, double dx_in, double dy_in, double dz_in,
                            int halo_depth, int do_local, int do_ghost, int sort, int *perm_out,
                            bool keep_f );
+// The same for the tiles of a batch: N->tg.W, E and ntiles are set, the
+// shape is not lowered (*built stays false where it does not fit).
+cmd_status tiles_build_batch( cmd_neigh *N, cmd_system *S, const TileSrc &src, bool *built );
+double tile_amax( const CellGrid &g, int E );
 cmd_status tiles_build( cmd_neigh *N, cmd_system *S, bool *built );
 cmd_status tiles_build_spec( cmd_neigh *N, cmd_system *S, bool *built );
 // Result words of the tiled build in the system's int scratch (sc.ires):

@@ -998,7 +998,7 @@ static void launch_tile_k( cmd_neigh *N, cmd_system *S, double4 *xn,
             k_tile_force<G, PREC, ONE, FUSED, ENERGY, true>
                 <<<N->tg.ntiles, 64 * N->tg.bw, lds, S->stream>>>(
                     N->tg, N->tile_info.p, N->grid_sort.start.p, N->cap, S->cap, slot_cap,
-                    S->x.p, S->xg.p, xn, S->v.p, S->f.p, N->row_counts(), N->tslab.p, Pd, c, mt,
+                    S->x.p, S->tile_ghosts(), xn, S->v.p, S->f.p, N->row_counts(), N->tslab.p, Pd, c, mt,
                     ctl, partial );
             return;
         }
@@ -1008,7 +1008,7 @@ static void launch_tile_k( cmd_neigh *N, cmd_system *S, double4 *xn,
         (size_t)slot_cap * ( TILE_REC + ( ONE ? 0 : sizeof( int ) ) ), 32 * sizeof( double ) );
     k_tile_force<G, PREC, ONE, FUSED, ENERGY, false><<<N->tg.ntiles, 64 * N->tg.bw, lds, S->stream>>>(
         N->tg, N->tile_info.p, N->grid_sort.start.p, N->cap, S->cap, slot_cap,
-        S->x.p, S->xg.p, xn, S->v.p, S->f.p, N->row_counts(), N->tslab.p, Pd, c, mt,
+        S->x.p, S->tile_ghosts(), xn, S->v.p, S->f.p, N->row_counts(), N->tslab.p, Pd, c, mt,
         ctl, partial );
 }
 

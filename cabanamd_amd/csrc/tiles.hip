@@ -72,20 +72,21 @@ static int max_force_slots( int rec )
 static constexpr int INFO_TPB = 1024;
 
 __global__ __launch_bounds__( INFO_TPB ) void k_tile_info(
-    TileGrid T, const int *__restrict__ ls, const int *__restrict__ gs, int apw,
-    const int *__restrict__ ghost_out, int *__restrict__ info, int *__restrict__ waves,
+    TileGrid T1, TileSrc src, int apw, int *__restrict__ info, int *__restrict__ waves,
     int *__restrict__ slots )
 {
+    const int *__restrict__ ls = src.ls, *__restrict__ gs = src.gs;
     __shared__ int s_max[5];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     if ( threadIdx.x < 5 )
         s_max[threadIdx.x] = 0;
     if ( blockIdx.x == 0 && threadIdx.x == 0 )
-        slots[TILE_RES_OUTSIDE] = *ghost_out;
+        slots[TILE_RES_OUTSIDE] = src.ghost_out ? *src.ghost_out : 0;
     __syncthreads();
-    const int t = blockIdx.x * ( INFO_TPB / 64 ) + wid;
-    if ( t < T.ntiles )
+    const int t = __builtin_amdgcn_readfirstlane( blockIdx.x * ( INFO_TPB / 64 ) + wid );
+    if ( t < T1.ntiles )
     {
+        const TileGrid T = src.grids ? src.grids[src.grid_of[t]] : T1;
         int a0, b0, e0, e1;
         tile_coords( T, t, a0, b0, e0, e1 );
         const int ea = max( e0 - 1, 0 ), eb = min( e1 + 1, T.g.n[2] );
@@ -507,9 +508,8 @@ __device__ __forceinline__ void build_atoms( const float ( &px )[BCH], const flo
 // instead of on occupancy it cannot reach.
 template <int G, bool HALF>
 __global__ __launch_bounds__( BTPB ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 ) ) ) void k_tile_build(
-    TileGrid T, const int *__restrict__ ls, const int *__restrict__ gs,
-    const int *__restrict__ info, const int *__restrict__ woff,
-    const double4 *__restrict__ x, const double4 *__restrict__ xg, double rc2, int rec,
+    TileGrid T1, TileSrc src, const int *__restrict__ info, const int *__restrict__ woff,
+    const double4 *__restrict__ x, double rc2, int rec,
     int cap, int slot_cap, int rows_cap, int waves_cap, unsigned short *__restrict__ slab,
     int *__restrict__ counts, int *__restrict__ hcounts, int *__restrict__ max_row,
     int *__restrict__ max_half, int *__restrict__ over, int *__restrict__ waves_total,
@@ -528,15 +528,18 @@ __global__ __launch_bounds__( BTPB ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 
     __shared__ int s_rf[BTPB / 64][MAXR];     // range starts in the force tile's slots
     __shared__ int s_rp[BTPB / 64][MAXR + 1]; // prefix of range lengths
     constexpr int APW = 64 / G;
-    const int W = T.W, S = W + 2, NA = W * W;
+    const int *__restrict__ ls = src.ls, *__restrict__ gs = src.gs;
+    const double4 *__restrict__ xg = src.xg;
+    const int W = T1.W, S = W + 2, NA = W * W;
     const int sub = xcd_tile( blockIdx.x, gridDim.x );
     const int t = sub / NA, c = sub % NA, ca = c / W, cb = c % W;
     if ( blockIdx.x == 0 && threadIdx.x == 0 )
-        *waves_total = woff[T.ntiles]; // read back with the build's results
+        *waves_total = woff[T1.ntiles]; // read back with the build's results
     load_head( info, t, W, H );
     const int nat_c = H.info[TI_AN + c];
     if ( nat_c == 0 )
         return; // block-uniform: an atom column outside the grid, or empty
+    const TileGrid T = src.grids ? src.grids[src.grid_of[t]] : T1;
     int a0, b0, e0, e1;
     tile_coords( T, t, a0, b0, e0, e1 );
     const int a = a0 + ca, b = b0 + cb;
@@ -704,8 +707,30 @@ __global__ __launch_bounds__( BTPB ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 
         }
         else
         {
-            // column q's ranges (lane q < 9), then their offsets in the list
-            const int nr_q = lane < 9 ? ( gh ? 2 * ( ehi - elo + 1 ) : 1 ) : 0;
+            // column q's ranges (lane q < 9): the locals and ghosts of its
+            // cells in turn, empty runs left out and runs of one kind that
+            // follow each other joined (a column holds ghosts at its ends,
+            // or nothing else: one or two ranges instead of six), then their
+            // offsets in the list
+            auto runs = [&]( auto &&begin, auto &&add )
+            {
+                int last = -1;
+                for ( int c2 = elo; c2 <= ehi; ++c2 )
+                    for ( int kind = 0; kind < 2; ++kind )
+                    {
+                        const int *cs = kind ? s_gcs[lane] : s_lcs[lane];
+                        const int n = cs[c2 + 1] - cs[c2];
+                        if ( n == 0 )
+                            continue;
+                        if ( kind != last )
+                            begin( kind, cs[c2] );
+                        last = kind;
+                        add( kind, c2, n );
+                    }
+            };
+            int nr_q = 0;
+            if ( lane < 9 )
+                runs( [&]( int, int ) { ++nr_q; }, []( int, int, int ) {} );
             int off = nr_q;
 #pragma unroll
             for ( int o = 1; o < 16; o <<= 1 )
@@ -715,34 +740,31 @@ __global__ __launch_bounds__( BTPB ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 
                     off += u;
             }
             nr = __builtin_amdgcn_readlane( off, 8 );
-            off -= nr_q;
-            const int off0 = off;
+            // the range of cell ce's locals and their place in it
+            int vb = 0, vo = 0;
             if ( lane < 9 )
             {
-                if ( !gh )
-                {
-                    rs[off] = s_lcs[lane][elo];
-                    rf[off] = ( s_lcs[lane][elo] + s_dl[lane] ) * ( HALF ? 2 : 1 );
-                    rp[off + 1] = s_lcs[lane][ehi + 1] - s_lcs[lane][elo];
-                }
-                else
-                {
-                    for ( int c2 = elo; c2 <= ehi; ++c2 )
+                int r = off - nr_q - 1, n = 0;
+                runs(
+                    [&]( int kind, int s0 )
                     {
-                        rs[off] = s_lcs[lane][c2];
-                        rf[off] = s_lcs[lane][c2] + s_dl[lane];
-                        rp[off + 1] = s_lcs[lane][c2 + 1] - s_lcs[lane][c2];
-                        rs[off + 1] = s_gcs[lane][c2];
-                        rf[off + 1] = s_gcs[lane][c2] + s_dg[lane];
+                        ++r;
+                        n = 0;
+                        rs[r] = s0;
+                        rf[r] = s0 + ( kind ? s_dg[lane] : s_dl[lane] );
                         if ( HALF ) // bit 0: ghosts
+                            rf[r] = 2 * rf[r] + kind;
+                    },
+                    [&]( int kind, int c2, int len )
+                    {
+                        if ( kind == 0 && c2 == ce )
                         {
-                            rf[off] *= 2;
-                            rf[off + 1] = 2 * rf[off + 1] + 1;
+                            vb = r;
+                            vo = n;
                         }
-                        rp[off + 2] = s_gcs[lane][c2 + 1] - s_gcs[lane][c2];
-                        off += 2;
-                    }
-                }
+                        n += len;
+                        rp[r + 1] = n;
+                    } );
             }
             __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
             // prefix of the range lengths (nr <= MAXR < 64: one range per lane)
@@ -764,15 +786,7 @@ __global__ __launch_bounds__( BTPB ) __attribute__( ( amdgpu_waves_per_eu( 2, 4 
                             : ( rf[lane] - t_p ) * rec;
             }
             // candidate index of the cell's first atom, in the centre
-            // column's (lane 4's) ranges: the locals of cell ce, its range
-            // 2 (ce - elo) where the column holds ghosts, else at offset
-            // ce - elo cells into its single range
-            int vb = 0, vo = 0;
-            if ( lane == 4 )
-            {
-                vb = gh ? off0 + 2 * ( ce - elo ) : off0;
-                vo = gh ? 0 : s_lcs[4][ce] - s_lcs[4][elo];
-            }
+            // column's (lane 4's) ranges
             const int rc = __builtin_amdgcn_readlane( vb, 4 );
             vbase = __builtin_amdgcn_readlane( t_p, rc ) + __builtin_amdgcn_readlane( vo, 4 );
             __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
@@ -1078,6 +1092,40 @@ cmd_status tiles_ghost_refresh( cmd_system *S )
 // local atoms the tiles cover, [2] most slab waves of a tile, [3] largest
 // staged count of one atom column's 3 x 3 columns, [4] most atoms of one
 // atom column.
+// Largest distance of a staged coordinate from its build block's origin: 1.5
+// cells across, half the staged cells along the column.
+double tile_amax( const CellGrid &g, int E )
+{
+    return 1.001 * std::max( { 1.5 / g.rd[0], 1.5 / g.rd[1], 0.5 * ( E + 2 ) / g.rd[2] } );
+}
+
+// The sources of a build on the system's binning grid.
+static TileSrc system_src( const cmd_neigh *N, const cmd_system *S )
+{
+    return { nullptr, nullptr, S->bins.start.p, S->gsort.start.p, S->xg.p, S->ghost_out.p,
+             tile_amax( N->tg.g, N->tg.E ) };
+}
+
+static cmd_status tile_info_run( cmd_neigh *N, cmd_system *S, const TileSrc &src )
+{
+    const TileGrid &T = N->tg;
+    CMD_TRY( N->tile_info.reserve( (size_t)T.ntiles * TI_WORDS ) );
+    CMD_TRY( S->sc.ires.reserve( TILE_RES_WORDS ) );
+    DevBuf<int> &waves = N->grid_sort.cursor; // scratch: waves per tile
+    CMD_TRY( waves.reserve( T.ntiles + 1 ) );
+    CMD_TRY( N->grid_sort.start.reserve( T.ntiles + 1 ) ); // scan of waves
+    // the maxima and the build's own words (longest row, capacity flag)
+    CMD_TRY( fill_i32( S->sc.ires.p, 0, TILE_RES_WORDS, S->stream ) );
+    const int apw = 64 / N->lanes;
+    constexpr int per = INFO_TPB / 64;
+    k_tile_info<<<( T.ntiles + per - 1 ) / per, INFO_TPB, 0, S->stream>>>(
+        T, src, apw, N->tile_info.p, waves.p, S->sc.ires.p );
+    CMD_LAUNCH_CHECK();
+    CMD_TRY( scan_exclusive( waves.p, N->grid_sort.start.p, T.ntiles, S->sc,
+                             S->stream, nullptr ) );
+    return CMD_OK;
+}
+
 static cmd_status tile_info_launch( cmd_neigh *N, cmd_system *S, int W, int E )
 {
     TileGrid &T = N->tg;
@@ -1092,22 +1140,7 @@ static cmd_status tile_info_launch( cmd_neigh *N, cmd_system *S, int W, int E )
     T.ntiles = T.nt0 * T.nt1 * T.tpc;
     CMD_REQUIRE( T.nc0 > 0 && T.nc1 > 0 && T.tpc > 0, CMD_ERR_ARG,
                  "binning grid has no interior cells" );
-    CMD_TRY( N->tile_info.reserve( (size_t)T.ntiles * TI_WORDS ) );
-    CMD_TRY( S->sc.ires.reserve( TILE_RES_WORDS ) );
-    DevBuf<int> &waves = N->grid_sort.cursor; // scratch: waves per tile
-    CMD_TRY( waves.reserve( T.ntiles + 1 ) );
-    CMD_TRY( N->grid_sort.start.reserve( T.ntiles + 1 ) ); // scan of waves
-    // the maxima and the build's own words (longest row, capacity flag)
-    CMD_TRY( fill_i32( S->sc.ires.p, 0, TILE_RES_WORDS, S->stream ) );
-    const int apw = 64 / N->lanes;
-    constexpr int per = INFO_TPB / 64;
-    k_tile_info<<<( T.ntiles + per - 1 ) / per, INFO_TPB, 0, S->stream>>>(
-        T, S->bins.start.p, S->gsort.start.p, apw, S->ghost_out.p, N->tile_info.p, waves.p,
-        S->sc.ires.p );
-    CMD_LAUNCH_CHECK();
-    CMD_TRY( scan_exclusive( waves.p, N->grid_sort.start.p, T.ntiles, S->sc,
-                             S->stream, nullptr ) );
-    return CMD_OK;
+    return tile_info_run( N, S, system_src( N, S ) );
 }
 
 // Reads the result words (res, TILE_RES_WORDS of them) and the slab waves
@@ -1191,19 +1224,16 @@ static size_t force_lds( int slots, int rec )
 }
 
 template <int G>
-static void launch_build( cmd_neigh *N, cmd_system *S, int slot_cap, int rows_cap,
-                          int waves_cap, size_t lds )
+static void launch_build( cmd_neigh *N, cmd_system *S, const TileSrc &src, int slot_cap,
+                          int rows_cap, int waves_cap, size_t lds )
 {
     const double rc2 = N->neigh_cut * N->neigh_cut;
     // the list build tests in FP32 about each block's origin: every
-    // staged coordinate lies within amax of it (1.5 cells across, half the
-    // staged cells along the column), so the FP32 r^2 is within
-    // 128 amax^2 2^-24 of the FP64 one (roundings of the coordinates, their
-    // differences, the squares and the sums); candidates within that band of
-    // rc^2 are tested again in FP64
-    const CellGrid &g = N->tg.g;
-    const double amax = 1.001 * std::max( { 1.5 / g.rd[0], 1.5 / g.rd[1],
-                                            0.5 * ( N->tg.E + 2 ) / g.rd[2] } );
+    // staged coordinate lies within amax of it (tile_amax), so the FP32 r^2
+    // is within 128 amax^2 2^-24 of the FP64 one (roundings of the
+    // coordinates, their differences, the squares and the sums); candidates
+    // within that band of rc^2 are tested again in FP64
+    const double amax = src.amax;
     double band = 128.0 * amax * amax * std::ldexp( 1.0, -24 ) + 1e-6 * rc2;
     // CMD_BUILD_BAND widens the band (never narrows it), so that tests can
     // send most candidates through the FP64 re-test
@@ -1219,20 +1249,20 @@ static void launch_build( cmd_neigh *N, cmd_system *S, int slot_cap, int rows_ca
     const int nb = N->tg.ntiles * N->tg.W * N->tg.W;
     if ( N->half )
         k_tile_build<G, true><<<nb, threads, lds, S->stream>>>(
-            N->tg, S->bins.start.p, S->gsort.start.p, N->tile_info.p,
-            N->grid_sort.start.p, S->x.p, S->xg.p, rc2, N->rec, N->cap, slot_cap, rows_cap,
+            N->tg, src, N->tile_info.p, N->grid_sort.start.p, S->x.p, rc2, N->rec, N->cap,
+            slot_cap, rows_cap,
             waves_cap, N->tslab.p, N->fcounts.p, N->counts.p, res + TILE_RES_MAXROW,
             res + TILE_RES_MAXHALF, res + TILE_RES_OVER, res + TILE_RES_WAVES, lo, hi, eps );
     else
         k_tile_build<G, false><<<nb, threads, lds, S->stream>>>(
-            N->tg, S->bins.start.p, S->gsort.start.p, N->tile_info.p,
-            N->grid_sort.start.p, S->x.p, S->xg.p, rc2, N->rec, N->cap, slot_cap, rows_cap,
+            N->tg, src, N->tile_info.p, N->grid_sort.start.p, S->x.p, rc2, N->rec, N->cap,
+            slot_cap, rows_cap,
             waves_cap, N->tslab.p, N->counts.p, nullptr, res + TILE_RES_MAXROW,
             res + TILE_RES_MAXHALF, res + TILE_RES_OVER, res + TILE_RES_WAVES, lo, hi, eps );
 }
 
-static cmd_status launch_build_g( cmd_neigh *N, cmd_system *S, int slot_cap, int rows_cap,
-                                  int waves_cap, size_t lds )
+static cmd_status launch_build_g( cmd_neigh *N, cmd_system *S, const TileSrc &src,
+                                  int slot_cap, int rows_cap, int waves_cap, size_t lds )
 {
     // a half list's rows hold the full neighbourhood: their lengths go to
     // fcounts, the half list's own to counts
@@ -1241,13 +1271,13 @@ static cmd_status launch_build_g( cmd_neigh *N, cmd_system *S, int slot_cap, int
     switch ( N->lanes )
     {
     case 2:
-        launch_build<2>( N, S, slot_cap, rows_cap, waves_cap, lds );
+        launch_build<2>( N, S, src, slot_cap, rows_cap, waves_cap, lds );
         break;
     case 4:
-        launch_build<4>( N, S, slot_cap, rows_cap, waves_cap, lds );
+        launch_build<4>( N, S, src, slot_cap, rows_cap, waves_cap, lds );
         break;
     default:
-        launch_build<8>( N, S, slot_cap, rows_cap, waves_cap, lds );
+        launch_build<8>( N, S, src, slot_cap, rows_cap, waves_cap, lds );
         break;
     }
     CMD_LAUNCH_CHECK();
@@ -1396,7 +1426,7 @@ cmd_status tiles_build( cmd_neigh *N, cmd_system *S, bool *built )
         N->max_tile_slots = h[0];
         // the slab sized for the next build's launch too (record_spec)
         CMD_TRY( N->tslab.reserve( tile_slab_entries( N, h[5] + std::max( 64, h[5] / 50 ) ) ) );
-        CMD_TRY( launch_build_g( N, S, h[3] + 1, h[4], h[5], lds ) );
+        CMD_TRY( launch_build_g( N, S, system_src( N, S ), h[3] + 1, h[4], h[5], lds ) );
         CMD_TRY( tile_results( N, S, res, &h[5], true ) );
         const int mr = res[TILE_RES_MAXROW];
         list_rows( N, res );
@@ -1411,6 +1441,53 @@ cmd_status tiles_build( cmd_neigh *N, cmd_system *S, bool *built )
             return CMD_OK;
         }
         // rows overflowed: larger rows, and the LDS fit rechecked
+        N->cap = std::max( N->max_neigh_guess, (int)( mr * 1.1 ) );
+    }
+    set_error( "neighbour rows kept growing during the tiled build" );
+    return CMD_ERR_CAPACITY;
+}
+
+cmd_status tiles_build_batch( cmd_neigh *N, cmd_system *S, const TileSrc &src, bool *built )
+{
+    *built = false;
+    N->spec.valid = false;
+    N->rec = TILE_REC;
+    if ( N->cap < 1 )
+        N->cap = std::max( 1, N->max_neigh_guess );
+    size_t hard = 0, lds_cu = 0;
+    lds_limits( &hard, &lds_cu );
+    CMD_TRY( tile_info_run( N, S, src ) );
+    int h[6] = { 0, 0, 0, 0, 0, 0 }, res[TILE_RES_WORDS];
+    CMD_TRY( tile_results( N, S, res, &h[5], false ) );
+    for ( int k = 0; k < 5; ++k )
+        h[k] = res[TILE_RES_INFO + k];
+    N->tg.bw = force_waves( N, h[2] );
+    if ( h[1] != S->n_local )
+        return CMD_OK; // an atom outside its system's interior cells
+    for ( int attempt = 0; attempt < 4; ++attempt )
+    {
+        const size_t lds = build_lds( N, h[3] + 1, h[4] );
+        bool fits = false;
+        int blocks = 0;
+        if ( !layout_ok( N, h, lds, hard, lds_cu, 1, &fits, &blocks ) || !fits )
+            return CMD_OK; // too dense for the tile shape
+        N->tile_blocks = blocks;
+        N->max_tile_slots = h[0];
+        CMD_TRY( N->tslab.reserve( tile_slab_entries( N, h[5] ) ) );
+        // the maxima of the build proper start afresh
+        CMD_TRY( fill_i32( S->sc.ires.p + TILE_RES_MAXROW, 0, 1, S->stream ) );
+        CMD_TRY( launch_build_g( N, S, src, h[3] + 1, h[4], h[5], lds ) );
+        int nw = 0;
+        CMD_TRY( tile_results( N, S, res, &nw, true ) );
+        const int mr = res[TILE_RES_MAXROW];
+        list_rows( N, res );
+        if ( mr <= N->cap )
+        {
+            *built = true;
+            N->tiled = true;
+            N->built_rec = N->rec;
+            return CMD_OK;
+        }
         N->cap = std::max( N->max_neigh_guess, (int)( mr * 1.1 ) );
     }
     set_error( "neighbour rows kept growing during the tiled build" );
@@ -1437,7 +1514,7 @@ cmd_status tiles_build_spec( cmd_neigh *N, cmd_system *S, bool *built )
     N->cap = P.cap; // grown ahead of the rows (record_spec)
     CMD_TRY( tile_info_launch( N, S, P.W, P.E ) );
     CMD_TRY( N->tslab.reserve( tile_slab_entries( N, P.slab_waves ) ) );
-    CMD_TRY( launch_build_g( N, S, P.slot_cap, P.rows, P.slab_waves, P.lds ) );
+    CMD_TRY( launch_build_g( N, S, system_src( N, S ), P.slot_cap, P.rows, P.slab_waves, P.lds ) );
     int res[TILE_RES_WORDS], h[6] = { 0, 0, 0, 0, 0, 0 };
     CMD_TRY( tile_results( N, S, res, &h[5], true ) );
     for ( int k = 0; k < 5; ++k )

@@ -48,6 +48,7 @@ __device__ __forceinline__ void tile_coords( const TileGrid &T, int t, int &a0,
     // tile columns in strips of TILE_STRIP rows of a, b outer and a inner
     // within a strip: the columns around a tile are staged by its neighbours
     // close together in time, so a staged column is mostly re-read from L2
+    t -= T.tile0;
     const int col = t / T.tpc, z = t % T.tpc;
     const int strip = col / ( TILE_STRIP * T.nt1 ), r = col % ( TILE_STRIP * T.nt1 );
     const int h = min( TILE_STRIP, T.nt0 - strip * TILE_STRIP );
@@ -59,7 +60,7 @@ __device__ __forceinline__ void tile_coords( const TileGrid &T, int t, int &a0,
 
 __device__ __forceinline__ int col_base( const TileGrid &T, int a, int b )
 {
-    return ( a * T.g.n[1] + b ) * T.g.n[2];
+    return T.cell0 + ( a * T.g.n[1] + b ) * T.g.n[2];
 }
 
 // Round-robin dispatch puts block b on XCD b % 8; give XCD k the k-th

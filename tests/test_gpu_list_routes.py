@@ -1,0 +1,128 @@
+"""List builds and layouts at the sizes where their routes change, through the
+C ABI: the global build against a search of all pairs, batches on tiled lists
+against the FP64 oracle and the global layout, and small boxes over several
+rebuilds."""
+import numpy as np
+import pytest
+from scipy.spatial import cKDTree
+
+import pyoracle as O
+from test_gpu_batch import SYSTEMS, _add, _min_image, _oracle, _params
+
+pytestmark = pytest.mark.gpu
+
+
+def _pairs(x, rc, half):
+    """Rows of all pairs within rc (accepted in FP64 as the engine does)."""
+    d = cKDTree(x).query_pairs(rc * (1 + 1e-9), output_type="ndarray")
+    i, j = np.concatenate([d, d[:, ::-1]]).T
+    e = x[i] - x[j]
+    ok = e[:, 0] ** 2 + e[:, 1] ** 2 + e[:, 2] ** 2 <= rc * rc
+    if half:  # j above i in x, then y, then z
+        up = [tuple(p) > tuple(q) for p, q in zip(x[j], x[i])]
+        ok &= np.array(up, bool)
+    i, j = i[ok], j[ok]
+    rows = [set() for _ in x]
+    for a, b in zip(i, j):
+        rows[a].add(b)
+    return rows
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("lanes", [1, 8])
+@pytest.mark.parametrize("n,side,ghosts", [
+    (1, 3.0, 0),       # one atom, one wave
+    (5, 4.0, 2),       # waves of four atoms, a part-full one
+    (700, 2.0, 60),    # one dense cell: two register passes
+    (8191, 22.0, 0),   # the row scan's single block, one below,
+    (8192, 22.0, 0),   # at
+    (8193, 22.0, 900), # and above its limit
+    (140000, 60.0, 0), # sixteen atoms a wave
+])
+def test_global_list_rows(gpu, n, side, ghosts, lanes, half):
+    M = gpu
+    if n > 100000 and (half or lanes > 1):
+        pytest.skip("one of the large case is enough")
+    rc = 1.3
+    rng = np.random.default_rng(n)
+    x = rng.uniform(0.0, side, (n + ghosts, 3))
+    x[: n // 3, 0] = np.round(x[: n // 3, 0], 1)  # equal coordinates
+    s = M.System(1)
+    s.create_domain([0, 0, 0], [side] * 3, rc)
+    s.upload(x, np.zeros_like(x), None, np.zeros(len(x), np.int32),
+             np.arange(1, len(x) + 1, dtype=np.int32), n_ghost=ghosts)
+    nl = M.NeighborVerlet(rc, half, 8, lanes=lanes)
+    nl.create(s)
+    off, idx = nl.get()
+    rows = _pairs(x, rc, half)[:n]
+    assert np.array_equal(np.diff(off), [len(r) for r in rows])
+    for i in range(n):
+        assert set(idx[off[i]:off[i + 1]].tolist()) == rows[i]
+
+
+@pytest.mark.parametrize("shape", ["2,2,3,0", "4,1,6,0", "8,3,2,0"])
+def test_batch_tiles_match_oracle(gpu, monkeypatch, shape):
+    """Two rebuilds on tiled lists, as the global layout's own test (the same
+    bounds); boxes of 3 to 5 cells, the lattice's atoms on the box faces."""
+    M = gpu
+    monkeypatch.setenv("CMD_TUNE", shape)
+    B = M.Batch(_params(M), M.PREC_FP64, lanes=0)
+    hs = [_add(M, B, s) for s in SYSTEMS]
+    B.run(50)
+    assert B.counts()["lanes"] == int(shape[0])
+    for h, spec in zip(hs, SYSTEMS):
+        L = np.array(spec[0]) * (4.0 / spec[1]) ** (1.0 / 3.0)
+        x, v, f, _, _ = B.download(h)
+        xo, vo, fo, tho = _oracle(spec, 50)
+        assert np.abs(_min_image(x - xo, L)).max() < 1e-9
+        assert np.abs(v - vo).max() < 1e-9
+        assert np.abs(f - fo).max() < 1e-7 * np.abs(fo).max()
+        for row in B.thermo(h):
+            ro = tho[tho[:, 0] == row[0]][0]
+            assert np.allclose(row[1:], ro[1:], rtol=1e-10, atol=1e-12), (row, ro)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_batch_tiles_alone_equals_in_mix(gpu, monkeypatch, prec):
+    """Members join and leave around a system on tiled lists: bit-identical
+    to the same system alone."""
+    M = gpu
+    monkeypatch.setenv("CMD_TUNE", "2,2,3,0")
+    P = M.PREC_FP64 if prec == "fp64" else M.PREC_MIXED
+    alone = M.Batch(_params(M), P, lanes=0)
+    ha = _add(M, alone, SYSTEMS[1])
+    mix = M.Batch(_params(M), P, lanes=0)
+    hb = _add(M, mix, SYSTEMS[0])
+    hm = _add(M, mix, SYSTEMS[1])
+    for k in (20, 20, 7):
+        alone.run(k)
+        mix.run(k)
+        if hb is not None:
+            mix.remove(hb)
+            _add(M, mix, SYSTEMS[3])
+            hb = None
+    for a, b in zip(alone.download(ha), mix.download(hm)):
+        assert np.array_equal(a, b)
+    assert np.array_equal(alone.thermo(ha), mix.thermo(hm))
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("ncells", [(4, 4, 4), (4, 5, 9)])
+def test_small_box_rebuilds(gpu, ncells, half):
+    """Boxes of two to five cells, every cell beside ghosts: the tiled list
+    over five rebuilds against the oracle's loop."""
+    M = gpu
+    kw = dict(ncells=ncells, nsteps=100, thermo=20, half=half)
+    md = M.CbnMD(M.lattice_params(**kw), precision=M.PREC_FP64, lanes=2)
+    md.init()
+    md.run(100)
+    ref = O.MD(O.lj_params(**kw))
+    ref.init()
+    ref.run(100)
+    n = md.n_local
+    assert np.allclose(md.thermo()[:, :4], ref.thermo(), rtol=1e-10, atol=1e-13)
+    x, v = md.arrays()[:2]
+    xo, vo = ref.arrays()[:2]
+    o, p = (np.argsort(m.arrays()[4][:n], kind="stable") for m in (md, ref))
+    assert np.abs(x[:n][o] - xo[:n][p]).max() < 1e-9
+    assert np.abs(v[:n][o] - vo[:n][p]).max() < 1e-9
