@@ -603,7 +603,7 @@ struct cmd_batch
     // Tiled lists (tiles.hip) where the layout is tuned: tiles of tile_w x
     // tile_w columns, tile_e cells tall (0: the global layout); every
     // system's tiles in one space, each with its system's grid.
-    bool may_tile = true;
+    bool may_tile = false; // ghosts are kept in cell order
     int tile_w = 0, tile_e = 0;
     DevBuf<TileGrid> tgrids;
     DevBuf<int> tgrid_of;
@@ -1064,67 +1064,109 @@ cmd_status autotune( cmd_batch *B )
     {
         int G, W, E;
     };
-    std::vector<Cand> cands{ { 1, 0, 0 }, { 2, 0, 0 }, { 4, 0, 0 },
-                             { 8, 0, 0 }, { 2, 2, 3 }, { 2, 2, 4 } };
+    std::vector<Cand> slabs{ { 1, 0, 0 }, { 2, 0, 0 }, { 4, 0, 0 }, { 8, 0, 0 } };
+    std::vector<Cand> tiles{ { 2, 2, 3 }, { 2, 2, 4 } };
     // CMD_TUNE=G,W,E,bw limits the search to one layout, as for one system
     if ( const char *e = std::getenv( "CMD_TUNE" ) )
     {
         Cand c{};
         if ( std::sscanf( e, "%d,%d,%d", &c.G, &c.W, &c.E ) == 3 )
-            cands.assign( 1, c );
+        {
+            slabs.assign( c.E == 0 ? 1 : 0, c );
+            tiles.assign( c.E > 0 ? 1 : 0, c );
+        }
     }
     hipEvent_t e0, e1;
     CMD_HIP( hipEventCreate( &e0 ) );
     CMD_HIP( hipEventCreate( &e1 ) );
-    float best = 1e30f;
-    Cand bestc = cands[0];
     StepCtl ctl{};
-    auto build = [&]( const Cand &c, bool *built ) -> cmd_status
+    // time of one force call on the list as built
+    auto step_ms = [&]( const Cand &c, float *ms ) -> cmd_status
     {
-        *built = true;
-        if ( c.E == 0 )
-        {
-            B->tile_w = B->tile_e = 0;
-            return build_list( B, c.G );
-        }
-        CMD_TRY( upload_tiles( B, c.W, c.E ) );
-        return build_tiles( B, c.G, built );
-    };
-    cmd_status st = CMD_OK;
-    for ( const Cand &c : cands )
-    {
-        bool built = false;
-        if ( ( st = build( c, &built ) ) != CMD_OK )
-            break;
-        if ( !built )
-            continue;
-        if ( ( st = lj_full( B->F, B->S, B->N, ctl, nullptr, nullptr, nullptr ) ) != CMD_OK )
-            break;
+        CMD_TRY( lj_full( B->F, B->S, B->N, ctl, nullptr, nullptr, nullptr ) );
         (void)hipEventRecord( e0, B->stream );
         for ( int r = 0; r < 3; ++r )
             (void)lj_full( B->F, B->S, B->N, ctl, nullptr, nullptr, nullptr );
         (void)hipEventRecord( e1, B->stream );
         (void)hipEventSynchronize( e1 );
-        float ms = 0.f;
-        (void)hipEventElapsedTime( &ms, e0, e1 );
+        (void)hipEventElapsedTime( ms, e0, e1 );
+        *ms /= 3;
         if ( std::getenv( "CMD_VERBOSE" ) )
             std::fprintf( stderr, "# batch lanes=%d tile=%dx%dx%d: %.4f ms\n", c.G, c.W, c.W,
-                          c.E, ms / 3 );
-        if ( ms < best )
+                          c.E, *ms );
+        return CMD_OK;
+    };
+    auto rebuild_ms = [&]( int G, float *ms ) -> cmd_status
+    {
+        (void)hipEventRecord( e0, B->stream );
+        CMD_TRY( rebuild( B, G ) );
+        (void)hipEventRecord( e1, B->stream );
+        (void)hipEventSynchronize( e1 );
+        (void)hipEventElapsedTime( ms, e0, e1 );
+        if ( std::getenv( "CMD_VERBOSE" ) )
+            std::fprintf( stderr, "# batch rebuild %.4f ms\n", *ms );
+        return CMD_OK;
+    };
+    auto run = [&]() -> cmd_status
+    {
+        Cand bs{}, bt{};
+        float fs = 1e30f, ft = 1e30f, rs = 0.f, rt = 0.f, ms = 0.f;
+        for ( const Cand &c : slabs )
         {
-            best = ms;
-            bestc = c;
+            CMD_TRY( build_list( B, c.G ) );
+            CMD_TRY( step_ms( c, &ms ) );
+            if ( ms < fs )
+            {
+                fs = ms;
+                bs = c;
+            }
         }
-    }
+        if ( bs.G > 0 )
+            CMD_TRY( rebuild_ms( bs.G, &rs ) );
+        B->may_tile = true;
+        bool sorted = false; // ghosts in cell order
+        for ( const Cand &c : tiles )
+        {
+            CMD_TRY( upload_tiles( B, c.W, c.E ) );
+            if ( sorted )
+            {
+                bool built = false;
+                CMD_TRY( build_tiles( B, c.G, &built ) );
+            }
+            else
+                CMD_TRY( rebuild( B, c.G ) );
+            sorted = true;
+            if ( !B->N->tiled )
+                continue;
+            CMD_TRY( step_ms( c, &ms ) );
+            if ( ms < ft )
+            {
+                ft = ms;
+                bt = c;
+            }
+        }
+        if ( bt.G > 0 )
+        {
+            CMD_TRY( upload_tiles( B, bt.W, bt.E ) );
+            CMD_TRY( rebuild_ms( bt.G, &rt ) );
+        }
+        // the step time and the rebuild's share of the steps it serves
+        const float every = (float)B->p.every;
+        if ( bt.G > 0 && ( bs.G == 0 || ft + rt / every < fs + rs / every ) )
+        {
+            B->lanes = bt.G;
+            return CMD_OK;
+        }
+        CMD_REQUIRE( bs.G > 0, CMD_ERR_STATE, "the requested tiles do not fit" );
+        B->may_tile = false;
+        B->tile_w = B->tile_e = 0;
+        B->lanes = bs.G;
+        return rebuild( B, bs.G );
+    };
+    const cmd_status st = run();
     (void)hipEventDestroy( e0 );
     (void)hipEventDestroy( e1 );
-    CMD_TRY( st );
-    B->lanes = bestc.G;
-    bool built = false;
-    CMD_TRY( build( bestc, &built ) );
-    CMD_REQUIRE( built, CMD_ERR_STATE, "the chosen tiled list was built before" );
-    B->may_tile = bestc.E > 0;
-    return CMD_OK;
+    return st;
 }
 
 // Membership changes at a rebuild boundary: leaving systems are dropped,
@@ -1239,8 +1281,6 @@ cmd_status apply_changes( cmd_batch *B )
     if ( B->nnp && B->lanes == 0 )
         B->lanes = 1; // the NNP kernels read the list as CSR
     const bool tune = B->lanes == 0 && S->n_local > 0;
-    if ( B->lanes != 0 && B->tile_e == 0 )
-        B->may_tile = false;
     if ( B->tile_e > 0 ) // the members' grids changed
         CMD_TRY( upload_tiles( B, B->tile_w, B->tile_e ) );
     CMD_TRY( rebuild( B, tune ? 1 : B->lanes ) );
