@@ -654,10 +654,11 @@ double now_s()
 }
 
 // Cell grid of one system: cells of at least neigh_cut over the system's
-// ghost shell, at most 1024 per dimension.  LJ systems: cells aligned with
-// the box and one around it on each side (boxes are longer than 2 depth, and
-// depth is neigh_cut, so these hold the ghosts); others: over [lo - depth,
-// hi + depth].
+// ghost shell [lo - depth, hi + depth], at most 1024 per dimension.  On tiles
+// the cells are aligned with the box, with one around it on each side (boxes
+// are longer than 2 depth, and depth is neigh_cut, so these hold the ghosts);
+// they are wider, so the global layout, which needs no aligned cells, tests
+// fewer candidates without.
 void grid_of( BSys &s, double depth, double cut, bool aligned )
 {
     s.aligned = aligned;
@@ -694,7 +695,7 @@ cmd_status upload_table( cmd_batch *B )
             s.hi[d] = m.hi[d];
             s.L[d] = m.hi[d] - m.lo[d];
         }
-        grid_of( s, depth, B->N->neigh_cut, !B->nnp );
+        grid_of( s, depth, B->N->neigh_cut, B->may_tile );
         s.cell_base = cb;
         cb += s.gn[0] * s.gn[1] * s.gn[2];
         s.a0 = a0;
@@ -708,6 +709,15 @@ cmd_status upload_table( cmd_batch *B )
         CMD_HIP( hipMemcpyAsync( B->tab.p, B->htab.data(), sizeof( BSys ) * B->htab.size(),
                                  hipMemcpyHostToDevice, B->stream ) );
     return CMD_OK;
+}
+
+// The systems' grids for tiled lists or the global layout.
+cmd_status set_tiling( cmd_batch *B, bool on )
+{
+    B->may_tile = on;
+    // (the table's last upload reads the host copy)
+    CMD_HIP( hipStreamSynchronize( B->stream ) );
+    return upload_table( B );
 }
 
 // Stable counting sort of n cell ids already in cs.cell_of.
@@ -1066,6 +1076,12 @@ cmd_status autotune( cmd_batch *B )
     };
     std::vector<Cand> slabs{ { 1, 0, 0 }, { 2, 0, 0 }, { 4, 0, 0 }, { 8, 0, 0 } };
     std::vector<Cand> tiles{ { 2, 2, 3 }, { 2, 2, 4 } };
+    // below this size the positions stay in the L2s and the search's own time
+    // is not won back (50 systems, 85,000 atoms, FP64: 0.025 ms a force call
+    // on 4 lanes, 0.026 on tiles; 60 systems, 220,000 atoms, mixed: 0.047 and
+    // 0.035)
+    if ( B->S->n_local < 65536 )
+        tiles.clear();
     // CMD_TUNE=G,W,E,bw limits the search to one layout, as for one system
     if ( const char *e = std::getenv( "CMD_TUNE" ) )
     {
@@ -1123,7 +1139,7 @@ cmd_status autotune( cmd_batch *B )
         }
         if ( bs.G > 0 )
             CMD_TRY( rebuild_ms( bs.G, &rs ) );
-        B->may_tile = true;
+        CMD_TRY( set_tiling( B, true ) );
         bool sorted = false; // ghosts in cell order
         for ( const Cand &c : tiles )
         {
@@ -1158,7 +1174,7 @@ cmd_status autotune( cmd_batch *B )
             return CMD_OK;
         }
         CMD_REQUIRE( bs.G > 0, CMD_ERR_STATE, "the requested tiles do not fit" );
-        B->may_tile = false;
+        CMD_TRY( set_tiling( B, false ) );
         B->tile_w = B->tile_e = 0;
         B->lanes = bs.G;
         return rebuild( B, bs.G );

@@ -16,7 +16,10 @@
 // in k_nnp_sf).  Candidate pairs rejected by the r_jk test and the
 // bookkeeping of the compacted pair stream are not counted: the model is
 // the useful work, and the hardware counters (SQ_INSTS_VALU_FLOPS_FP32)
-// measure what is issued.
+// measure what is issued.  The builds for zeta = 1, 2, 4 and 16 (k_nnp_sf_pow,
+// k_nnp_force_pow) do the same useful work with fewer operations: squarings
+// in place of log2 and exp2, and one combination of two vectors per triplet
+// in place of a gradient per function.
 #pragma once
 
 namespace cmd

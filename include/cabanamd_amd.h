@@ -207,9 +207,9 @@ cmd_status cmd_force_virial( cmd_force *f, cmd_system *s, cmd_neigh *n,
  * are written to local and ghost rows; fold them with cmd_comm_update_force,
  * as the reference does after an NNP force (cabanamd_impl.h:346-353).
  * cmd_force_set_precision: CMD_PREC_MIXED runs the network layers as BF16
- * MFMA GEMMs with FP32 accumulation (default), CMD_PREC_FP64 runs them in
- * FP32 on the vector units; symmetry functions and forces are FP32 either
- * way, forces are accumulated in FP64. */
+ * MFMA GEMMs with FP32 accumulation (default), CMD_PREC_FP64 runs them as
+ * FP32 MFMA GEMMs; symmetry functions and forces are FP32 either way, forces
+ * are accumulated in FP64. */
 typedef struct cmd_nnp_model cmd_nnp_model;
 
 cmd_status cmd_nnp_model_create( int nelem, int n_hidden, const int *hidden,
