@@ -726,8 +726,31 @@ cmd_status sort_cells( cmd_batch *B, CellSort &cs, int n )
     return cell_sort_ids( n, B->ncell, cs, B->S->sc, B->stream );
 }
 
-// The tile grids of the batch's systems for tiles of W x W columns, E cells
-// tall (after a change of members or of the shape).
+// The tallest tile, up to E cells, whose staged neighbourhood is expected to
+// fit its LDS records in a system: the densest one spans W + 2 columns each
+// way and E + 2 cells, or the whole box and its ghost shell where that is
+// less; 12 % are left for fluctuations.  (Small boxes have cells up to half
+// again as wide as the cutoff: at E = 3 a few of them would send the whole
+// batch to the global layout.)
+int tile_height( const BSys &s, double depth, int W, int E )
+{
+    auto extent = [&]( int d, int cells )
+    {
+        const int n = s.gn[d] - 2;
+        const double w = s.L[d] / n;
+        if ( n >= cells )
+            return cells * w;
+        return s.L[d] + ( n == cells - 1 ? depth : 2.0 * depth );
+    };
+    const double rho = s.na / ( s.L[0] * s.L[1] * s.L[2] );
+    while ( E > 1 && 1.12 * rho * extent( 0, W + 2 ) * extent( 1, W + 2 ) * extent( 2, E + 2 ) >
+                         tile_max_slots() )
+        --E;
+    return E;
+}
+
+// The tile grids of the batch's systems for tiles of W x W columns, up to E
+// cells tall (after a change of members or of the shape).
 cmd_status upload_tiles( cmd_batch *B, int W, int E )
 {
     B->tile_w = W;
@@ -752,13 +775,13 @@ cmd_status upload_tiles( cmd_batch *B, int W, int E )
         T.W = W;
         T.nt0 = ( T.nc0 + W - 1 ) / W;
         T.nt1 = ( T.nc1 + W - 1 ) / W;
-        T.E = E;
-        T.tpc = ( s.gn[2] - 2 + E - 1 ) / E;
+        T.E = tile_height( s, B->N->neigh_cut, W, E );
+        T.tpc = ( s.gn[2] - 2 + T.E - 1 ) / T.E;
         T.ntiles = T.nt0 * T.nt1 * T.tpc;
         T.cell0 = s.cell_base;
         T.tile0 = (int)of.size();
         of.insert( of.end(), T.ntiles, (int)k );
-        B->tile_amax = std::max( B->tile_amax, tile_amax( T.g, E ) );
+        B->tile_amax = std::max( B->tile_amax, tile_amax( T.g, T.E ) );
     }
     B->ntiles = (int)of.size();
     CMD_TRY( B->tgrids.reserve( std::max<size_t>( 1, grids.size() ) ) );

@@ -571,6 +571,7 @@ cmd_status binning_create( cmd_system *s, double dx_in, double dy_in, double dz_
 // shape is not lowered (*built stays false where it does not fit).
 cmd_status tiles_build_batch( cmd_neigh *N, cmd_system *S, const TileSrc &src, bool *built );
 double tile_amax( const CellGrid &g, int E );
+int tile_max_slots(); // staged FP64 records of a tile
 cmd_status tiles_build( cmd_neigh *N, cmd_system *S, bool *built );
 cmd_status tiles_build_spec( cmd_neigh *N, cmd_system *S, bool *built );
 // Result words of the tiled build in the system's int scratch (sc.ires):

@@ -56,6 +56,8 @@ static int max_force_slots( int rec )
     return rec == TILE_REC32 ? MAX_SLOTS32 : MAX_SLOTS;
 }
 
+int tile_max_slots() { return MAX_SLOTS; }
+
 // Per-tile runs, atom columns and staged count; slab waves per tile.
 // slots[0] gets the largest staged count of a tile, slots[1] the number of
 // local atoms the tiles cover (all of them only when every local atom sits
