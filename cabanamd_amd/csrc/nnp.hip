@@ -655,10 +655,12 @@ __device__ __forceinline__ void pair_of( int p, int n, int &a, int &q )
 // with every lane busy (lane l takes entries l*per .. l*per + per - 1).
 // Used where the body keeps many accumulators in registers.
 // A wave that shares the atom with others takes every its-th test from it0.
+// With ALL the body runs in every lane of the wave, as body(a, q, ok): lanes
+// past the list repeat its last pair with ok false.
 // With PAIRS the body takes two pairs at once, (a0, q0) and (a1, q1), the
 // second valid when ok1 (else a repeat of the first): the two gradient
 // chains are independent, so their latencies overlap.
-template <bool PAIRS = false, int CAP = TCAP, class Body>
+template <bool PAIRS = false, int CAP = TCAP, bool ALL = false, class Body>
 __device__ __forceinline__ void for_triplets( const NbLds &L, int n, float rc2,
                                              unsigned short *buf, Body body,
                                              int *count = nullptr, int it0 = 0, int its = 1 )
@@ -738,6 +740,15 @@ __device__ __forceinline__ void for_triplets( const NbLds &L, int n, float rc2,
                 }
             }
         }
+        else if constexpr ( ALL )
+        {
+            for ( int j = 0; j < per; ++j )
+            {
+                const int e = lane * per + j;
+                const unsigned c = buf[min( e, cnt - 1 )];
+                body( (int)( c & 0xffu ), (int)( c >> 8 ), e < cnt );
+            }
+        }
         else
         {
             for ( int j = 0; j < per; ++j )
@@ -759,8 +770,9 @@ __device__ __forceinline__ void for_triplets( const NbLds &L, int n, float rc2,
 // (1 <= d <= n / 2) pairs neighbour l with neighbour (l + d) mod n in lane l,
 // so a row's test reads the partners from consecutive LDS records and its
 // valid pairs are one 64-bit mask.  The valid pairs of consecutive rows are
-// compacted into a ring of PAIR_RING codes; step(slot, l, p) runs on 64 of
-// them at a time.  Once all pairs of a row are done, row(d, mask, start) may
+// compacted into a ring of PAIR_RING codes; step(slot, l, p, ok) runs on 64 of
+// them at a time: in every lane of the wave with ROWS (lanes past the last pair
+// repeat it with ok false), else in the lanes that have one.  Once all pairs of a row are done, row(d, mask, start) may
 // collect what step left at ring slots start, start + 1, ... (one per mask
 // bit in lane order) -- each neighbour meets each of its pairs there in its
 // own lane, which replaces reactions added with LDS atomics: at 192,000 atoms
@@ -835,11 +847,11 @@ __device__ __forceinline__ int pair_ring( const NbLds &L, int n, float rc2, int 
         while ( prod - comp >= 64 || ( made > nrow && comp < prod ) )
         {
             const int e = comp + lane;
-            if ( e < prod )
+            if ( ROWS || e < prod )
             {
-                const int slot = e & ( PAIR_RING - 1 );
+                const int slot = min( e, prod - 1 ) & ( PAIR_RING - 1 );
                 const unsigned c = code[slot];
-                step( slot, (int)( c & 0xffu ), (int)( c >> 8 ) );
+                step( slot, (int)( c & 0xffu ), (int)( c >> 8 ), e < prod );
             }
             comp = min( comp + 64, prod );
         }
@@ -1107,7 +1119,7 @@ __global__ __launch_bounds__( NNP_TPB ) void k_nnp_sf_pow(
     int ntrip = 0;
     if ( n <= 64 )
         ntrip = pair_ring<false, WPA>(
-            L, n, rc2, part, tbuf[wv], [&]( int, int a, int q ) { triplet( a, q ); },
+            L, n, rc2, part, tbuf[wv], [&]( int, int a, int q, bool ) { triplet( a, q ); },
             []( int, unsigned long long, int ) {} );
     else
         for_triplets( L, n, rc2, tbuf[wv], triplet, &ntrip, part, WPA );
@@ -1778,7 +1790,7 @@ __global__ __launch_bounds__( NNP_TPB, 5 ) void k_nnp_force_pow(
     __builtin_amdgcn_fence( __ATOMIC_SEQ_CST, "wavefront" );
     const float krev = 0.5f / rc; // pi r / rc in revolutions
     const float kd = -0.5f * kpi;
-    // pa, pb and pm of the triplet (i, a, q)
+    // pa, pb and pm of the triplet (i, a, q); run by all lanes of the wave
     auto grad = [&]( const float4 &A, const float4 &B, const float4 &Ea, const float4 &Eb,
                      float &pa, float &pb, float &pm )
     {
@@ -1800,7 +1812,11 @@ __global__ __launch_bounds__( NNP_TPB, 5 ) void k_nnp_force_pow(
         // matrix cores: in 16 blocks of 4 x 4 with the coefficients as rows
         // and the Gaussians as columns, lane l is column l % 4 of block
         // l / 4 and receives its own triplet's four sums, so no operand
-        // changes lanes (a lane outside the exec mask fills only its own)
+        // changes lanes.  The coefficient rows of a block come from all four
+        // of its lanes, also where only some of them have a pair, and an MFMA
+        // reads a lane's registers whether it is in the exec mask or not: so
+        // every lane of the wave runs this (the compiler keeps the values of
+        // masked-out lanes only by chance)
         f32x4 T[2] = { { 0.f, 0.f, 0.f, 0.f }, { 0.f, 0.f, 0.f, 0.f } }, U[2] = { T[0], T[0] };
 #pragma unroll
         for ( int g = 0; g < NAG; ++g )
@@ -1854,12 +1870,15 @@ __global__ __launch_bounds__( NNP_TPB, 5 ) void k_nnp_force_pow(
         float sp = srad[0], sx = 0.f, sy = 0.f, sz = 0.f;
         pair_ring<true, WPA>(
             L, n, rc2, part, buf[wv].ring.code,
-            [&]( int slot, int a, int q ) {
+            [&]( int slot, int a, int q, bool ok ) {
                 float pa, pb, pm;
                 grad( L.d[a], L.d[q], L.e[a], L.e[q], pa, pb, pm );
-                rpa[slot] = pa;
-                rpm[slot] = pm;
-                rpb[slot] = pb;
+                if ( ok )
+                {
+                    rpa[slot] = pa;
+                    rpm[slot] = pm;
+                    rpb[slot] = pb;
+                }
             },
             [&]( int d, unsigned long long m, int s0 ) {
                 // as the pair's first neighbour, the partner d further on
@@ -1933,10 +1952,13 @@ __global__ __launch_bounds__( NNP_TPB, 5 ) void k_nnp_force_pow(
             atomicAdd( &sF[cur][1], -( spa * A.y + by ) );
             atomicAdd( &sF[cur][2], -( spa * A.z + bz ) );
         };
-        for_triplets<false, PAIR_RING>( L, n, rc2, buf[wv].flat.code, [&]( int a, int q ) {
+        for_triplets<false, PAIR_RING, true>( L, n, rc2, buf[wv].flat.code,
+                                              [&]( int a, int q, bool ok ) {
             const float4 A = L.d[a], B = L.d[q];
             float pa, pb, pm;
             grad( A, B, L.e[a], L.e[q], pa, pb, pm );
+            if ( !ok )
+                return;
             if ( a != cur )
             {
                 if ( cur >= 0 )

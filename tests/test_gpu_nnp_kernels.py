@@ -133,6 +133,25 @@ def test_neighbour_counts(gpu, n, pl):
     _check(gpu, m, x, t, "fp32")
 
 
+@pytest.mark.parametrize("neta", [1, 5, 8])
+@pytest.mark.parametrize("n", [64, 66, 67, 100, 127])
+def test_one_wave_past_64_neighbours(gpu, n, neta):
+    """A cluster of n atoms, every one a neighbour of every other, among
+    atoms with none: too few neighbours on average for four waves on an atom,
+    so one wave walks 63 to 126 neighbours, with pair counts of every
+    remainder by 4 (the lanes that share a block of matrix products)."""
+    x, t = _cluster(n, 1, n)
+    x = BOX / 2 + (x - BOX / 2) * min(1.0, 4.0 / np.ptp(x, axis=0).max())
+    g = np.arange(5.0, BOX, 10.0)
+    lone = np.array([(a, b, c) for a in g for b in g for c in g])
+    lone = lone[np.linalg.norm(lone - BOX / 2, axis=1) > 15.0]
+    assert n * (n - 1) < 48 * (n + len(lone))
+    x = np.vstack([x, lone])
+    t = np.zeros(len(x), np.int32)
+    m = _model(1, [0.01 * (k + 1) for k in range(neta)], POW2, rc=8.0)
+    _check(gpu, m, x, t, "fp32")
+
+
 def test_one_wave_per_atom_at_62_neighbours(gpu):
     """3,375 atoms, past the sizes that put four waves on an atom: the ring
     walk with most lanes in use, forces within 1e-5 of the oracle."""
