@@ -585,7 +585,8 @@ enum
     TILE_RES_OUTSIDE = 7,  // 1: a ghost lies outside the binning grid
     TILE_RES_WAVES = 8,    // slab waves of all tiles (written by the build)
     TILE_RES_MAXHALF = 9,  // longest row of a half list
-    TILE_RES_WORDS = 10
+    TILE_RES_SAME = 10,    // 1: a half list's atom has another at its very place
+    TILE_RES_WORDS = 11
 };
 static_assert( HW_TILE + TILE_RES_WORDS <= HW_WORDS, "tile results fit the pinned words" );
 cmd_status tiles_csr( cmd_neigh *N, int64_t *nnz );

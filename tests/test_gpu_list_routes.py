@@ -126,3 +126,47 @@ def test_small_box_rebuilds(gpu, ncells, half):
     o, p = (np.argsort(m.arrays()[4][:n], kind="stable") for m in (md, ref))
     assert np.abs(x[:n][o] - xo[:n][p]).max() < 1e-9
     assert np.abs(v[:n][o] - vo[:n][p]).max() < 1e-9
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("lanes,width", [(2, 1), (2, 2), (8, 2)])
+def test_half_list_skips_atoms_at_one_place(gpu, lanes, width, prec):
+    """Two atoms at the same coordinates are no pair of a half list (neither
+    is above the other), so they exert no force on each other: a list that
+    asks for tiles, whose forces walk both sides of each pair, against the
+    global layout, whose kernel walks the half rows."""
+    M = gpu
+    P = M.PREC_FP64 if prec == "fp64" else M.PREC_MIXED
+    x, _, _, _, _, hi = M.fcc_system((7, 7, 8), 0.8442, 1.0, 5)
+    hi = np.array(hi)
+    rng = np.random.default_rng(5)
+    x = np.mod(x + rng.normal(0, 0.05, x.shape), hi)
+    # copies inside the box, beside a face and beside an edge (their ghosts
+    # coincide too), and a triple
+    twin = [700, int(np.argmin(x[:, 0])), int(np.argmin(x[:, 1] + x[:, 2])), 300, 300]
+    x = np.vstack([x, x[twin]])
+    n = len(x)
+    out = []
+    for kw in (dict(lanes=1), dict(lanes=lanes, tile_width=width)):
+        s = M.System(1)
+        s.create_domain([0, 0, 0], hi, 2.8)
+        s.upload(x, None, None, np.zeros(n, np.int32), np.arange(1, n + 1, dtype=np.int32))
+        M.Binning(s).create_binning(2.8, 2.8, 2.8, 1, True, False, True)
+        comm = M.Comm(s, 2.8)
+        comm.exchange_halo()
+        nl = M.NeighborVerlet(2.8, True, 50, **kw)
+        nl.create(s)
+        F = M.ForceLJ(s, P)
+        F.init_coeff([["pair_coeff", "1", "1", "1.0", "1.0", "2.5"]])
+        F.compute(s, nl)
+        comm.update_force()
+        off, idx = nl.get()
+        out.append((s.download()[2][:n], off, idx, F.compute_energy(s, nl)))
+    (f1, off1, idx1, e1), (f, off, idx, e) = out
+    assert np.array_equal(off, off1)
+    for i in range(n):
+        assert np.array_equal(*(np.sort(k[off[i]:off[i + 1]]) for k in (idx, idx1)))
+    assert np.isfinite(f).all()
+    tol = 1e-12 if prec == "fp64" else 1e-5
+    assert np.abs(f - f1).max() < tol * np.abs(f1).max()
+    assert abs(e - e1) < 1e-12 * abs(e1)
