@@ -1105,15 +1105,16 @@ cmd_status autotune( cmd_batch *B )
     // 0.035)
     if ( B->S->n_local < 65536 )
         tiles.clear();
-    // CMD_TUNE=G,W,E,bw limits the search to one layout, as for one system
-    if ( const char *e = std::getenv( "CMD_TUNE" ) )
+    bool given = false;
+    Cand c{};
+    int bw = 0;
+    CMD_TRY( tune_request( &given, &c.G, &c.W, &c.E, &bw ) );
+    if ( given )
     {
-        Cand c{};
-        if ( std::sscanf( e, "%d,%d,%d", &c.G, &c.W, &c.E ) == 3 )
-        {
-            slabs.assign( c.E == 0 ? 1 : 0, c );
-            tiles.assign( c.E > 0 ? 1 : 0, c );
-        }
+        CMD_REQUIRE( c.E == 0 || ( c.G >= 2 && c.W >= 1 ), CMD_ERR_ARG,
+                     "CMD_TUNE: tiles have 2, 4 or 8 lanes and 1 to 3 columns" );
+        slabs.assign( c.E == 0 ? 1 : 0, c );
+        tiles.assign( c.E > 0 ? 1 : 0, c );
     }
     hipEvent_t e0, e1;
     CMD_HIP( hipEventCreate( &e0 ) );

@@ -1276,6 +1276,23 @@ cmd_status lj_energy_virial( const cmd_force *F, cmd_system *S,
     return CMD_OK;
 }
 
+// CMD_TUNE=G,W,E,bw limits a layout search to one layout (for measurements):
+// lanes per atom, tile width and height in cells (0: the default, in a batch
+// the global layout) and waves per block (0: by the tile).  *set says whether
+// the variable holds four numbers; values that no kernel has are an error.
+cmd_status tune_request( bool *set, int *G, int *W, int *E, int *bw )
+{
+    const char *e = std::getenv( "CMD_TUNE" );
+    *set = e && std::sscanf( e, "%d,%d,%d,%d", G, W, E, bw ) == 4;
+    CMD_REQUIRE( !*set || ( ( *G == 1 || *G == 2 || *G == 4 || *G == 8 ) && *W >= 0 && *W <= 3 &&
+                            *E >= 0 && *E <= 14 && *bw >= 0 && *bw <= 8 ),
+                 CMD_ERR_ARG,
+                 "CMD_TUNE=%s: lanes 1, 2, 4 or 8, tile width up to 3, height up to 14 cells, up "
+                 "to 8 waves per block",
+                 e );
+    return CMD_OK;
+}
+
 // Build the list in each layout -- lanes per atom 1, 2, 4, 8 and, for the
 // LDS-tiled layout, tiles of 2 x 2 columns 2 to 4 cells tall and of one
 // column 4 to 8 cells tall -- time the force kernel on it and keep the
@@ -1306,16 +1323,14 @@ cmd_status autotune_lanes( cmd_force *F, cmd_system *S, cmd_neigh *N, int every 
                                 { 2, 1, 4, 4 }, { 4, 1, 1, 4 }, { 4, 1, 2, 4 }, { 8, 1, 1, 8 },
                                 { 8, 1, 2, 8 } };
     const bool small = S->n_local <= 65536 && F->prec == CMD_PREC_FP64;
-    // CMD_TUNE=G,W,E,bw limits the search to one layout (for measurements)
     std::vector<Cand> cv( std::begin( all ), std::end( all ) );
     if ( small )
         cv.assign( std::begin( few ), std::end( few ) );
-    if ( const char *e = std::getenv( "CMD_TUNE" ) )
-    {
-        Cand c{};
-        if ( std::sscanf( e, "%d,%d,%d,%d", &c.G, &c.W, &c.E, &c.bw ) == 4 )
-            cv.assign( 1, c );
-    }
+    bool given = false;
+    Cand one{};
+    CMD_TRY( tune_request( &given, &one.G, &one.W, &one.E, &one.bw ) );
+    if ( given )
+        cv.assign( 1, one );
     const Cand *cands = cv.data();
     const size_t ncand = cv.size();
     N->occ_blocks = 0;

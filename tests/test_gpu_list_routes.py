@@ -170,3 +170,21 @@ def test_half_list_skips_atoms_at_one_place(gpu, lanes, width, prec):
     tol = 1e-12 if prec == "fp64" else 1e-5
     assert np.abs(f - f1).max() < tol * np.abs(f1).max()
     assert abs(e - e1) < 1e-12 * abs(e1)
+
+
+@pytest.mark.parametrize("shape", ["2,4,3,0", "2,0,3,0", "1,2,3,0", "3,2,3,0", "2,2,15,0",
+                                   "2,2,3,9", "2,2,-1,0"])
+@pytest.mark.parametrize("batch", [True, False])
+def test_layouts_without_a_kernel_are_refused(gpu, monkeypatch, batch, shape):
+    """CMD_TUNE values that no kernel has raise, in a batch and in CbnMD."""
+    M = gpu
+    monkeypatch.setenv("CMD_TUNE", shape)
+    if batch:
+        B = M.Batch(_params(M), M.PREC_FP64, lanes=0)
+        _add(M, B, SYSTEMS[0])
+        with pytest.raises(RuntimeError, match="CMD_TUNE"):
+            B.run(1)
+    elif shape not in ("2,0,3,0", "1,2,3,0"):  # one system: W 0 is the default
+        md = M.CbnMD(M.lattice_params(ncells=(6, 6, 6)), precision=M.PREC_FP64)
+        with pytest.raises(RuntimeError, match="CMD_TUNE"):
+            md.init()
