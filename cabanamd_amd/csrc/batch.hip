@@ -1515,9 +1515,6 @@ cmd_status cmd_batch_remove( cmd_batch *b, int handle )
     return CMD_ERR_ARG;
 }
 
-// Systems added or removed since the last call join or leave now when the
-// batch sits on a rebuild boundary (else at the first call that starts on
-// one).  Thermo rows are taken every thermo_rate steps and at the last step.
 // Capture two plain steps (refresh ghosts, fused step into x_alt; the
 // same from x_alt back into x) as one graph.  The capture runs nothing; the
 // host-side buffer swaps it makes are undone by the second.  Only kernels
@@ -1558,6 +1555,54 @@ static cmd_status capture_plain_pair( cmd_batch *b, const StepCtl &ctl,
     return CMD_OK;
 }
 
+// CbnMD::run's order (cabanamd_impl.h:285-399) of an NNP batch; a step's final
+// half kick and the next one's half kick and drift are one kernel except at a
+// thermo row, and no step waits on the device.
+static cmd_status nnp_steps( cmd_batch *b, int s0, int s1 )
+{
+    cmd_system *S = b->S;
+    cmd_nnp *M = b->F->nnp;
+    const cmd_params &p = b->p;
+    const int G = b->N->lanes;
+    StepCtl ctl{};
+    ctl.dtf = 0.5 * S->dt / S->mvv2e;
+    ctl.dtv = S->dt;
+    ctl.do_final = 1;
+    bool started = false;
+    for ( int s = s0; s <= s1; ++s )
+    {
+        b->step = s;
+        if ( !started )
+            CMD_TRY( cmd_nve_initial( S ) );
+        if ( s % p.every == 0 )
+        {
+            CMD_TRY( wrap( b, S->x.p ) );
+            CMD_TRY( rebuild( b, G ) );
+            CMD_TRY( nnp_run_check( M, false ) ); // (it waited: the steps before are in)
+        }
+        else
+            CMD_TRY( refresh( b ) );
+        CMD_TRY( forces( b, false ) );
+        const bool th = s == s1 || ( p.thermo_rate > 0 && s % p.thermo_rate == 0 );
+        started = !th;
+        nnp_run_gate( M, ctl, s );
+        ctl.do_next_initial = started ? 1 : 0;
+        CMD_TRY( S->x_alt.reserve( S->cap ) );
+        CMD_TRY( nve_final_initial( S, ctl, S->x_alt.p, nullptr, nullptr ) );
+        if ( started )
+            S->x.swap( S->x_alt );
+        if ( th )
+        {
+            CMD_TRY( nnp_run_check( M, true ) );
+            CMD_TRY( thermo( b, nullptr ) );
+        }
+    }
+    return CMD_OK;
+}
+
+// Systems added or removed since the last call join or leave now when the
+// batch sits on a rebuild boundary (else at the first call that starts on
+// one).  Thermo rows are taken every thermo_rate steps and at the last step.
 cmd_status cmd_batch_run( cmd_batch *b, int nsteps )
 {
     CMD_REQUIRE( b && nsteps >= 0, CMD_ERR_ARG, "bad argument" );
@@ -1577,46 +1622,20 @@ cmd_status cmd_batch_run( cmd_batch *b, int nsteps )
     const int s0 = b->step + 1, s1 = b->step + nsteps;
     if ( b->nnp )
     {
-        // CbnMD::run's order (cabanamd_impl.h:285-399); a step's final half
-        // kick and the next one's half kick and drift are one kernel except
-        // at a thermo row, and the force's check is read at the end
-        StepCtl ctl{};
-        ctl.dtf = 0.5 * S->dt / S->mvv2e;
-        ctl.dtv = S->dt;
-        ctl.do_final = 1;
-        ctl.do_next_initial = 1;
-        CMD_TRY( nnp_check_begin( b->F->nnp, st ) );
-        bool started = false;
-        for ( int s = s0; s <= s1; ++s )
+        // an atom past the neighbour limit ends the call at its step, as in
+        // CbnMD (md.hip)
+        cmd_nnp *M = b->F->nnp;
+        CMD_TRY( nnp_run_begin( M, st ) );
+        cmd_status rc = nnp_steps( b, s0, s1 );
+        if ( const int stopped = nnp_run_stop( M ) )
         {
-            b->step = s;
-            if ( !started )
-                CMD_TRY( cmd_nve_initial( S ) );
-            if ( s % p.every == 0 )
-            {
-                CMD_TRY( wrap( b, S->x.p ) );
-                CMD_TRY( rebuild( b, G ) );
-            }
-            else
-                CMD_TRY( refresh( b ) );
-            CMD_TRY( forces( b, false ) );
-            const bool th = s == s1 || ( p.thermo_rate > 0 && s % p.thermo_rate == 0 );
-            started = !th;
-            if ( started )
-            {
-                CMD_TRY( S->x_alt.reserve( S->cap ) );
-                CMD_TRY( nve_final_initial( S, ctl, S->x_alt.p, nullptr, nullptr ) );
-                S->x.swap( S->x_alt );
-            }
-            else
-            {
-                CMD_TRY( cmd_nve_final( S ) );
-                CMD_TRY( thermo( b, nullptr ) );
-            }
+            rc = nnp_run_check( M, false );
+            b->step = stopped;
+            (void)refresh( b );
+            (void)hipStreamSynchronize( st );
         }
-        CMD_TRY( nnp_check_end( b->F->nnp, st ) );
         b->timers[1] += now_s() - t0;
-        return CMD_OK;
+        return rc;
     }
     StepCtl ctl{};
     ctl.dtf = 0.5 * S->dt / S->mvv2e;

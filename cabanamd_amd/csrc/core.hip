@@ -541,8 +541,8 @@ __device__ void block_partials4( double a, double b, double c, double d,
 }
 
 // Fused final kick of this step, thermo partials, and (optionally) the next
-// step's half kick + drift (+ wrap) into x_next.  Used after half-list
-// forces, whose per-atom totals are only known after the atomics finish.
+// step's half kick + drift (+ wrap) into x_next.  Used after half-list and
+// NNP forces, whose per-atom totals are only known after the atomics finish.
 __global__ void k_final_initial( int n, int cap, const double4 *__restrict__ x,
                                  double4 *__restrict__ x_next,
                                  double *__restrict__ v,
@@ -551,15 +551,25 @@ __global__ void k_final_initial( int n, int cap, const double4 *__restrict__ x,
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     double mv2 = 0.0;
+    const int stopped = ctl.stop ? *ctl.stop : 0; // (used after the loads below)
     if ( i < n )
     {
         double4 p = x[i];
         const double m = mt.m[(int)p.w];
         const double dtfm = ctl.dtf / m;
         const double fx = f[i], fy = f[cap + i], fz = f[2 * cap + i];
-        double vx = v[i] + dtfm * fx;
-        double vy = v[cap + i] + dtfm * fy;
-        double vz = v[2 * cap + i] + dtfm * fz;
+        double vx = v[i], vy = v[cap + i], vz = v[2 * cap + i];
+        if ( stopped )
+        {
+            if ( i == 0 && *ctl.stop_step == 0 )
+                *ctl.stop_step = ctl.step;
+            if ( ctl.do_next_initial )
+                x_next[i] = p;
+            return;
+        }
+        vx = vx + dtfm * fx;
+        vy = vy + dtfm * fy;
+        vz = vz + dtfm * fz;
         mv2 = ( vx * vx + vy * vy + vz * vz ) * m;
         if ( ctl.do_next_initial )
         {
@@ -591,7 +601,7 @@ __global__ void k_final_initial( int n, int cap, const double4 *__restrict__ x,
         v[cap + i] = vy;
         v[2 * cap + i] = vz;
     }
-    if ( ctl.thermo )
+    if ( ctl.thermo ) // (never with a stop: all threads get here)
         block_partials4( mv2, 0.0, 0.0, 0.0, partial );
 }
 

@@ -503,6 +503,12 @@ struct StepCtl
     double4 *xg_next = nullptr;
     const int2 *img_rng = nullptr;  // per local atom: first and past-the-last entry of img_pk
     const int *img_pk = nullptr;    // sorted slot | code << IMG_CODE_SHIFT
+    // (integrator) when set and nonzero, the step's forces are not whole: the
+    // positions and velocities stay as they are and *stop_step gets the step,
+    // unless an earlier one is there
+    const int *stop = nullptr;
+    int *stop_step = nullptr;
+    int step = 0;
 };
 
 // LJ kernels (lj.hip)
@@ -515,12 +521,20 @@ cmd_status lj_energy_virial( const cmd_force *F, cmd_system *S,
                              const cmd_neigh *N, double *pe, double *w );
 
 // NNP force (nnp.hip)
-// check: wait for the result and report an atom with too many neighbours; a
-// time loop passes false and brackets its calls with nnp_check_begin and
-// nnp_check_end, so that its steps queue without a host wait.
+// check: wait for the result and report an atom with too many neighbours.  A
+// time loop passes false and leaves the check to these, so that its steps
+// queue without a host wait of their own:
+//   nnp_run_begin  before the first step;
+//   nnp_run_gate   the integrator of a step with such an atom, and of those
+//                  queued behind it, leaves the state of that step;
+//   nnp_run_check  fails if there was one, by what the device has reported (or
+//                  after waiting for it);
+//   nnp_run_stop   the step that stopped (0: none), after waiting.
 cmd_status nnp_compute( cmd_nnp *M, cmd_system *S, cmd_neigh *N, bool check = true );
-cmd_status nnp_check_begin( cmd_nnp *M, hipStream_t st );
-cmd_status nnp_check_end( cmd_nnp *M, hipStream_t st );
+cmd_status nnp_run_begin( cmd_nnp *M, hipStream_t st );
+void nnp_run_gate( cmd_nnp *M, StepCtl &ctl, int step );
+cmd_status nnp_run_check( cmd_nnp *M, bool wait );
+int nnp_run_stop( cmd_nnp *M );
 cmd_status nnp_reference_energy( cmd_nnp *M, cmd_system *S, double *pe );
 cmd_status nnp_energy_sum( cmd_nnp *M, cmd_system *S, double *sum );
 // Atomic energies E_i of the last compute as FP64 into out[0..n) (device).

@@ -212,23 +212,20 @@ static cmd_status thermo_now( cmd_md *md, int step )
 
 // The reference's step order (cabanamd_impl.h:285-399) for the NNP force.
 // The final half kick of a step and the half kick and drift of the next (with
-// the wrap before a rebuild) run as one kernel, except around a thermo row;
-// no step waits on the device: the force's neighbour-count check is read at
-// the end of the call.
-static cmd_status run_steps_plain( cmd_md *md, int nsteps )
+// the wrap before a rebuild) run as one kernel, except around a thermo row.
+// No step waits on the device: the force's neighbour-count check is read at
+// rebuilds, thermo rows and the end, and stops the integration by itself.
+static cmd_status plain_steps( cmd_md *md, int s0, int s1, int *nghost )
 {
     cmd_system *S = md->S;
+    cmd_nnp *M = md->F->nnp;
     const cmd_params &p = md->p;
-    const int s0 = md->step + 1, s1 = md->step + nsteps;
-    auto t0 = std::chrono::steady_clock::now();
     StepCtl ctl{};
     ctl.dtf = 0.5 * S->dt / S->mvv2e;
     ctl.dtv = S->dt;
     for ( int k = 0; k < 3; ++k )
         ctl.L[k] = S->dom.L[k];
     ctl.do_final = 1;
-    ctl.do_next_initial = 1;
-    CMD_TRY( nnp_check_begin( md->F->nnp, S->stream ) );
     bool started = false; // the last step's kernel began this one
     for ( int s = s0; s <= s1; ++s )
     {
@@ -247,15 +244,19 @@ static cmd_status run_steps_plain( cmd_md *md, int nsteps )
             }
         }
         if ( rb )
+        {
             CMD_TRY( rebuild( md ) );
+            CMD_TRY( nnp_run_check( M, false ) ); // (it waited: the steps before are in)
+        }
         else
         {
             k = md->begin( PH_COMM );
             CMD_TRY( cmd_comm_update_halo( S ) );
             md->end( k );
         }
+        *nghost = S->n_ghost;
         k = md->begin( PH_FORCE );
-        CMD_TRY( nnp_compute( md->F->nnp, S, md->N, false ) );
+        CMD_TRY( nnp_compute( M, S, md->N, false ) );
         md->end( k );
         k = md->begin( PH_COMM );
         CMD_TRY( cmd_comm_update_force( S ) );
@@ -263,11 +264,16 @@ static cmd_status run_steps_plain( cmd_md *md, int nsteps )
         const bool th = p.thermo_rate > 0 && s % p.thermo_rate == 0;
         started = s < s1 && !th && S->n_local > 0;
         k = md->begin( PH_INT );
-        if ( started )
+        nnp_run_gate( M, ctl, s );
+        ctl.do_next_initial = started ? 1 : 0;
+        ctl.wrap_next = started && ( s + 1 ) % p.every == 0 ? 1 : 0;
+        if ( S->n_local > 0 )
         {
-            ctl.wrap_next = ( s + 1 ) % p.every == 0 ? 1 : 0;
             CMD_TRY( S->x_alt.reserve( S->cap ) );
             CMD_TRY( nve_final_initial( S, ctl, S->x_alt.p, nullptr, nullptr ) );
+        }
+        if ( started )
+        {
             S->x.swap( S->x_alt );
             S->bin_grid_valid = false; // atoms leave the cells they were sorted into
             if ( ctl.wrap_next )
@@ -276,19 +282,44 @@ static cmd_status run_steps_plain( cmd_md *md, int nsteps )
                 S->xg_valid = false;
             }
         }
-        else
-            CMD_TRY( cmd_nve_final( S ) );
         md->end( k );
+        if ( th || s == s1 )
+            CMD_TRY( nnp_run_check( M, true ) );
         if ( th )
             CMD_TRY( thermo_now( md, s ) );
     }
-    CMD_TRY( nnp_check_end( md->F->nnp, S->stream ) );
+    return CMD_OK;
+}
+
+// A step with an atom past the neighbour limit ends the call as the check
+// after each force did: with the positions of that step, half-kicked
+// velocities and no thermo row from its forces.
+static cmd_status run_steps_plain( cmd_md *md, int nsteps )
+{
+    cmd_system *S = md->S;
+    cmd_nnp *M = md->F->nnp;
+    const int s1 = md->step + nsteps;
+    auto t0 = std::chrono::steady_clock::now();
+    int nghost = S->n_ghost;
+    CMD_TRY( nnp_run_begin( M, S->stream ) );
+    cmd_status st = plain_steps( md, md->step + 1, s1, &nghost );
+    const int stopped = nnp_run_stop( M );
     md->timers[5] +=
         std::chrono::duration<double>( std::chrono::steady_clock::now() - t0 )
             .count();
     md->collect();
-    md->step = s1;
-    return CMD_OK;
+    if ( stopped )
+    {
+        // (whatever else failed after that step)
+        st = nnp_run_check( M, false );
+        md->step = stopped;
+        S->n_ghost = nghost;
+        (void)cmd_comm_update_halo( S );
+        (void)hipStreamSynchronize( S->stream );
+    }
+    if ( st == CMD_OK )
+        md->step = s1;
+    return st;
 }
 
 static cmd_status run_steps( cmd_md *md, int nsteps )

@@ -149,6 +149,9 @@ struct cmd_nnp
     cmd::DevBuf<int4> terms; // per atom: neighbours, triplets, element (last compute)
     int cap = 0;
     int n_last = 0;
+    // a time loop's stream and (pinned) the step that stopped it
+    hipStream_t run_stream = nullptr;
+    cmd::HostWords stop;
 };
 
 namespace cmd
@@ -2054,24 +2057,58 @@ static cmd_status nnp_prepare( cmd_nnp *M, int n_local, hipStream_t st )
     return CMD_OK;
 }
 
-// The neighbour-count check of one or several force calls: begin clears the
-// flag that the kernels raise, end waits for the stream and reads it.
-cmd_status nnp_check_begin( cmd_nnp *M, hipStream_t st )
+// The neighbour-count check of a force call: begin clears the flag that the
+// kernels raise, end waits for the stream and reads it.
+static cmd_status too_many_neighbours()
+{
+    set_error( "an atom has more than %d neighbours inside the NNP cutoff", NN_MAX );
+    return CMD_ERR_CAPACITY;
+}
+
+static cmd_status nnp_check_begin( cmd_nnp *M, hipStream_t st )
 {
     CMD_TRY( M->flag.reserve( 1 ) );
     return fill_i32( M->flag.p, 0, 1, st );
 }
 
-cmd_status nnp_check_end( cmd_nnp *M, hipStream_t st )
+static cmd_status nnp_check_end( cmd_nnp *M, hipStream_t st )
 {
     int fl = 0;
     CMD_HIP( hipMemcpyAsync( &fl, M->flag.p, sizeof( int ),
                              hipMemcpyDeviceToHost, st ) );
     CMD_HIP( hipStreamSynchronize( st ) );
-    CMD_REQUIRE( fl == 0, CMD_ERR_CAPACITY,
-                 "an atom has more than %d neighbours inside the NNP cutoff",
-                 NN_MAX );
-    return CMD_OK;
+    return fl == 0 ? CMD_OK : too_many_neighbours();
+}
+
+// The same for the steps of a time loop (internal.h).  The flag stays up once
+// raised, so every later integrator of the loop leaves the state alone too.
+cmd_status nnp_run_begin( cmd_nnp *M, hipStream_t st )
+{
+    CMD_TRY( M->stop.init( 1 ) );
+    // (no step of an earlier loop is unfinished: loops end with nnp_run_stop)
+    M->stop.p[0] = 0;
+    M->run_stream = st;
+    return nnp_check_begin( M, st );
+}
+
+void nnp_run_gate( cmd_nnp *M, StepCtl &ctl, int step )
+{
+    ctl.stop = M->flag.p;
+    ctl.stop_step = M->stop.d;
+    ctl.step = step;
+}
+
+cmd_status nnp_run_check( cmd_nnp *M, bool wait )
+{
+    if ( wait )
+        CMD_HIP( hipStreamSynchronize( M->run_stream ) );
+    return *(volatile int *)M->stop.p == 0 ? CMD_OK : too_many_neighbours();
+}
+
+int nnp_run_stop( cmd_nnp *M )
+{
+    (void)hipStreamSynchronize( M->run_stream );
+    return *(volatile int *)M->stop.p;
 }
 
 // Up to this many atoms, and from this many listed neighbours on average, the

@@ -199,3 +199,58 @@ def test_joined_kicks_match_separate_ones(gpu, batch):
             out.append([k[:n][o] for k in a[:3]])
     for a, b in zip(*out):
         assert np.abs(a - b).max() < 1e-11 * np.abs(b).max()
+
+
+@pytest.mark.parametrize("thermo", [3, 100])
+@pytest.mark.parametrize("every", [7, 4, 50])
+@pytest.mark.parametrize("batch", [False, True])
+def test_neighbour_overflow_stops_at_its_step(gpu, batch, every, thermo):
+    """A cluster that shrinks evenly (a network of negligible forces) until an
+    atom has more than 128 neighbours inside the cutoff, at step 6: the run
+    ends with the positions of that step and with no thermo row from it or
+    later ones, whether a rebuild, a thermo row or the last step follows."""
+    M = gpu
+    m = _model(1, (0.01,), POW2, rc=4.0)
+    m["W"][0][2] *= 1e-9
+    n, dt, rate = 400, 0.01, 0.6
+    x, t = _cluster(n, 1, 7)
+    c = np.full(3, BOX / 2)
+
+    def most(s):
+        d = np.linalg.norm(x[:, None] - x[None], axis=2) * (1 - rate * dt * s)
+        return (d < 4.0).sum(1).max() - 1
+
+    # a size from which the limit is passed some steps later
+    while most(0) > 120:
+        x = c + (x - c) * 1.01
+    over = next(s for s in range(1, 100) if most(s) > 128)
+    assert over == 6
+    v = -rate * (x - c)
+    p = M.nnp_params(ntypes=1, cutoff=4.0, skin=2.0, thermo=thermo, dt=dt, every=every,
+                     max_neigh_guess=300)
+    model = _engine_model(M, m)
+    ids = np.arange(1, n + 1, dtype=np.int32)
+    if batch:
+        B = M.Batch(p, M.PREC_MIXED, nnp_model=model)
+        h = B.add(x, t, [0, 0, 0], [BOX] * 3, v=v, id=ids)
+        run, rows = B.run, lambda: B.thermo(h)
+        state = lambda: B.download(h)[:2]
+    else:
+        md = M.CbnMD(p, M.PREC_MIXED)
+        md.set_nnp_model(model)
+        md.set_initial_state(x, t, [0, 0, 0], [BOX] * 3, v=v, id=ids)
+        md.init()
+        run, rows = md.run, md.thermo
+
+        def state():
+            a = md.arrays()
+            o = np.argsort(a[4][:n])
+            return a[0][:n][o], a[1][:n][o]
+    with pytest.raises(RuntimeError, match="more than 128 neighbours"):
+        run(60)
+    assert rows()[-1, 0] == (over - 1) // thermo * thermo
+    xs, vs = state()
+    assert np.abs(xs - (x + v * dt * over)).max() < 1e-9
+    assert np.abs(vs - v).max() < 1e-9
+    if batch:
+        assert B.counts()["step"] == over
