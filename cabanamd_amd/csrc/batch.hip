@@ -1161,6 +1161,11 @@ cmd_status autotune( cmd_batch *B )
                 bs = c;
             }
         }
+        if ( tiles.empty() ) // nothing to compare a rebuild with
+        {
+            B->lanes = bs.G;
+            return build_list( B, bs.G );
+        }
         if ( bs.G > 0 )
             CMD_TRY( rebuild_ms( bs.G, &rs ) );
         CMD_TRY( set_tiling( B, true ) );

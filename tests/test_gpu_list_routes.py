@@ -188,3 +188,17 @@ def test_layouts_without_a_kernel_are_refused(gpu, monkeypatch, batch, shape):
         md = M.CbnMD(M.lattice_params(ncells=(6, 6, 6)), precision=M.PREC_FP64)
         with pytest.raises(RuntimeError, match="CMD_TUNE"):
             md.init()
+
+
+def test_small_batch_search_rebuilds_nothing(gpu, monkeypatch, capfd):
+    """A batch too small for tiles compares lanes on one set of cells: the
+    search neither times a rebuild nor makes one."""
+    M = gpu
+    monkeypatch.setenv("CMD_VERBOSE", "1")
+    B = M.Batch(_params(M), M.PREC_FP64, lanes=0)
+    for spec in SYSTEMS:
+        _add(M, B, spec)
+    B.run(1)
+    err = capfd.readouterr().err
+    assert err.count("# batch lanes=") == 4, err
+    assert "# batch rebuild" not in err, err
