@@ -603,6 +603,7 @@ struct cmd_batch
     // Tiled lists (tiles.hip) where the layout is tuned: tiles of tile_w x
     // tile_w columns, tile_e cells tall (0: the global layout); every
     // system's tiles in one space, each with its system's grid.
+    bool no_tiles = false; // another batch shares the device (batch_no_tiles)
     bool may_tile = false; // ghosts are kept in cell order
     int tile_w = 0, tile_e = 0;
     DevBuf<TileGrid> tgrids;
@@ -1103,7 +1104,7 @@ cmd_status autotune( cmd_batch *B )
     // is not won back (50 systems, 85,000 atoms, FP64: 0.025 ms a force call
     // on 4 lanes, 0.026 on tiles; 60 systems, 220,000 atoms, mixed: 0.047 and
     // 0.035)
-    if ( B->S->n_local < 65536 )
+    if ( B->S->n_local < 65536 || B->no_tiles )
         tiles.clear();
     bool given = false;
     Cand c{};
@@ -1341,6 +1342,16 @@ cmd_status apply_changes( cmd_batch *B )
     return CMD_OK;
 }
 } // namespace
+
+// For a batch that runs beside an NNP batch: its search leaves tiles out.  The
+// NNP force kernel's six blocks hold a CU's whole LDS (6 x 26.6 of 160 KB), and
+// a tile's block (about 36 KB) starts only where two of them end together,
+// while the global layout's kernel, which has no LDS, fits beside them.  16 LJ
+// jobs (0.75 million atoms) beside 8 NNP jobs (0.4 million): a force call 2.6
+// to 3.8 ms on tiles and 0.20 ms without, the 24 jobs' median latency 1.65 s
+// and 0.36 s (without the NNP jobs 0.15 s and 0.18 s).  A search under such a
+// load took either, so it is not left to the search.
+void cmd::batch_no_tiles( cmd_batch *B ) { B->no_tiles = true; }
 
 extern "C" {
 

@@ -574,6 +574,7 @@ size_t slab_entries( int n_local, int cap, int lanes );
 // Layout search for the fused full-list step; a layout scores its step
 // time plus its list build time over the `every` steps the list serves.
 cmd_status autotune_lanes( cmd_force *F, cmd_system *S, cmd_neigh *N, int every );
+void batch_no_tiles( cmd_batch *B );
 cmd_status tune_request( bool *set, int *G, int *W, int *E, int *bw );
 // tiles.hip
 cmd_status tiles_prepare_ghosts( cmd_system *S );

@@ -30,6 +30,7 @@
 namespace cmd
 {
 void set_error( const char *fmt, ... );
+void batch_no_tiles( cmd_batch *b );
 }
 
 namespace
@@ -298,6 +299,8 @@ cmd_status cmd_server_create( const cmd_params *lj, const cmd_params *nnp,
         st = cmd_batch_create( nnp, &s->nnp );
     if ( st == CMD_OK && nnp )
         st = cmd_batch_set_nnp_model( s->nnp, model );
+    if ( st == CMD_OK && nnp )
+        cmd::batch_no_tiles( s->lj ); // the two step at the same time
     if ( st != CMD_OK )
     {
         cmd_server_destroy( s );

@@ -145,3 +145,23 @@ def test_server_nnp_job_conserves_energy(gpu, nnp_model):
     e = pe + ke
     assert th[0, 0] == 0 and th[-1, 0] == 200
     assert np.abs(e - e[0]).max() / np.abs(e).max() < 1e-2
+
+
+@pytest.mark.parametrize("mixed", [True, False])
+def test_lj_jobs_beside_nnp_jobs_stay_off_tiles(gpu, nnp_model, monkeypatch, capfd, mixed):
+    """NNP force blocks leave no LDS for a tile's block, so a server of both
+    kinds runs its LJ jobs on the global layout at any size; one of LJ jobs
+    alone searches tiles from 65,536 atoms."""
+    M = gpu
+    monkeypatch.setenv("CMD_VERBOSE", "1")
+    kw = dict(precision=M.PREC_MIXED, lanes=0)
+    S = (M.Server(_lj_params(M), M.nnp_params(thermo=100), nnp_model, **kw) if mixed
+         else M.Server(_lj_params(M), **kw))
+    if mixed:
+        _submit_nnp(M, S, NNP_B, 20)
+    j = _submit_lj(M, S, ((26, 26, 26), 0.8, 1.4, 31), 20)
+    S.drain(60)
+    assert S.job(j)["state"] == 3  # done
+    err = capfd.readouterr().err
+    assert "# batch lanes=8 tile=0x0x0" in err, err
+    assert ("tile=2x2" in err) == (not mixed), err
