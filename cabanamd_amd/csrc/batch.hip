@@ -1573,7 +1573,7 @@ static cmd_status capture_plain_pair( cmd_batch *b, const StepCtl &ctl,
 
 // CbnMD::run's order (cabanamd_impl.h:285-399) of an NNP batch; a step's final
 // half kick and the next one's half kick and drift are one kernel except at a
-// thermo row, and no step waits on the device.
+// thermo row, and the host queues a step or two ahead.
 static cmd_status nnp_steps( cmd_batch *b, int s0, int s1 )
 {
     cmd_system *S = b->S;
@@ -1607,6 +1607,7 @@ static cmd_status nnp_steps( cmd_batch *b, int s0, int s1 )
         CMD_TRY( nve_final_initial( S, ctl, S->x_alt.p, nullptr, nullptr ) );
         if ( started )
             S->x.swap( S->x_alt );
+        CMD_TRY( nnp_run_mark( M, S->n_local ) );
         if ( th )
         {
             CMD_TRY( nnp_run_check( M, true ) );

@@ -529,11 +529,13 @@ cmd_status lj_energy_virial( const cmd_force *F, cmd_system *S,
 //                  queued behind it, leaves the state of that step;
 //   nnp_run_check  fails if there was one, by what the device has reported (or
 //                  after waiting for it);
+//   nnp_run_mark   after a step's launches: bounds how far the host is ahead;
 //   nnp_run_stop   the step that stopped (0: none), after waiting.
 cmd_status nnp_compute( cmd_nnp *M, cmd_system *S, cmd_neigh *N, bool check = true );
 cmd_status nnp_run_begin( cmd_nnp *M, hipStream_t st );
 void nnp_run_gate( cmd_nnp *M, StepCtl &ctl, int step );
 cmd_status nnp_run_check( cmd_nnp *M, bool wait );
+cmd_status nnp_run_mark( cmd_nnp *M, int n_local );
 int nnp_run_stop( cmd_nnp *M );
 cmd_status nnp_reference_energy( cmd_nnp *M, cmd_system *S, double *pe );
 cmd_status nnp_energy_sum( cmd_nnp *M, cmd_system *S, double *sum );

@@ -213,8 +213,8 @@ static cmd_status thermo_now( cmd_md *md, int step )
 // The reference's step order (cabanamd_impl.h:285-399) for the NNP force.
 // The final half kick of a step and the half kick and drift of the next (with
 // the wrap before a rebuild) run as one kernel, except around a thermo row.
-// No step waits on the device: the force's neighbour-count check is read at
-// rebuilds, thermo rows and the end, and stops the integration by itself.
+// The host queues a step or two ahead (nnp_run_mark) and reads the force's
+// neighbour-count check on the way, which stops the integration by itself.
 static cmd_status plain_steps( cmd_md *md, int s0, int s1, int *nghost )
 {
     cmd_system *S = md->S;
@@ -283,6 +283,7 @@ static cmd_status plain_steps( cmd_md *md, int s0, int s1, int *nghost )
             }
         }
         md->end( k );
+        CMD_TRY( nnp_run_mark( M, S->n_local ) );
         if ( th || s == s1 )
             CMD_TRY( nnp_run_check( M, true ) );
         if ( th )
