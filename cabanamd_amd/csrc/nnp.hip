@@ -2174,7 +2174,12 @@ cmd_status nnp_compute( cmd_nnp *M, cmd_system *S, cmd_neigh *N, bool check )
     if ( check )
         CMD_TRY( nnp_check_begin( M, st ) );
     if ( n == 0 )
-        return CMD_OK; // no atoms, no ghosts: no force rows
+    {
+        // no kernel below clears the rows of uploaded ghosts
+        for ( int c = 0; c < 3; ++c )
+            CMD_TRY( fill_f64( S->f.p + (size_t)c * S->cap, 0.0, nt, st ) );
+        return CMD_OK;
+    }
     CMD_TRY( M->terms.reserve( std::max( n, 1 ) ) );
     M->n_last = n;
     const int nbw = ( n + NNP_TPB / 64 - 1 ) / ( NNP_TPB / 64 );

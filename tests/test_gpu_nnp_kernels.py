@@ -254,3 +254,18 @@ def test_neighbour_overflow_stops_at_its_step(gpu, batch, every, thermo):
     assert np.abs(vs - v).max() < 1e-9
     if batch:
         assert B.counts()["step"] == over
+
+
+def test_ghosts_alone_get_zero_forces(gpu):
+    """A system of uploaded ghosts and no local atom: force rows cleared."""
+    M = gpu
+    m = _model(1, (0.01,), POW2)
+    x = np.random.default_rng(1).uniform(0, 10, (9, 3))
+    s = M.System(1)
+    s.create_domain([0, 0, 0], [10.0] * 3, 3.3)
+    s.upload(x, None, np.ones_like(x), np.zeros(9, np.int32),
+             np.arange(1, 10, dtype=np.int32), n_ghost=9)
+    nl = M.NeighborVerlet(3.3, False, 50, lanes=1)
+    nl.create(s)
+    M.ForceNNP(_engine_model(M, m)).compute(s, nl)
+    assert not s.download()[2].any()
