@@ -19,10 +19,11 @@
 // Independence: a system's atoms, ghosts and list rows depend only on that
 // system (cells belong to one system, sorts are stable by flat index, ghost
 // images are emitted per atom in a fixed direction order, reductions run one
-// block per system in a fixed order), so on one list layout its trajectory is
-// bit-identical whether it runs alone or beside others (lists are tiled where
-// the tuned layout says so and every member's tiles fit in LDS, else in the
-// global layout).  Systems join and leave only at a rebuild boundary.
+// block per system in a fixed order), and so does its place on tiled lists
+// where the tuned layout has them: its tile height, and whether its tiles fit
+// at all (else it is on the global layout beside the others' tiles).  So on one
+// tuned layout its trajectory is bit-identical whether it runs alone or beside
+// others.  Systems join and leave only at a rebuild boundary.
 #include "internal.h"
 #include "tiles_dev.h"
 
@@ -281,7 +282,9 @@ __global__ __launch_bounds__( 256 ) void k_b_neigh_cell(
     int mrow = 0;
     const int c0 = c < ncell ? __builtin_amdgcn_readfirstlane( lstart[c] ) : 0;
     const int c1 = c < ncell ? __builtin_amdgcn_readfirstlane( lstart[c + 1] ) : 0;
-    if ( c1 > c0 )
+    // (the systems on tiles, whose cells are aligned with the box, have no rows
+    // here)
+    if ( c1 > c0 && !T[__builtin_amdgcn_readfirstlane( sys[c0] )].aligned )
     {
         const BSys &s = T[__builtin_amdgcn_readfirstlane( sys[c0] )];
         const int lc = c - s.cell_base;
@@ -415,6 +418,8 @@ __global__ void k_b_atom_thermo( int n_local, int scap, int cap, const double4 *
     const int R = ( cap + G - 1 ) / G;
     const int *row = slab + (size_t)( i / APW ) * R * 64 + i % APW;
     const int n = counts[i];
+    if ( n < 0 )
+        return; // on tiles
     double e = 0.0;
     for ( int k = 0; k < n; ++k )
     {
@@ -517,6 +522,16 @@ __global__ __launch_bounds__( 512 ) void k_b_tile_thermo(
     }
 }
 
+// The longest row of each system (every third word of out, cleared before).
+__global__ void k_b_row_max( int n_local, const int *__restrict__ counts,
+                             const int *__restrict__ sys, const BSys *__restrict__ T,
+                             int *__restrict__ out )
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if ( i < n_local && T[sys[i]].aligned )
+        raise_max( out + 3 * sys[i], counts[i] );
+}
+
 __global__ void k_b_mv2( int n_local, int scap, const double4 *__restrict__ x,
                          const double *__restrict__ v, MassTable mt, double *__restrict__ mv2 )
 {
@@ -585,6 +600,9 @@ struct BMember
     int join_step;
     int a0;
     std::vector<double> thermo; // rows: local step, T, PE/N, (PE+KE)/N
+    // tiled layouts: the system's tile height in cells, lowered where its tiles
+    // do not fit (0: on the global layout; -1: not chosen yet)
+    int tile_h = -1;
 };
 } // namespace cmd
 
@@ -612,6 +630,13 @@ struct cmd_batch
     DevBuf<int> root_alt, code_alt;
     double tile_amax = 0.0;
     int ntiles = 0;
+    int n_tiled = 0; // atoms of the systems on tiles
+    // the list of those that are not (made when the first one is): rows of -1
+    // for the others' atoms
+    cmd_neigh *rest = nullptr;
+    int rest_lanes = 4;
+    bool has_rest() const { return tile_e > 0 && n_tiled < S->n_local; }
+    DevBuf<int> fit;
     int step = 0;
     int next_handle = 1;
     std::vector<BMember> members;
@@ -696,7 +721,7 @@ cmd_status upload_table( cmd_batch *B )
             s.hi[d] = m.hi[d];
             s.L[d] = m.hi[d] - m.lo[d];
         }
-        grid_of( s, depth, B->N->neigh_cut, B->may_tile );
+        grid_of( s, depth, B->N->neigh_cut, B->may_tile && m.tile_h != 0 );
         s.cell_base = cb;
         cb += s.gn[0] * s.gn[1] * s.gn[2];
         s.a0 = a0;
@@ -712,10 +737,13 @@ cmd_status upload_table( cmd_batch *B )
     return CMD_OK;
 }
 
-// The systems' grids for tiled lists or the global layout.
+// The systems' grids for tiled lists (every system's height chosen afresh) or
+// the global layout.
 cmd_status set_tiling( cmd_batch *B, bool on )
 {
     B->may_tile = on;
+    for ( BMember &m : B->members )
+        m.tile_h = -1;
     // (the table's last upload reads the host copy)
     CMD_HIP( hipStreamSynchronize( B->stream ) );
     return upload_table( B );
@@ -730,9 +758,8 @@ cmd_status sort_cells( cmd_batch *B, CellSort &cs, int n )
 // The tallest tile, up to E cells, whose staged neighbourhood is expected to
 // fit its LDS records in a system: the densest one spans W + 2 columns each
 // way and E + 2 cells, or the whole box and its ghost shell where that is
-// less; 12 % are left for fluctuations.  (Small boxes have cells up to half
-// again as wide as the cutoff: at E = 3 a few of them would send the whole
-// batch to the global layout.)
+// less; 12 % are left for fluctuations.  Where it does not fit after all, the
+// system's tiles are lowered at the build (lower_tiles).
 int tile_height( const BSys &s, double depth, int W, int E )
 {
     auto extent = [&]( int d, int cells )
@@ -751,7 +778,7 @@ int tile_height( const BSys &s, double depth, int W, int E )
 }
 
 // The tile grids of the batch's systems for tiles of W x W columns, up to E
-// cells tall (after a change of members or of the shape).
+// cells tall (after a change of members, of the shape or of a system's height).
 cmd_status upload_tiles( cmd_batch *B, int W, int E )
 {
     B->tile_w = W;
@@ -759,11 +786,17 @@ cmd_status upload_tiles( cmd_batch *B, int W, int E )
     std::vector<TileGrid> grids( B->htab.size() );
     std::vector<int> of;
     B->tile_amax = 0.0;
+    B->n_tiled = 0;
     for ( size_t k = 0; k < grids.size(); ++k )
     {
         const BSys &s = B->htab[k];
         TileGrid &T = grids[k];
         T = TileGrid{};
+        int &height = B->members[k].tile_h;
+        if ( height == 0 )
+            continue;
+        if ( height < 0 )
+            height = tile_height( s, B->N->neigh_cut, W, E );
         for ( int d = 0; d < 3; ++d )
         {
             T.g.min[d] = s.gmin[d];
@@ -776,13 +809,14 @@ cmd_status upload_tiles( cmd_batch *B, int W, int E )
         T.W = W;
         T.nt0 = ( T.nc0 + W - 1 ) / W;
         T.nt1 = ( T.nc1 + W - 1 ) / W;
-        T.E = tile_height( s, B->N->neigh_cut, W, E );
+        T.E = height;
         T.tpc = ( s.gn[2] - 2 + T.E - 1 ) / T.E;
         T.ntiles = T.nt0 * T.nt1 * T.tpc;
         T.cell0 = s.cell_base;
         T.tile0 = (int)of.size();
         of.insert( of.end(), T.ntiles, (int)k );
         B->tile_amax = std::max( B->tile_amax, tile_amax( T.g, T.E ) );
+        B->n_tiled += s.na;
     }
     B->ntiles = (int)of.size();
     CMD_TRY( B->tgrids.reserve( std::max<size_t>( 1, grids.size() ) ) );
@@ -799,36 +833,95 @@ cmd_status upload_tiles( cmd_batch *B, int W, int E )
     return CMD_OK;
 }
 
-// The tiled list of the sorted atoms and ghosts; *built stays false where
-// the tiles do not apply (an atom outside its box, a tile too dense for LDS).
-cmd_status build_tiles( cmd_batch *B, int G, bool *built )
+// After a build that did not fit: the systems whose tiles or rows exceed the
+// bounds get shorter tiles, or (an atom outside the box, a row too long, tiles
+// of one cell too full) leave the tiles for good.  *resort: one left, so that
+// its atoms go into other cells.
+cmd_status lower_tiles( cmd_batch *B, const TileSrc &src, TileFit why, bool *resort )
+{
+    cmd_neigh *N = B->N;
+    const size_t ns = B->members.size();
+    const TileBounds lim = tile_bounds( N->lanes );
+    CMD_TRY( B->fit.reserve( 3 * ns ) );
+    CMD_TRY( fill_i32( B->fit.p, 0, 3 * ns, B->stream ) );
+    if ( why == TILES_FULL )
+        CMD_TRY( tile_maxima( N, src, B->fit.p, B->stream ) );
+    else
+    {
+        k_b_row_max<<<nblk( B->S->n_local ), TPB, 0, B->stream>>>(
+            B->S->n_local, N->counts.p, B->sys.p, B->tab.p, B->fit.p );
+        CMD_LAUNCH_CHECK();
+    }
+    std::vector<int> h( 3 * ns );
+    CMD_HIP( hipMemcpyAsync( h.data(), B->fit.p, sizeof( int ) * h.size(),
+                             hipMemcpyDeviceToHost, B->stream ) );
+    CMD_HIP( hipStreamSynchronize( B->stream ) );
+    int changed = 0;
+    for ( size_t k = 0; k < ns; ++k )
+    {
+        BMember &m = B->members[k];
+        if ( m.tile_h == 0 )
+            continue;
+        const int *o = &h[3 * k];
+        const bool out = why == TILES_FULL ? o[2] != m.n : o[0] > lim.row;
+        const bool full = why == TILES_FULL && ( o[0] > lim.slots || o[1] > lim.column );
+        if ( !out && !full )
+            continue;
+        ++changed;
+        m.tile_h = out ? 0 : m.tile_h - 1;
+        if ( m.tile_h == 0 )
+            *resort = true;
+        if ( std::getenv( "CMD_VERBOSE" ) )
+            std::fprintf( stderr, "# batch system %d: tile height %d\n", m.handle, m.tile_h );
+    }
+    CMD_REQUIRE( changed > 0, CMD_ERR_STATE, "no system of the batch exceeds the tiles' bounds" );
+    return CMD_OK;
+}
+
+// The tiled list of the sorted atoms and ghosts of the systems on tiles;
+// *resort: a system left the tiles, and the atoms are to be sorted again.
+cmd_status build_tiles( cmd_batch *B, int G, bool *resort )
 {
     cmd_system *S = B->S;
     cmd_neigh *N = B->N;
     N->lanes = G;
     N->half = 0;
-    N->tiled = false;
+    N->tiled = true;
     N->csr_valid = false;
     N->nnz = -1;
     N->n_rows = S->n_local;
     N->stream = B->stream;
     CMD_TRY( N->counts.reserve( std::max( S->n_local, 1 ) ) );
-    N->tg = TileGrid{};
-    N->tg.W = B->tile_w;
-    N->tg.E = B->tile_e;
-    N->tg.ntiles = B->ntiles;
     S->ghosts_in_x = true;
     S->xg_valid = true;
-    const TileSrc src{ B->tgrids.p,         B->tgrid_of.p,        B->lsort.start.p,
-                       B->gsort.start.p,    S->x.p + S->n_local,  nullptr,
-                       B->tile_amax };
-    return tiles_build_batch( N, S, src, built );
+    for ( ;; )
+    {
+        N->tg = TileGrid{};
+        N->tg.W = B->tile_w;
+        N->tg.E = B->tile_e;
+        N->tg.ntiles = B->ntiles;
+        if ( B->ntiles == 0 )
+            return CMD_OK;
+        const TileSrc src{ B->tgrids.p,      B->tgrid_of.p,       B->lsort.start.p,
+                           B->gsort.start.p, S->x.p + S->n_local, nullptr,
+                           B->tile_amax };
+        TileFit fit = TILES_BUILT;
+        CMD_TRY( tiles_build_batch( N, S, src, B->n_tiled, &fit ) );
+        if ( fit == TILES_BUILT )
+            return CMD_OK;
+        CMD_TRY( lower_tiles( B, src, fit, resort ) );
+        if ( *resort )
+            CMD_TRY( upload_table( B ) );
+        CMD_TRY( upload_tiles( B, B->tile_w, B->tile_e ) );
+        if ( *resort )
+            return CMD_OK;
+    }
 }
 
-cmd_status build_list( cmd_batch *B, int G )
+// The list of the systems that are not on tiles, in the global layout.
+cmd_status build_list( cmd_batch *B, cmd_neigh *N, int G )
 {
     cmd_system *S = B->S;
-    cmd_neigh *N = B->N;
     const int n = S->n_local;
     const double rc2 = N->neigh_cut * N->neigh_cut;
     N->lanes = G;
@@ -845,6 +938,8 @@ cmd_status build_list( cmd_batch *B, int G )
     {
         CMD_TRY( N->slab.reserve( slab_entries( n, N->cap, G ) ) );
         CMD_TRY( fill_i32( B->max_row.p, 0, 1, B->stream ) );
+        if ( B->has_rest() )
+            CMD_TRY( fill_i32( N->counts.p, -1, n, B->stream ) );
         if ( n > 0 )
         {
 #define CMD_BN( GG )                                                                   \
@@ -881,10 +976,9 @@ cmd_status build_list( cmd_batch *B, int G )
 
 // Rebuild of every system from wrapped positions: binning sort of the owned
 // atoms, ghost images, cell sort of all atoms, Verlet list.
-cmd_status rebuild( cmd_batch *B, int G )
+// *resort: a system left the tiles, and the sort is to be made again.
+cmd_status rebuild_once( cmd_batch *B, int G, bool *resort )
 {
-    ++B->epoch; // captured steps hold this build's buffers and sizes
-    const double t0 = now_s();
     cmd_system *S = B->S;
     const hipStream_t st = B->stream;
     const int n = S->n_local;
@@ -942,13 +1036,9 @@ cmd_status rebuild( cmd_batch *B, int G )
         }
         if ( B->tile_e > 0 )
         {
-            bool built = false;
-            CMD_TRY( build_tiles( B, G, &built ) );
-            if ( built )
-            {
-                B->timers[0] += now_s() - t0;
+            CMD_TRY( build_tiles( B, G, resort ) );
+            if ( *resort || !B->has_rest() )
                 return CMD_OK;
-            }
         }
     }
     // candidates: all atoms in their system's cells
@@ -960,8 +1050,37 @@ cmd_status rebuild( cmd_batch *B, int G )
     CMD_TRY( B->xs.reserve( nt ) );
     k_b_gather<<<nblk( nt ), TPB, 0, st>>>( nt, B->asort.perm.p, S->x.p, B->xs.p );
     CMD_LAUNCH_CHECK();
-    CMD_TRY( build_list( B, G ) );
+    if ( B->tile_e == 0 )
+        return build_list( B, B->N, G );
+    if ( !B->rest )
+    {
+        CMD_TRY( cmd_neigh_create( B->N->neigh_cut, 0, B->p.max_neigh_guess, &B->rest ) );
+        B->rest->stream = st;
+    }
+    return build_list( B, B->rest, B->rest_lanes );
+}
+
+cmd_status rebuild( cmd_batch *B, int G )
+{
+    ++B->epoch; // captured steps hold this build's buffers and sizes
+    const double t0 = now_s();
+    for ( bool resort = true; resort; )
+    {
+        resort = false;
+        CMD_TRY( rebuild_once( B, G, &resort ) );
+    }
     B->timers[0] += now_s() - t0;
+    return CMD_OK;
+}
+
+// The LJ forces (or the fused step) of every system: of those on tiles and of
+// those on the global layout.
+cmd_status lj_step( cmd_batch *B, const StepCtl &ctl, double4 *x_next )
+{
+    if ( B->tile_e == 0 || B->ntiles > 0 )
+        CMD_TRY( lj_full( B->F, B->S, B->N, ctl, x_next, nullptr, nullptr ) );
+    if ( B->has_rest() )
+        CMD_TRY( lj_full( B->F, B->S, B->rest, ctl, x_next, nullptr, nullptr ) );
     return CMD_OK;
 }
 
@@ -1019,24 +1138,28 @@ cmd_status thermo( cmd_batch *B, const std::vector<char> *which )
         S->x.p, S->tile_ghosts(), S->v.p, N->counts.p, N->tslab.p, B->Pd.p, S->mass_table(), \
         B->pe.p, B->mv2.p )
 #define CMD_BT( GG )                                                                        \
-    k_b_atom_thermo<GG><<<nblk( n ), TPB, 0, B->stream>>>( n, S->cap, N->cap, S->x.p, S->v.p, \
-                                                           N->counts.p, N->slab.p, B->Pd.p,   \
+    k_b_atom_thermo<GG><<<nblk( n ), TPB, 0, B->stream>>>( n, S->cap, R->cap, S->x.p, S->v.p, \
+                                                           R->counts.p, R->slab.p, B->Pd.p,   \
                                                            S->mass_table(), B->pe.p, B->mv2.p )
-        if ( N->tiled )
+        const cmd_neigh *R = B->tile_e == 0 ? N : B->rest;
+        if ( B->ntiles > 0 && B->tile_e > 0 )
+        {
             switch ( N->lanes )
             {
             case 2: CMD_BTT( 2 ); break;
             case 4: CMD_BTT( 4 ); break;
             default: CMD_BTT( 8 ); break;
             }
-        else
-        switch ( N->lanes )
-        {
-        case 1: CMD_BT( 1 ); break;
-        case 2: CMD_BT( 2 ); break;
-        case 4: CMD_BT( 4 ); break;
-        default: CMD_BT( 8 ); break;
+            CMD_LAUNCH_CHECK();
         }
+        if ( B->tile_e == 0 || B->has_rest() )
+            switch ( R->lanes )
+            {
+            case 1: CMD_BT( 1 ); break;
+            case 2: CMD_BT( 2 ); break;
+            case 4: CMD_BT( 4 ); break;
+            default: CMD_BT( 8 ); break;
+            }
 #undef CMD_BT
 #undef CMD_BTT
         CMD_LAUNCH_CHECK();
@@ -1081,8 +1204,7 @@ cmd_status forces( cmd_batch *B, bool check = true )
         CMD_TRY( nnp_compute( B->F->nnp, B->S, B->N, check ) );
         return cmd_comm_update_force( B->S );
     }
-    StepCtl ctl{};
-    return lj_full( B->F, B->S, B->N, ctl, nullptr, nullptr, nullptr );
+    return lj_step( B, StepCtl{}, nullptr );
 }
 
 // Times the force kernel on each list layout and keeps the fastest: lanes per
@@ -1124,10 +1246,10 @@ cmd_status autotune( cmd_batch *B )
     // time of one force call on the list as built
     auto step_ms = [&]( const Cand &c, float *ms ) -> cmd_status
     {
-        CMD_TRY( lj_full( B->F, B->S, B->N, ctl, nullptr, nullptr, nullptr ) );
+        CMD_TRY( lj_step( B, ctl, nullptr ) );
         (void)hipEventRecord( e0, B->stream );
         for ( int r = 0; r < 3; ++r )
-            (void)lj_full( B->F, B->S, B->N, ctl, nullptr, nullptr, nullptr );
+            (void)lj_step( B, ctl, nullptr );
         (void)hipEventRecord( e1, B->stream );
         (void)hipEventSynchronize( e1 );
         (void)hipEventElapsedTime( ms, e0, e1 );
@@ -1154,7 +1276,7 @@ cmd_status autotune( cmd_batch *B )
         float fs = 1e30f, ft = 1e30f, rs = 0.f, rt = 0.f, ms = 0.f;
         for ( const Cand &c : slabs )
         {
-            CMD_TRY( build_list( B, c.G ) );
+            CMD_TRY( build_list( B, B->N, c.G ) );
             CMD_TRY( step_ms( c, &ms ) );
             if ( ms < fs )
             {
@@ -1165,24 +1287,28 @@ cmd_status autotune( cmd_batch *B )
         if ( tiles.empty() ) // nothing to compare a rebuild with
         {
             B->lanes = bs.G;
-            return build_list( B, bs.G );
+            return build_list( B, B->N, bs.G );
         }
         if ( bs.G > 0 )
+        {
             CMD_TRY( rebuild_ms( bs.G, &rs ) );
-        CMD_TRY( set_tiling( B, true ) );
-        bool sorted = false; // ghosts in cell order
+            B->rest_lanes = bs.G;
+        }
+        bool sorted = false; // on the grids of tiles, ghosts in cell order
         for ( const Cand &c : tiles )
         {
+            // (a system that left the last shape's tiles gets its cells back)
+            if ( sorted && B->n_tiled < B->S->n_local )
+                sorted = false;
+            bool resort = !sorted;
+            CMD_TRY( set_tiling( B, true ) );
             CMD_TRY( upload_tiles( B, c.W, c.E ) );
             if ( sorted )
-            {
-                bool built = false;
-                CMD_TRY( build_tiles( B, c.G, &built ) );
-            }
-            else
+                CMD_TRY( build_tiles( B, c.G, &resort ) );
+            if ( resort )
                 CMD_TRY( rebuild( B, c.G ) );
             sorted = true;
-            if ( !B->N->tiled )
+            if ( B->ntiles == 0 )
                 continue;
             CMD_TRY( step_ms( c, &ms ) );
             if ( ms < ft )
@@ -1193,6 +1319,7 @@ cmd_status autotune( cmd_batch *B )
         }
         if ( bt.G > 0 )
         {
+            CMD_TRY( set_tiling( B, true ) );
             CMD_TRY( upload_tiles( B, bt.W, bt.E ) );
             CMD_TRY( rebuild_ms( bt.G, &rt ) );
         }
@@ -1204,8 +1331,8 @@ cmd_status autotune( cmd_batch *B )
             return CMD_OK;
         }
         CMD_REQUIRE( bs.G > 0, CMD_ERR_STATE, "the requested tiles do not fit" );
-        CMD_TRY( set_tiling( B, false ) );
         B->tile_w = B->tile_e = 0;
+        CMD_TRY( set_tiling( B, false ) );
         B->lanes = bs.G;
         return rebuild( B, bs.G );
     };
@@ -1429,6 +1556,8 @@ cmd_status cmd_batch_destroy( cmd_batch *b )
         cmd_force_destroy( b->F );
     if ( b->N )
         cmd_neigh_destroy( b->N );
+    if ( b->rest )
+        cmd_neigh_destroy( b->rest );
     b->Pd.release();
     b->tab.release();
     if ( b->S )
@@ -1566,7 +1695,7 @@ static cmd_status capture_plain_pair( cmd_batch *b, const StepCtl &ctl,
         if ( rc == CMD_OK )
             rc = refresh( b );
         if ( rc == CMD_OK )
-            rc = lj_full( b->F, S, b->N, ctl, S->x_alt.p, nullptr, nullptr );
+            rc = lj_step( b, ctl, S->x_alt.p );
         S->x.swap( S->x_alt );
     }
     hipGraph_t g = nullptr;
@@ -1732,7 +1861,7 @@ cmd_status cmd_batch_run( cmd_batch *b, int nsteps )
             ctl.do_next_initial = 0;
             ctl.write_f = 1;
             CMD_TRY( S->x_alt.reserve( S->cap ) );
-            CMD_TRY( lj_full( b->F, S, N, ctl, S->x_alt.p, nullptr, nullptr ) );
+            CMD_TRY( lj_step( b, ctl, S->x_alt.p ) );
             CMD_TRY( thermo( b, nullptr ) );
             if ( !last )
             {
@@ -1746,7 +1875,7 @@ cmd_status cmd_batch_run( cmd_batch *b, int nsteps )
             ctl.do_next_initial = 1;
             ctl.write_f = 0;
             CMD_TRY( S->x_alt.reserve( S->cap ) );
-            CMD_TRY( lj_full( b->F, S, N, ctl, S->x_alt.p, nullptr, nullptr ) );
+            CMD_TRY( lj_step( b, ctl, S->x_alt.p ) );
             if ( ( s + 1 ) % p.every == 0 )
                 CMD_TRY( wrap( b, S->x_alt.p ) );
             // ghosts are refreshed (or rebuilt) into the new buffer next step

@@ -585,9 +585,26 @@ cmd_status tiles_prepare_ghosts( cmd_system *S );
 cmd_status binning_create( cmd_system *s, double dx_in, double dy_in, double dz_in,
                            int halo_depth, int do_local, int do_ghost, int sort, int *perm_out,
                            bool keep_f );
-// The same for the tiles of a batch: N->tg.W, E and ntiles are set, the
-// shape is not lowered (*built stays false where it does not fit).
-cmd_status tiles_build_batch( cmd_neigh *N, cmd_system *S, const TileSrc &src, bool *built );
+// The same for the tiles of a batch: N->tg.W, E and ntiles are set, the shape
+// is not lowered.  A grid fits where each of its tiles and rows stays within
+// fixed bounds, whatever the batch's other grids hold: *fit says what exceeded
+// them (n_atoms: the atoms of the batch's tiled grids).
+struct TileBounds
+{
+    int slots, column, row; // staged positions, atoms of a tile's column, row length
+};
+enum TileFit
+{
+    TILES_BUILT,
+    TILES_FULL, // a tile or a column, or an atom lies in no tile
+    TILES_ROWS  // a row (the lengths are in N->counts)
+};
+TileBounds tile_bounds( int lanes );
+cmd_status tiles_build_batch( cmd_neigh *N, cmd_system *S, const TileSrc &src, int n_atoms,
+                              TileFit *fit );
+// Of the tiles of each grid, after tiles_build_batch: the most staged positions,
+// the most atoms of a column and all atoms (3 words a grid, cleared before).
+cmd_status tile_maxima( cmd_neigh *N, const TileSrc &src, int *out, hipStream_t st );
 double tile_amax( const CellGrid &g, int E );
 int tile_max_slots(); // staged FP64 records of a tile
 cmd_status tiles_build( cmd_neigh *N, cmd_system *S, bool *built );

@@ -412,7 +412,7 @@ __global__ __launch_bounds__( TPB ) void k_lj_full(
     constexpr int APW = 64 / G;
     const SlabLane L = slab_lane<G>( xcd_remap( blockIdx.x, gridDim.x ) );
     const int i = L.i;
-    const bool active = i < n_local;
+    bool active = i < n_local;
     const bool energy = FUSED && ctl.thermo;
     double fx = 0.0, fy = 0.0, fz = 0.0, pe = 0.0, vir = 0.0;
     double4 xi = make_double4( 0.0, 0.0, 0.0, 0.0 );
@@ -421,6 +421,7 @@ __global__ __launch_bounds__( TPB ) void k_lj_full(
         xi = x[i];
         const int ti = (int)xi.w;
         const int n = counts[i];
+        active = n >= 0; // an atom with no row is another list's (batch.hip)
         const int nr = n > L.s ? ( n - L.s + G - 1 ) / G : 0;
         const int R = ( lcap + G - 1 ) / G;
         const int *row = slab + (size_t)L.wave * R * 64 + L.s * APW + L.a;

@@ -13,8 +13,9 @@
 //              end, whichever comes first; new jobs join at a boundary;
 //   retire  -- a job that has run its steps is copied out (positions and
 //              velocities by atom id, thermo rows), timestamped and removed.
-// A job's trajectory does not depend on the other jobs (batch.hip), so its
-// result is the same alone or in any mix.
+// On the list layout chosen when the first jobs of a kind join (or set), a
+// job's trajectory does not depend on the other jobs (batch.hip): its result is
+// the same alone or in any mix.
 #include "../../include/cabanamd_amd.h"
 
 #include <algorithm>

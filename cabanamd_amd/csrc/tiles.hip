@@ -1477,13 +1477,32 @@ cmd_status tiles_build( cmd_neigh *N, cmd_system *S, bool *built )
     return CMD_ERR_CAPACITY;
 }
 
-cmd_status tiles_build_batch( cmd_neigh *N, cmd_system *S, const TileSrc &src, bool *built )
+// A batch's grids share one launch, and its LDS holds the largest planes, the
+// most rows and the longest rows of any of them: with the longest row for which
+// MAX_SLOTS planes and BATCH_COLUMN rows fit (152 KB: 288 entries and more; LJ
+// at its melting point has rows of 80 and columns of 70), what a grid may hold
+// does not depend on the others.
+static constexpr int BATCH_COLUMN = 192;
+
+TileBounds tile_bounds( int lanes )
 {
-    *built = false;
+    size_t hard = 0, lds_cu = 0;
+    lds_limits( &hard, &lds_cu );
+    int row = 4;
+    while ( build_lds_cap( lanes, row + 4, MAX_SLOTS + 1, BATCH_COLUMN ) <= hard )
+        row += 4;
+    return { MAX_SLOTS, BATCH_COLUMN, row };
+}
+
+cmd_status tiles_build_batch( cmd_neigh *N, cmd_system *S, const TileSrc &src, int n_atoms,
+                              TileFit *fit )
+{
     N->spec.valid = false;
     N->rec = TILE_REC;
+    const TileBounds lim = tile_bounds( N->lanes );
     if ( N->cap < 1 )
         N->cap = std::max( 1, N->max_neigh_guess );
+    N->cap = std::min( N->cap, lim.row );
     size_t hard = 0, lds_cu = 0;
     lds_limits( &hard, &lds_cu );
     CMD_TRY( tile_info_run( N, S, src ) );
@@ -1492,36 +1511,62 @@ cmd_status tiles_build_batch( cmd_neigh *N, cmd_system *S, const TileSrc &src, b
     for ( int k = 0; k < 5; ++k )
         h[k] = res[TILE_RES_INFO + k];
     N->tg.bw = force_waves( N, h[2] );
-    if ( h[1] != S->n_local )
-        return CMD_OK; // an atom outside its system's interior cells
+    *fit = TILES_FULL;
+    if ( h[1] != n_atoms || h[0] > lim.slots || h[4] > lim.column )
+        return CMD_OK;
+    N->tile_blocks = (int)std::min( lds_cu / ( force_lds( h[0], N->rec ) + 1024 ),
+                                    (size_t)( 32 / N->tg.bw ) );
+    N->max_tile_slots = h[0];
     for ( int attempt = 0; attempt < 4; ++attempt )
     {
-        const size_t lds = build_lds( N, h[3] + 1, h[4] );
-        bool fits = false;
-        int blocks = 0;
-        if ( !layout_ok( N, h, lds, hard, lds_cu, 1, &fits, &blocks ) || !fits )
-            return CMD_OK; // too dense for the tile shape
-        N->tile_blocks = blocks;
-        N->max_tile_slots = h[0];
         CMD_TRY( N->tslab.reserve( tile_slab_entries( N, h[5] ) ) );
         // the maxima of the build proper start afresh
         CMD_TRY( fill_i32( S->sc.ires.p + TILE_RES_MAXROW, 0, 1, S->stream ) );
-        CMD_TRY( launch_build_g( N, S, src, h[3] + 1, h[4], h[5], lds ) );
+        CMD_TRY( launch_build_g( N, S, src, h[3] + 1, h[4], h[5],
+                                 build_lds( N, h[3] + 1, h[4] ) ) );
         int nw = 0;
         CMD_TRY( tile_results( N, S, res, &nw, true ) );
         const int mr = res[TILE_RES_MAXROW];
         list_rows( N, res );
         if ( mr <= N->cap )
         {
-            *built = true;
+            *fit = TILES_BUILT;
             N->tiled = true;
             N->built_rec = N->rec;
             return CMD_OK;
         }
-        N->cap = std::max( N->max_neigh_guess, (int)( mr * 1.1 ) );
+        *fit = TILES_ROWS;
+        if ( mr > lim.row )
+            return CMD_OK;
+        N->cap = std::min( std::max( N->max_neigh_guess, (int)( mr * 1.1 ) ), lim.row );
     }
     set_error( "neighbour rows kept growing during the tiled build" );
     return CMD_ERR_CAPACITY;
+}
+
+__global__ void k_tile_maxima( int ntiles, int W, const int *__restrict__ info,
+                               const int *__restrict__ grid_of, int *__restrict__ out )
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if ( t >= ntiles )
+        return;
+    const int *I = info + (size_t)t * TI_WORDS;
+    int col = 0;
+    for ( int c = 0; c < W * W; ++c )
+        col = max( col, I[TI_AN + c] );
+    int *o = out + 3 * grid_of[t];
+    atomicMax( o, I[TI_TOTAL] );
+    atomicMax( o + 1, col );
+    atomicAdd( o + 2, I[TI_NAT] );
+}
+
+cmd_status tile_maxima( cmd_neigh *N, const TileSrc &src, int *out, hipStream_t st )
+{
+    const int n = N->tg.ntiles;
+    k_tile_maxima<<<( n + TPB - 1 ) / TPB, TPB, 0, st>>>( n, N->tg.W, N->tile_info.p,
+                                                          src.grid_of, out );
+    CMD_LAUNCH_CHECK();
+    return CMD_OK;
 }
 
 // The tiled build launched with the sizes of the last one (record_spec) and

@@ -202,3 +202,150 @@ def test_small_batch_search_rebuilds_nothing(gpu, monkeypatch, capfd):
     err = capfd.readouterr().err
     assert err.count("# batch lanes=") == 4, err
     assert "# batch rebuild" not in err, err
+
+
+def _gas_params(M, odd):
+    """Atoms of diameter 0.5 (0.2) inside the same cutoff: dense boxes stay
+    calm."""
+    p = _params(M)
+    p.coeff_sigma[0] = 0.2 if odd == "clump" else 0.5
+    return p
+
+
+def _boxed(x, v, hi):
+    n = len(x)
+    return dict(x=x, type=np.zeros(n, np.int32), lo=[0.0] * 3, hi=list(hi), v=v,
+                id=np.arange(1, n + 1, dtype=np.int32))
+
+
+def _odd_members(M):
+    """Systems whose tiles do not fit as the batch's shape has them: one too
+    dense for tiles of one cell, one dense in half of its box (fits with
+    shorter tiles than its mean density suggests), one whose rows alone are
+    too long (a clump around a corner of its cells), one with an atom that
+    crosses its box between rebuilds."""
+    dense = M.fcc_system((13, 12, 12), 2.9, 0.3, 7)
+    half = M.fcc_system((11, 11, 24), 1.9, 0.3, 8)
+    keep = half[0][:, 2] < 0.5 * half[5][2]
+    x = np.array([[1.0, 1, 1], [5, 1, 1], [1, 5, 1], [5, 5, 1], [1, 4, 4.5]])
+    v = np.zeros_like(x)
+    v[4, 0] = 300.0
+    g = 0.35 * (np.arange(7) - 3.0)
+    c = np.array([(5.65 + a, 5.65 + b, 5.0 + e) for a in g for b in g for e in g])
+    c = np.vstack([c, c[:49] - [0.35, 0, 0]])
+    return dict(dense=_boxed(dense[0], dense[1], dense[5]),
+                clump=_boxed(c, np.zeros_like(c), [11.3] * 3),
+                half=_boxed(half[0][keep], half[1][keep], half[5]),
+                fast=_boxed(x, v, [9.0] * 3))
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("odd", ["dense", "half", "clump", "fast"])
+def test_batch_member_off_tiles_changes_no_other(gpu, monkeypatch, capfd, odd, prec):
+    """A system that the tiles cannot hold joins a tiled batch: it gets shorter
+    tiles or the global layout by itself, the others stay where they are, and
+    both trajectories are the bits they are alone."""
+    M = gpu
+    monkeypatch.setenv("CMD_TUNE", "2,2,3,0")
+    monkeypatch.setenv("CMD_VERBOSE", "1")
+    P = M.PREC_FP64 if prec == "fp64" else M.PREC_MIXED
+    calm = M.fcc_system((9, 9, 10), 1.2, 0.5, 3)
+    member = _odd_members(M)[odd]
+    alone = M.Batch(_gas_params(M, odd), P, lanes=0)
+    ha = alone.add(**_boxed(calm[0], calm[1], calm[5]))
+    single = M.Batch(_gas_params(M, odd), P, lanes=0)
+    single.add(**_boxed(calm[0], calm[1], calm[5]))  # tunes the batch
+    mix = M.Batch(_gas_params(M, odd), P, lanes=0)
+    hm = mix.add(**_boxed(calm[0], calm[1], calm[5]))
+    for B in (alone, mix, single):
+        B.run(20)
+    capfd.readouterr()
+    ho = mix.add(**member)
+    for k in (20, 20, 7):
+        alone.run(k)
+        mix.run(k)
+    err = capfd.readouterr().err
+    lowered = [int(l.split()[-1]) for l in err.splitlines() if "tile height" in l]
+    for a, b in zip(alone.download(ha), mix.download(hm)):
+        assert np.array_equal(a, b)
+    assert np.array_equal(alone.thermo(ha), mix.thermo(hm))
+    if odd == "half":
+        assert lowered in ([2], [2, 1]), err
+    else:  # (the mean density gives the uniformly dense box tiles of one cell at once)
+        assert lowered == [0], err
+    # the odd one against the same system with other company
+    extra = M.fcc_system((8, 8, 8), 0.9, 0.5, 5)
+    single.add(**_boxed(extra[0], extra[1], extra[5]))
+    hs = single.add(**member)
+    for k in (20, 20, 7):
+        single.run(k)
+    for a, b in zip(single.download(hs), mix.download(ho)):
+        assert np.array_equal(a, b)
+    assert np.array_equal(single.thermo(hs), mix.thermo(ho))
+    # and against the global layout
+    g = M.Batch(_gas_params(M, odd), P, lanes=4)
+    hg = g.add(**member)
+    g.run(47)
+    x, xg = mix.download(ho)[0], g.download(hg)[0]
+    assert np.abs(_min_image(x - xg, np.array(member["hi"]))).max() < 1e-7
+    if odd == "fast":
+        assert np.abs(_min_image(x[4] - (member["x"][4] + [300 * 0.005 * 47, 0, 0]),
+                                 np.array(member["hi"]))).max() < 1e-9
+
+
+def _two_types(M):
+    p = _params(M, thermo=10)
+    p.ntypes = 2
+    p.mass[1] = 2.0
+    p.ncoeff = 3
+    for k, (a, b, eps, sig) in enumerate(((1, 1, 1.0, 1.0), (1, 2, 0.8, 1.1),
+                                          (2, 2, 1.2, 0.95))):
+        p.coeff_i[k], p.coeff_j[k] = a, b
+        p.coeff_eps[k], p.coeff_sigma[k], p.coeff_cut[k] = eps, sig, 2.5
+    return p
+
+
+@pytest.mark.parametrize("shape", ["2,2,3,0", "4,1,4,0"])
+def test_batch_tiles_two_types(gpu, monkeypatch, shape):
+    """Two atom types with their own masses and cross coefficients: forces,
+    positions and thermo rows on tiles against the global layout (FP64; the
+    same sums in another order over 30 steps)."""
+    M = gpu
+    out = []
+    for lanes in (0, 4):
+        monkeypatch.setenv("CMD_TUNE", shape)
+        B = M.Batch(_two_types(M), M.PREC_FP64, lanes=lanes)
+        hs = []
+        for cells, rho, temp, seed in SYSTEMS:
+            x, v, t, i, lo, hi = M.fcc_system(cells, rho, temp, seed)
+            t = t.copy()
+            t[::3] = 1
+            hs.append(B.add(x, t, lo, hi, v=v, id=i))
+        B.run(30)
+        out.append([(*B.download(h)[:3], B.thermo(h)) for h in hs])
+    for a, b in zip(*out):
+        for u, w in zip(a, b):
+            assert np.abs(u - w).max() < 1e-9 * max(np.abs(w).max(), 1.0)
+
+
+def test_batch_layout_search_with_tiles(gpu, monkeypatch, capfd):
+    """A batch above the size from which the search times tiles too (and
+    rebuilds on the loser's cells and back): against the fixed global layout,
+    FP64, over two rebuilds."""
+    M = gpu
+    monkeypatch.setenv("CMD_VERBOSE", "1")
+    spec = [((9 + k % 4, 10, 11), 0.7 + 0.02 * k, 0.8 + 0.1 * k, 200 + k) for k in range(15)]
+    out = []
+    for lanes in (0, 4):
+        B = M.Batch(_params(M), M.PREC_FP64, lanes=lanes)
+        hs = [_add(M, B, s) for s in spec]
+        B.run(45)
+        assert B.counts()["atoms"] > 65536
+        out.append([(*B.download(h)[:3], B.thermo(h)) for h in hs])
+    err = capfd.readouterr().err
+    assert "tile=2x2x3" in err and "# batch rebuild" in err, err
+    for s, a, b in zip(spec, *out):
+        L = np.array(s[0]) * (4.0 / s[1]) ** (1.0 / 3.0)
+        assert np.abs(_min_image(a[0] - b[0], L)).max() < 1e-9
+        for u, w in zip(a[1:], b[1:]):
+            assert np.abs(u - w).max() < 1e-8 * np.abs(w).max()
