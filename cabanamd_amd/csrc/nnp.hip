@@ -1712,7 +1712,7 @@ __global__ __launch_bounds__( NNP_TPB ) void k_nnp_force(
 
 // LDS of a wave's pair walk beyond its neighbours'.  Up to 64 neighbours
 // leave the upper halves of L.d and L.e free: the ring's records (pa, pm,
-// pb) lie there and here, which keeps five blocks on a CU.
+// pb) lie there and here, which keeps six blocks on a CU.
 union ForceBuf
 {
     float coef[NSF_LD];
@@ -2146,14 +2146,28 @@ int nnp_run_stop( cmd_nnp *M )
     return *(volatile int *)M->stop.p;
 }
 
-// Up to this many atoms, and from this many listed neighbours on average, the
-// power-of-two kernels put four waves on an atom: one wave each leaves SIMDs
-// with too few waves to cover their latencies, but the gather and set-up are
-// repeated, which costs more where there are few pairs or many atoms.
-// Forces / symmetry functions, one wave and four: 512 atoms of 62 neighbours
-// 49 / 30 and 27 / 15 us, 3,000 atoms 61 / 39 and 59 / 34 us, 5,832 atoms
-// 86 / 56 and 91 / 53 us; 2,048 atoms of 23 neighbours 12 / 8 and 19 / 13 us.
-static constexpr int NNP_SPLIT_MAX = 3072, NNP_SPLIT_NEIGH = 48;
+// Where the power-of-two kernels put four waves on an atom.  One wave each
+// leaves SIMDs with too few waves to cover their latencies, but the gather and
+// set-up are repeated in each of the four.  A block is then an atom, and up to
+// 1,536 of them (six to a CU) run in one round; with few pairs to share the
+// repeats win there too.  Beyond that only atoms past the ring's 64 neighbours
+// gain, whose walk with LDS atomics one wave does slowly.  In systems with
+// thermal displacements (0.25 on a spacing of 2.5) they are some from about 66
+// listed on average (near a perfect lattice from 72), and the gain is down to
+// 5 % at 3,072 atoms.  Step with four waves / with one (us), by atoms and
+// listed neighbours:
+//              24          36          53          61          69          76
+//   729      52 / 53
+//   1,331    59 / 57     62 / 63     69 / 73     71 / 78     86 / 115   118 / 154
+//   1,728    67 / 57     71 / 63     76 / 72     79 / 79     92 / 118   139 / 157
+//   2,744    73 / 59     77 / 66     84 / 78     89 / 84    112 / 121   173 / 184
+//   4,096    87 / 62     94 / 71    103 / 84    109 / 93    133 / 140   223 / 217
+//   4,913    98 / 65    103 / 75    114 / 90    121 / 100   147 / 146   254 / 247
+static bool nnp_split( int n, int64_t listed )
+{
+    return ( n <= 1536 && listed >= 32 * (int64_t)n ) ||
+           ( n <= 3072 && listed >= 66 * (int64_t)n );
+}
 
 cmd_status nnp_compute( cmd_nnp *M, cmd_system *S, cmd_neigh *N, bool check )
 {
@@ -2202,7 +2216,7 @@ cmd_status nnp_compute( cmd_nnp *M, cmd_system *S, cmd_neigh *N, bool check )
     // operations wherever the grid allows them
     const bool pow = nag >= 1 && rs0 && pow2;
     const bool g58 = nag == 5 && nap8;
-    const bool split = n <= NNP_SPLIT_MAX && N->nnz >= (int64_t)NNP_SPLIT_NEIGH * n;
+    const bool split = nnp_split( n, N->nnz );
 #define CMD_POW( LAUNCH )                                                                 \
     switch ( nag )                                                                        \
     {                                                                                     \

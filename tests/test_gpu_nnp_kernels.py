@@ -137,15 +137,15 @@ def test_neighbour_counts(gpu, n, pl):
 @pytest.mark.parametrize("n", [64, 66, 67, 100, 127])
 def test_one_wave_past_64_neighbours(gpu, n, neta):
     """A cluster of n atoms, every one a neighbour of every other, among
-    atoms with none: too few neighbours on average for four waves on an atom,
-    so one wave walks 63 to 126 neighbours, with pair counts of every
+    atoms with six at most: too few neighbours on average for four waves on an
+    atom, so one wave walks 63 to 126 neighbours, with pair counts of every
     remainder by 4 (the lanes that share a block of matrix products)."""
     x, t = _cluster(n, 1, n)
     x = BOX / 2 + (x - BOX / 2) * min(1.0, 4.0 / np.ptp(x, axis=0).max())
-    g = np.arange(5.0, BOX, 10.0)
+    g = np.arange(9.0, 52.0, 6.0)
     lone = np.array([(a, b, c) for a in g for b in g for c in g])
-    lone = lone[np.linalg.norm(lone - BOX / 2, axis=1) > 15.0]
-    assert n * (n - 1) < 48 * (n + len(lone))
+    lone = lone[np.linalg.norm(lone - BOX / 2, axis=1) > 12.0]
+    assert n * (n - 1) + 6 * len(lone) < 32 * (n + len(lone))
     x = np.vstack([x, lone])
     t = np.zeros(len(x), np.int32)
     m = _model(1, [0.01 * (k + 1) for k in range(neta)], POW2, rc=8.0)
@@ -159,6 +159,25 @@ def test_one_wave_per_atom_at_62_neighbours(gpu):
     M = gpu
     x, t, _ = M.nnp_lattice((15, 15, 15), spacing=2.5, jitter=0.1, seed=5)
     L = [37.5] * 3
+    model = _fitted_benchmark_model(M, x, t, L)
+    m = model.describe(2)
+    m.update(act="ttl", smin=0.0, smax=1.0, scale=True)
+    s, comm, nl = _system(M, x, t, L, 6.3)
+    r = _run(M, s, comm, nl, M.ForceNNP(model, M.PREC_MIXED), m)
+    assert (np.linalg.norm(r["f"] - r["fo"]) <
+            1e-5 * np.linalg.norm(r["fo"]))
+
+
+@pytest.mark.parametrize("cells,spacing", [((11, 11, 12), 2.7), ((11, 12, 12), 2.7),
+                                           ((14, 14, 15), 2.5), ((11, 12, 12), 3.5)])
+def test_waves_per_atom(gpu, cells, spacing):
+    """Around the sizes where an atom gets four waves: 1,452 (four) and 1,584
+    atoms (one) of 55 listed neighbours, 2,940 of 75 (four) and 1,584 of 24
+    (one): forces within 1e-5 of the oracle."""
+    from test_gpu_nnp import _fitted_benchmark_model, _run
+    M = gpu
+    x, t, _ = M.nnp_lattice(cells, spacing=spacing, jitter=0.1, seed=5)
+    L = [spacing * c for c in cells]
     model = _fitted_benchmark_model(M, x, t, L)
     m = model.describe(2)
     m.update(act="ttl", smin=0.0, smax=1.0, scale=True)
