@@ -191,7 +191,10 @@ cmd_status cmd_force_set_precision( cmd_force *f, int prec );
  * 0 = autotune at init by timing each layout. */
 cmd_status cmd_force_set_lanes( cmd_force *f, int lanes );
 cmd_status cmd_force_get_lanes( const cmd_force *f, int *lanes );
-/* f = 0 over local+ghost, then accumulate (cabanamd_impl.h:336-341). */
+/* f = 0 over local+ghost, then accumulate (cabanamd_impl.h:336-341).  With a
+ * half list the ghost rows hold the reactions on the ghosts where the list is
+ * in the global layout, and stay 0 where it is tiled (the local rows are whole
+ * there); cmd_comm_update_force after it gives the same forces on both. */
 cmd_status cmd_force_compute( cmd_force *f, cmd_system *s, cmd_neigh *n );
 /* Shifted pair energy with the reference's list weights (impl.h:261-377). */
 cmd_status cmd_force_energy( cmd_force *f, cmd_system *s, cmd_neigh *n,
