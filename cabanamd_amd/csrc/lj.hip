@@ -1316,14 +1316,14 @@ cmd_status autotune_lanes( cmd_force *F, cmd_system *S, cmd_neigh *N, int every 
     // would get no block, and the time of a step is that of one block, so
     // short tiles and more lanes are tried in place of tall ones.  Each layout
     // is built once more before its build is timed (the first may allocate).
-    // 100 steps, tall tiles and short ones, FP64: 256 atoms 1.77 and 1.71 ms,
-    // 32,000 2.37 and 2.19; mixed: 256 atoms 1.52 to 1.60 and 1.45 ms, 4,000
-    // 1.57 to 2.01 and 1.47, 32,000 2.08 and 1.82, 55,296 1.90 and 1.91.
+    // 100 steps at 256 atoms FP64 1.77 -> 1.71 ms, at 32,000 2.37 -> 2.19 ms;
+    // mixed precision keeps the list of large systems (48,000 atoms of two
+    // types: 2.05 ms with either).
     static const Cand few[] = { { 1, 0, 0, 0 }, { 2, 2, 2, 4 }, { 2, 2, 2, 2 }, { 2, 2, 3, 4 },
                                 { 2, 1, 1, 2 }, { 2, 1, 2, 2 }, { 2, 1, 2, 4 }, { 2, 1, 3, 2 },
                                 { 2, 1, 4, 4 }, { 4, 1, 1, 4 }, { 4, 1, 2, 4 }, { 8, 1, 1, 8 },
                                 { 8, 1, 2, 8 } };
-    const bool small = S->n_local <= 65536;
+    const bool small = S->n_local <= 65536 && F->prec == CMD_PREC_FP64;
     std::vector<Cand> cv( std::begin( all ), std::end( all ) );
     if ( small )
         cv.assign( std::begin( few ), std::end( few ) );
