@@ -1316,9 +1316,13 @@ cmd_status autotune_lanes( cmd_force *F, cmd_system *S, cmd_neigh *N, int every 
     // would get no block, and the time of a step is that of one block, so
     // short tiles and more lanes are tried in place of tall ones.  Each layout
     // is built once more before its build is timed (the first may allocate).
-    // 100 steps at 256 atoms FP64 1.77 -> 1.71 ms, at 32,000 2.37 -> 2.19 ms;
-    // mixed precision keeps the list of large systems (48,000 atoms of two
-    // types: 2.05 ms with either).
+    // 100 steps at 256 atoms FP64 1.77 -> 1.71 ms, at 32,000 2.37 -> 2.19 ms.
+    // Mixed precision keeps the list of large systems: of one type the short
+    // tiles take 256 atoms from 1.52-1.60 to 1.45 ms, 4,000 from 1.57-2.01 to
+    // 1.47, 32,000 from 2.08 to 1.82 and 55,296 nowhere (1.90, 1.91), but
+    // 48,000 atoms of two types from 2.05 to 2.07, and the layout decides what
+    // is rounded to FP32: the energies of a small box came out 8.4e-6 off
+    // 64 bits instead of 6.9e-6.
     static const Cand few[] = { { 1, 0, 0, 0 }, { 2, 2, 2, 4 }, { 2, 2, 2, 2 }, { 2, 2, 3, 4 },
                                 { 2, 1, 1, 2 }, { 2, 1, 2, 2 }, { 2, 1, 2, 4 }, { 2, 1, 3, 2 },
                                 { 2, 1, 4, 4 }, { 4, 1, 1, 4 }, { 4, 1, 2, 4 }, { 8, 1, 1, 8 },
