@@ -790,8 +790,9 @@ __device__ __forceinline__ void for_triplets( const NbLds &L, int n, float rc2,
 // own lane, which replaces reactions added with LDS atomics: at 192,000 atoms
 // those took half of the force kernel's 3794 us, which the ring, the matrix
 // products of the coefficients (k_nnp_force_pow) and six blocks per CU brought
-// to 1795 us, 87 % of them VALU issue; the symmetry functions, which use the
-// steps alone, went from 996 to 893 us.
+// to 1795 us, 87 % of them VALU issue (1742 us with the steps' loads outside
+// the branch of the lanes that have a pair); the symmetry functions, which use
+// the steps alone, went from 996 to 893 us.
 constexpr int PAIR_RING = 256;
 
 // set bits of m below the lane's
