@@ -6,9 +6,8 @@ list, FP64 with the half list.  At this size
 the checks are properties that do not depend on the size:
 - the step with the ghost refresh fused into it equals the separate
   refresh pass bit for bit (positions, velocities, forces, thermo rows;
-  the half list always takes the separate pass, and its reactions are
-  summed with FP64 atomics, so two of its runs may differ in the last
-  bits);
+  compared with the full list here, with the half list at a smaller size in
+  test_gpu_list_routes.py);
 - net momentum stays zero (pair forces are exact negatives, so only the
   rounding of the per-atom sums is left);
 - the thermo rows (T, PE/N, E/N every 5 steps, over two list rebuilds)

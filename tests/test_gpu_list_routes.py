@@ -349,3 +349,22 @@ def test_batch_layout_search_with_tiles(gpu, monkeypatch, capfd):
         assert np.abs(_min_image(a[0] - b[0], L)).max() < 1e-9
         for u, w in zip(a[1:], b[1:]):
             assert np.abs(u - w).max() < 1e-8 * np.abs(w).max()
+
+
+@pytest.mark.parametrize("width", [1, 2])
+def test_half_list_ghost_images_in_the_step(gpu, width):
+    """A tiled half list's step writes the next step's ghosts as a full
+    list's does: 90 steps over four rebuilds equal the separate refresh bit
+    for bit, ghost rows included."""
+    M = gpu
+    out = []
+    for fuse in (True, False):
+        md = M.CbnMD(M.lattice_params(ncells=(9, 8, 10), thermo=15, half=True),
+                     precision=M.PREC_FP64, lanes=2, tile_width=width, fuse_ghosts=fuse)
+        md.init()
+        for k in (7, 33, 50):
+            md.run(k)
+        assert md.neighbor.layout()["tiled"]
+        out.append((*md.arrays(), md.thermo()))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)

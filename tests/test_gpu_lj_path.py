@@ -227,9 +227,9 @@ def test_neighbor_on_binning_grid_exact(gpu, half, lanes, width):
     nl.create(s)
     off, idx = nl.get()
     lay = nl.layout()
-    # a half list on 3 x 3 tiles stages FP64 records and reactions for 25
-    # columns, which may exceed a block's LDS at every height (then the
-    # global layout): only its rows are checked
+    # a half list on 3 x 3 tiles stages FP64 records for 25 columns, which may
+    # exceed a block's LDS at every height (then the global layout): only its
+    # rows are checked
     if not (half and width == 3):
         assert lay["tiled"] == (lanes > 1)
         assert lay["tile_width"] == (width if lanes > 1 else 0)
@@ -333,10 +333,10 @@ def test_lj_tiled_force(gpu, prec, lanes, wrapped, shape):
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
 @pytest.mark.parametrize("lanes", [2, 4, 8])
 def test_lj_tiled_half_force(gpu, prec, lanes):
-    """Half list on the binning grid with 2+ lanes per atom: the tiled
-    kernel sums reactions per staged atom in LDS and adds them to f with
-    atomics; after the ghost fold, forces, energy and virial against the
-    oracle's half-list force and fold (force_lj_cabana_neigh_impl.h:205-259,
+    """Half list on the binning grid with 2+ lanes per atom: the tiled rows
+    hold every neighbour, so each atom's force is whole in its own row and
+    the ghost rows stay 0; after the ghost fold, forces, energy and virial
+    against the oracle's half-list force and fold (force_lj_cabana_neigh_impl.h:205-259,
     comm_mpi_impl.h:410-441)."""
     M = gpu
     ncells = (10, 9, 8)
@@ -373,9 +373,9 @@ def test_lj_tiled_half_force(gpu, prec, lanes):
 
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
 def test_md_loop_half_tiled(gpu, prec):
-    """CbnMD with a half list and two lanes per atom (the tiled half kernel,
-    its thermo energy with the reference's 1/2 weight for ghost pairs, and
-    the ghost fold) against the FP64 oracle's loop."""
+    """CbnMD with a half list and two lanes per atom (the fused step on tiled
+    half rows, its thermo energy with the reference's 1/2 weight for ghost
+    pairs) against the FP64 oracle's loop."""
     M = gpu
     kw = dict(ncells=(10, 10, 10), nsteps=100, thermo=10, half=True)
     md = M.CbnMD(M.lattice_params(**kw),
